@@ -1,5 +1,6 @@
 // Attention input-pullback for P cotangent basis directions (gfx950): C ABI entry points
 // and the choice between the MFMA kernels and the generic kernels.
+#include "lbi_attn_f32.h"
 #include "lbi_attn_generic.h"
 #include "lbi_attn_mfma.h"
 #include "lbi_attn_dkdv128.h"
@@ -113,6 +114,8 @@ extern "C" int lbi_attn_pullback(const void* q, const void* k, const void* v, co
                    ? attn_mfma::launch<_Float16>(q, k, v, d_out, dq, dk, dv, ws, b, h, t, dh, p, softmax_scale, causal, stream)
                    : attn_mfma::launch<bf16_raw>(q, k, v, d_out, dq, dk, dv, ws, b, h, t, dh, p, softmax_scale, causal, stream);
     }
+    if (attn_f32::supports(dh, dtype))
+        return attn_f32::launch(q, k, v, d_out, dq, dk, dv, ws, b, h, t, dh, p, softmax_scale, causal, stream);
     switch (dtype) {
         case LBI_F32: return attn_generic::launch<float>(q, k, v, d_out, dq, dk, dv, ws, b, h, t, dh, p, softmax_scale, causal, stream);
         case LBI_F16: return attn_generic::launch<_Float16>(q, k, v, d_out, dq, dk, dv, ws, b, h, t, dh, p, softmax_scale, causal, stream);

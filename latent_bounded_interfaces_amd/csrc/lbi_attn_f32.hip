@@ -1,0 +1,585 @@
+// Attention input-pullback for fp32 storage on the fp32 matrix cores: any T, head dim <= 128, causal or not.
+//
+// Bound: v_mfma_f32_32x32x2_f32 does 64 flop per cycle and SIMD (157 TFLOP/s on the part); a product is 64 cycles,
+// so LDS, softmax and address work of a tile fit under its products and one wave per SIMD is enough.
+//
+// Operand layout of that instruction (lane = 32*h + m):
+//   A (32 x 2): lane holds A[m][h]      B (2 x 32): lane holds B[h][m]
+//   C (32 x 32): register i of the lane holds C[row(i)][m],  row(i) = 8*(i/4) + 4*h + i%4
+// Which two k a product takes is free as long as A and B agree, which gives the two forms used here:
+//   * reduction over the head dim ("dot" form): product t takes column t of the lower and of the upper half of the
+//     head dim, so a lane's operand is one contiguous half row: 16-byte LDS reads, or registers for the operand
+//     that stays with the wave;
+//   * reduction over the rows of an accumulator tile ("chain" form): product t takes rows row(t) of both lane halves,
+//     so register t of the tile IS the operand, and the other side is one 4-byte LDS read of row row(t), 32
+//     consecutive columns per lane half.  P and dS never leave the registers.
+//
+// Three kernels per call, every output with one owner and a fixed summation order (no atomics, reruns bit-identical):
+//   stats   lse2[b,h,i] (log2 domain) and O = softmax(..) V; O is parked in the dk slice of direction 0, which the
+//           last kernel overwrites, so the workspace is no larger than that of the scalar kernels
+//   dq      a wave owns 32 queries x PB directions (S^T orientation: lanes are queries); also leaves
+//           delta[b,p,h,i] = d_out . O for the next kernel
+//   dkdv    a wave owns 32 keys x PB directions (S orientation: lanes are keys)
+// The streamed tiles pass through two LDS buffers (the next tile waits in registers during the products of the current
+// one; one barrier per tile) and are shared by the four waves of a workgroup, which own different directions of the same
+// rows as far as there are any: under the causal mask neighbouring row tiles end at different steps and the waves of the
+// shorter ones wait (B=4 H=8 T=512 Dh=64 P=8: dq 145 -> 125 us, dkdv 189 -> 175 us against four row tiles).  Two
+// directions per wave share one S tile, at one wave per SIMD; one direction at two waves per SIMD took 176 / 201 us.
+// Whole call there: 5.43 ms on the scalar kernels (lbi_attn_generic.h), 0.333 ms here (53 TFLOP/s algorithmic).
+#include "lbi_attn_f32.h"
+
+#include <initializer_list>
+
+namespace lbi {
+namespace attn_f32 {
+namespace {
+
+constexpr int NWAVE = 4, NT = 64 * NWAVE, TILE = 32;
+constexpr float LOG2E = 1.4426950408889634f;
+
+__device__ __forceinline__ int acc_row(int i, int h) { return 8 * (i >> 2) + 4 * h + (i & 3); }
+__device__ __forceinline__ f32x16 mma(float a, float b, f32x16 c) {
+    return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ f32x16 zero16() {
+    f32x16 z;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) z[e] = 0.0f;
+    return z;
+}
+
+// Products over the head dim: acc[p] += tile (32 rows in LDS) . own[p]^T.  The 16-byte LDS read of the next four products
+// is issued ahead of the current ones (a wave has the SIMD to itself, nothing else would hide its latency), and
+// `side(i)` for i = 0 .. 15, vector work that does not depend on these products, runs in their shadow.
+template <int DH, int N, typename Side>
+__device__ __forceinline__ void dot_form(f32x16 (&acc)[N], const float* lane_tile, const float (&own)[N][DH / 2],
+                                         Side side) {
+    constexpr int ROUNDS = DH / 8;
+    f32x4 a[2];
+    a[0] = *reinterpret_cast<const f32x4*>(lane_tile);
+#pragma unroll
+    for (int c = 0; c < ROUNDS; ++c) {
+        if (c + 1 < ROUNDS) a[(c + 1) & 1] = *reinterpret_cast<const f32x4*>(lane_tile + 4 * (c + 1));
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int p = 0; p < N; ++p) acc[p] = mma(a[c & 1][e], own[p][4 * c + e], acc[p]);
+#pragma unroll
+        for (int i = 16 * c / ROUNDS; i < 16 * (c + 1) / ROUNDS; ++i) side(i);
+    }
+}
+
+// Products over the rows of accumulator tiles: acc[p][n] += x[p]^T . tile[:, 32n ...] (OUT_T: the transposed product).
+// `lane_tile` points at row 4h, column m of the tile.  `side(i)` runs in the shadow of the products of register i - 2
+// (i = 0, 1: in front of them), so it may also form x[p][i].
+template <int NB, int PITCH, int N, bool OUT_T, typename Side>
+__device__ __forceinline__ void chain_form(f32x16 (&acc)[N][NB], const float* lane_tile, const f32x16 (&x)[N],
+                                           Side side) {
+    float b[2][2][NB];   // two rows per round, two rounds
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+#pragma unroll
+        for (int n = 0; n < NB; ++n) b[0][u][n] = lane_tile[acc_row(u, 0) * PITCH + 32 * n];
+        side(u);
+    }
+#pragma unroll
+    for (int i = 0; i < 16; i += 2) {
+        if (i + 2 < 16)
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int n = 0; n < NB; ++n) b[((i >> 1) + 1) & 1][u][n] = lane_tile[acc_row(i + 2 + u, 0) * PITCH + 32 * n];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int n = 0; n < NB; ++n)
+#pragma unroll
+                for (int p = 0; p < N; ++p) {
+                    const float t = b[(i >> 1) & 1][u][n];
+                    acc[p][n] = OUT_T ? mma(t, x[p][i + u], acc[p][n]) : mma(x[p][i + u], t, acc[p][n]);
+                }
+        if (i + 2 < 16) {
+            side(i + 2);
+            side(i + 3);
+        }
+    }
+}
+constexpr auto nothing = [](int) __attribute__((always_inline)) {};
+
+// Four consecutive elements of a row-major [T, dh] matrix from (row, c), zero outside it.  The load itself is never
+// predicated: it reads a clamped address and `keep` says whether the value counts, so that nothing waits for a load
+// before its value is needed (a load under a branch is waited for at the join).  VEC: dh is a multiple of four and the
+// matrix 16-byte aligned.
+template <bool VEC>
+__device__ __forceinline__ f32x4 load_piece(const float* __restrict__ src, int row, int c, int T_len, int dh) {
+    const float* p = src + (size_t)min(row, T_len - 1) * dh;
+    if constexpr (VEC) {
+        return *reinterpret_cast<const f32x4*>(p + min(c, dh - 4));
+    } else {
+        f32x4 v;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = p[min(c + e, dh - 1)];
+        return v;
+    }
+}
+__device__ __forceinline__ f32x4 keep(f32x4 v, bool row_ok, int c, int dh) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = row_ok && c + e < dh ? v[e] : 0.0f;
+    return v;
+}
+
+// A 32 x DH tile on its way from memory to LDS (pitch DH + 4 floats: the half-row reads of a lane group spread over all
+// banks).  Rows past `rows_end` and columns past dh become zero.
+template <int DH, bool VEC>
+struct TileStage {
+    static constexpr int PITCH = DH + 4, PIECES = TILE * DH / 4 / NT;
+    f32x4 reg[PIECES];
+    __device__ __forceinline__ void fetch(const float* __restrict__ src, int row0, int T_len, int dh, int tid) {
+#pragma unroll
+        for (int u = 0; u < PIECES; ++u) {
+            const int piece = tid + NT * u;
+            reg[u] = load_piece<VEC>(src, row0 + piece / (DH / 4), 4 * (piece % (DH / 4)), T_len, dh);
+        }
+    }
+    __device__ __forceinline__ void commit(float* lds, int row0, int rows_end, int dh, int tid) const {
+#pragma unroll
+        for (int u = 0; u < PIECES; ++u) {
+            const int piece = tid + NT * u, row = piece / (DH / 4), c = 4 * (piece % (DH / 4));
+            *reinterpret_cast<f32x4*>(lds + row * PITCH + c) = keep(reg[u], row0 + row < rows_end, c, dh);
+        }
+    }
+};
+
+// The lane's half row (columns h*DH/2 ...) of row `row`, zero outside the matrix.
+template <int DH, bool VEC>
+__device__ __forceinline__ void load_half_row(float (&dst)[DH / 2], const float* __restrict__ src, int row, int h,
+                                              int T_len, int dh, bool live = true) {
+#pragma unroll
+    for (int q = 0; q < DH / 8; ++q) {
+        const int c = h * (DH / 2) + 4 * q;
+        const f32x4 v = keep(load_piece<VEC>(src, row, c, T_len, dh), live && row < T_len, c, dh);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) dst[4 * q + e] = v[e];
+    }
+}
+
+// Rows and groups of a launch: workgroup id -> (row tile, group), all groups of the longest row tile first, so that the
+// short tiles of a causal call fill the end of the launch.
+struct Place {
+    int tile, group;
+};
+__device__ __forceinline__ Place place(int id, int tiles, int groups, bool last_first) {
+    const int t = id / groups;
+    return {last_first ? tiles - 1 - t : t, id - t * groups};
+}
+
+template <int DH, bool VEC>
+__global__ __launch_bounds__(NT) void stats_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                                                   const float* __restrict__ v, float* __restrict__ o_park,
+                                                   float* __restrict__ lse2, int H, int P, int T_len, int dh,
+                                                   float scale, int causal, int tiles, int groups) {
+    using Stage = TileStage<DH, VEC>;
+    constexpr int ROWS = NWAVE * TILE;
+    constexpr int PITCH = Stage::PITCH, BUF = 2 * TILE * PITCH, NB = DH / 32;
+    extern __shared__ __align__(16) float lds[];  // [2][K tile, V tile]
+    const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, h = lane >> 5, wave = tid >> 6;
+    const Place at = place(blockIdx.x, tiles, groups, causal);
+    const size_t base = (size_t)at.group * T_len * dh;
+    const int q0 = at.tile * ROWS + wave * TILE, query = q0 + m;
+    float qf[1][DH / 2];
+    load_half_row<DH, VEC>(qf[0], q + base, query, h, T_len, dh);
+    f32x16 o_acc[1][NB];  // O^T: lanes are queries
+#pragma unroll
+    for (int n = 0; n < NB; ++n) o_acc[0][n] = zero16();
+    float m_run = -INFINITY, l_run = 0.0f;
+    const float sc2 = scale * LOG2E;
+    const int end = causal ? min(T_len, (at.tile + 1) * ROWS) : T_len;
+    const int steps = (end + TILE - 1) / TILE;
+    Stage ks, vs;
+    ks.fetch(k + base, 0, T_len, dh, tid);
+    vs.fetch(v + base, 0, T_len, dh, tid);
+    ks.commit(lds, 0, T_len, dh, tid);
+    vs.commit(lds + TILE * PITCH, 0, T_len, dh, tid);
+    __syncthreads();
+    auto begin = [&](int it) {  // the next tile sets out
+        if (it + 1 < steps) {
+            ks.fetch(k + base, (it + 1) * TILE, T_len, dh, tid);
+            vs.fetch(v + base, (it + 1) * TILE, T_len, dh, tid);
+        }
+    };
+    auto finish = [&](int it) {
+        if (it + 1 < steps) {
+            float* next = lds + ((it + 1) & 1) * BUF;
+            ks.commit(next, (it + 1) * TILE, T_len, dh, tid);
+            vs.commit(next + TILE * PITCH, (it + 1) * TILE, T_len, dh, tid);
+        }
+        __syncthreads();
+    };
+    // this wave's own tiles first, then the rest of the workgroup's (no branch around the products: the accumulators
+    // would be copied at its join on every step)
+    const int mine = q0 >= T_len ? 0 : causal ? min(steps, q0 / TILE + 1) : steps;
+    for (int it = 0; it < mine; ++it) {
+        const int j0 = it * TILE;
+        begin(it);
+        const float* kt = lds + (it & 1) * BUF;
+        const float* vt = kt + TILE * PITCH;
+        f32x16 ss[1] = {zero16()};
+        f32x16& s = ss[0];
+        dot_form<DH, 1>(ss, kt + m * PITCH + h * (DH / 2), qf, nothing);
+        float top = m_run;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const int key = j0 + acc_row(i, h);
+            s[i] = (key < T_len && (!causal || key <= query)) ? s[i] * sc2 : -INFINITY;
+            top = fmaxf(top, s[i]);
+        }
+        top = fmaxf(top, __shfl_xor(top, 32, 64));
+        // key 0 is visible to every query, so the maximum is finite from the first tile on
+        const float alpha = exp2f(m_run - top);
+        m_run = top;
+        l_run *= alpha;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            s[i] = exp2f(s[i] - top);
+            l_run += s[i];
+        }
+#pragma unroll
+        for (int n = 0; n < NB; ++n) o_acc[0][n] *= alpha;
+        chain_form<NB, PITCH, 1, true>(o_acc, vt + 4 * h * PITCH + m, ss, nothing);
+        finish(it);
+    }
+    for (int it = mine; it < steps; ++it) {
+        begin(it);
+        finish(it);
+    }
+    if (query >= T_len) return;
+    const float l_all = l_run + __shfl_xor(l_run, 32, 64);
+    if (h == 0) lse2[(size_t)at.group * T_len + query] = m_run + log2f(l_all);
+    const float inv = 1.0f / l_all;
+    const int b = at.group / H, head = at.group - b * H;
+    float* o_row = o_park + (((size_t)b * P * H + head) * T_len + query) * dh;
+#pragma unroll
+    for (int n = 0; n < NB; ++n)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int c = 32 * n + 8 * g + 4 * h;
+            const f32x4 v4 = {o_acc[0][n][4 * g] * inv, o_acc[0][n][4 * g + 1] * inv, o_acc[0][n][4 * g + 2] * inv,
+                              o_acc[0][n][4 * g + 3] * inv};
+            if constexpr (VEC) {
+                if (c < dh) *reinterpret_cast<f32x4*>(o_row + c) = v4;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (c + e < dh) o_row[c + e] = v4[e];
+            }
+        }
+}
+
+// DW of the four waves own different direction groups of the same rows, 4 / DW different row tiles.  A group of the
+// launch is (b, DW * PB directions, head); directions past P in the last group compute on zeros and store nothing.
+template <int DH, int PB, int DW, bool VEC>
+__global__ __launch_bounds__(NT) void dq_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                                                const float* __restrict__ v, const float* __restrict__ d_out,
+                                                const float* __restrict__ o_park, const float* __restrict__ lse2,
+                                                float* __restrict__ delta, float* __restrict__ dq, int H, int P,
+                                                int T_len, int dh, float scale, int causal, int tiles,
+                                                int groups) {
+    using Stage = TileStage<DH, VEC>;
+    constexpr int ROWS = NWAVE / DW * TILE;
+    constexpr int PITCH = Stage::PITCH, BUF = 2 * TILE * PITCH, NB = DH / 32;
+    extern __shared__ __align__(16) float lds[];  // [2][K tile, V tile]
+    const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const Place at = place(blockIdx.x, tiles, groups, causal);
+    const int pgroups = (P + DW * PB - 1) / (DW * PB);
+    const int head = at.group % H, b = at.group / (H * pgroups);
+    const int p0 = ((at.group / H) % pgroups * DW + wave % DW) * PB;  // the wave's first direction
+    const size_t rows = (size_t)T_len, kv_base = ((size_t)b * H + head) * rows * dh;
+    const int q0 = at.tile * ROWS + wave / DW * TILE, query = q0 + m;
+    float qf[1][DH / 2], gf[PB][DH / 2], dl[PB];
+    load_half_row<DH, VEC>(qf[0], q + kv_base, query, h, T_len, dh);
+    {
+        float of[DH / 2];
+        load_half_row<DH, VEC>(of, o_park + ((size_t)b * P * H + head) * rows * dh, query, h, T_len, dh);
+#pragma unroll
+        for (int p = 0; p < PB; ++p) {
+            const bool live = p0 + p < P;
+            const size_t bph = ((size_t)b * P + min(p0 + p, P - 1)) * H + head;
+            load_half_row<DH, VEC>(gf[p], d_out + bph * rows * dh, query, h, T_len, dh, live);
+            float acc = 0.0f;
+#pragma unroll
+            for (int t = 0; t < DH / 2; ++t) acc = fmaf(gf[p][t], of[t], acc);
+            dl[p] = acc + __shfl_xor(acc, 32, 64);
+            if (live && h == 0 && query < T_len) delta[bph * rows + query] = dl[p];
+        }
+    }
+    const float my_lse = query < T_len ? lse2[((size_t)b * H + head) * rows + query] : INFINITY;  // P = 0 past the end
+    f32x16 acc[PB][NB];
+#pragma unroll
+    for (int p = 0; p < PB; ++p)
+#pragma unroll
+        for (int n = 0; n < NB; ++n) acc[p][n] = zero16();
+    const float sc2 = scale * LOG2E;
+    const int end = causal ? min(T_len, (at.tile + 1) * ROWS) : T_len;
+    const int steps = (end + TILE - 1) / TILE;
+    Stage ks, vs;
+    ks.fetch(k + kv_base, 0, T_len, dh, tid);
+    vs.fetch(v + kv_base, 0, T_len, dh, tid);
+    ks.commit(lds, 0, T_len, dh, tid);
+    vs.commit(lds + TILE * PITCH, 0, T_len, dh, tid);
+    __syncthreads();
+    auto begin = [&](int it) {  // the next tile sets out
+        if (it + 1 < steps) {
+            ks.fetch(k + kv_base, (it + 1) * TILE, T_len, dh, tid);
+            vs.fetch(v + kv_base, (it + 1) * TILE, T_len, dh, tid);
+        }
+    };
+    auto finish = [&](int it) {
+        if (it + 1 < steps) {
+            float* next = lds + ((it + 1) & 1) * BUF;
+            ks.commit(next, (it + 1) * TILE, T_len, dh, tid);
+            vs.commit(next + TILE * PITCH, (it + 1) * TILE, T_len, dh, tid);
+        }
+        __syncthreads();
+    };
+    // this wave's own tiles first, then the rest of the workgroup's (no branch around the products: the accumulators
+    // would be copied at its join on every step)
+    const int mine = q0 >= T_len ? 0 : causal ? min(steps, q0 / TILE + 1) : steps;
+    for (int it = 0; it < mine; ++it) {
+        const int j0 = it * TILE;
+        begin(it);
+        const float* kt = lds + (it & 1) * BUF;
+        const float* vt = kt + TILE * PITCH;
+        f32x16 ss[1] = {zero16()}, dp[PB];
+#pragma unroll
+        for (int p = 0; p < PB; ++p) dp[p] = zero16();
+        dot_form<DH, 1>(ss, kt + m * PITCH + h * (DH / 2), qf, nothing);
+        const bool masked = (causal && j0 + TILE - 1 > q0) || j0 + TILE > T_len;  // the same in all lanes
+        f32x16& prob = ss[0];
+        dot_form<DH, PB>(dp, vt + m * PITCH + h * (DH / 2), gf, [&](int i) __attribute__((always_inline)) {
+            prob[i] = exp2f(prob[i] * sc2 - my_lse);
+        });
+        if (masked) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int key = j0 + acc_row(i, h);
+                if (key >= T_len || (causal && key > query)) prob[i] = 0.0f;
+            }
+        }
+        chain_form<NB, PITCH, PB, false>(acc, kt + 4 * h * PITCH + m, dp, [&](int i) __attribute__((always_inline)) {
+#pragma unroll
+            for (int p = 0; p < PB; ++p) dp[p][i] = prob[i] * (dp[p][i] - dl[p]);
+        });
+        finish(it);
+    }
+    for (int it = mine; it < steps; ++it) {
+        begin(it);
+        finish(it);
+    }
+#pragma unroll
+    for (int p = 0; p < PB; ++p) {
+        if (p0 + p >= P) break;
+        float* out = dq + (((size_t)b * P + p0 + p) * H + head) * rows * dh;
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int row = q0 + acc_row(i, h), c = 32 * n + m;
+                if (row < T_len && c < dh) out[(size_t)row * dh + c] = acc[p][n][i] * scale;
+            }
+    }
+}
+
+template <int DH, int PB, int DW, bool VEC>
+__global__ __launch_bounds__(NT) void dkdv_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                                                  const float* __restrict__ v, const float* __restrict__ d_out,
+                                                  const float* __restrict__ lse2, const float* __restrict__ delta,
+                                                  float* __restrict__ dk, float* __restrict__ dv, int H, int P,
+                                                  int T_len, int dh, float scale, int causal, int tiles,
+                                                  int groups) {
+    using Stage = TileStage<DH, VEC>;
+    constexpr int PITCH = Stage::PITCH, NB = DH / 32, ROWS = NWAVE / DW * TILE;
+    constexpr int ND = DW * PB;  // directions of the workgroup
+    constexpr int MATS = (1 + ND) * TILE * PITCH, BUF = MATS + 2 * NT;
+    extern __shared__ __align__(16) float lds[];  // [2][Q tile, ND d_out tiles, lse of the rows, ND deltas of the rows]
+    const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const Place at = place(blockIdx.x, tiles, groups, false);  // the first keys see the most queries
+    const int pgroups = (P + ND - 1) / ND;
+    const int head = at.group % H, b = at.group / (H * pgroups);
+    const int dir0 = (at.group / H) % pgroups * ND;                   // the workgroup's first direction
+    const int d0 = wave % DW * PB;                                    // the wave's first one behind it
+    const size_t rows = (size_t)T_len, bh = (size_t)b * H + head, kv_base = bh * rows * dh;
+    const int k0 = at.tile * ROWS + wave / DW * TILE, key = k0 + m;
+    float kf[1][DH / 2], vf[1][DH / 2];
+    load_half_row<DH, VEC>(kf[0], k + kv_base, key, h, T_len, dh);
+    load_half_row<DH, VEC>(vf[0], v + kv_base, key, h, T_len, dh);
+    f32x16 acc_k[PB][1][NB], acc_v[PB][1][NB];
+#pragma unroll
+    for (int p = 0; p < PB; ++p)
+#pragma unroll
+        for (int n = 0; n < NB; ++n) acc_k[p][0][n] = acc_v[p][0][n] = zero16();
+    const float sc2 = scale * LOG2E;
+    const int first = causal ? at.tile * (ROWS / TILE) : 0;
+    const int steps = (T_len + TILE - 1) / TILE;
+    Stage qs, gs[ND];
+    float row_value[2];  // lse and deltas of the next tile's rows, one or two per thread
+    auto fetch = [&](int it) {
+        const int i0 = it * TILE;
+        qs.fetch(q + kv_base, i0, T_len, dh, tid);
+#pragma unroll
+        for (int p = 0; p < ND; ++p) {
+            const size_t bph = ((size_t)b * P + min(dir0 + p, P - 1)) * H + head;
+            gs[p].fetch(d_out + bph * rows * dh, i0, T_len, dh, tid);
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int which = min((tid + NT * u) / TILE, ND), row = min(i0 + tid % TILE, T_len - 1);
+            const int p = min(dir0 + which - 1, P - 1);
+            row_value[u] = *(which == 0 ? lse2 + bh * rows + row : delta + (((size_t)b * P + p) * H + head) * rows + row);
+        }
+    };
+    auto commit = [&](int it) {
+        const int i0 = it * TILE;
+        float* dst = lds + (it & 1) * BUF;
+        qs.commit(dst, i0, T_len, dh, tid);
+#pragma unroll
+        for (int p = 0; p < ND; ++p)
+            gs[p].commit(dst + (1 + p) * TILE * PITCH, i0, dir0 + p < P ? T_len : 0, dh, tid);
+        // rows past the end: lse = +inf makes their P zero
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+            dst[MATS + tid + NT * u] = i0 + tid % TILE < T_len ? row_value[u] : tid + NT * u < TILE ? INFINITY : 0.0f;
+    };
+    fetch(first);
+    commit(first);
+    __syncthreads();
+    // the steps of the workgroup's earlier keys first, then this wave's own (no branch around the products: the
+    // accumulators would be copied at its join on every step)
+    const int own = k0 >= T_len ? steps : causal ? k0 / TILE : first;
+    for (int it = first; it < own; ++it) {
+        if (it + 1 < steps) fetch(it + 1);
+        if (it + 1 < steps) commit(it + 1);
+        __syncthreads();
+    }
+    for (int it = own; it < steps; ++it) {
+        const int i0 = it * TILE;
+        if (it + 1 < steps) fetch(it + 1);
+        const float* qt = lds + (it & 1) * BUF;
+        const float* stat = qt + MATS;
+        f32x16 ss[1] = {zero16()};
+        f32x16& s = ss[0];
+        dot_form<DH, 1>(ss, qt + m * PITCH + h * (DH / 2), kf, nothing);
+        const bool masked = causal && i0 < k0 + TILE - 1;  // the same in all lanes
+        f32x4 lse4[4];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) lse4[g] = *reinterpret_cast<const f32x4*>(stat + 8 * g + 4 * h);
+#pragma unroll
+        for (int p = 0; p < PB; ++p) {
+            const float* gt = qt + (1 + d0 + p) * TILE * PITCH;
+            f32x16 dps[1] = {zero16()};
+            f32x16& dp = dps[0];
+            if (p == 0)
+                dot_form<DH, 1>(dps, gt + m * PITCH + h * (DH / 2), vf, [&](int i) __attribute__((always_inline)) {
+                    s[i] = exp2f(s[i] * sc2 - lse4[i >> 2][i & 3]);
+                    if (masked && key > i0 + acc_row(i, h)) s[i] = 0.0f;
+                });
+            else
+                dot_form<DH, 1>(dps, gt + m * PITCH + h * (DH / 2), vf, nothing);
+            f32x4 d4[4];
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+                d4[g] = *reinterpret_cast<const f32x4*>(stat + (1 + d0 + p) * TILE + 8 * g + 4 * h);
+            chain_form<NB, PITCH, 1, false>(acc_v[p], gt + 4 * h * PITCH + m, ss, [&](int i) __attribute__((always_inline)) {
+                dp[i] = s[i] * (dp[i] - d4[i >> 2][i & 3]);
+            });
+            chain_form<NB, PITCH, 1, false>(acc_k[p], qt + 4 * h * PITCH + m, dps, nothing);
+        }
+        if (it + 1 < steps) commit(it + 1);
+        __syncthreads();
+    }
+#pragma unroll
+    for (int p = 0; p < PB; ++p) {
+        if (dir0 + d0 + p >= P) break;
+        const size_t base = (((size_t)b * P + dir0 + d0 + p) * H + head) * rows * dh;
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const int row = k0 + acc_row(i, h), c = 32 * n + m;
+                if (row < T_len && c < dh) {
+                    dk[base + (size_t)row * dh + c] = acc_k[p][0][n][i] * scale;
+                    dv[base + (size_t)row * dh + c] = acc_v[p][0][n][i];
+                }
+            }
+    }
+}
+
+struct Args {
+    const float *q, *k, *v, *d_out;
+    float *dq, *dk, *dv, *lse2, *delta;
+    int B, H, T_len, dh, P, causal;
+    float scale;
+    hipStream_t stream;
+};
+
+template <int DH, int PB, int DW, bool VEC>
+int launch_with(const Args& a) {
+    constexpr int PITCH = TileStage<DH, VEC>::PITCH, ROWS = NWAVE / DW * TILE, ND = DW * PB;
+    constexpr size_t kv_bytes = (size_t)4 * TILE * PITCH * sizeof(float);
+    constexpr size_t qg_bytes = (size_t)2 * ((1 + ND) * TILE * PITCH + 2 * NT) * sizeof(float);
+    static_assert(qg_bytes <= 160 * 1024 && (1 + ND) * TILE <= 2 * NT, "LDS budget");
+    const int heads = a.B * a.H, groups = heads * ((a.P + ND - 1) / ND);
+    const int tiles = (a.T_len + ROWS - 1) / ROWS, stat_tiles = (a.T_len + NWAVE * TILE - 1) / (NWAVE * TILE);
+    if ((double)tiles * groups > 2.0e9) return fail(LBI_ERR_UNSUPPORTED, "lbi_attn_pullback: too many row tiles");
+    if (int rc = ensure_dynamic_lds<&stats_kernel<DH, VEC>>(kv_bytes)) return rc;
+    if (int rc = ensure_dynamic_lds<&dq_kernel<DH, PB, DW, VEC>>(kv_bytes)) return rc;
+    if (int rc = ensure_dynamic_lds<&dkdv_kernel<DH, PB, DW, VEC>>(qg_bytes)) return rc;
+    hipLaunchKernelGGL((stats_kernel<DH, VEC>), dim3((unsigned)(stat_tiles * heads)), dim3(NT), kv_bytes, a.stream,
+                       a.q, a.k, a.v, a.dk, a.lse2, a.H, a.P, a.T_len, a.dh, a.scale, a.causal, stat_tiles, heads);
+    hipLaunchKernelGGL((dq_kernel<DH, PB, DW, VEC>), dim3((unsigned)(tiles * groups)), dim3(NT), kv_bytes, a.stream,
+                       a.q, a.k, a.v, a.d_out, a.dk, a.lse2, a.delta, a.dq, a.H, a.P, a.T_len, a.dh, a.scale, a.causal,
+                       tiles, groups);
+    hipLaunchKernelGGL((dkdv_kernel<DH, PB, DW, VEC>), dim3((unsigned)(tiles * groups)), dim3(NT), qg_bytes, a.stream,
+                       a.q, a.k, a.v, a.d_out, a.lse2, a.delta, a.dk, a.dv, a.H, a.P, a.T_len, a.dh, a.scale, a.causal,
+                       tiles, groups);
+    LBI_HIP_CHECK(hipGetLastError());
+    return LBI_OK;
+}
+
+// How many waves of a workgroup take different directions: as many as there are direction groups (MAX at most: what the
+// d_out tiles leave of the LDS), fewer where that leaves fewer waves without a direction.
+template <int DH, int PB, int MAX>
+int launch_directions(const Args& a) {
+    const int pgroups = (a.P + PB - 1) / PB;
+    auto padded = [&](int dw) { return (pgroups + dw - 1) / dw * dw; };
+    if constexpr (MAX >= 4)
+        if (padded(4) == padded(2) && pgroups > 2) return launch_with<DH, PB, 4, true>(a);
+    if (padded(2) == pgroups || pgroups > 2) return launch_with<DH, PB, 2, true>(a);
+    return launch_with<DH, PB, 1, true>(a);
+}
+
+}  // namespace
+
+int launch(const void* q, const void* k, const void* v, const void* d_out, void* dq, void* dk, void* dv,
+                  float* workspace, int B, int H, int T_len, int dh, int P, float scale, int causal,
+                  hipStream_t stream) {
+    const Args a{static_cast<const float*>(q), static_cast<const float*>(k), static_cast<const float*>(v),
+                 static_cast<const float*>(d_out), static_cast<float*>(dq), static_cast<float*>(dk),
+                 static_cast<float*>(dv), workspace, workspace + (size_t)B * H * T_len, B, H, T_len, dh, P, causal,
+                 scale, stream};
+    uintptr_t bits = 0;
+    for (const void* p : {q, k, v, d_out, (const void*)dk}) bits |= reinterpret_cast<uintptr_t>(p);
+    if (dh % 4 != 0 || bits % 16 != 0) {
+        if (dh <= 32) return launch_with<32, 1, 1, false>(a);
+        if (dh <= 64) return launch_with<64, 1, 1, false>(a);
+        return dh <= 96 ? launch_with<96, 1, 1, false>(a) : launch_with<128, 1, 1, false>(a);
+    }
+    if (dh <= 32) return P >= 2 ? launch_directions<32, 2, 4>(a) : launch_with<32, 1, 1, true>(a);
+    if (dh <= 64) return P >= 2 ? launch_directions<64, 2, 4>(a) : launch_with<64, 1, 1, true>(a);
+    if (dh <= 96) return launch_directions<96, 1, 4>(a);
+    return launch_directions<128, 1, 2>(a);
+}
+
+}  // namespace attn_f32
+}  // namespace lbi

@@ -68,6 +68,31 @@ def test_fp32_matches_oracle(seed, shape, basis, causal, device):
         assert torch.allclose(a.double(), c, atol=2e-5, rtol=2e-5)
 
 
+# fp32 matrix-core kernels: lengths around the 32-row tiles and the 128-row workgroups, head dims at and between the
+# compiled widths (33 and 130: scalar loads / the scalar kernels), direction counts that fill one, two or four waves of a
+# workgroup with directions and leave the last group a remainder
+FP32_MFMA_CASES = [
+    ((1, 2, 31, 32), 1), ((2, 1, 32, 64), 2), ((1, 2, 33, 64), 3), ((1, 1, 128, 64), 4), ((1, 1, 129, 64), 5),
+    ((1, 2, 160, 36), 6), ((1, 1, 95, 33), 3), ((1, 1, 64, 96), 1), ((1, 1, 97, 80), 2), ((1, 1, 65, 96), 3),
+    ((1, 1, 127, 128), 4), ((1, 1, 225, 128), 1), ((1, 1, 70, 100), 5), ((2, 2, 1, 128), 3), ((1, 2, 258, 64), 9),
+    ((1, 3, 200, 32), 8), ((1, 1, 40, 130), 2),
+]
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("shape,basis", FP32_MFMA_CASES)
+def test_fp32_tile_edges_against_fp64(shape, basis, causal, device):
+    q, k, v, g = oattn.make_attention_inputs(*shape, basis, dtype=torch.float32, seed=shape[2] * 131 + basis)
+    scale = 1.0 / math.sqrt(shape[-1])
+    got = _run(q, k, v, g, device, scale=scale, causal=causal)
+    truth = oattn.attention_pullback_dense(q, k, v, g, softmax_scale=scale, causal=causal, dtype=torch.float64)
+    bound = (shape[2] + 2 * shape[3]) * 2.0 ** -24  # a rounding per term of the sums over keys and over the head dim
+    for name, a, c in zip(("dq", "dk", "dv"), got, truth):
+        # against the largest cotangent where a result vanishes (one token: dq = dk = 0)
+        err = float((a.double() - c).abs().max()) / max(float(c.abs().max()), float(g.abs().max()))
+        assert err <= bound, (name, err, bound)
+
+
 # 16-bit storage: the MFMA kernels (T % 64 == 0, Dh in {64, 128}; one fused launch for Dh = 64, T <= 128) and the
 # generic ones otherwise.
 # (121, (1, 2, 16, 64), P) are the reference's fp16 cases (tests/test_cuda_attention_pullback.py:178-243);
