@@ -83,6 +83,14 @@ template <> struct Pack<bf16_raw, 8> {
     }
 };
 
+// VEC elements as loaded, widened where they are used: a load that is still in flight costs its registers only.
+// `p` must be aligned to VEC elements.
+template <typename T, int VEC> struct alignas(sizeof(T) * VEC) Raw {
+    T e[VEC];
+    __device__ __forceinline__ void load(const T* p) { *this = *reinterpret_cast<const Raw*>(p); }
+    __device__ __forceinline__ float at(int i) const { return to_f32(e[i]); }
+};
+
 // Elements of T in a 16-byte access.
 template <typename T> constexpr int wide() { return 16 / (int)sizeof(T); }
 
@@ -226,6 +234,42 @@ __device__ __forceinline__ void qkv_unit_offsets(bool rotary, int half, int j, i
     off1 = (rotary && !INTERLEAVED) ? half + j : 2 * j + VEC;
 }
 
+// Transposed rotation of VEC pairs; a0 | a1 are the values at in-head offsets off0.. / off1..
+template <int VEC, bool INTERLEAVED>
+__device__ __forceinline__ void qkv_unrotate(const float (&a0)[VEC], const float (&a1)[VEC], const float (&cs)[VEC],
+                                             const float (&sn)[VEC], float (&y0)[VEC], float (&y1)[VEC]) {
+    float ge[VEC], go[VEC];
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+        if (INTERLEAVED) {  // a0|a1 holds pairs (2i, 2i+1) of the 2 VEC span
+            const int e = 2 * i, o = 2 * i + 1;
+            ge[i] = e < VEC ? a0[e % VEC] : a1[e % VEC];
+            go[i] = o < VEC ? a0[o % VEC] : a1[o % VEC];
+        } else {
+            ge[i] = a0[i];
+            go[i] = a1[i];
+        }
+    }
+    float re[VEC], ro[VEC];
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+        // explicit fused steps: every caller rounds the same way whatever the compiler would contract
+        re[i] = fmaf(ge[i], cs[i], go[i] * sn[i]);
+        ro[i] = fmaf(go[i], cs[i], -(ge[i] * sn[i]));
+    }
+#pragma unroll
+    for (int i = 0; i < VEC; ++i) {
+        if (INTERLEAVED) {
+            const int e = 2 * i, o = 2 * i + 1;
+            if (e < VEC) y0[e % VEC] = re[i]; else y1[e % VEC] = re[i];
+            if (o < VEC) y0[o % VEC] = ro[i]; else y1[o % VEC] = ro[i];
+        } else {
+            y0[i] = re[i];
+            y1[i] = ro[i];
+        }
+    }
+}
+
 template <typename T, int VEC, bool INTERLEAVED>
 __device__ __forceinline__ void qkv_unit_values(const T* __restrict__ dq, const T* __restrict__ dk,
                                                 const T* __restrict__ dv, const float* __restrict__ cos_t,
@@ -270,36 +314,7 @@ __device__ __forceinline__ void qkv_unit_values(const T* __restrict__ dq, const 
     Pack<float, VEC> cs, sn;
     cs.load(cos_t + (long long)t * half + j);
     sn.load(sin_t + (long long)t * half + j);
-    float ge[VEC], go[VEC];
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-        if (INTERLEAVED) {  // a0|a1 holds pairs (2i, 2i+1) of the 2 VEC span
-            const int e = 2 * i, o = 2 * i + 1;
-            ge[i] = e < VEC ? a0[e % VEC] : a1[e % VEC];
-            go[i] = o < VEC ? a0[o % VEC] : a1[o % VEC];
-        } else {
-            ge[i] = a0[i];
-            go[i] = a1[i];
-        }
-    }
-    float re[VEC], ro[VEC];
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-        // explicit fused steps: every caller rounds the same way whatever the compiler would contract
-        re[i] = fmaf(ge[i], cs.v[i], go[i] * sn.v[i]);
-        ro[i] = fmaf(go[i], cs.v[i], -(ge[i] * sn.v[i]));
-    }
-#pragma unroll
-    for (int i = 0; i < VEC; ++i) {
-        if (INTERLEAVED) {
-            const int e = 2 * i, o = 2 * i + 1;
-            if (e < VEC) y0[e % VEC] = re[i]; else y1[e % VEC] = re[i];
-            if (o < VEC) y0[o % VEC] = ro[i]; else y1[o % VEC] = ro[i];
-        } else {
-            y0[i] = re[i];
-            y1[i] = ro[i];
-        }
-    }
+    qkv_unrotate<VEC, INTERLEAVED>(a0, a1, cs.v, sn.v, y0, y1);
 }
 
 template <typename T, int VEC, bool INTERLEAVED>
@@ -336,7 +351,15 @@ __global__ __launch_bounds__(256) void qkv_pullback_kernel(const T* __restrict__
 // The same projection cotangent pulled back through the depthwise causal convolution that follows the packed
 // projection (see the transposed convolution below), without storing the intermediate: one thread forms the
 // projection cotangent of its 2 VEC channels at RUN + KMAX - 1 consecutive positions and accumulates RUN outputs.
-template <typename T, int VEC, int KMAX, int RUN, bool INTERLEAVED, bool EXACT>
+//
+// Bound: memory.  The rows of a run form a serial chain only through registers, so their loads are all independent:
+// they are issued AHEAD rows before their use, from clamped addresses and under no branch (a load under a branch is
+// waited for at the join, which made every row cost a full memory latency).  REP is the number of query heads of a
+// key/value group, 0 for "any": then the heads are added up in a loop inside the row.  Heads of q have one source; the
+// other REP - 1 loads repeat its address and count as zero.  Consecutive workgroups share the halo rows of their runs,
+// so a contiguous eighth of them is dealt to each XCD.  bf16, H = 12, Dh = 64, T = 1024, B P = 512: 1.34 -> 1.05 ms
+// (4.6 TB/s); H = 4, Hkv = 2, T = 128, B P = 16, in runs of 4 instead of 16: 28.5 -> 7.7 us.
+template <typename T, int VEC, int KMAX, int RUN, bool INTERLEAVED, bool EXACT, int REP>
 __global__ __launch_bounds__(256) void qkv_conv_pullback_kernel(const T* __restrict__ dq, const T* __restrict__ dk,
                                                                 const T* __restrict__ dv,
                                                                 const float* __restrict__ cos_t,
@@ -344,7 +367,10 @@ __global__ __launch_bounds__(256) void qkv_conv_pullback_kernel(const T* __restr
                                                                 const T* __restrict__ weight, T* __restrict__ out,
                                                                 long long n_units, int T_len, int H, int Hkv, int Dh,
                                                                 int ksize) {
-    const long long unit = (long long)blockIdx.x * 256 + threadIdx.x;
+    constexpr int ROWS = RUN + KMAX - 1, AHEAD = sizeof(T) == 4 ? 4 : 6;
+    const unsigned per_xcd = gridDim.x / 8;
+    const unsigned block = blockIdx.x < 8 * per_xcd ? blockIdx.x % 8 * per_xcd + blockIdx.x / 8 : blockIdx.x;
+    const long long unit = (long long)block * 256 + threadIdx.x;
     if (unit >= n_units) return;
     const int half = Dh / 2;
     const int upr = half / VEC;
@@ -393,21 +419,66 @@ __global__ __launch_bounds__(256) void qkv_conv_pullback_kernel(const T* __restr
 #pragma unroll
         for (int e = 0; e < VEC; ++e) acc0[r][e] = acc1[r][e] = 0.0f;
     T* o = out + (n * T_len + s0) * (long long)C;
+    const bool rotary = head < H + Hkv;
+    const int rep = H / Hkv;
+    const int count = head < H ? 1 : rep;  // heads of dq / dk / dv that this packed head sums
+    const int first = head < H ? head : (head < H + Hkv ? head - H : head - H - Hkv) * rep;
+    const T* src = (head < H ? dq : rotary ? dk : dv) + (n * H + first) * (long long)T_len * Dh;
+    const long long head_stride = (long long)T_len * Dh;
+    constexpr int HEADS = REP > 0 ? REP : 1;
+    Raw<T, VEC> x0[AHEAD][HEADS], x1[AHEAD][HEADS];
+    Raw<float, VEC> cs[AHEAD], sn[AHEAD];
+    auto request = [&](int jj) __attribute__((always_inline)) {
+        const int t = min(s0 + jj, T_len - 1), slot = jj % AHEAD;
+        const T* p = src + (long long)t * Dh;
 #pragma unroll
-    for (int jj = 0; jj < RUN + KMAX - 1; ++jj) {
-        float g0[VEC], g1[VEC];
-        if (s0 + jj < T_len && jj < RUN + ksize - 1) {
-            qkv_unit_values<T, VEC, INTERLEAVED>(dq, dk, dv, cos_t, sin_t, n, s0 + jj, T_len, H, Hkv, Dh, head, j, g0,
-                                                 g1);
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) {  // the stored intermediate of the two-kernel form is rounded to T
-                g0[e] = round_via<T>(g0[e]);
-                g1[e] = round_via<T>(g1[e]);
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < VEC; ++e) g0[e] = g1[e] = 0.0f;
+        for (int g = 0; g < HEADS; ++g) {
+            const T* pg = p + (g < count ? g : 0) * head_stride;
+            x0[slot][g].load(pg + off0);
+            x1[slot][g].load(pg + off1);
         }
+        cs[slot].load(cos_t + (long long)t * half + j);
+        sn[slot].load(sin_t + (long long)t * half + j);
+    };
+#pragma unroll
+    for (int jj = 0; jj < AHEAD; ++jj) request(jj);
+#pragma unroll
+    for (int jj = 0; jj < ROWS; ++jj) {
+        const int slot = jj % AHEAD;
+        const bool live = s0 + jj < T_len && jj < RUN + ksize - 1;
+        float a0[VEC], a1[VEC], c[VEC], s[VEC], g0[VEC], g1[VEC];
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {
+            a0[e] = a1[e] = 0.0f;
+#pragma unroll
+            for (int g = 0; g < HEADS; ++g) {
+                a0[e] += g < count ? x0[slot][g].at(e) : 0.0f;
+                a1[e] += g < count ? x1[slot][g].at(e) : 0.0f;
+            }
+            c[e] = cs[slot].at(e);
+            s[e] = sn[slot].at(e);
+        }
+        if (REP == 0) {
+            const T* p = src + (long long)min(s0 + jj, T_len - 1) * Dh;
+            for (int g = 1; g < count; ++g) {
+                Raw<T, VEC> m0, m1;
+                m0.load(p + g * head_stride + off0);
+                m1.load(p + g * head_stride + off1);
+#pragma unroll
+                for (int e = 0; e < VEC; ++e) {
+                    a0[e] += m0.at(e);
+                    a1[e] += m1.at(e);
+                }
+            }
+        }
+        qkv_unrotate<VEC, INTERLEAVED>(a0, a1, c, s, g0, g1);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) {  // the stored intermediate of the two-kernel form is rounded to T
+            g0[e] = live ? round_via<T>(rotary ? g0[e] : a0[e]) : 0.0f;
+            g1[e] = live ? round_via<T>(rotary ? g1[e] : a1[e]) : 0.0f;
+        }
+        if (jj + AHEAD < ROWS) request(jj + AHEAD);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int r = 0; r < RUN; ++r) {
             const int i = jj - r;
@@ -587,14 +658,13 @@ int launch_qkv(const void* dq, const void* dk, const void* dv, const float* cos_
     return LBI_OK;
 }
 
-template <typename T, int VEC, int KMAX, bool INTERLEAVED, bool EXACT>
+template <typename T, int VEC, int KMAX, int RUN, bool INTERLEAVED, bool EXACT, int REP>
 int launch_qkv_conv_as(const void* dq, const void* dk, const void* dv, const float* cos_t, const float* sin_t,
                        const void* weight, void* out, long long n_seq, int T_len, int H, int Hkv, int Dh, int ksize,
                        hipStream_t stream) {
-    constexpr int RUN = KMAX <= 4 ? 16 : 8;  // longer runs spill
     const long long units = n_seq * ((T_len + RUN - 1) / RUN) * (long long)(H + 2 * Hkv) * (Dh / 2 / VEC);
     if (!fits_grid(units, 256)) return fail(LBI_ERR_UNSUPPORTED, "lbi_attn_qkv_conv_pullback: too many elements");
-    hipLaunchKernelGGL((qkv_conv_pullback_kernel<T, VEC, KMAX, RUN, INTERLEAVED, EXACT>), dim3(blocks_for(units, 256)),
+    hipLaunchKernelGGL((qkv_conv_pullback_kernel<T, VEC, KMAX, RUN, INTERLEAVED, EXACT, REP>), dim3(blocks_for(units, 256)),
                        dim3(256), 0, stream, (const T*)dq, (const T*)dk, (const T*)dv, cos_t, sin_t, (const T*)weight,
                        (T*)out, units, T_len, H, Hkv, Dh, ksize);
     LBI_HIP_CHECK(hipGetLastError());
@@ -608,15 +678,28 @@ int launch_qkv_conv_il(const void* dq, const void* dk, const void* dv, const flo
     const bool vec = (Dh / 2) % 4 == 0;
     // the 4 x 4 weights of a channel group are contiguous; 4-element loads of them need 4-element alignment
     const bool exact = vec && ksize == 4 && reinterpret_cast<uintptr_t>(weight) % (4 * sizeof(T)) == 0;
-    if (exact)
-        return launch_qkv_conv_as<T, 4, 4, INTERLEAVED, true>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
+    if (exact) {
+        // A run of RUN outputs reads RUN + 3 rows, so long runs read least; short ones where long ones would leave
+        // compute units without a workgroup.
+        const long long long_units = n_seq * ((T_len + 15) / 16) * (long long)(H + 2 * Hkv) * (Dh / 8);
+        const bool short_runs = long_units < 4LL * 256 * device_compute_units();
+        const int rep = H / Hkv;
+        if (short_runs) {
+            if (rep == 1) return launch_qkv_conv_as<T, 4, 4, 4, INTERLEAVED, true, 1>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
+            if (rep == 2) return launch_qkv_conv_as<T, 4, 4, 4, INTERLEAVED, true, 2>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
+            return launch_qkv_conv_as<T, 4, 4, 4, INTERLEAVED, true, 0>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
+        }
+        if (rep == 1) return launch_qkv_conv_as<T, 4, 4, 16, INTERLEAVED, true, 1>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
+        if (rep == 2) return launch_qkv_conv_as<T, 4, 4, 16, INTERLEAVED, true, 2>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
+        return launch_qkv_conv_as<T, 4, 4, 16, INTERLEAVED, true, 0>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
+    }
     if (vec && ksize <= 4)
-        return launch_qkv_conv_as<T, 4, 4, INTERLEAVED, false>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
+        return launch_qkv_conv_as<T, 4, 4, 16, INTERLEAVED, false, 0>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
     if (vec)
-        return launch_qkv_conv_as<T, 4, 8, INTERLEAVED, false>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
+        return launch_qkv_conv_as<T, 4, 8, 8, INTERLEAVED, false, 0>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);  // longer runs spill
     if (ksize <= 4)
-        return launch_qkv_conv_as<T, 1, 4, INTERLEAVED, false>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
-    return launch_qkv_conv_as<T, 1, 8, INTERLEAVED, false>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
+        return launch_qkv_conv_as<T, 1, 4, 16, INTERLEAVED, false, 0>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
+    return launch_qkv_conv_as<T, 1, 8, 8, INTERLEAVED, false, 0>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
 }
 
 template <typename T>
