@@ -101,8 +101,8 @@ __device__ __forceinline__ float wave_sum(float x) {
 }
 
 // ---------------------------------------------------------------------------------------
-// RMSNorm pullback.  One wave per cotangent row (b, p, t); the row is read twice (sums,
-// then outputs), the second time from cache.  x is first rounded to the storage type the
+// RMSNorm pullback, any width, residual or not.  One wave per cotangent row (b, p, t); the row is read twice
+// (sums, then outputs), the second time from cache.  x is first rounded to the storage type the
 // norm ran in (TB), as the forward does.
 // ---------------------------------------------------------------------------------------
 template <typename TB, typename TX, int VEC>
@@ -156,6 +156,95 @@ __global__ __launch_bounds__(256) void rmsnorm_pullback_kernel(const TB* __restr
         }
         if (g_sum != nullptr) of.store(g_sum + row * D + j);
         if (g_sum_branch != nullptr) ob.store(g_sum_branch + row * D + j);
+    }
+}
+
+// The same with a residual, for rows of up to 256 * NIT elements (D a multiple of four): one wave takes DIRS directions
+// of a token.  Bound: memory.  x, the weight and sum x^2 are read and formed once for the DIRS rows, a row is read once
+// and stays in registers between the sums and the outputs, and the next direction's row and residual are requested
+// before this one's reductions.  Same arithmetic and summation order as above.  bf16 branch, fp32 residual and x,
+// D = 768, 512 K rows (mean over residual shared / per row): 1.01 -> 0.81 ms (5.3 TB/s).
+template <typename TB, typename TX, int NIT, int DIRS>
+__global__ __launch_bounds__(256) void rmsnorm_pullback_rows_kernel(const TB* __restrict__ g_out,
+                                                                    const TX* __restrict__ x,
+                                                                    const TB* __restrict__ weight,
+                                                                    const float* g_residual, float* g_sum,
+                                                                    TB* __restrict__ g_sum_branch, unsigned n_waves,
+                                                                    int P, int T_len, int D, float eps,
+                                                                    int res_bcast) {
+    const unsigned id = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (id >= n_waves) return;
+    const unsigned groups = (unsigned)(P + DIRS - 1) / DIRS, rest = id / (unsigned)T_len;
+    const int t = (int)(id - rest * (unsigned)T_len), p0 = (int)(rest % groups) * DIRS, last = min(DIRS, P - p0) - 1;
+    const long long b = rest / groups, bp0 = b * P + p0;
+    const int lane = threadIdx.x & 63;
+    int col[NIT];  // past the end of the row: a load from its last elements that counts as zero
+    bool ok[NIT];
+#pragma unroll
+    for (int k = 0; k < NIT; ++k) {
+        const int j = (k * 64 + lane) * 4;
+        ok[k] = j < D;
+        col[k] = min(j, D - 4);
+    }
+    Raw<TB, 4> g[2][NIT], wr[NIT];
+    Raw<float, 4> res[2][NIT];
+    Raw<TX, 4> xraw[NIT];
+    auto request = [&](int d) __attribute__((always_inline)) {
+        const long long bp = bp0 + min(d, last), row = bp * T_len + t;
+#pragma unroll
+        for (int k = 0; k < NIT; ++k) {
+            g[d & 1][k].load(g_out + row * D + col[k]);
+            res[d & 1][k].load(g_residual + (res_bcast ? bp : row) * D + col[k]);  // [B,P,D] or [B,P,T,D]
+        }
+    };
+#pragma unroll
+    for (int k = 0; k < NIT; ++k) {
+        xraw[k].load(x + (b * T_len + t) * D + col[k]);
+        wr[k].load(weight + col[k]);
+    }
+    request(0);
+    float xr[NIT][4], ss = 0.0f;
+#pragma unroll
+    for (int k = 0; k < NIT; ++k)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            xr[k][i] = ok[k] ? round_via<TB>(xraw[k].at(i)) : 0.0f;
+            ss = fmaf(xr[k][i], xr[k][i], ss);
+        }
+    ss = wave_sum(ss);
+    const float r = rsqrtf(ss / (float)D + eps);
+#pragma unroll
+    for (int d = 0; d < DIRS; ++d) {
+        if (d > last) break;
+        if (d + 1 < DIRS) request(d + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        float wg[NIT][4], dot = 0.0f;
+#pragma unroll
+        for (int k = 0; k < NIT; ++k)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                wg[k][i] = ok[k] ? wr[k].at(i) * g[d & 1][k].at(i) : 0.0f;
+                dot = fmaf(xr[k][i], wg[k][i], dot);
+            }
+        dot = wave_sum(dot);
+        const float c = r * r * r * dot / (float)D;
+        const long long row = (bp0 + d) * T_len + t;
+#pragma unroll
+        for (int k = 0; k < NIT; ++k) {
+            Pack<TB, 4> ob;
+            Pack<float, 4> of;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float o = r * wg[k][i] - xr[k][i] * c;
+                o += res[d & 1][k].at(i);
+                of.v[i] = o;
+                ob.v[i] = o;
+            }
+            if (ok[k]) {
+                of.store(g_sum + row * D + col[k]);
+                if (g_sum_branch != nullptr) ob.store(g_sum_branch + row * D + col[k]);
+            }
+        }
     }
 }
 
@@ -591,6 +680,28 @@ int launch_rmsnorm(const void* g_out, const void* x, const void* weight, const v
                    void* g_sum_branch, long long n_rows, int P, int T_len, int D, float eps, int res_bcast,
                    hipStream_t stream) {
     const dim3 grid(blocks_for(n_rows, 4)), block(256);
+    // Rows that fit the registers (1024 elements; longer ones would leave one wave per SIMD).  Four directions per wave
+    // as soon as that still gives every SIMD four waves.
+    const uintptr_t rows_align = reinterpret_cast<uintptr_t>(x) % (4 * sizeof(TX)) |
+                                 (reinterpret_cast<uintptr_t>(g_out) | reinterpret_cast<uintptr_t>(weight) |
+                                  reinterpret_cast<uintptr_t>(g_sum_branch)) % (4 * sizeof(TB)) |
+                                 (reinterpret_cast<uintptr_t>(g_residual) | reinterpret_cast<uintptr_t>(g_sum)) % 16;
+    if (D % 4 == 0 && D <= 1024 && g_residual != nullptr && g_sum != nullptr && rows_align == 0 && n_rows <= 0x7fffffff) {
+        const long long tokens = n_rows / P, fours = tokens * ((P + 3) / 4);
+        const bool four = P >= 2 && fours >= 16LL * device_compute_units();
+        const unsigned waves = (unsigned)(four ? fours : n_rows);
+#define LBI_RMSNORM_ROWS(NIT, DIRS)                                                                                    \
+    hipLaunchKernelGGL((rmsnorm_pullback_rows_kernel<TB, TX, NIT, DIRS>), dim3(blocks_for(waves, 4)), block, 0, stream, \
+                       (const TB*)g_out, (const TX*)x, (const TB*)weight, (const float*)g_residual, (float*)g_sum,     \
+                       (TB*)g_sum_branch, waves, P, T_len, D, eps, res_bcast)
+        if (D <= 256) { if (four) LBI_RMSNORM_ROWS(1, 4); else LBI_RMSNORM_ROWS(1, 1); }
+        else if (D <= 512) { if (four) LBI_RMSNORM_ROWS(2, 4); else LBI_RMSNORM_ROWS(2, 1); }
+        else if (D <= 768) { if (four) LBI_RMSNORM_ROWS(3, 4); else LBI_RMSNORM_ROWS(3, 1); }
+        else { if (four) LBI_RMSNORM_ROWS(4, 4); else LBI_RMSNORM_ROWS(4, 1); }
+#undef LBI_RMSNORM_ROWS
+        LBI_HIP_CHECK(hipGetLastError());
+        return LBI_OK;
+    }
     if (D % 4 == 0)
         hipLaunchKernelGGL((rmsnorm_pullback_kernel<TB, TX, 4>), grid, block, 0, stream, (const TB*)g_out, (const TX*)x,
                            (const TB*)weight, (const float*)g_residual, (float*)g_sum, (TB*)g_sum_branch, n_rows, P,

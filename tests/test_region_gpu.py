@@ -55,6 +55,30 @@ def test_rmsnorm_pullback(dtype, dim, device):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("dim", [4, 256, 260, 1020, 1024, 1028])
+def test_rmsnorm_pullback_several_directions_per_wave(dtype, dim, device):
+    """Enough tokens for four directions per wave, with a last group of one, at the edges of the register-held widths
+    and one past them; one direction alone has to give the same bits."""
+    from latent_bounded_interfaces_amd.hip.transformer import region
+
+    torch.manual_seed(dim)
+    b, p, t = 2, 5, 1025
+    g = torch.randn(b, p, t, dim, device=device).to(dtype)
+    x = torch.randn(b, t, dim, device=device)
+    w = (1 + 0.1 * torch.randn(dim, device=device)).to(dtype)
+    res = torch.randn(b, p, t, dim, device=device)
+    total, branch = region.rmsnorm_pullback(g, x, w, 1e-5, res.clone(), want_branch=True)
+    xr, wg = x.to(dtype).double().unsqueeze(1), w.double() * g.double()
+    r = torch.rsqrt(xr.pow(2).mean(-1, keepdim=True) + 1e-5)
+    want = r * wg - xr * r.pow(3) * (xr * wg).mean(-1, keepdim=True) + res.double()
+    assert _max_rel(total, want) <= 2e-5 and _max_rel(branch, want) <= _tol(dtype)
+    for i in (0, p - 1):
+        one, one_branch = region.rmsnorm_pullback(g[-1:, i:i + 1].contiguous(), x[-1:], w, 1e-5,
+                                                  res[-1:, i:i + 1].contiguous(), want_branch=True)
+        assert torch.equal(one[0, 0], total[-1, i]) and torch.equal(one_branch[0, 0], branch[-1, i])
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("hidden", [24, 27, 3072])
 def test_gated_mlp_pullback(dtype, hidden, device):
     from latent_bounded_interfaces_amd.hip.transformer import region
