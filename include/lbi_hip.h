@@ -158,6 +158,22 @@ int lbi_attn_pullback(const void* q, const void* k, const void* v, const void* d
                       float softmax_scale, int causal, int dtype, void* stream);
 
 /*
+ * lbi_attn_pullback for sequences and head dims that end inside a tile, on the matrix-core kernels: any T, Dh a
+ * multiple of 8 up to 128, 16-bit storage, causal (short sequences, which need no workspace: causal or not).
+ * The results are those of lbi_attn_pullback on copies padded with zeros to T = 64 n and Dh = 64 or 128, without the
+ * copies.  (lbi_attn_pullback itself runs such sizes on kernels that keep the probabilities in fp32, at a small
+ * fraction of the speed.)  All seven tensors 16-byte aligned; other calls return LBI_ERR_UNSUPPORTED.
+ */
+size_t lbi_attn_pullback_edge_workspace_bytes(int64_t B, int64_t H, int64_t T, int64_t Dh,
+                                              int64_t P, int dtype);
+
+int lbi_attn_pullback_edge(const void* q, const void* k, const void* v, const void* d_out,
+                           void* dq, void* dk, void* dv,
+                           void* workspace, size_t workspace_bytes,
+                           int64_t B, int64_t H, int64_t T, int64_t Dh, int64_t P,
+                           float softmax_scale, int causal, int dtype, void* stream);
+
+/*
  * lbi_attn_pullback without a workspace argument and without any allocation: the scratch memory (softmax
  * statistics, -delta, the fp32 forward output) lives in a static device array of
  * LBI_ATTN_STATIC_SCRATCH_BYTES inside the library, one copy per GPU, held until the process ends.

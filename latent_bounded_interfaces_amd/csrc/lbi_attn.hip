@@ -123,6 +123,53 @@ extern "C" int lbi_attn_pullback(const void* q, const void* k, const void* v, co
     }
 }
 
+extern "C" size_t lbi_attn_pullback_edge_workspace_bytes(int64_t B, int64_t H, int64_t T, int64_t Dh, int64_t P,
+                                                         int dtype) {
+    using namespace lbi;
+    if (check_attn_dims(B, H, T, Dh, P, dtype) != LBI_OK) return 0;
+    if (B == 0 || H == 0 || T == 0 || Dh == 0 || P == 0 || !attn_mfma::supports_edge((int)T, (int)Dh, dtype)) return 0;
+    const int wide = Dh > 64 ? 128 : 64;
+    if (use_small_path((int)T, wide, dtype)) return 0;
+    return (attn_mfma::workspace_floats(B, H, attn_mfma::edge_len((int)T), wide, P) * sizeof(float) + 255) & ~(size_t)255;
+}
+
+// Lengths and head dims that end inside a tile, on the matrix-core kernels.  Short ones take the single launch, as
+// whole tiles do; the streaming kernels have the form for causal calls only, since a key past the end is told from a
+// real one by the causal mask alone.
+extern "C" int lbi_attn_pullback_edge(const void* q, const void* k, const void* v, const void* d_out, void* dq, void* dk,
+                                      void* dv, void* workspace, size_t workspace_bytes, int64_t B, int64_t H, int64_t T,
+                                      int64_t Dh, int64_t P, float softmax_scale, int causal, int dtype, void* stream_v) {
+    using namespace lbi;
+    clear_error();
+    if (int rc = check_attn_dims(B, H, T, Dh, P, dtype)) return rc;
+    if (B == 0 || H == 0 || T == 0 || Dh == 0 || P == 0) return LBI_OK;
+    if (!q || !k || !v || !d_out || !dq || !dk || !dv)
+        return fail(LBI_ERR_INVALID, "lbi_attn_pullback_edge: null tensor pointer");
+    const int b = (int)B, h = (int)H, t = (int)T, dh = (int)Dh, p = (int)P;
+    const int wide = dh > 64 ? 128 : 64;
+    const bool small = attn_mfma::supports_edge(t, dh, dtype) &&
+                       (use_small_path(t, wide, dtype) || (!causal && attn_small::supports(t, wide, dtype)));
+    if (!attn_mfma::supports_edge(t, dh, dtype) || !(small || causal))
+        return fail(LBI_ERR_UNSUPPORTED, "lbi_attn_pullback_edge: needs half or bfloat16, Dh a multiple of 8 up to 128, "
+                                         "and a causal call or a short sequence");
+    for (const void* ptr : {q, k, v, d_out, (const void*)dq, (const void*)dk, (const void*)dv})
+        if (reinterpret_cast<uintptr_t>(ptr) % 16)
+            return fail(LBI_ERR_INVALID, "lbi_attn_pullback_edge: tensors must be 16-byte aligned");
+    hipStream_t stream = static_cast<hipStream_t>(stream_v);
+    if (small)
+        return dtype == LBI_F16
+                   ? attn_small::launch<_Float16>(q, k, v, d_out, dq, dk, dv, b, h, t, dh, p, softmax_scale, causal, stream)
+                   : attn_small::launch<bf16_raw>(q, k, v, d_out, dq, dk, dv, b, h, t, dh, p, softmax_scale, causal, stream);
+    const size_t need = lbi_attn_pullback_edge_workspace_bytes(B, H, T, Dh, P, dtype);
+    if (!workspace || workspace_bytes < need || reinterpret_cast<uintptr_t>(workspace) % 16 != 0)
+        return fail(LBI_ERR_WORKSPACE, "lbi_attn_pullback_edge: 16-byte aligned workspace of %zu bytes needed, %zu given",
+                    need, workspace_bytes);
+    float* ws = static_cast<float*>(workspace);
+    return dtype == LBI_F16
+               ? attn_mfma::launch_edge<_Float16>(q, k, v, d_out, dq, dk, dv, ws, b, h, t, dh, p, softmax_scale, stream)
+               : attn_mfma::launch_edge<bf16_raw>(q, k, v, d_out, dq, dk, dv, ws, b, h, t, dh, p, softmax_scale, stream);
+}
+
 extern "C" int lbi_attn_pullback_static(const void* q, const void* k, const void* v, const void* d_out, void* dq,
                                         void* dk, void* dv, int64_t B, int64_t H, int64_t T, int64_t Dh, int64_t P,
                                         float softmax_scale, int causal, int dtype, void* stream_v) {

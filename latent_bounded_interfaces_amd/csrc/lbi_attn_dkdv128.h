@@ -45,12 +45,12 @@ __device__ __forceinline__ void dma16_at(const void* lane_ptr, unsigned lds_base
                  : "memory");
 }
 
-template <typename T, int DH, bool CAUSAL>
+template <typename T, int DH, bool CAUSAL, bool EDGE>
 __global__ __launch_bounds__(256) void dkdv_ring_kernel(const T* __restrict__ q, const T* __restrict__ k,
                                                       const T* __restrict__ v, const T* __restrict__ d_out,
                                                       const float* __restrict__ lse2, const float* __restrict__ delta,
                                                       T* __restrict__ dk, T* __restrict__ dv, int n_bh, int H, int P,
-                                                      int T_len, float scale) {
+                                                      int T_len, float scale, int t_rows, int dh) {
     constexpr int KS = DH / 16, ND = DH / 32;
     constexpr int RB = DH * 2;                     // bytes per tile row
     constexpr int CPR = DH / 8;                    // 16-byte chunks per tile row
@@ -71,12 +71,14 @@ __global__ __launch_bounds__(256) void dkdv_ring_kernel(const T* __restrict__ q,
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, m = lane & 31, h = lane >> 5;
     const bool active = kb * 256 + wave * 64 < T_len;
     const int j0w = min(kb * 256 + wave * 64, T_len - 64);
-    const size_t base = (size_t)bh * T_len * DH;
-    const size_t prow = (((size_t)b * P + p) * H + hh) * T_len;
+    const Extent<DH, EDGE> ext(T_len, t_rows, dh);
+    const size_t base = (size_t)bh * ext.t_rows * ext.dh;
+    const size_t slice = ((size_t)b * P + p) * H + hh;
+    const size_t prow = slice * ext.t_rows;
     const T* q_bh = q + base;
-    const T* g_p = d_out + prow * DH;
+    const T* g_p = d_out + prow * ext.dh;
     const float* lse_bh = lse2 + (size_t)bh * T_len;
-    const float* delta_p = delta + prow;
+    const float* delta_p = delta + slice * T_len;
 
     // ---- lane constants of the LDS addressing -------------------------------------------
     // nat: tile_off(m, 2ks + h) == lane_nat ^ (ks << 5).  tr: the address of the transpose read for
@@ -95,18 +97,18 @@ __global__ __launch_bounds__(256) void dkdv_ring_kernel(const T* __restrict__ q,
     for (int x = 0; x < NX; ++x) {
         const int sigma = 64 * (NX * wave + x) + lane;
         const int r = sigma / CPR;
-        dma_off[x] = r * RB + (((sigma % CPR) ^ swz<DH>(r)) << 4);
+        dma_off[x] = ext.chunk_off(r, (sigma % CPR) ^ swz<DH>(r));
     }
     // lanes 0-7: lse2 float4 #lane, lanes 8-15: delta float4 #(lane-8); the two arrays need not
     // share an allocation, so each lane carries its own 64-bit address
     const float* stat_ptr = (lane < 8 ? lse_bh : delta_p) + 4 * (lane & 7);
     const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char*)smem;
     auto issue_tile = [&](int i_row, unsigned stage_base) __attribute__((always_inline)) {
-        const unsigned row_bytes = (unsigned)i_row * RB;
 #pragma unroll
         for (int x = 0; x < NX; ++x) {
-            dma16(q_bh, row_bytes + dma_off[x], lds0 + stage_base + 1024 * (NX * wave + x));
-            dma16(g_p, row_bytes + dma_off[x], lds0 + stage_base + TILE + 1024 * (NX * wave + x));
+            const unsigned off = ext.source_off(dma_off[x], (64 * (NX * wave + x) + lane) / CPR, i_row);
+            dma16(q_bh, off, lds0 + stage_base + 1024 * (NX * wave + x));
+            dma16(g_p, off, lds0 + stage_base + TILE + 1024 * (NX * wave + x));
         }
         // Every wave keeps its own copy of the 64 row statistics: no cross-wave dependency.
         if (lane < 16) dma16_at(stat_ptr + i_row, lds0 + stage_base + 2 * TILE + 256 * wave);
@@ -120,14 +122,14 @@ __global__ __launch_bounds__(256) void dkdv_ring_kernel(const T* __restrict__ q,
     for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
-            kf[t][ks] = *reinterpret_cast<const u32x4*>(k + base + (size_t)(j0w + 32 * t + m) * DH + 16 * ks + 8 * h);
+            kf[t][ks] = ext.resident(k + base, j0w + 32 * t + m, 16 * ks + 8 * h);
     {
         char* vt_w = smem + R * STAGE + wave * 2 * TILE;
 #pragma unroll
         for (int u = 0; u < CPR; ++u) {
             const int slot = 64 * u + lane;  // 16-byte slot of the wave's 64-row block
             const int r = slot / CPR, c = slot % CPR;
-            const u32x4 val = *reinterpret_cast<const u32x4*>(v + base + (size_t)(j0w + r) * DH + 8 * c);
+            const u32x4 val = ext.resident(v + base, j0w + r, 8 * c);
             *reinterpret_cast<u32x4*>(vt_w + (r >> 5) * TILE + tile_off<DH>(r & 31, c)) = val;
         }
     }
@@ -360,8 +362,8 @@ __global__ __launch_bounds__(256) void dkdv_ring_kernel(const T* __restrict__ q,
     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
 
     if (active) {
-        unsigned short* ok = reinterpret_cast<unsigned short*>(dk + (prow + j0w) * DH);
-        unsigned short* ov = reinterpret_cast<unsigned short*>(dv + (prow + j0w) * DH);
+        unsigned short* ok = reinterpret_cast<unsigned short*>(dk + (prow + j0w) * ext.dh);
+        unsigned short* ov = reinterpret_cast<unsigned short*>(dv + (prow + j0w) * ext.dh);
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -370,12 +372,16 @@ __global__ __launch_bounds__(256) void dkdv_ring_kernel(const T* __restrict__ q,
                 for (int r = 0; r < 16; r += 2) {
                     const unsigned k2 = Mma<T>::pack2(acc_k[t][nd][r] * scale, acc_k[t][nd][r + 1] * scale);
                     const unsigned v2 = Mma<T>::pack2(acc_v[t][nd][r], acc_v[t][nd][r + 1]);
-                    const size_t o0 = (size_t)(32 * t + c_row(r, h)) * DH + 32 * nd + m;
-                    const size_t o1 = (size_t)(32 * t + c_row(r + 1, h)) * DH + 32 * nd + m;
-                    ok[o0] = (unsigned short)(k2 & 0xffffu);
-                    ok[o1] = (unsigned short)(k2 >> 16);
-                    ov[o0] = (unsigned short)(v2 & 0xffffu);
-                    ov[o1] = (unsigned short)(v2 >> 16);
+                    const int r0 = 32 * t + c_row(r, h), r1 = 32 * t + c_row(r + 1, h), col = 32 * nd + m;
+                    const size_t o0 = (size_t)r0 * ext.dh + col, o1 = (size_t)r1 * ext.dh + col;
+                    if (ext.stored(j0w + r0, col)) {
+                        ok[o0] = (unsigned short)(k2 & 0xffffu);
+                        ov[o0] = (unsigned short)(v2 & 0xffffu);
+                    }
+                    if (ext.stored(j0w + r1, col)) {
+                        ok[o1] = (unsigned short)(k2 >> 16);
+                        ov[o1] = (unsigned short)(v2 >> 16);
+                    }
                 }
     }
 }
@@ -384,15 +390,16 @@ template <int DH> constexpr size_t dkdv_ring_lds_bytes() {
     return 4 * (2 * 32 * DH * 2 + 4 * 256) + 4 * 2 * 32 * DH * 2;  // 4 stages + V of 256 keys
 }
 
-template <typename T, int DH, bool CAUSAL>
+template <typename T, int DH, bool CAUSAL, bool EDGE>
 int launch_dkdv(const T* q, const T* k, const T* v, const T* g, const float* lse2, const float* delta, T* dk, T* dv,
-                 int n_bh, int H, int P, int T_len, float scale, hipStream_t stream) {
+                 int n_bh, int H, int P, int T_len, float scale, int t_rows, int dh,
+                hipStream_t stream) {
     const int n_kb = (T_len + 255) / 256;
     constexpr size_t lds_bytes = dkdv_ring_lds_bytes<DH>();
     static_assert(lds_bytes <= 160 * 1024, "LDS budget");
-    if (int rc = ensure_dynamic_lds<&dkdv_ring_kernel<T, DH, CAUSAL>>(lds_bytes)) return rc;
-    hipLaunchKernelGGL((dkdv_ring_kernel<T, DH, CAUSAL>), dim3(grid_size(n_kb * P, n_bh)), dim3(256), lds_bytes, stream,
-                       q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale);
+    if (int rc = ensure_dynamic_lds<&dkdv_ring_kernel<T, DH, CAUSAL, EDGE>>(lds_bytes)) return rc;
+    hipLaunchKernelGGL((dkdv_ring_kernel<T, DH, CAUSAL, EDGE>), dim3(grid_size(n_kb * P, n_bh)), dim3(256), lds_bytes, stream,
+                       q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, t_rows, dh);
     return LBI_OK;
 }
 

@@ -32,12 +32,12 @@
 namespace lbi {
 namespace attn_mfma {
 
-template <typename T, int DH, bool CAUSAL, int DW = 1>
+template <typename T, int DH, bool CAUSAL, int DW, bool EDGE>
 __global__ __launch_bounds__(256) void dkdv_pair_kernel(const T* __restrict__ q, const T* __restrict__ k,
                                                       const T* __restrict__ v, const T* __restrict__ d_out,
                                                       const float* __restrict__ lse2, const float* __restrict__ delta,
                                                       T* __restrict__ dk, T* __restrict__ dv, int n_bh, int H, int P,
-                                                      int T_len, float scale) {
+                                                      int T_len, float scale, int t_rows, int dh) {
     constexpr int KS = DH / 16, ND = DH / 32;
     constexpr int RB = DH * 2;                       // bytes per tile row
     constexpr int CPR = DH / 8;                      // 16-byte chunks per tile row
@@ -78,12 +78,13 @@ __global__ __launch_bounds__(256) void dkdv_pair_kernel(const T* __restrict__ q,
     size_t prow_own[DW];
     const int j0w = min(j0 + 64 * kh, T_len - 64);   // this wave's 64 keys (dP, dV, dK)
     const int j0s = min(j0 + 32 * wave, T_len - 32); // this wave's S tile (equals j0w + 32 d inside the sequence)
-    const size_t base = (size_t)bh * T_len * DH;
+    const Extent<DH, EDGE> ext(T_len, t_rows, dh);
+    const size_t base = (size_t)bh * ext.t_rows * ext.dh;
     const T* q_bh = q + base;
     const float* lse_bh = lse2 + (size_t)bh * T_len;
     size_t prow[2 * DW];
 #pragma unroll
-    for (int e = 0; e < 2 * DW; ++e) prow[e] = (((size_t)b * P + min(p_first + e, P - 1)) * H + hh) * T_len;
+    for (int e = 0; e < 2 * DW; ++e) prow[e] = (((size_t)b * P + min(p_first + e, P - 1)) * H + hh) * ext.t_rows;
 #pragma unroll
     for (int e = 0; e < DW; ++e) {
         active[e] = (j0 + 64 * kh < T_len) && (p_first + d + 2 * e < P);
@@ -110,18 +111,21 @@ __global__ __launch_bounds__(256) void dkdv_pair_kernel(const T* __restrict__ q,
         const int tile = c / CPT, u = c % CPT;
         const int sigma = 64 * u + lane;
         const int r = sigma / CPR;
-        dma_off[x] = r * RB + (((sigma % CPR) ^ swz<DH>(r)) << 4);
+        dma_off[x] = ext.chunk_off(r, (sigma % CPR) ^ swz<DH>(r));
         dma_dst[x] = tile * TILE + 1024 * u;
-        dma_src[x] = tile == 0 ? q_bh : d_out + prow[tile - 1] * DH;
+        dma_src[x] = tile == 0 ? q_bh : d_out + prow[tile - 1] * ext.dh;
     }
     // lanes 0-7: lse2, 8-15: -delta of statistics slot 1, 16-23: of slot 2 (float4 each)
     const int slot_dir = DW == 1 ? (lane < 16 ? 0 : 1) : d + (lane < 16 ? 0 : 2);
-    const float* stat_ptr = (lane < 8 ? lse_bh : delta + prow[slot_dir]) + 4 * (lane & 7);
+    const size_t stat_row = (((size_t)b * P + min(p_first + slot_dir, P - 1)) * H + hh) * T_len;
+    const float* stat_ptr = (lane < 8 ? lse_bh : delta + stat_row) + 4 * (lane & 7);
     const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char*)smem;
     auto issue_tile = [&](int i_row, unsigned stage_base) __attribute__((always_inline)) {
-        const unsigned row_bytes = (unsigned)i_row * RB;
 #pragma unroll
-        for (int x = 0; x < NXW; ++x) dma16(dma_src[x], row_bytes + dma_off[x], lds0 + stage_base + dma_dst[x]);
+        for (int x = 0; x < NXW; ++x) {
+            const int r = (64 * ((wave + 4 * x) % CPT) + lane) / CPR;
+            dma16(dma_src[x], ext.source_off(dma_off[x], r, i_row), lds0 + stage_base + dma_dst[x]);
+        }
         if (lane < 24) dma16_at(stat_ptr + i_row, lds0 + stage_base + NTILE * TILE + 512 * wave);
     };
 
@@ -147,14 +151,14 @@ __global__ __launch_bounds__(256) void dkdv_pair_kernel(const T* __restrict__ q,
     for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
-            vf[t][ks] = *reinterpret_cast<const u32x4*>(v + base + (size_t)(j0w + 32 * t + m) * DH + 16 * ks + 8 * h);
+            vf[t][ks] = ext.resident(v + base, j0w + 32 * t + m, 16 * ks + 8 * h);
     {
         char* kt_w = smem + KT0 + wave * TILE;       // wave w writes the tile it will read
 #pragma unroll
         for (int u = 0; u < CPR / 2; ++u) {
             const int slot = 64 * u + lane;
             const int r = slot / CPR, c = slot % CPR;
-            const u32x4 val = *reinterpret_cast<const u32x4*>(k + base + (size_t)(j0s + r) * DH + 8 * c);
+            const u32x4 val = ext.resident(k + base, j0s + r, 8 * c);
             *reinterpret_cast<u32x4*>(kt_w + tile_off<DH>(r, c)) = val;
         }
     }
@@ -427,8 +431,8 @@ __global__ __launch_bounds__(256) void dkdv_pair_kernel(const T* __restrict__ q,
 #pragma unroll
     for (int e = 0; e < DW; ++e) {
         if (!active[e]) continue;
-        unsigned short* ok = reinterpret_cast<unsigned short*>(dk + (prow_own[e] + j0w) * DH);
-        unsigned short* ov = reinterpret_cast<unsigned short*>(dv + (prow_own[e] + j0w) * DH);
+        unsigned short* ok = reinterpret_cast<unsigned short*>(dk + (prow_own[e] + j0w) * ext.dh);
+        unsigned short* ov = reinterpret_cast<unsigned short*>(dv + (prow_own[e] + j0w) * ext.dh);
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -437,12 +441,16 @@ __global__ __launch_bounds__(256) void dkdv_pair_kernel(const T* __restrict__ q,
                 for (int r = 0; r < 16; r += 2) {
                     const unsigned k2 = Mma<T>::pack2(acc_k[e][t][nd][r] * scale, acc_k[e][t][nd][r + 1] * scale);
                     const unsigned v2 = Mma<T>::pack2(acc_v[e][t][nd][r], acc_v[e][t][nd][r + 1]);
-                    const size_t o0 = (size_t)(32 * t + c_row(r, h)) * DH + 32 * nd + m;
-                    const size_t o1 = (size_t)(32 * t + c_row(r + 1, h)) * DH + 32 * nd + m;
-                    ok[o0] = (unsigned short)(k2 & 0xffffu);
-                    ok[o1] = (unsigned short)(k2 >> 16);
-                    ov[o0] = (unsigned short)(v2 & 0xffffu);
-                    ov[o1] = (unsigned short)(v2 >> 16);
+                    const int r0 = 32 * t + c_row(r, h), r1 = 32 * t + c_row(r + 1, h), col = 32 * nd + m;
+                    const size_t o0 = (size_t)r0 * ext.dh + col, o1 = (size_t)r1 * ext.dh + col;
+                    if (ext.stored(j0w + r0, col)) {
+                        ok[o0] = (unsigned short)(k2 & 0xffffu);
+                        ov[o0] = (unsigned short)(v2 & 0xffffu);
+                    }
+                    if (ext.stored(j0w + r1, col)) {
+                        ok[o1] = (unsigned short)(k2 >> 16);
+                        ov[o1] = (unsigned short)(v2 >> 16);
+                    }
                 }
     }
 }
@@ -452,28 +460,30 @@ template <int DH, int DW = 1> constexpr size_t dkdv_pair_lds_bytes() {
     return 4 * ((1 + 2 * DW) * 32 * DH * 2 + 4 * 512) + 4 * 32 * DH * 2 + 2 * 8 * 1024;
 }
 
-template <typename T, int DH, bool CAUSAL, int DW>
+template <typename T, int DH, bool CAUSAL, int DW, bool EDGE>
 int launch_dkdv_pair_as(const T* q, const T* k, const T* v, const T* g, const float* lse2, const float* delta, T* dk,
-                        T* dv, int n_bh, int H, int P, int T_len, float scale, hipStream_t stream) {
+                        T* dv, int n_bh, int H, int P, int T_len, float scale, int t_rows, int dh,
+                     hipStream_t stream) {
     const int n_kb = (T_len + 127) / 128;
     const int n_pp = (P + 2 * DW - 1) / (2 * DW);
     constexpr size_t lds_bytes = dkdv_pair_lds_bytes<DH, DW>();
     static_assert(lds_bytes <= 160 * 1024, "LDS budget");
-    if (int rc = ensure_dynamic_lds<&dkdv_pair_kernel<T, DH, CAUSAL, DW>>(lds_bytes)) return rc;
-    hipLaunchKernelGGL((dkdv_pair_kernel<T, DH, CAUSAL, DW>), dim3(grid_size(n_kb * n_pp, n_bh)), dim3(256), lds_bytes,
-                       stream, q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale);
+    if (int rc = ensure_dynamic_lds<&dkdv_pair_kernel<T, DH, CAUSAL, DW, EDGE>>(lds_bytes)) return rc;
+    hipLaunchKernelGGL((dkdv_pair_kernel<T, DH, CAUSAL, DW, EDGE>), dim3(grid_size(n_kb * n_pp, n_bh)), dim3(256), lds_bytes,
+                       stream, q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, t_rows, dh);
     return LBI_OK;
 }
 
 // Head dim 64 with three directions or more: two directions per wave (four per workgroup).
-template <typename T, int DH, bool CAUSAL>
+template <typename T, int DH, bool CAUSAL, bool EDGE>
 int launch_dkdv_pair(const T* q, const T* k, const T* v, const T* g, const float* lse2, const float* delta, T* dk,
-                      T* dv, int n_bh, int H, int P, int T_len, float scale, hipStream_t stream) {
+                      T* dv, int n_bh, int H, int P, int T_len, float scale, int t_rows, int dh,
+                     hipStream_t stream) {
     if constexpr (DH == 64) {
         if (P >= 3)
-            return launch_dkdv_pair_as<T, DH, CAUSAL, 2>(q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, stream);
+            return launch_dkdv_pair_as<T, DH, CAUSAL, 2, EDGE>(q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, t_rows, dh, stream);
     }
-    return launch_dkdv_pair_as<T, DH, CAUSAL, 1>(q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, stream);
+    return launch_dkdv_pair_as<T, DH, CAUSAL, 1, EDGE>(q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, t_rows, dh, stream);
 }
 
 }  // namespace attn_mfma

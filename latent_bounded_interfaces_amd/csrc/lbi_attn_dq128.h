@@ -24,12 +24,12 @@
 namespace lbi {
 namespace attn_mfma {
 
-template <typename T, int DH, int PB, bool CAUSAL>
+template <typename T, int DH, int PB, bool CAUSAL, bool EDGE>
 __global__ __launch_bounds__(256) void dq_ring_kernel(const T* __restrict__ q, const T* __restrict__ k,
                                                     const T* __restrict__ v, const T* __restrict__ d_out,
                                                     const float* __restrict__ lse2, const float* __restrict__ o32,
                                                     float* __restrict__ delta, T* __restrict__ dq, int n_bh, int H,
-                                                    int P, int T_len, float scale) {
+                                                    int P, int T_len, float scale, int t_rows, int dh) {
     constexpr int KS = DH / 16, ND = DH / 32;
     constexpr int RB = DH * 2;               // bytes per tile row
     constexpr int CPR = DH / 8;              // 16-byte chunks per tile row
@@ -50,7 +50,8 @@ __global__ __launch_bounds__(256) void dq_ring_kernel(const T* __restrict__ q, c
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, m = lane & 31, h = lane >> 5;
     const bool active = qb * 128 + wave * 32 < T_len;
     const int i0w = min(qb * 128 + wave * 32, T_len - 32);
-    const size_t base = (size_t)bh * T_len * DH;
+    const Extent<DH, EDGE> ext(T_len, t_rows, dh);
+    const size_t base = (size_t)bh * ext.t_rows * ext.dh;
     const T* k_bh = k + base;
     const T* v_bh = v + base;
 
@@ -64,15 +65,15 @@ __global__ __launch_bounds__(256) void dq_ring_kernel(const T* __restrict__ q, c
     for (int x = 0; x < NX; ++x) {
         const int sigma = 64 * (NX * wave + x) + lane;
         const int r = sigma / CPR;
-        dma_off[x] = r * RB + (((sigma % CPR) ^ swz<DH>(r)) << 4);
+        dma_off[x] = ext.chunk_off(r, (sigma % CPR) ^ swz<DH>(r));
     }
     const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char*)smem;
     auto issue_tile = [&](int j_row, unsigned stage_base) __attribute__((always_inline)) {
-        const unsigned row_bytes = (unsigned)j_row * RB;
 #pragma unroll
         for (int x = 0; x < NX; ++x) {
-            dma16(k_bh, row_bytes + dma_off[x], lds0 + stage_base + 1024 * (NX * wave + x));
-            dma16(v_bh, row_bytes + dma_off[x], lds0 + stage_base + TILE + 1024 * (NX * wave + x));
+            const unsigned off = ext.source_off(dma_off[x], (64 * (NX * wave + x) + lane) / CPR, j_row);
+            dma16(k_bh, off, lds0 + stage_base + 1024 * (NX * wave + x));
+            dma16(v_bh, off, lds0 + stage_base + TILE + 1024 * (NX * wave + x));
         }
     };
 
@@ -82,20 +83,19 @@ __global__ __launch_bounds__(256) void dq_ring_kernel(const T* __restrict__ q, c
     // (negated) for the dK/dV kernel: every (direction, query) has exactly one owner wave.
     u32x4 qf[KS];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-        qf[ks] = *reinterpret_cast<const u32x4*>(q + base + (size_t)(i0w + m) * DH + 16 * ks + 8 * h);
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = ext.resident(q + base, i0w + m, 16 * ks + 8 * h);
     const float my_lse = lse2[(size_t)bh * T_len + i0w + m];
     float my_delta[PB];
     char* gf_w = smem + GF0 + wave * PB * TILE;
 #pragma unroll
     for (int pp = 0; pp < PB; ++pp) {
         const int p = min(p0 + pp, P - 1);  // surplus slots redo the last direction; never stored
-        const size_t row0 = (((size_t)b * P + p) * H + hh) * T_len + i0w;
+        const T* g_p = d_out + (((size_t)b * P + p) * H + hh) * ext.t_rows * ext.dh;
 #pragma unroll
         for (int u = 0; u < CPR / 2; ++u) {
             const int slot = 64 * u + lane;
             const int r = slot / CPR, c = slot % CPR;
-            const u32x4 val = *reinterpret_cast<const u32x4*>(d_out + (row0 + r) * DH + 8 * c);
+            const u32x4 val = ext.resident(g_p, i0w + r, 8 * c);
             *reinterpret_cast<u32x4*>(gf_w + pp * TILE + tile_off<DH>(r, c)) = val;
         }
         my_delta[pp] = 0.0f;
@@ -103,7 +103,7 @@ __global__ __launch_bounds__(256) void dq_ring_kernel(const T* __restrict__ q, c
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // the tiles are the wave's own: LDS runs in order
     __builtin_amdgcn_wave_barrier();
     {
-        const float* o_row = o32 + base + (size_t)(i0w + m) * DH + h * (DH / 2);
+        const float* o_row = o32 + ((size_t)bh * T_len + i0w + m) * DH + h * (DH / 2);
 #pragma unroll
         for (int c = 0; c < CPR / 2; ++c) {
             const f32x4 o_lo = *reinterpret_cast<const f32x4*>(o_row + 8 * c);
@@ -275,14 +275,15 @@ __global__ __launch_bounds__(256) void dq_ring_kernel(const T* __restrict__ q, c
         for (int pp = 0; pp < PB; ++pp) {
             if (p0 + pp >= P) break;
             unsigned short* o =
-                reinterpret_cast<unsigned short*>(dq + ((((size_t)b * P + p0 + pp) * H + hh) * T_len + i0w) * DH);
+                reinterpret_cast<unsigned short*>(dq + ((((size_t)b * P + p0 + pp) * H + hh) * ext.t_rows + i0w) * ext.dh);
 #pragma unroll
             for (int nd = 0; nd < ND; ++nd)
 #pragma unroll
                 for (int r = 0; r < 16; r += 2) {
                     const unsigned two = Mma<T>::pack2(acc[pp][nd][r] * scale, acc[pp][nd][r + 1] * scale);
-                    o[(size_t)c_row(r, h) * DH + 32 * nd + m] = (unsigned short)(two & 0xffffu);
-                    o[(size_t)c_row(r + 1, h) * DH + 32 * nd + m] = (unsigned short)(two >> 16);
+                    const int r0 = c_row(r, h), r1 = c_row(r + 1, h), col = 32 * nd + m;
+                    if (ext.stored(i0w + r0, col)) o[(size_t)r0 * ext.dh + col] = (unsigned short)(two & 0xffffu);
+                    if (ext.stored(i0w + r1, col)) o[(size_t)r1 * ext.dh + col] = (unsigned short)(two >> 16);
                 }
         }
     }
@@ -294,17 +295,18 @@ template <int DH, int PB> constexpr size_t dq_ring_lds_bytes() {
 
 // PB is the direction block of the caller's choice (1, 2, 4, and 8 for head dim 64); head dim 128 has
 // accumulation registers for four.
-template <typename T, int DH, int PB, bool CAUSAL>
+template <typename T, int DH, int PB, bool CAUSAL, bool EDGE>
 int launch_dq(const T* q, const T* k, const T* v, const T* g, const float* lse2, const float* o32, float* delta, T* dq,
-               int n_bh, int H, int P, int T_len, float scale, hipStream_t stream) {
+               int n_bh, int H, int P, int T_len, float scale, int t_rows, int dh,
+               hipStream_t stream) {
     constexpr int PBK = (DH == 128 && PB > 4) ? 4 : PB;
     const int n_qb = (T_len + 127) / 128;
     const int n_pb = (P + PBK - 1) / PBK;
     constexpr size_t lds_bytes = dq_ring_lds_bytes<DH, PBK>();
     static_assert(lds_bytes <= 160 * 1024, "LDS budget");
-    if (int rc = ensure_dynamic_lds<&dq_ring_kernel<T, DH, PBK, CAUSAL>>(lds_bytes)) return rc;
-    hipLaunchKernelGGL((dq_ring_kernel<T, DH, PBK, CAUSAL>), dim3(grid_size(n_qb * n_pb, n_bh)), dim3(256), lds_bytes,
-                       stream, q, k, v, g, lse2, o32, delta, dq, n_bh, H, P, T_len, scale);
+    if (int rc = ensure_dynamic_lds<&dq_ring_kernel<T, DH, PBK, CAUSAL, EDGE>>(lds_bytes)) return rc;
+    hipLaunchKernelGGL((dq_ring_kernel<T, DH, PBK, CAUSAL, EDGE>), dim3(grid_size(n_qb * n_pb, n_bh)), dim3(256), lds_bytes,
+                       stream, q, k, v, g, lse2, o32, delta, dq, n_bh, H, P, T_len, scale, t_rows, dh);
     return LBI_OK;
 }
 

@@ -124,18 +124,55 @@ template <int DH> __device__ __forceinline__ int tile_off(int r, int chunk) {
     return r * (DH * 2) + ((chunk ^ swz<DH>(r)) << 4);
 }
 
+// EDGE forms of the kernels (causal calls): sequences that end inside a tile, head dims (multiples of 8) below the
+// tile's DH.  The tile loops run over T_len, the length rounded up to 64, and the workspace has T_len rows and DH
+// columns; the caller's tensors have t_rows rows of dh elements.  Copies padded to the tile cost one extra pass over
+// every tensor and one over every result (bf16 B=8 H=12 T=1000 Dh=64 P=16: 1.19 -> 0.98 ms without them), so
+// the tiles are padded on chip instead, and the results are those of the padded call:
+//  * a row past the end is read from the last row.  As a key it lies above the diagonal of every real query; as a
+//    query its lse2 is +infinity, so its P and dS are 0 and it adds 0 to dK and dV (a value that is not finite in the
+//    last row reaches the same sums through the row itself);
+//  * the resident operands (K and V of the dK/dV kernels, Q and d_out of the dQ kernel, Q of the statistics) are
+//    zero in the columns past dh, so what a streamed tile holds there (the row's last 16 bytes again) is multiplied
+//    by zero;
+//  * neither rows nor columns past the end are stored.
+template <int DH, bool EDGE> struct Extent {
+    int t_rows, dh;
+    __device__ __forceinline__ Extent(int T_len, int t_rows_, int dh_)
+        : t_rows(EDGE ? t_rows_ : T_len), dh(EDGE ? dh_ : DH) {}
+    __device__ __forceinline__ int row(int r) const { return EDGE ? min(r, t_rows - 1) : r; }
+    // eight elements at column c of row r of a resident operand
+    __device__ __forceinline__ u32x4 resident(const void* base, int r, int c) const {
+        const int col = EDGE ? min(c, dh - 8) : c;
+        u32x4 v = *reinterpret_cast<const u32x4*>(static_cast<const char*>(base) + ((size_t)row(r) * dh + col) * 2);
+        if (EDGE && c >= dh) v = u32x4{0u, 0u, 0u, 0u};
+        return v;
+    }
+    // byte offset of 16-byte chunk `chunk` of tile row r in the source tile (row 0 of the tile at offset 0)
+    __device__ __forceinline__ unsigned chunk_off(int r, int chunk) const {
+        return (unsigned)(r * dh * 2 + ((EDGE ? min(chunk, dh / 8 - 1) : chunk) << 4));
+    }
+    // the same, plus where the tile starts: row i_row, or less for a row that would lie past the end
+    __device__ __forceinline__ unsigned source_off(unsigned off, int r, int i_row) const {
+        if (!EDGE) return (unsigned)i_row * (DH * 2) + off;
+        return __umul24((unsigned)(min(i_row + r, t_rows - 1)), (unsigned)(dh * 2)) + off - (unsigned)(r * dh * 2);
+    }
+    __device__ __forceinline__ bool stored(int r, int c) const { return !EDGE || (r < t_rows && c < dh); }
+};
+
 template <int DH> struct TileLoader {
     static constexpr int CHUNKS_PER_ROW = DH / 8;
     static constexpr int N = 32 * CHUNKS_PER_ROW / 256;  // 16-byte chunks per thread
     u32x4 regs[N];
-    // rows row0 .. row0+31 of a row-major [T][DH] 16-bit matrix
-    __device__ __forceinline__ void fetch(const void* base, int row0, int tid) {
+    // rows row0 .. row0+31 of a row-major 16-bit matrix
+    template <bool EDGE> __device__ __forceinline__ void fetch(const Extent<DH, EDGE>& ext, const void* base, int row0, int tid) {
 #pragma unroll
         for (int u = 0; u < N; ++u) {
             const int id = tid + 256 * u;
             const int r = id / CHUNKS_PER_ROW, c = id % CHUNKS_PER_ROW;
+            const int col = EDGE ? min(c * 8, ext.dh - 8) : c * 8;
             regs[u] = *reinterpret_cast<const u32x4*>(static_cast<const char*>(base) +
-                                                      ((size_t)(row0 + r) * DH + c * 8) * 2);
+                                                      ((size_t)ext.row(row0 + r) * ext.dh + col) * 2);
         }
     }
     __device__ __forceinline__ void commit(char* tile, int tid) const {
@@ -212,10 +249,11 @@ inline unsigned grid_size(int per_bh, int n_bh) { return (unsigned)(((n_bh + 7) 
 // stats_kernel: one wave = 32 queries, workgroup = 128 queries, K/V streamed in 32-key tiles.
 // S^T tile: lanes = queries, registers = keys, so softmax statistics are per lane.
 // ---------------------------------------------------------------------------------------
-template <typename T, int DH, bool CAUSAL>
+template <typename T, int DH, bool CAUSAL, bool EDGE>
 __global__ __launch_bounds__(256) void stats_kernel(const T* __restrict__ q, const T* __restrict__ k,
                                                     const T* __restrict__ v, float* __restrict__ lse2,
-                                                    float* __restrict__ o32, int n_bh, int T_len, float scale) {
+                                                    float* __restrict__ o32, int n_bh, int T_len, float scale,
+                                                    int t_rows, int dh) {
     constexpr int KS = DH / 16, ND = DH / 32, TILE_BYTES = 32 * DH * 2;
     extern __shared__ __align__(16) char smem[];  // [2][K tile, V tile]
     int bh, qb;
@@ -227,14 +265,14 @@ __global__ __launch_bounds__(256) void stats_kernel(const T* __restrict__ q, con
     // loop body is branch-free so the accumulators stay in place.
     const bool active = qb * 128 + wave * 32 < T_len;
     const int i0w = min(qb * 128 + wave * 32, T_len - 32);
-    const size_t base = (size_t)bh * T_len * DH;
+    const Extent<DH, EDGE> ext(T_len, t_rows, dh);
+    const size_t base = (size_t)bh * ext.t_rows * ext.dh;
     const T* k_bh = k + base;
     const T* v_bh = v + base;
 
     u32x4 qf[KS];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
-        qf[ks] = *reinterpret_cast<const u32x4*>(q + base + (size_t)(i0w + m) * DH + 16 * ks + 8 * h);
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = ext.resident(q + base, i0w + m, 16 * ks + 8 * h);
     f32x16 o_t[ND];
 #pragma unroll
     for (int nd = 0; nd < ND; ++nd) o_t[nd] = zero16();
@@ -244,8 +282,8 @@ __global__ __launch_bounds__(256) void stats_kernel(const T* __restrict__ q, con
     const int j_end = CAUSAL ? min(T_len, qb * 128 + 128) : T_len;
     const int n_it = j_end / 32;
     TileLoader<DH> kl, vl;
-    kl.fetch(k_bh, 0, tid);
-    vl.fetch(v_bh, 0, tid);
+    kl.fetch(ext, k_bh, 0, tid);
+    vl.fetch(ext, v_bh, 0, tid);
     kl.commit(smem, tid);
     vl.commit(smem + TILE_BYTES, tid);
     __syncthreads();
@@ -255,8 +293,8 @@ __global__ __launch_bounds__(256) void stats_kernel(const T* __restrict__ q, con
         const char* vt = kt + TILE_BYTES;
         {
             const int j_next = min(j0 + 32, T_len - 32);  // the last trip re-reads a valid tile
-            kl.fetch(k_bh, j_next, tid);
-            vl.fetch(v_bh, j_next, tid);
+            kl.fetch(ext, k_bh, j_next, tid);
+            vl.fetch(ext, v_bh, j_next, tid);
         }
         {
             // A tile that lies wholly above the diagonal masks to all -inf and changes nothing.
@@ -315,8 +353,9 @@ __global__ __launch_bounds__(256) void stats_kernel(const T* __restrict__ q, con
     }
     if (active) {
         const float inv = 1.0f / l_run;
-        if (h == 0) lse2[(size_t)bh * T_len + i0w + m] = m_run + log2f(l_run);
-        float* o_row = o32 + base + (size_t)(i0w + m) * DH;
+        if (h == 0)
+            lse2[(size_t)bh * T_len + i0w + m] = EDGE && i0w + m >= ext.t_rows ? INFINITY : m_run + log2f(l_run);
+        float* o_row = o32 + ((size_t)bh * T_len + i0w + m) * DH;
 #pragma unroll
         for (int nd = 0; nd < ND; ++nd)
 #pragma unroll
@@ -338,41 +377,45 @@ inline size_t workspace_floats(int64_t B, int64_t H, int64_t T, int64_t Dh, int6
 }
 
 // dK/dV launch (kernel in lbi_attn_dkdv128.h).
-template <typename T, int DH, bool CAUSAL>
+template <typename T, int DH, bool CAUSAL, bool EDGE>
 int launch_dkdv(const T* q, const T* k, const T* v, const T* g, const float* lse2, const float* delta, T* dk, T* dv,
-                 int n_bh, int H, int P, int T_len, float scale, hipStream_t stream);
+                 int n_bh, int H, int P, int T_len, float scale, int t_rows, int dh,
+                hipStream_t stream);
 
 // dK/dV launch for two or more directions (kernel in lbi_attn_dkdv_pair.h).
-template <typename T, int DH, bool CAUSAL>
+template <typename T, int DH, bool CAUSAL, bool EDGE>
 int launch_dkdv_pair(const T* q, const T* k, const T* v, const T* g, const float* lse2, const float* delta, T* dk,
-                      T* dv, int n_bh, int H, int P, int T_len, float scale, hipStream_t stream);
+                      T* dv, int n_bh, int H, int P, int T_len, float scale, int t_rows, int dh,
+                hipStream_t stream);
 
 // dQ launch (kernel in lbi_attn_dq128.h); PB = directions per wave.
-template <typename T, int DH, int PB, bool CAUSAL>
+template <typename T, int DH, int PB, bool CAUSAL, bool EDGE>
 int launch_dq(const T* q, const T* k, const T* v, const T* g, const float* lse2, const float* o32, float* delta, T* dq,
-               int n_bh, int H, int P, int T_len, float scale, hipStream_t stream);
+               int n_bh, int H, int P, int T_len, float scale, int t_rows, int dh,
+                hipStream_t stream);
 
-template <typename T, int DH, bool CAUSAL>
+// T_len: the length in tiles (a multiple of 64); t_rows, dh: rows and head dim of the tensors (EDGE).
+template <typename T, int DH, bool CAUSAL, bool EDGE = false>
 int launch_typed(const T* q, const T* k, const T* v, const T* g, T* dq, T* dk, T* dv, float* workspace, int B,
-                 int H, int T_len, int P, float scale, hipStream_t stream) {
+                 int H, int T_len, int P, float scale, int t_rows, int dh, hipStream_t stream) {
     constexpr size_t lds_bytes = 4 * 32 * DH * 2;
     const int n_bh = B * H;
     float* lse2 = workspace;
     float* delta = lse2 + (size_t)n_bh * T_len;
     float* o32 = delta + (size_t)n_bh * P * T_len;
     const int n_qb = (T_len + 127) / 128;
-    hipLaunchKernelGGL((stats_kernel<T, DH, CAUSAL>), dim3(grid_size(n_qb, n_bh)), dim3(256), lds_bytes, stream, q, k,
-                       v, lse2, o32, n_bh, T_len, scale);
+    hipLaunchKernelGGL((stats_kernel<T, DH, CAUSAL, EDGE>), dim3(grid_size(n_qb, n_bh)), dim3(256), lds_bytes, stream, q, k,
+                       v, lse2, o32, n_bh, T_len, scale, t_rows, dh);
     // the dQ kernel runs first: it writes -delta, which the dK/dV kernel reads
     // directions per wave of the dQ kernel: as many as share one S tile, without idle slots for one or two directions
     int rc;
-    if (P == 1) rc = launch_dq<T, DH, 1, CAUSAL>(q, k, v, g, lse2, o32, delta, dq, n_bh, H, P, T_len, scale, stream);
-    else if (P == 2) rc = launch_dq<T, DH, 2, CAUSAL>(q, k, v, g, lse2, o32, delta, dq, n_bh, H, P, T_len, scale, stream);
-    else if (DH == 64 && P > 4) rc = launch_dq<T, DH, 8, CAUSAL>(q, k, v, g, lse2, o32, delta, dq, n_bh, H, P, T_len, scale, stream);
-    else rc = launch_dq<T, DH, 4, CAUSAL>(q, k, v, g, lse2, o32, delta, dq, n_bh, H, P, T_len, scale, stream);
+    if (P == 1) rc = launch_dq<T, DH, 1, CAUSAL, EDGE>(q, k, v, g, lse2, o32, delta, dq, n_bh, H, P, T_len, scale, t_rows, dh, stream);
+    else if (P == 2) rc = launch_dq<T, DH, 2, CAUSAL, EDGE>(q, k, v, g, lse2, o32, delta, dq, n_bh, H, P, T_len, scale, t_rows, dh, stream);
+    else if (DH == 64 && P > 4) rc = launch_dq<T, DH, 8, CAUSAL, EDGE>(q, k, v, g, lse2, o32, delta, dq, n_bh, H, P, T_len, scale, t_rows, dh, stream);
+    else rc = launch_dq<T, DH, 4, CAUSAL, EDGE>(q, k, v, g, lse2, o32, delta, dq, n_bh, H, P, T_len, scale, t_rows, dh, stream);
     if (rc) return rc;
-    if (P >= 2) rc = launch_dkdv_pair<T, DH, CAUSAL>(q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, stream);
-    else rc = launch_dkdv<T, DH, CAUSAL>(q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, stream);
+    if (P >= 2) rc = launch_dkdv_pair<T, DH, CAUSAL, EDGE>(q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, t_rows, dh, stream);
+    else rc = launch_dkdv<T, DH, CAUSAL, EDGE>(q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, t_rows, dh, stream);
     if (rc) return rc;
     LBI_HIP_CHECK(hipGetLastError());
     return LBI_OK;
@@ -389,11 +432,32 @@ int launch(const void* q, const void* k, const void* v, const void* g, void* dq,
     T* dkp = static_cast<T*>(dk);
     T* dvp = static_cast<T*>(dv);
     if (dh == 128) {
-        return causal ? launch_typed<T, 128, true>(qp, kp, vp, gp, dqp, dkp, dvp, workspace, B, H, T_len, P, scale, stream)
-                      : launch_typed<T, 128, false>(qp, kp, vp, gp, dqp, dkp, dvp, workspace, B, H, T_len, P, scale, stream);
+        return causal ? launch_typed<T, 128, true>(qp, kp, vp, gp, dqp, dkp, dvp, workspace, B, H, T_len, P, scale, T_len, dh, stream)
+                      : launch_typed<T, 128, false>(qp, kp, vp, gp, dqp, dkp, dvp, workspace, B, H, T_len, P, scale, T_len, dh, stream);
     }
-    return causal ? launch_typed<T, 64, true>(qp, kp, vp, gp, dqp, dkp, dvp, workspace, B, H, T_len, P, scale, stream)
-                  : launch_typed<T, 64, false>(qp, kp, vp, gp, dqp, dkp, dvp, workspace, B, H, T_len, P, scale, stream);
+    return causal ? launch_typed<T, 64, true>(qp, kp, vp, gp, dqp, dkp, dvp, workspace, B, H, T_len, P, scale, T_len, dh, stream)
+                  : launch_typed<T, 64, false>(qp, kp, vp, gp, dqp, dkp, dvp, workspace, B, H, T_len, P, scale, T_len, dh, stream);
+}
+
+// What the EDGE forms take: lengths and head dims of causal 16-bit calls that the plain forms leave out.
+inline int edge_len(int T_len) { return (T_len + 63) / 64 * 64; }
+inline bool supports_edge(int T_len, int dh, int dtype) {
+    return (dtype == LBI_F16 || dtype == LBI_BF16) && dh >= 8 && dh <= 128 && dh % 8 == 0 && T_len >= 1;
+}
+
+template <typename T>
+int launch_edge(const void* q, const void* k, const void* v, const void* g, void* dq, void* dk, void* dv,
+                float* workspace, int B, int H, int t_rows, int dh, int P, float scale, hipStream_t stream) {
+    const T* qp = static_cast<const T*>(q);
+    const T* kp = static_cast<const T*>(k);
+    const T* vp = static_cast<const T*>(v);
+    const T* gp = static_cast<const T*>(g);
+    T* dqp = static_cast<T*>(dq);
+    T* dkp = static_cast<T*>(dk);
+    T* dvp = static_cast<T*>(dv);
+    const int T_len = edge_len(t_rows);
+    return dh > 64 ? launch_typed<T, 128, true, true>(qp, kp, vp, gp, dqp, dkp, dvp, workspace, B, H, T_len, P, scale, t_rows, dh, stream)
+                   : launch_typed<T, 64, true, true>(qp, kp, vp, gp, dqp, dkp, dvp, workspace, B, H, T_len, P, scale, t_rows, dh, stream);
 }
 
 }  // namespace attn_mfma

@@ -13,6 +13,7 @@
 //     dV = P^T dO, dK = scale dS^T Q
 // A length that is no multiple of 32 fills its last tile with zero rows: as keys they are masked out (the causal
 // mask already does that), as queries they carry a zero cotangent and add nothing; their outputs are not stored.
+// A head dim (a multiple of 8) below the tile's is filled with zero columns, which add nothing to any product.
 // Every output tile has one owner and every sum a fixed order: reruns are bit-identical.
 #pragma once
 
@@ -46,7 +47,7 @@ template <typename T, int DH, int MAX_TILES, bool CAUSAL>
 __global__ __launch_bounds__(256, (DH == 64 && MAX_TILES == 4) ? 2 : 1) void small_seq_kernel(const T* __restrict__ q, const T* __restrict__ k,
                                                         const T* __restrict__ v, const T* __restrict__ d_out,
                                                         T* __restrict__ dq, T* __restrict__ dk, T* __restrict__ dv,
-                                                        int n_bh, int H, int P, int T_len, float scale) {
+                                                        int n_bh, int H, int P, int T_len, int dh, float scale) {
     constexpr int KS = DH / 16, ND = DH / 32, TILE_BYTES = 32 * DH * 2, OPERAND_BYTES = MAX_TILES * TILE_BYTES;
     constexpr int MAX_T = 32 * MAX_TILES, OWNED = MAX_TILES / 4;
     static_assert(MAX_TILES == 4 || MAX_TILES == 8, "a wave owns one or two tiles");
@@ -64,19 +65,20 @@ __global__ __launch_bounds__(256, (DH == 64 && MAX_TILES == 4) ? 2 : 1) void sma
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int b = bh / H, hh = bh - b * H;
-    const size_t base = (size_t)bh * T_len * DH;                               // q, k, v
-    const size_t gbase = (((size_t)b * P + p) * H + hh) * (size_t)T_len * DH;  // d_out, dq, dk, dv
+    const size_t base = (size_t)bh * T_len * dh;                               // q, k, v
+    const size_t gbase = (((size_t)b * P + p) * H + hh) * (size_t)T_len * dh;  // d_out, dq, dk, dv
     const float sc2 = scale * LOG2E;
 
     {
-        // rows past the end of the sequence (last tile of a ragged length) are zero
+        // rows past the end of the sequence (last tile of a ragged length) and columns past dh are zero
         auto fetch = [&](TileLoader<DH>& ld, const T* src, int row0) __attribute__((always_inline)) {
             constexpr int CPR = DH / 8;
 #pragma unroll
             for (int u = 0; u < TileLoader<DH>::N; ++u) {
                 const int id = tid + 256 * u;
                 const int r = row0 + id / CPR, c = id % CPR;
-                ld.regs[u] = r < T_len ? *reinterpret_cast<const u32x4*>(src + (size_t)r * DH + c * 8) : u32x4{0u, 0u, 0u, 0u};
+                ld.regs[u] = r < T_len && c * 8 < dh ? *reinterpret_cast<const u32x4*>(src + (size_t)r * dh + c * 8)
+                                                     : u32x4{0u, 0u, 0u, 0u};
             }
         };
         TileLoader<DH> lq[MAX_TILES], lk[MAX_TILES], lv[MAX_TILES], lg[MAX_TILES];
@@ -175,11 +177,12 @@ __global__ __launch_bounds__(256, (DH == 64 && MAX_TILES == 4) ? 2 : 1) void sma
                 }
             }
         if (32 * qt + m < T_len) {
-            T* dq_row = dq + gbase + (size_t)(32 * qt + m) * DH;
+            T* dq_row = dq + gbase + (size_t)(32 * qt + m) * dh;
 #pragma unroll
             for (int nd = 0; nd < ND; ++nd)
 #pragma unroll
-                for (int g = 0; g < 4; ++g) store4<T>(dq_row + 32 * nd + 8 * g + 4 * h, dq_t[nd], g, scale);
+                for (int g = 0; g < 4; ++g)
+                    if (32 * nd + 8 * g + 4 * h < dh) store4<T>(dq_row + 32 * nd + 8 * g + 4 * h, dq_t[nd], g, scale);
         }
         if (h == 0) {
             lse_lds[32 * qt + m] = row_max + log2f(row_sum);
@@ -241,12 +244,13 @@ __global__ __launch_bounds__(256, (DH == 64 && MAX_TILES == 4) ? 2 : 1) void sma
             }
         }
         if (32 * kt + m < T_len) {
-            T* dk_row = dk + gbase + (size_t)(32 * kt + m) * DH;
-            T* dv_row = dv + gbase + (size_t)(32 * kt + m) * DH;
+            T* dk_row = dk + gbase + (size_t)(32 * kt + m) * dh;
+            T* dv_row = dv + gbase + (size_t)(32 * kt + m) * dh;
 #pragma unroll
             for (int nd = 0; nd < ND; ++nd)
 #pragma unroll
                 for (int g = 0; g < 4; ++g) {
+                    if (32 * nd + 8 * g + 4 * h >= dh) continue;
                     store4<T>(dk_row + 32 * nd + 8 * g + 4 * h, dk_t[nd], g, scale);
                     store4<T>(dv_row + 32 * nd + 8 * g + 4 * h, dv_t[nd], g, 1.0f);
                 }
@@ -256,14 +260,14 @@ __global__ __launch_bounds__(256, (DH == 64 && MAX_TILES == 4) ? 2 : 1) void sma
 
 template <typename T, int DH, int MAX_TILES>
 int launch_sized(const void* q, const void* k, const void* v, const void* g, void* dq, void* dk, void* dv, int B,
-                 int H, int T_len, int P, float scale, int causal, hipStream_t stream) {
+                 int H, int T_len, int dh, int P, float scale, int causal, hipStream_t stream) {
     constexpr size_t lds = lds_bytes<DH, MAX_TILES>();
     const int n_bh = B * H;
     const dim3 grid(grid_size(P, n_bh));
     auto run = [&](auto kern) {
         hipLaunchKernelGGL(kern, grid, dim3(256), lds, stream, static_cast<const T*>(q), static_cast<const T*>(k),
                            static_cast<const T*>(v), static_cast<const T*>(g), static_cast<T*>(dq), static_cast<T*>(dk),
-                           static_cast<T*>(dv), n_bh, H, P, T_len, scale);
+                           static_cast<T*>(dv), n_bh, H, P, T_len, dh, scale);
     };
     if (causal) {
         if (int rc = ensure_dynamic_lds<&small_seq_kernel<T, DH, MAX_TILES, true>>(lds)) return rc;
@@ -276,13 +280,13 @@ int launch_sized(const void* q, const void* k, const void* v, const void* g, voi
     return LBI_OK;
 }
 
-// T_len, dh as accepted by supports().
+// T_len as accepted by supports() for the tile's head dim; dh a multiple of 8 up to 128.
 template <typename T>
 int launch(const void* q, const void* k, const void* v, const void* g, void* dq, void* dk, void* dv, int B, int H,
            int T_len, int dh, int P, float scale, int causal, hipStream_t stream) {
-    if (dh == 128) return launch_sized<T, 128, 4>(q, k, v, g, dq, dk, dv, B, H, T_len, P, scale, causal, stream);
-    if (T_len <= 128) return launch_sized<T, 64, 4>(q, k, v, g, dq, dk, dv, B, H, T_len, P, scale, causal, stream);
-    return launch_sized<T, 64, 8>(q, k, v, g, dq, dk, dv, B, H, T_len, P, scale, causal, stream);
+    if (dh > 64) return launch_sized<T, 128, 4>(q, k, v, g, dq, dk, dv, B, H, T_len, dh, P, scale, causal, stream);
+    if (T_len <= 128) return launch_sized<T, 64, 4>(q, k, v, g, dq, dk, dv, B, H, T_len, dh, P, scale, causal, stream);
+    return launch_sized<T, 64, 8>(q, k, v, g, dq, dk, dv, B, H, T_len, dh, P, scale, causal, stream);
 }
 
 }  // namespace attn_small

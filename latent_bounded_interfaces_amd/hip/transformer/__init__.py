@@ -46,6 +46,35 @@ def _validate(q, k, v, output_cotangent_basis) -> None:
         raise ValueError("output_cotangent_basis must have shape [B, P, H, T, Dh] matching q/k/v")
 
 
+def _launch(q, k, v, d_out, softmax_scale, causal, dtype, edge):
+    """One call of ``lbi_attn_pullback`` or (``edge``) ``lbi_attn_pullback_edge`` on contiguous tensors."""
+    dq = torch.empty_like(d_out)
+    dk = torch.empty_like(d_out)
+    dv = torch.empty_like(d_out)
+    if d_out.numel() == 0:
+        return dq, dk, dv
+    bsz, heads, seqlen, head_dim = q.shape
+    basis = d_out.shape[1]
+    lib = _lib.load()
+    workspace_bytes, entry = ((lib.lbi_attn_pullback_edge_workspace_bytes, lib.lbi_attn_pullback_edge) if edge else
+                              (lib.lbi_attn_pullback_workspace_bytes, lib.lbi_attn_pullback))
+    with torch.cuda.device(q.device):
+        need = int(workspace_bytes(bsz, heads, seqlen, head_dim, basis, dtype))
+        # short sequences run as one launch that needs none
+        workspace = torch.empty(need, device=q.device, dtype=torch.uint8) if need > 0 else None
+        status = entry(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(),
+            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+            workspace.data_ptr() if need > 0 else None, need,
+            bsz, heads, seqlen, head_dim, basis,
+            float(softmax_scale), int(bool(causal)), dtype, _lib.current_stream_ptr(q.device),
+        )
+    _lib.check(status, "lbi_attn_pullback_edge" if edge else "lbi_attn_pullback")
+    # The workspace is only used by kernels already queued on this stream; torch's
+    # caching allocator reuses it in stream order, so releasing it here is safe.
+    return dq, dk, dv
+
+
 def attention_input_pullback_basis(
     q: torch.Tensor,
     k: torch.Tensor,
@@ -86,9 +115,9 @@ def attention_input_pullback_basis(
     wide_dim = next((w for w in _MFMA_HEAD_DIMS if w >= head_dim), head_dim)
     single_launch = seqlen <= _SINGLE_LAUNCH_MAX_SEQ.get(wide_dim, 0)
     if q.dtype in (torch.float16, torch.bfloat16) and d_out.numel() and (single_launch or seqlen > _MFMA_SEQ_MULTIPLE // 2):
-        # The matrix-core kernels take head dims 64 and 128 and sequence lengths that are multiples of 64 (short
-        # sequences, which run as a single launch, any length); everything else runs on the generic kernels, at a
-        # small fraction of their speed.  Two paddings are exact:
+        # The matrix-core kernels work on tiles of head dim 64 or 128 and 64 positions (short sequences, which run as
+        # a single launch, any length); what does not fill them is padded, since the generic kernels run at a small
+        # fraction of their speed.  Two paddings are exact:
         # * zero columns appended to the head dim add nothing to any dot product (the scale is passed explicitly)
         #   and receive zero cotangents;
         # * under the causal mask, zero rows appended after the sequence are invisible to every real query, and as
@@ -98,32 +127,15 @@ def attention_input_pullback_basis(
         long_seq = seqlen + (multiple - seqlen % multiple) if (ragged and causal) else seqlen
         if (wide_dim != head_dim or long_seq != seqlen) and long_seq % multiple == 0 \
                 and wide_dim in _MFMA_HEAD_DIMS:
+            # head dims of whole 16-byte pieces on aligned tensors: the kernels pad their tiles on chip
+            if (causal or single_launch) and head_dim % 8 == 0 and all(t.data_ptr() % 16 == 0 for t in (q, k, v, d_out)):
+                return _launch(q, k, v, d_out, softmax_scale, causal, dtype, True)
             pads = (0, wide_dim - head_dim, 0, long_seq - seqlen)
             padded = [torch.nn.functional.pad(t, pads) for t in (q, k, v, d_out)]
             outs = attention_input_pullback_basis(*padded, softmax_scale=softmax_scale, causal=causal,
                                                   use_cuda=use_cuda, kernel_mode="hip")
             return tuple(o[..., :seqlen, :head_dim].contiguous() for o in outs)
-    dq = torch.empty_like(d_out)
-    dk = torch.empty_like(d_out)
-    dv = torch.empty_like(d_out)
-    if d_out.numel() == 0:
-        return dq, dk, dv
-    lib = _lib.load()
-    with torch.cuda.device(q.device):
-        need = int(lib.lbi_attn_pullback_workspace_bytes(bsz, heads, seqlen, head_dim, basis, dtype))
-        # short sequences run as one launch that needs none
-        workspace = torch.empty(need, device=q.device, dtype=torch.uint8) if need > 0 else None
-        status = lib.lbi_attn_pullback(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), d_out.data_ptr(),
-            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-            workspace.data_ptr() if need > 0 else None, need,
-            bsz, heads, seqlen, head_dim, basis,
-            float(softmax_scale), int(bool(causal)), dtype, _lib.current_stream_ptr(q.device),
-        )
-    _lib.check(status, "lbi_attn_pullback")
-    # The workspace is only used by kernels already queued on this stream; torch's
-    # caching allocator reuses it in stream order, so releasing it here is safe.
-    return dq, dk, dv
+    return _launch(q, k, v, d_out, softmax_scale, causal, dtype, False)
 
 
 def attention_input_pullback_basis_static(

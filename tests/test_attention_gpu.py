@@ -226,6 +226,34 @@ def test_results_do_not_depend_on_how_directions_are_grouped(shape, basis, dtype
             assert torch.equal(a, b[:, lo:hi]), (name, lo, hi)
 
 
+# lengths around the tiles of 32, 64 and 128 positions and past the single launch; head dims of one to sixteen pieces
+EDGE_CASES = [((1, 2, 257, 64), 1), ((2, 3, 319, 64), 2), ((1, 3, 1000, 64), 5), ((1, 9, 385, 64), 9),
+              ((1, 2, 129, 128), 1), ((2, 1, 191, 128), 3), ((1, 2, 545, 128), 2), ((1, 2, 320, 32), 3),
+              ((2, 2, 333, 8), 4), ((1, 2, 384, 56), 1), ((1, 3, 450, 80), 11), ((1, 2, 256, 96), 4),
+              ((1, 2, 161, 120), 2), ((2, 2, 48, 32), 3), ((1, 2, 250, 40), 2), ((2, 1, 77, 96), 3), ((1, 1, 1, 72), 2)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape,basis", EDGE_CASES)
+def test_tiles_padded_on_chip_equal_padded_copies(shape, basis, dtype, device):
+    """Zero rows and columns appended by hand give the same bits: the sums are the same, in the same order."""
+    from latent_bounded_interfaces_amd.hip.transformer import attention_input_pullback_basis
+
+    gen = torch.Generator().manual_seed(31)
+    bsz, heads, seqlen, dim = shape
+    q, k, v = (torch.randn(*shape, generator=gen).to(dtype).to(device) for _ in range(3))
+    g = torch.randn(bsz, basis, *shape[1:], generator=gen).to(dtype).to(device)
+    wide = 64 if dim <= 64 else 128
+    single = seqlen <= {64: 256, 128: 128}[wide]
+    pads = (0, wide - dim, 0, 0 if single else -seqlen % 64)
+    for causal in (True, False) if single else (True,):
+        got = attention_input_pullback_basis(q, k, v, g, softmax_scale=0.2, causal=causal, kernel_mode="hip")
+        want = attention_input_pullback_basis(*(torch.nn.functional.pad(t, pads) for t in (q, k, v, g)),
+                                              softmax_scale=0.2, causal=causal, kernel_mode="hip")
+        for name, a, b in zip(("dq", "dk", "dv"), got, want):
+            assert a.shape == g.shape and torch.equal(a, b[..., :seqlen, :dim]), (name, causal)
+
+
 def test_long_context_properties(device):
     """bf16, T=4096, Dh=128, P=16 on two (b, h) slices: size-independent checks."""
     from latent_bounded_interfaces_amd.hip.transformer import attention_input_pullback_basis
