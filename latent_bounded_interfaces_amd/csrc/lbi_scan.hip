@@ -596,6 +596,87 @@ __global__ __launch_bounds__(256) void cotangent_staged_kernel(const Tin* __rest
 }
 
 // ---------------------------------------------------------------------------------------
+// Cotangent chain for widths up to 256 that neither fit the staged kernel (fp32 above d = 180) nor have rows of whole
+// 16-byte pieces.  One row at a time per wave, as the any-width kernel goes, a step is a serial chain of 13-32 memory
+// latencies.  The matrices do not depend on the chain, so a wave of the sixteen keeps its rows (4 NJ at most, NJ
+// elements per lane, each load 64 neighbouring elements) of the next matrix in flight in registers and refills each
+// as soon as it has been used, as cotangent256_kernel does; the sums of a lane are folded by a halving butterfly.
+// What is left is one CU's streaming rate, a batch element being one workgroup.
+// fp32 B=12 K=6 d=198: 173 -> 56 us.
+// ---------------------------------------------------------------------------------------
+template <typename Tin, int NJ>
+__global__ __launch_bounds__(1024) void cotangent_rows_kernel(const Tin* __restrict__ mats, const float* __restrict__ g,
+                                                              float* __restrict__ out, int K, int d) {
+    constexpr int NW = 16, R = NJ >= 3 ? 16 : 4 * NJ;  // rows of a wave
+    constexpr int SHIFT = R == 16 ? 2 : (R == 8 ? 3 : 4);  // 6 - log2 R
+    __shared__ float vbuf[2][64 * NJ];
+    const int b = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const Tin* mats_b = mats + (size_t)b * K * d * d;
+    float* out_b = out + (size_t)b * (K + 1) * d;
+    if (tid < 64 * NJ) {
+        const float val = tid < d ? g[(size_t)b * d + tid] : 0.0f;
+        vbuf[0][tid] = val;
+        vbuf[1][tid] = 0.0f;
+        if (tid < d) out_b[(size_t)K * d + tid] = val;
+    }
+    if (K == 0) return;
+    int col[NJ];  // lanes past the row read its last element; the product leaves it out
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) col[j] = min(64 * j + lane, d - 1);
+    Tin buf[R][NJ];
+    auto load_row = [&](int r, int i) __attribute__((always_inline)) {
+        const Tin* a = mats_b + (size_t)r * d * d + (size_t)min(wave + NW * i, d - 1) * d;
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) buf[i][j] = a[col[j]];
+    };
+#pragma unroll
+    for (int i = 0; i < R; ++i) load_row(K - 1, i);
+    // LDS writes visible to the workgroup; loads already in flight are not waited for
+    auto lds_barrier = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    lds_barrier();
+    int cur = 0;
+    for (int r = K - 1; r >= 0; --r) {
+        const int r_next = r > 0 ? r - 1 : 0;  // a harmless re-read at the end
+        float vv[NJ], vals[R];
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) vv[j] = vbuf[cur][64 * j + lane];
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            float acc = 0.0f;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) {
+                const float a = to_f32(buf[i][j]);
+                acc = fmaf(j < NJ - 1 || 64 * j + lane < d ? a : 0.0f, vv[j], acc);
+            }
+            vals[i] = acc;
+            load_row(r_next, i);
+        }
+        // halving butterfly: lane bit `off` keeps the upper or lower half of the rows it holds
+#pragma unroll
+        for (int n = R / 2, off = 32; n >= 1; n >>= 1, off >>= 1) {
+            const bool up = (lane & off) != 0;
+#pragma unroll
+            for (int i = 0; i < n; ++i) {
+                const float send = up ? vals[i] : vals[i + n], keep = up ? vals[i + n] : vals[i];
+                vals[i] = keep + __shfl_xor(send, off, 64);
+            }
+        }
+        float sum = vals[0];
+#pragma unroll
+        for (int off = 32 / R; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, 64);
+        const int row = wave + NW * (lane >> SHIFT);
+        if ((lane & ((1 << SHIFT) - 1)) == 0 && row < d) {
+            vbuf[cur ^ 1][row] = sum;
+            out_b[(size_t)r * d + row] = sum;
+        }
+        lds_barrier();
+        cur ^= 1;
+    }
+}
+
+// ---------------------------------------------------------------------------------------
 // Cotangent chain for d = 256, fp32: the HBM-bound case that matters.  One workgroup of
 // 8 waves per batch element; a wave takes rows wave, wave+8, ... (32 per step), one row
 // (1 KiB) per load instruction.  The matrices do not depend on the chain, so a wave keeps its
@@ -1281,6 +1362,18 @@ int launch_cotangent(const void* mats, const void* g, void* out, int B, int K, i
         if (int rc = ensure_dynamic_lds<&cotangent_staged_kernel<Tin>>(staged_bytes)) return rc;
         hipLaunchKernelGGL(kern, dim3(B), dim3(256), staged_bytes, stream, static_cast<const Tin*>(mats),
                            static_cast<const float*>(g), static_cast<float*>(out), K, d);
+        LBI_HIP_CHECK(hipGetLastError());
+        return LBI_OK;
+    }
+    if (d <= 256 && d > 16) {
+        auto run = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(B), dim3(1024), 0, stream, static_cast<const Tin*>(mats),
+                               static_cast<const float*>(g), static_cast<float*>(out), K, d);
+        };
+        if (d <= 64) run(cotangent_rows_kernel<Tin, 1>);
+        else if (d <= 128) run(cotangent_rows_kernel<Tin, 2>);
+        else if (d <= 192) run(cotangent_rows_kernel<Tin, 3>);
+        else run(cotangent_rows_kernel<Tin, 4>);
         LBI_HIP_CHECK(hipGetLastError());
         return LBI_OK;
     }

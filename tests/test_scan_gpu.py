@@ -127,6 +127,25 @@ def test_cotangent_chain_matches_oracle(shape, dtype, device):
     assert torch.equal(got.cpu(), torch.tensor(case["cotangents"]))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rank", [17, 63, 65, 127, 129, 191, 193, 198, 254, 255])
+@pytest.mark.parametrize("bsz,count", [(1, 1), (3, 9)])
+def test_cotangent_chain_rows_in_registers(rank, bsz, count, dtype, device):
+    """Widths up to 256 whose rows are no whole 16-byte pieces: edges of the 64-column blocks a lane holds."""
+    from latent_bounded_interfaces_amd.hip.interface import suffix_scan_cotangents
+
+    mats, g = oscan.make_scan_inputs(bsz, count, rank, kind="randn", seed=rank)
+    mats = mats.to(dtype)
+    mats[0, 0, 0, rank - 1] = float("inf")   # reaches the one entry that multiplies it, from the row's last column
+    out = suffix_scan_cotangents(mats.to(device), g.to(device)).cpu()
+    truth = oscan.suffix_cotangents_sequential(mats.double(), g.double())
+    assert torch.equal(out[:, count], g)
+    finite = torch.isfinite(truth)
+    assert torch.equal(torch.isinf(out), torch.isinf(truth)) and not torch.isnan(out).any()
+    scale = truth.where(finite, torch.zeros(())).abs().amax(dim=-1, keepdim=True).clamp_min(1e-30)
+    assert float(((out.double() - truth).abs() / scale)[finite].max()) <= 1e-5
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("bsz,count", [(1, 2), (3, 5), (13, 128), (64, 128), (64, 9), (65, 11)])
 def test_cotangent_chain_on_four_workgroups_per_element(bsz, count, dtype, device):
