@@ -5,6 +5,7 @@ no fallback: if it is missing or a call fails, an exception is raised.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import threading
 from pathlib import Path
@@ -156,5 +157,15 @@ def check(status: int, what: str) -> None:
         raise LbiLibraryError(f"{what} failed (status {status}): {message}")
 
 
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def device_guard(device: torch.device):
+    """``with`` this, calls go to ``device``.  Entering and leaving torch's own guard takes about 3 us, a good part of a
+    short call, so it is entered only where ``device`` (of a tensor: it has an index) is not current already."""
+    return _SAME_DEVICE if device.index == torch.cuda.current_device() else torch.cuda.device(device)
+
+
 def current_stream_ptr(device: torch.device) -> int:
-    return int(torch.cuda.current_stream(device).cuda_stream)
+    """The current stream of ``device`` (of a tensor), without building a stream object."""
+    return torch._C._cuda_getCurrentRawStream(device.index)

@@ -62,7 +62,7 @@ def suffix_scan_pullbacks(mats: torch.Tensor, *, exact_suffix: bool = False) -> 
     if out.numel() == 0:
         return out
     lib = _lib.load()
-    with torch.cuda.device(mats.device):
+    with _lib.device_guard(mats.device):
         status = lib.lbi_suffix_scan_ex(
             mats.data_ptr(), None, out.data_ptr(), None, bsz, count, rank, _lib.dtype_code(mats.dtype), _lib.LBI_F32,
             _lib.LBI_SCAN_EXACT_SUFFIX if exact_suffix else 0, _lib.current_stream_ptr(mats.device),
@@ -86,7 +86,7 @@ def suffix_scan_cotangents(mats: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
     if out.numel() == 0:
         return out
     lib = _lib.load()
-    with torch.cuda.device(mats.device):
+    with _lib.device_guard(mats.device):
         status = lib.lbi_suffix_cotangents(
             mats.data_ptr(), g32.data_ptr(), out.data_ptr(), bsz, count, rank,
             _lib.dtype_code(mats.dtype), _lib.current_stream_ptr(mats.device),
@@ -117,7 +117,7 @@ def suffix_scan_pullbacks_and_cotangents(mats: torch.Tensor, g: torch.Tensor, *,
     if out.numel() == 0:
         return out, cot
     lib = _lib.load()
-    with torch.cuda.device(mats.device):
+    with _lib.device_guard(mats.device):
         status = lib.lbi_suffix_scan_ex(
             mats.data_ptr(), g32.data_ptr(), out.data_ptr(), cot.data_ptr(), bsz, count, rank,
             _lib.dtype_code(mats.dtype), _lib.LBI_F32, _lib.LBI_SCAN_EXACT_SUFFIX if exact_suffix else 0,
@@ -143,7 +143,7 @@ def suffix_apply(suffix: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
     if out.numel() == 0:
         return out
     lib = _lib.load()
-    with torch.cuda.device(suffix.device):
+    with _lib.device_guard(suffix.device):
         status = lib.lbi_suffix_apply(suffix.data_ptr(), g32.data_ptr(), out.data_ptr(), bsz, count, rank,
                                       _lib.current_stream_ptr(suffix.device))
     _lib.check(status, "lbi_suffix_apply")
@@ -176,7 +176,7 @@ def matrix_norms(mats: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     lib = _lib.load()
     need = int(lib.lbi_matrix_norms_workspace_bytes(count, rank))
     workspace = torch.empty(max(need, 16), device=mats.device, dtype=torch.uint8)
-    with torch.cuda.device(mats.device):
+    with _lib.device_guard(mats.device):
         status = lib.lbi_matrix_norms(
             mats.data_ptr(), spectral.data_ptr(), frobenius.data_ptr(), workspace.data_ptr(), workspace.numel(),
             count, rank, _lib.dtype_code(mats.dtype), _lib.current_stream_ptr(mats.device),

@@ -58,7 +58,7 @@ def _launch(q, k, v, d_out, softmax_scale, causal, dtype, edge):
     lib = _lib.load()
     workspace_bytes, entry = ((lib.lbi_attn_pullback_edge_workspace_bytes, lib.lbi_attn_pullback_edge) if edge else
                               (lib.lbi_attn_pullback_workspace_bytes, lib.lbi_attn_pullback))
-    with torch.cuda.device(q.device):
+    with _lib.device_guard(q.device):
         need = int(workspace_bytes(bsz, heads, seqlen, head_dim, basis, dtype))
         # short sequences run as one launch that needs none
         workspace = torch.empty(need, device=q.device, dtype=torch.uint8) if need > 0 else None
@@ -163,7 +163,7 @@ def attention_input_pullback_basis_static(
         return out
     bsz, heads, seqlen, head_dim = q.shape
     lib = _lib.load()
-    with torch.cuda.device(q.device):
+    with _lib.device_guard(q.device):
         status = lib.lbi_attn_pullback_static(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), output_cotangent_basis.data_ptr(),
             out[0].data_ptr(), out[1].data_ptr(), out[2].data_ptr(),

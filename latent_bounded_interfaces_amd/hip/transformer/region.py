@@ -67,7 +67,7 @@ def rmsnorm_pullback(g_out: torch.Tensor, x: torch.Tensor, weight: torch.Tensor,
             raise ValueError("rmsnorm_pullback: g_residual must be shaped like g_out, or [B, P, 1, D]")
         res_ptr = g_residual.data_ptr()
     branch = torch.empty_like(g_out) if want_branch else None
-    with torch.cuda.device(g_out.device):
+    with _lib.device_guard(g_out.device):
         status = _lib.load().lbi_rmsnorm_pullback(
             g_out.data_ptr(), x.data_ptr(), weight.data_ptr(), res_ptr, total.data_ptr(),
             branch.data_ptr() if branch is not None else None, bsz, basis, seqlen, dim, float(eps), shared,
@@ -90,7 +90,7 @@ def gated_mlp_pullback(g_down_input: torch.Tensor, fc1_output: torch.Tensor) -> 
     shared = int(g_len == 1 and seqlen != 1)
     g_down_input, fc1_output = g_down_input.contiguous(), fc1_output.contiguous()
     out = torch.empty((bsz, basis, seqlen, 2 * hidden), device=g_down_input.device, dtype=g_down_input.dtype)
-    with torch.cuda.device(out.device):
+    with _lib.device_guard(out.device):
         status = _lib.load().lbi_gated_mlp_pullback(
             g_down_input.data_ptr(), fc1_output.data_ptr(), out.data_ptr(), bsz, basis, seqlen, hidden, shared,
             _lib.dtype_code(out.dtype), _stream(out))
@@ -106,7 +106,7 @@ def attn_heads_split(g_merged: torch.Tensor, n_heads: int, head_dim: int) -> tor
         raise ValueError("attn_heads_split: last dimension must be n_heads * head_dim")
     g_merged = g_merged.contiguous()
     out = torch.empty((bsz, basis, n_heads, seqlen, head_dim), device=g_merged.device, dtype=g_merged.dtype)
-    with torch.cuda.device(out.device):
+    with _lib.device_guard(out.device):
         status = _lib.load().lbi_attn_heads_split(g_merged.data_ptr(), out.data_ptr(), bsz, basis, seqlen, n_heads,
                                                   head_dim, _lib.dtype_code(out.dtype), _stream(out))
     _lib.check(status, "lbi_attn_heads_split")
@@ -147,7 +147,7 @@ def attn_qkv_pullback(dq: torch.Tensor, dk: torch.Tensor, dv: torch.Tensor, *, n
     dq, dk, dv = dq.contiguous(), dk.contiguous(), dv.contiguous()
     cos, sin = rope_tables(seqlen, head_dim, rope_base, dq.device)
     out = torch.empty((bsz, basis, seqlen, (heads + 2 * n_kv_heads) * head_dim), device=dq.device, dtype=dq.dtype)
-    with torch.cuda.device(out.device):
+    with _lib.device_guard(out.device):
         status = _lib.load().lbi_attn_qkv_pullback(
             dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), cos.data_ptr(), sin.data_ptr(), out.data_ptr(), bsz, basis,
             seqlen, heads, n_kv_heads, head_dim, int(bool(rope_interleaved)), _lib.dtype_code(out.dtype), _stream(out))
@@ -164,7 +164,7 @@ def causal_conv1d_pullback(g_out: torch.Tensor, weight: torch.Tensor) -> torch.T
     g_out = g_out.contiguous()
     weight = weight.to(g_out.dtype).contiguous()
     out = torch.empty_like(g_out)
-    with torch.cuda.device(out.device):
+    with _lib.device_guard(out.device):
         status = _lib.load().lbi_causal_conv1d_pullback(g_out.data_ptr(), weight.data_ptr(), out.data_ptr(),
                                                         bsz * basis, seqlen, channels, weight.shape[-1],
                                                         _lib.dtype_code(out.dtype), _stream(out))
@@ -195,7 +195,7 @@ def attn_qkv_conv_pullback(dq: torch.Tensor, dk: torch.Tensor, dv: torch.Tensor,
     weight = conv_weight.to(dq.dtype).contiguous()
     cos, sin = rope_tables(seqlen, head_dim, rope_base, dq.device)
     out = torch.empty((bsz, basis, seqlen, channels), device=dq.device, dtype=dq.dtype)
-    with torch.cuda.device(out.device):
+    with _lib.device_guard(out.device):
         status = _lib.load().lbi_attn_qkv_conv_pullback(
             dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), cos.data_ptr(), sin.data_ptr(), weight.data_ptr(),
             out.data_ptr(), bsz, basis, seqlen, heads, n_kv_heads, head_dim, int(bool(rope_interleaved)),
@@ -223,7 +223,7 @@ def rmsnorm_weight_grad(g_out: torch.Tensor, x: torch.Tensor, eps: float) -> tor
     rows = g_out.numel() // width
     out = torch.empty(width, device=g_out.device, dtype=torch.float32)
     lib = _lib.load()
-    with torch.cuda.device(out.device):
+    with _lib.device_guard(out.device):
         need = int(lib.lbi_rmsnorm_weight_grad_workspace_bytes(rows, width))
         workspace = torch.empty(max(need, 16), device=out.device, dtype=torch.uint8)
         status = lib.lbi_rmsnorm_weight_grad(g_out.data_ptr(), x.data_ptr(), out.data_ptr(), workspace.data_ptr(),
@@ -243,7 +243,7 @@ def causal_conv1d_weight_grad(g_out: torch.Tensor, x: torch.Tensor, ksize: int) 
     g_out, x = g_out.contiguous(), x.contiguous()
     out = torch.empty(channels * ksize + channels, device=g_out.device, dtype=torch.float32)
     lib = _lib.load()
-    with torch.cuda.device(out.device):
+    with _lib.device_guard(out.device):
         need = int(lib.lbi_causal_conv1d_weight_grad_workspace_bytes(bsz, seqlen, channels, ksize))
         workspace = torch.empty(max(need, 16), device=out.device, dtype=torch.uint8)
         status = lib.lbi_causal_conv1d_weight_grad(g_out.data_ptr(), x.data_ptr(), out.data_ptr(), workspace.data_ptr(),
@@ -467,11 +467,9 @@ def region_parameter_vjp_with_input_cotangent(backend: Any, cache: Any, output_c
             g_input = _pull_back_region(backend, cache, output_cotangent.unsqueeze(1), kernel_mode, by_id)[:, 0]
     else:
         g_input = output_cotangent.detach().float()
-    wanted = {id(p) for layer_cache in cache.layer_caches
-              for p in backend.backbone.blocks[layer_cache.layer_index].parameters() if p.requires_grad}
     out: dict[str, torch.Tensor] = {}
     for name, param in backend.named_parameters():
-        if id(param) in wanted and id(param) in by_id:
+        if param.requires_grad and id(param) in by_id:  # gradients were formed for the region's blocks only
             out[name] = by_id[id(param)].detach()
     return out, g_input
 
