@@ -255,7 +255,8 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
 
     // mats chunks are prefetched RING-1 chunks ahead into a register ring; the ring
     // index of a chunk is kc % RING, the same in every step because RING divides NCH.
-    constexpr int RING = (NCH % 4 == 0) ? 4 : 2;
+    constexpr int RING = NCH == 1 ? 2 : NCH % 4 == 0 ? 4 : NCH % 3 == 0 ? 3 : NCH % 2 == 0 ? 2 : NCH;
+    static_assert(NCH == 1 || NCH % RING == 0, "a chunk keeps its slot from step to step");
     constexpr int AHEAD = RING - 1;
     f32x4 a_ring[RING][RTILES][4];
     // Chunk number c (0 <= c < AHEAD) counted from the start of step r_top; when NCH == 1
@@ -1235,6 +1236,15 @@ int launch_scan(const void* mats, void* out, const void* g, void* cot, int B, in
         case 128:
             if (plan_chunks(B, K, 4, &plan)) return launch_chunked<Tin, 128, 32, 32>(mats, out, g, cot, B, K, plan, stream);
             break;
+        case 192:
+            if (plan_chunks(B, K, 6, &plan)) return launch_chunked<Tin, 192, 32, 32>(mats, out, g, cot, B, K, plan, stream);
+            break;
+        case 160:
+            if (plan_chunks(B, K, 5, &plan)) return launch_chunked<Tin, 160, 32, 32>(mats, out, g, cot, B, K, plan, stream);
+            break;
+        case 96:
+            if (plan_chunks(B, K, 3, &plan)) return launch_chunked<Tin, 96, 32, 32>(mats, out, g, cot, B, K, plan, stream);
+            break;
         case 64:
             if (plan_chunks(B, K, 2, &plan)) return launch_chunked<Tin, 64, 32, 32>(mats, out, g, cot, B, K, plan, stream);
             break;
@@ -1303,6 +1313,14 @@ int launch_scan(const void* mats, void* out, const void* g, void* cot, int B, in
             if (B >= wide_block_batch()) return launch_mfma<Tin, 64, 32, 64>(mats, out, g, cot, B, K, stream);
             return launch_mfma<Tin, 64, 32, 32>(mats, out, g, cot, B, K, stream);
         case 32: return launch_mfma<Tin, 32, 32, 32>(mats, out, g, cot, B, K, stream);
+        // Widths between the powers of two: on matrices padded to the next one they cost three copies and
+        // (128/96)^3 = 2.4, (256/160)^3 = 4.1 or (256/192)^3 = 2.4 times the products.
+        // Matrices and cotangents, whole calls, padded -> here: fp32 B=16 K=50 d=96: 0.135 -> 0.068 ms; B=64 K=128,
+        // d=96 / 160 / 192: 0.78 -> 0.36, 3.1 -> 1.4, 3.4 -> 1.6 ms.  16-bit storage gains the same at 96; bf16 at 160
+        // and 192, whose padded form runs on the 16-bit matrix cores, from 1.56 to 1.50 and 1.80 to 1.70 ms.
+        case 96: return launch_mfma<Tin, 96, 32, 32>(mats, out, g, cot, B, K, stream);
+        case 160: return launch_mfma<Tin, 160, 32, 32>(mats, out, g, cot, B, K, stream);
+        case 192: return launch_mfma<Tin, 192, 32, 32>(mats, out, g, cot, B, K, stream);
         default: break;
     }
     if (cot) {

@@ -30,7 +30,7 @@ def _validate(mats: torch.Tensor) -> tuple[int, int, int]:
 
 
 #: interface widths the matrix-core scan kernels are built for
-_MFMA_WIDTHS = (32, 64, 128, 256, 512)
+_MFMA_WIDTHS = (32, 64, 96, 128, 160, 192, 256, 512)
 
 
 def _padded_width(rank: int) -> int:
@@ -39,6 +39,11 @@ def _padded_width(rank: int) -> int:
     if rank <= 16 or rank in _MFMA_WIDTHS:
         return rank
     return next((w for w in _MFMA_WIDTHS if w > rank), rank)
+
+
+def _aligned(t: torch.Tensor, rank: int) -> torch.Tensor:
+    """Widths whose calls on a tensor off the 16-byte grid used to run on its padded copy: on a plain copy now."""
+    return t.clone() if rank in (96, 160, 192) and t.data_ptr() % 16 else t
 
 
 def suffix_scan_pullbacks(mats: torch.Tensor, *, exact_suffix: bool = False) -> torch.Tensor:
@@ -57,7 +62,7 @@ def suffix_scan_pullbacks(mats: torch.Tensor, *, exact_suffix: bool = False) -> 
         pad = width - rank
         wide = suffix_scan_pullbacks(torch.nn.functional.pad(mats, (0, pad, 0, pad)), exact_suffix=exact_suffix)
         return wide[:, :, :rank, :rank].contiguous()
-    mats = mats.contiguous()
+    mats = _aligned(mats.contiguous(), rank)
     out = torch.empty((bsz, count + 1, rank, rank), device=mats.device, dtype=torch.float32)
     if out.numel() == 0:
         return out
@@ -110,8 +115,8 @@ def suffix_scan_pullbacks_and_cotangents(mats: torch.Tensor, g: torch.Tensor, *,
                                                               torch.nn.functional.pad(g, (0, pad)),
                                                               exact_suffix=exact_suffix)
         return wide[:, :, :rank, :rank].contiguous(), wide_cot[:, :, :rank].contiguous()
-    mats = mats.contiguous()
-    g32 = g.to(device=mats.device, dtype=torch.float32).contiguous()
+    mats = _aligned(mats.contiguous(), rank)
+    g32 = _aligned(g.to(device=mats.device, dtype=torch.float32).contiguous(), rank)
     out = torch.empty((bsz, count + 1, rank, rank), device=mats.device, dtype=torch.float32)
     cot = torch.empty((bsz, count + 1, rank), device=mats.device, dtype=torch.float32)
     if out.numel() == 0:

@@ -128,6 +128,34 @@ def test_cotangent_chain_matches_oracle(shape, dtype, device):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rank", [65, 95, 96, 129, 160, 161, 191, 192, 193])
+@pytest.mark.parametrize("bsz,count", [(1, 1), (2, 2), (1, 40), (3, 13), (45, 14)])
+def test_widths_between_powers_of_two(rank, bsz, count, dtype, device):
+    """Both forms of the scan (one chain; chunks side by side) at 96, 160 and 192 columns and what is padded to them,
+    on tensors that start off the 16-byte grid too."""
+    from latent_bounded_interfaces_amd.hip.interface import suffix_scan_pullbacks, suffix_scan_pullbacks_and_cotangents
+
+    mats, g = oscan.make_scan_inputs(bsz, count, rank, kind="randn", seed=rank + count)
+    mats = mats.to(dtype).to(device)
+    off = torch.empty(mats.numel() + 1, dtype=dtype, device=device)[1:].view(mats.shape).copy_(mats)
+    g_off = torch.empty(g.numel() + 1, device=device)[1:].view(g.shape).copy_(g)
+    out, cot = suffix_scan_pullbacks_and_cotangents(mats, g.to(device))
+    out_off, cot_off = suffix_scan_pullbacks_and_cotangents(off, g_off)
+    assert torch.equal(out, out_off) and torch.equal(cot, cot_off)
+    only = suffix_scan_pullbacks(mats)
+    truth = oscan.suffix_scan_sequential(mats.cpu(), dtype=torch.float64)
+    want = oscan.suffix_cotangents_sequential(mats.cpu().double(), g.double())
+    bar = 2e-4 if dtype == torch.bfloat16 and rank > 192 else 1e-5   # bf16 at 193: the width-256 kernel's two planes
+    for result in (out, only):
+        result = result.cpu()
+        err = (result.double() - truth).abs().flatten(2).amax(2) / truth.abs().flatten(2).amax(2)
+        assert float(err.max()) <= bar
+        assert torch.equal(result[:, count], torch.eye(rank).expand(bsz, -1, -1))
+    scale = want.abs().amax(dim=-1, keepdim=True)
+    assert float(((cot.cpu().double() - want).abs() / scale).max()) <= max(bar, 3e-5)   # products applied to g
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rank", [17, 63, 65, 127, 129, 191, 193, 198, 254, 255])
 @pytest.mark.parametrize("bsz,count", [(1, 1), (3, 9)])
 def test_cotangent_chain_rows_in_registers(rank, bsz, count, dtype, device):
