@@ -165,27 +165,33 @@ __device__ __forceinline__ void load_half_row(float (&dst)[DH / 2], const float*
     }
 }
 
-// Rows and groups of a launch: workgroup id -> (row tile, group), all groups of the longest row tile first, so that the
-// short tiles of a causal call fill the end of the launch.
+// Workgroup -> (row tile, group).  The groups lie along x, which is dealt first, and the row tiles along y and z: all
+// groups of the longest row tile come first, so that the short tiles of a causal call fill the end of the launch.  A grid
+// may hold fewer than 2^32 threads along x and 65535 workgroups along y and z, so neither lies along x alone.
 struct Place {
     int tile, group;
 };
-__device__ __forceinline__ Place place(int id, int tiles, int groups, bool last_first) {
-    const int t = id / groups;
-    return {last_first ? tiles - 1 - t : t, id - t * groups};
+__device__ __forceinline__ Place place(int tiles, bool last_first) {
+    const int t = (int)(blockIdx.z * gridDim.y + blockIdx.y);  // past `tiles` in the last row of z: no work
+    return {last_first ? tiles - 1 - t : t, (int)blockIdx.x};
+}
+inline dim3 grid_of(int tiles, int groups) {
+    const int rows = tiles < 65535 ? tiles : 65535;
+    return dim3((unsigned)groups, (unsigned)rows, (unsigned)((tiles + rows - 1) / rows));
 }
 
 template <int DH, bool VEC>
 __global__ __launch_bounds__(NT) void stats_kernel(const float* __restrict__ q, const float* __restrict__ k,
                                                    const float* __restrict__ v, float* __restrict__ o_park,
                                                    float* __restrict__ lse2, int H, int P, int T_len, int dh,
-                                                   float scale, int causal, int tiles, int groups) {
+                                                   float scale, int causal, int tiles) {
     using Stage = TileStage<DH, VEC>;
     constexpr int ROWS = NWAVE * TILE;
     constexpr int PITCH = Stage::PITCH, BUF = 2 * TILE * PITCH, NB = DH / 32;
     extern __shared__ __align__(16) float lds[];  // [2][K tile, V tile]
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, h = lane >> 5, wave = tid >> 6;
-    const Place at = place(blockIdx.x, tiles, groups, causal);
+    const Place at = place(tiles, causal);
+    if (at.tile < 0 || at.tile >= tiles) return;
     const size_t base = (size_t)at.group * T_len * dh;
     const int q0 = at.tile * ROWS + wave * TILE, query = q0 + m;
     float qf[1][DH / 2];
@@ -284,14 +290,14 @@ __global__ __launch_bounds__(NT) void dq_kernel(const float* __restrict__ q, con
                                                 const float* __restrict__ v, const float* __restrict__ d_out,
                                                 const float* __restrict__ o_park, const float* __restrict__ lse2,
                                                 float* __restrict__ delta, float* __restrict__ dq, int H, int P,
-                                                int T_len, int dh, float scale, int causal, int tiles,
-                                                int groups) {
+                                                int T_len, int dh, float scale, int causal, int tiles) {
     using Stage = TileStage<DH, VEC>;
     constexpr int ROWS = NWAVE / DW * TILE;
     constexpr int PITCH = Stage::PITCH, BUF = 2 * TILE * PITCH, NB = DH / 32;
     extern __shared__ __align__(16) float lds[];  // [2][K tile, V tile]
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const Place at = place(blockIdx.x, tiles, groups, causal);
+    const Place at = place(tiles, causal);
+    if (at.tile < 0 || at.tile >= tiles) return;
     const int pgroups = (P + DW * PB - 1) / (DW * PB);
     const int head = at.group % H, b = at.group / (H * pgroups);
     const int p0 = ((at.group / H) % pgroups * DW + wave % DW) * PB;  // the wave's first direction
@@ -396,15 +402,15 @@ __global__ __launch_bounds__(NT) void dkdv_kernel(const float* __restrict__ q, c
                                                   const float* __restrict__ v, const float* __restrict__ d_out,
                                                   const float* __restrict__ lse2, const float* __restrict__ delta,
                                                   float* __restrict__ dk, float* __restrict__ dv, int H, int P,
-                                                  int T_len, int dh, float scale, int causal, int tiles,
-                                                  int groups) {
+                                                  int T_len, int dh, float scale, int causal, int tiles) {
     using Stage = TileStage<DH, VEC>;
     constexpr int PITCH = Stage::PITCH, NB = DH / 32, ROWS = NWAVE / DW * TILE;
     constexpr int ND = DW * PB;  // directions of the workgroup
     constexpr int MATS = (1 + ND) * TILE * PITCH, BUF = MATS + 2 * NT;
     extern __shared__ __align__(16) float lds[];  // [2][Q tile, ND d_out tiles, lse of the rows, ND deltas of the rows]
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const Place at = place(blockIdx.x, tiles, groups, false);  // the first keys see the most queries
+    const Place at = place(tiles, false);  // the first keys see the most queries
+    if (at.tile >= tiles) return;
     const int pgroups = (P + ND - 1) / ND;
     const int head = at.group % H, b = at.group / (H * pgroups);
     const int dir0 = (at.group / H) % pgroups * ND;                   // the workgroup's first direction
@@ -531,18 +537,19 @@ int launch_with(const Args& a) {
     static_assert(qg_bytes <= 160 * 1024 && (1 + ND) * TILE <= 2 * NT, "LDS budget");
     const int heads = a.B * a.H, groups = heads * ((a.P + ND - 1) / ND);
     const int tiles = (a.T_len + ROWS - 1) / ROWS, stat_tiles = (a.T_len + NWAVE * TILE - 1) / (NWAVE * TILE);
-    if ((double)tiles * groups > 2.0e9) return fail(LBI_ERR_UNSUPPORTED, "lbi_attn_pullback: too many row tiles");
+    if ((long long)groups * NT >= 1LL << 32)  // before the first launch: a refused call writes nothing
+        return fail(LBI_ERR_UNSUPPORTED, "lbi_attn_pullback: too many (batch, head, direction) groups for one launch");
     if (int rc = ensure_dynamic_lds<&stats_kernel<DH, VEC>>(kv_bytes)) return rc;
     if (int rc = ensure_dynamic_lds<&dq_kernel<DH, PB, DW, VEC>>(kv_bytes)) return rc;
     if (int rc = ensure_dynamic_lds<&dkdv_kernel<DH, PB, DW, VEC>>(qg_bytes)) return rc;
-    hipLaunchKernelGGL((stats_kernel<DH, VEC>), dim3((unsigned)(stat_tiles * heads)), dim3(NT), kv_bytes, a.stream,
-                       a.q, a.k, a.v, a.dk, a.lse2, a.H, a.P, a.T_len, a.dh, a.scale, a.causal, stat_tiles, heads);
-    hipLaunchKernelGGL((dq_kernel<DH, PB, DW, VEC>), dim3((unsigned)(tiles * groups)), dim3(NT), kv_bytes, a.stream,
+    hipLaunchKernelGGL((stats_kernel<DH, VEC>), grid_of(stat_tiles, heads), dim3(NT), kv_bytes, a.stream,
+                       a.q, a.k, a.v, a.dk, a.lse2, a.H, a.P, a.T_len, a.dh, a.scale, a.causal, stat_tiles);
+    hipLaunchKernelGGL((dq_kernel<DH, PB, DW, VEC>), grid_of(tiles, groups), dim3(NT), kv_bytes, a.stream,
                        a.q, a.k, a.v, a.d_out, a.dk, a.lse2, a.delta, a.dq, a.H, a.P, a.T_len, a.dh, a.scale, a.causal,
-                       tiles, groups);
-    hipLaunchKernelGGL((dkdv_kernel<DH, PB, DW, VEC>), dim3((unsigned)(tiles * groups)), dim3(NT), qg_bytes, a.stream,
+                       tiles);
+    hipLaunchKernelGGL((dkdv_kernel<DH, PB, DW, VEC>), grid_of(tiles, groups), dim3(NT), qg_bytes, a.stream,
                        a.q, a.k, a.v, a.d_out, a.lse2, a.delta, a.dk, a.dv, a.H, a.P, a.T_len, a.dh, a.scale, a.causal,
-                       tiles, groups);
+                       tiles);
     LBI_HIP_CHECK(hipGetLastError());
     return LBI_OK;
 }

@@ -124,6 +124,17 @@ def test_region_and_norm_entry_points_validate_on_the_host():
     assert f"#define LBI_ATTN_STATIC_SCRATCH_BYTES ({_lib.ATTN_STATIC_SCRATCH_BYTES >> 20}u << 20)" in header
 
 
+def test_fp32_attention_refuses_what_no_grid_holds():
+    """More groups than a grid may have threads for: refused on the host, before a kernel has written anything."""
+    lib = _lib.load()
+    one = ctypes.c_void_p(256)  # never dereferenced
+    need = lib.lbi_attn_pullback_workspace_bytes(1024, 1024, 1, 3, 64, _lib.LBI_F32)
+    assert need > 0
+    assert lib.lbi_attn_pullback(one, one, one, one, one, one, one, one, need, 1024, 1024, 1, 3, 64, 0.1, 1, _lib.LBI_F32,
+                                 None) == -2
+    assert b"groups" in lib.lbi_last_error()
+
+
 def test_wrappers_reject_bad_input_before_touching_the_device():
     import torch
 
