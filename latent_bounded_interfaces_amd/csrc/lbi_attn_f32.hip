@@ -14,18 +14,19 @@
 //     so register t of the tile IS the operand, and the other side is one 4-byte LDS read of row row(t), 32
 //     consecutive columns per lane half.  P and dS never leave the registers.
 //
-// Three kernels per call, every output with one owner and a fixed summation order (no atomics, reruns bit-identical):
-//   stats   lse2[b,h,i] (log2 domain) and O = softmax(..) V; O is parked in the dk slice of direction 0, which the
-//           last kernel overwrites, so the workspace is no larger than that of the scalar kernels
-//   dq      a wave owns 32 queries x PB directions (S^T orientation: lanes are queries); also leaves
-//           delta[b,p,h,i] = d_out . O for the next kernel
+// Four kernels per call, every output with one owner and a fixed summation order (no atomics, reruns bit-identical):
+//   stats   lse2[b,h,i] (log2 domain)
+//   delta   delta[b,p,h,i] = sum_j P dP
+//   dq      a wave owns 32 queries x PB directions (S^T orientation: lanes are queries), as in stats and delta
 //   dkdv    a wave owns 32 keys x PB directions (S orientation: lanes are keys)
 // The streamed tiles pass through two LDS buffers (the next tile waits in registers during the products of the current
 // one; one barrier per tile) and are shared by the four waves of a workgroup, which own different directions of the same
 // rows as far as there are any: under the causal mask neighbouring row tiles end at different steps and the waves of the
 // shorter ones wait (B=4 H=8 T=512 Dh=64 P=8: dq 145 -> 125 us, dkdv 189 -> 175 us against four row tiles).  Two
 // directions per wave share one S tile, at one wave per SIMD; one direction at two waves per SIMD took 176 / 201 us.
-// Whole call there: 5.43 ms on the scalar kernels (lbi_attn_generic.h), 0.333 ms here (53 TFLOP/s algorithmic).
+// Whole call there: 5.41 ms on the scalar kernels (lbi_attn_generic.h), 0.388 ms here (46 TFLOP/s algorithmic), with the
+// error of the scalar kernels: relative 2-norm against 64 bits 3.9e-7 / 6.0e-7 / 5.9e-7 in dQ / dK / dV, and 0.98 to 1.02
+// times theirs over T = 24 ... 3000, head dims 16 ... 128, V with and without an offset.
 #include "lbi_attn_f32.h"
 
 #include <initializer_list>
@@ -40,6 +41,13 @@ constexpr float LOG2E = 1.4426950408889634f;
 __device__ __forceinline__ int acc_row(int i, int h) { return 8 * (i >> 2) + 4 * h + (i & 3); }
 __device__ __forceinline__ f32x16 mma(float a, float b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
+}
+// P of a score: the product is rounded before the subtraction, as in the statistics (a fused step would leave its rounding
+// in P: with one visible key, P would not be exactly one).
+__device__ __forceinline__ float prob_of(float score, float sc2, float lse) {
+#pragma clang fp contract(off)
+    const float x = score * sc2;
+    return exp2f(x - lse);
 }
 __device__ __forceinline__ f32x16 zero16() {
     f32x16 z;
@@ -70,10 +78,10 @@ __device__ __forceinline__ void dot_form(f32x16 (&acc)[N], const float* lane_til
     }
 }
 
-// Products over the rows of accumulator tiles: acc[p][n] += x[p]^T . tile[:, 32n ...] (OUT_T: the transposed product).
+// Products over the rows of accumulator tiles: acc[p][n] += x[p]^T . tile[:, 32n ...].
 // `lane_tile` points at row 4h, column m of the tile.  `side(i)` runs in the shadow of the products of register i - 2
 // (i = 0, 1: in front of them), so it may also form x[p][i].
-template <int NB, int PITCH, int N, bool OUT_T, typename Side>
+template <int NB, int PITCH, int N, typename Side>
 __device__ __forceinline__ void chain_form(f32x16 (&acc)[N][NB], const float* lane_tile, const f32x16 (&x)[N],
                                            Side side) {
     float b[2][2][NB];   // two rows per round, two rounds
@@ -98,7 +106,7 @@ __device__ __forceinline__ void chain_form(f32x16 (&acc)[N][NB], const float* la
 #pragma unroll
                 for (int p = 0; p < N; ++p) {
                     const float t = b[(i >> 1) & 1][u][n];
-                    acc[p][n] = OUT_T ? mma(t, x[p][i + u], acc[p][n]) : mma(x[p][i + u], t, acc[p][n]);
+                    acc[p][n] = mma(x[p][i + u], t, acc[p][n]);
                 }
         if (i + 2 < 16) {
             side(i + 2);
@@ -180,15 +188,53 @@ inline dim3 grid_of(int tiles, int groups) {
     return dim3((unsigned)groups, (unsigned)rows, (unsigned)((tiles + rows - 1) / rows));
 }
 
+// N matrices streamed through LDS in tiles of 32 rows: two buffers of N tiles, the next tile in registers during the
+// products of the current one, one barrier per tile.
+template <int DH, bool VEC, int N>
+struct TileStream {
+    using Stage = TileStage<DH, VEC>;
+    static constexpr int MAT = TILE * Stage::PITCH, BUF = N * MAT;
+    static constexpr size_t LDS_BYTES = 2 * BUF * sizeof(float);
+    const float* src[N];
+    float* lds;
+    int T_len, dh, tid, steps;
+    Stage stage[N];
+    __device__ __forceinline__ void fetch(int it) {
+#pragma unroll
+        for (int n = 0; n < N; ++n) stage[n].fetch(src[n], it * TILE, T_len, dh, tid);
+    }
+    __device__ __forceinline__ void commit(int it) {
+#pragma unroll
+        for (int n = 0; n < N; ++n) stage[n].commit(lds + (it & 1) * BUF + n * MAT, it * TILE, T_len, dh, tid);
+    }
+    __device__ __forceinline__ void start() {
+        fetch(0);
+        commit(0);
+        __syncthreads();
+    }
+    __device__ __forceinline__ void begin(int it) {  // the next tile sets out
+        if (it + 1 < steps) fetch(it + 1);
+    }
+    __device__ __forceinline__ void finish(int it) {
+        if (it + 1 < steps) commit(it + 1);
+        __syncthreads();
+    }
+    __device__ __forceinline__ const float* tile(int it, int n) const { return lds + (it & 1) * BUF + n * MAT; }
+};
+
+__device__ __forceinline__ float sum16(const f32x16& x) {
+    float t[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) t[i] = (x[i] + x[i + 4]) + (x[i + 8] + x[i + 12]);
+    return (t[0] + t[1]) + (t[2] + t[3]);
+}
+
 template <int DH, bool VEC>
 __global__ __launch_bounds__(NT) void stats_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                   const float* __restrict__ v, float* __restrict__ o_park,
-                                                   float* __restrict__ lse2, int H, int P, int T_len, int dh,
-                                                   float scale, int causal, int tiles) {
-    using Stage = TileStage<DH, VEC>;
-    constexpr int ROWS = NWAVE * TILE;
-    constexpr int PITCH = Stage::PITCH, BUF = 2 * TILE * PITCH, NB = DH / 32;
-    extern __shared__ __align__(16) float lds[];  // [2][K tile, V tile]
+                                                   float* __restrict__ lse2, int T_len, int dh, float scale, int causal,
+                                                   int tiles) {
+    constexpr int ROWS = NWAVE * TILE, PITCH = TileStage<DH, VEC>::PITCH;
+    extern __shared__ __align__(16) float lds[];  // [2][K tile]
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, h = lane >> 5, wave = tid >> 6;
     const Place at = place(tiles, causal);
     if (at.tile < 0 || at.tile >= tiles) return;
@@ -196,44 +242,20 @@ __global__ __launch_bounds__(NT) void stats_kernel(const float* __restrict__ q, 
     const int q0 = at.tile * ROWS + wave * TILE, query = q0 + m;
     float qf[1][DH / 2];
     load_half_row<DH, VEC>(qf[0], q + base, query, h, T_len, dh);
-    f32x16 o_acc[1][NB];  // O^T: lanes are queries
-#pragma unroll
-    for (int n = 0; n < NB; ++n) o_acc[0][n] = zero16();
     float m_run = -INFINITY, l_run = 0.0f;
     const float sc2 = scale * LOG2E;
     const int end = causal ? min(T_len, (at.tile + 1) * ROWS) : T_len;
-    const int steps = (end + TILE - 1) / TILE;
-    Stage ks, vs;
-    ks.fetch(k + base, 0, T_len, dh, tid);
-    vs.fetch(v + base, 0, T_len, dh, tid);
-    ks.commit(lds, 0, T_len, dh, tid);
-    vs.commit(lds + TILE * PITCH, 0, T_len, dh, tid);
-    __syncthreads();
-    auto begin = [&](int it) {  // the next tile sets out
-        if (it + 1 < steps) {
-            ks.fetch(k + base, (it + 1) * TILE, T_len, dh, tid);
-            vs.fetch(v + base, (it + 1) * TILE, T_len, dh, tid);
-        }
-    };
-    auto finish = [&](int it) {
-        if (it + 1 < steps) {
-            float* next = lds + ((it + 1) & 1) * BUF;
-            ks.commit(next, (it + 1) * TILE, T_len, dh, tid);
-            vs.commit(next + TILE * PITCH, (it + 1) * TILE, T_len, dh, tid);
-        }
-        __syncthreads();
-    };
+    TileStream<DH, VEC, 1> keys{{k + base}, lds, T_len, dh, tid, (end + TILE - 1) / TILE};
+    keys.start();
     // this wave's own tiles first, then the rest of the workgroup's (no branch around the products: the accumulators
     // would be copied at its join on every step)
-    const int mine = q0 >= T_len ? 0 : causal ? min(steps, q0 / TILE + 1) : steps;
+    const int mine = q0 >= T_len ? 0 : causal ? min(keys.steps, q0 / TILE + 1) : keys.steps;
     for (int it = 0; it < mine; ++it) {
         const int j0 = it * TILE;
-        begin(it);
-        const float* kt = lds + (it & 1) * BUF;
-        const float* vt = kt + TILE * PITCH;
+        keys.begin(it);
         f32x16 ss[1] = {zero16()};
         f32x16& s = ss[0];
-        dot_form<DH, 1>(ss, kt + m * PITCH + h * (DH / 2), qf, nothing);
+        dot_form<DH, 1>(ss, keys.tile(it, 0) + m * PITCH + h * (DH / 2), qf, nothing);
         float top = m_run;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
@@ -245,82 +267,121 @@ __global__ __launch_bounds__(NT) void stats_kernel(const float* __restrict__ q, 
         // key 0 is visible to every query, so the maximum is finite from the first tile on
         const float alpha = exp2f(m_run - top);
         m_run = top;
-        l_run *= alpha;
+        // the terms of a tile in a tree of their own: the running sum rounds once per tile
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            s[i] = exp2f(s[i] - top);
-            l_run += s[i];
-        }
-#pragma unroll
-        for (int n = 0; n < NB; ++n) o_acc[0][n] *= alpha;
-        chain_form<NB, PITCH, 1, true>(o_acc, vt + 4 * h * PITCH + m, ss, nothing);
-        finish(it);
+        for (int i = 0; i < 16; ++i) s[i] = exp2f(s[i] - top);
+        l_run = l_run * alpha + sum16(s);
+        keys.finish(it);
     }
-    for (int it = mine; it < steps; ++it) {
-        begin(it);
-        finish(it);
+    for (int it = mine; it < keys.steps; ++it) {
+        keys.begin(it);
+        keys.finish(it);
     }
     if (query >= T_len) return;
     const float l_all = l_run + __shfl_xor(l_run, 32, 64);
     if (h == 0) lse2[(size_t)at.group * T_len + query] = m_run + log2f(l_all);
-    const float inv = 1.0f / l_all;
-    const int b = at.group / H, head = at.group - b * H;
-    float* o_row = o_park + (((size_t)b * P * H + head) * T_len + query) * dh;
-#pragma unroll
-    for (int n = 0; n < NB; ++n)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-            const int c = 32 * n + 8 * g + 4 * h;
-            const f32x4 v4 = {o_acc[0][n][4 * g] * inv, o_acc[0][n][4 * g + 1] * inv, o_acc[0][n][4 * g + 2] * inv,
-                              o_acc[0][n][4 * g + 3] * inv};
-            if constexpr (VEC) {
-                if (c < dh) *reinterpret_cast<f32x4*>(o_row + c) = v4;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (c + e < dh) o_row[c + e] = v4[e];
-            }
-        }
 }
 
-// DW of the four waves own different direction groups of the same rows, 4 / DW different row tiles.  A group of the
-// launch is (b, DW * PB directions, head); directions past P in the last group compute on zeros and store nothing.
+// The wave's share of a dq or delta launch.  DW of the four waves own different direction groups of the same rows, 4 / DW
+// different row tiles.  A group of the launch is (b, DW * PB directions, head); directions past P in the last group compute
+// on zeros and store nothing.
+template <int PB, int DW> struct QueryShare {
+    int head, b, p0, q0;
+    size_t kv;  // first row of (b, head) in units of rows
+    __device__ __forceinline__ QueryShare(const Place& at, int wave, int H, int P, int T_len) {
+        const int pgroups = (P + DW * PB - 1) / (DW * PB);
+        head = at.group % H;
+        b = at.group / (H * pgroups);
+        p0 = ((at.group / H) % pgroups * DW + wave % DW) * PB;  // the wave's first direction
+        kv = ((size_t)b * H + head) * T_len;
+        q0 = at.tile * (NWAVE / DW * TILE) + wave / DW * TILE;
+    }
+    __device__ __forceinline__ size_t row_of(int p, int H, int P, int T_len) const {  // first row of (b, direction, head)
+        return (((size_t)b * P + min(p0 + p, P - 1)) * H + head) * T_len;
+    }
+};
+
+// delta[b,p,h,i] = sum_j P_ij dP_ij from the very P and dP that the next two kernels subtract it from, so that their
+// rounding cancels as far as it can (one visible key: dS is exactly zero).  Taken as d_out . O, with O from the statistics
+// kernel, it saves these products (the whole call above 0.330 ms), but the error of dQ is 1.04 to 1.14 times as large, and
+// with an offset in V up to 1.9 times.
 template <int DH, int PB, int DW, bool VEC>
-__global__ __launch_bounds__(NT) void dq_kernel(const float* __restrict__ q, const float* __restrict__ k,
-                                                const float* __restrict__ v, const float* __restrict__ d_out,
-                                                const float* __restrict__ o_park, const float* __restrict__ lse2,
-                                                float* __restrict__ delta, float* __restrict__ dq, int H, int P,
-                                                int T_len, int dh, float scale, int causal, int tiles) {
-    using Stage = TileStage<DH, VEC>;
-    constexpr int ROWS = NWAVE / DW * TILE;
-    constexpr int PITCH = Stage::PITCH, BUF = 2 * TILE * PITCH, NB = DH / 32;
+__global__ __launch_bounds__(NT) void delta_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                                                   const float* __restrict__ v, const float* __restrict__ d_out,
+                                                   const float* __restrict__ lse2, float* __restrict__ delta, int H, int P,
+                                                   int T_len, int dh, float scale, int causal, int tiles) {
+    constexpr int ROWS = NWAVE / DW * TILE, PITCH = TileStage<DH, VEC>::PITCH;
     extern __shared__ __align__(16) float lds[];  // [2][K tile, V tile]
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const Place at = place(tiles, causal);
     if (at.tile < 0 || at.tile >= tiles) return;
-    const int pgroups = (P + DW * PB - 1) / (DW * PB);
-    const int head = at.group % H, b = at.group / (H * pgroups);
-    const int p0 = ((at.group / H) % pgroups * DW + wave % DW) * PB;  // the wave's first direction
-    const size_t rows = (size_t)T_len, kv_base = ((size_t)b * H + head) * rows * dh;
-    const int q0 = at.tile * ROWS + wave / DW * TILE, query = q0 + m;
-    float qf[1][DH / 2], gf[PB][DH / 2], dl[PB];
-    load_half_row<DH, VEC>(qf[0], q + kv_base, query, h, T_len, dh);
-    {
-        float of[DH / 2];
-        load_half_row<DH, VEC>(of, o_park + ((size_t)b * P * H + head) * rows * dh, query, h, T_len, dh);
+    const QueryShare<PB, DW> own(at, wave, H, P, T_len);
+    const int query = own.q0 + m;
+    float qf[1][DH / 2], gf[PB][DH / 2], sum[PB];
+    load_half_row<DH, VEC>(qf[0], q + own.kv * dh, query, h, T_len, dh);
+#pragma unroll
+    for (int p = 0; p < PB; ++p) {
+        load_half_row<DH, VEC>(gf[p], d_out + own.row_of(p, H, P, T_len) * dh, query, h, T_len, dh, own.p0 + p < P);
+        sum[p] = 0.0f;
+    }
+    const float my_lse = query < T_len ? lse2[own.kv + query] : INFINITY;
+    const float sc2 = scale * LOG2E;
+    const int end = causal ? min(T_len, (at.tile + 1) * ROWS) : T_len;
+    TileStream<DH, VEC, 2> keys{{k + own.kv * dh, v + own.kv * dh}, lds, T_len, dh, tid, (end + TILE - 1) / TILE};
+    keys.start();
+    const int mine = own.q0 >= T_len ? 0 : causal ? min(keys.steps, own.q0 / TILE + 1) : keys.steps;
+    const int last_key = causal ? min(query, T_len - 1) : T_len - 1;
+    for (int it = 0; it < mine; ++it) {
+        keys.begin(it);
+        f32x16 ss[1] = {zero16()}, dp[PB];
+#pragma unroll
+        for (int p = 0; p < PB; ++p) dp[p] = zero16();
+        dot_form<DH, 1>(ss, keys.tile(it, 0) + m * PITCH + h * (DH / 2), qf, nothing);
+        f32x16& prob = ss[0];
+        dot_form<DH, PB>(dp, keys.tile(it, 1) + m * PITCH + h * (DH / 2), gf, [&](int i) __attribute__((always_inline)) {
+            prob[i] = prob_of(prob[i], sc2, my_lse);
+        });
 #pragma unroll
         for (int p = 0; p < PB; ++p) {
-            const bool live = p0 + p < P;
-            const size_t bph = ((size_t)b * P + min(p0 + p, P - 1)) * H + head;
-            load_half_row<DH, VEC>(gf[p], d_out + bph * rows * dh, query, h, T_len, dh, live);
-            float acc = 0.0f;
 #pragma unroll
-            for (int t = 0; t < DH / 2; ++t) acc = fmaf(gf[p][t], of[t], acc);
-            dl[p] = acc + __shfl_xor(acc, 32, 64);
-            if (live && h == 0 && query < T_len) delta[bph * rows + query] = dl[p];
+            for (int i = 0; i < 16; ++i) dp[p][i] = it * TILE + acc_row(i, h) <= last_key ? prob[i] * dp[p][i] : 0.0f;
+            sum[p] += sum16(dp[p]);
         }
+        keys.finish(it);
     }
-    const float my_lse = query < T_len ? lse2[((size_t)b * H + head) * rows + query] : INFINITY;  // P = 0 past the end
+    for (int it = mine; it < keys.steps; ++it) {
+        keys.begin(it);
+        keys.finish(it);
+    }
+#pragma unroll
+    for (int p = 0; p < PB; ++p) {
+        const float all = sum[p] + __shfl_xor(sum[p], 32, 64);
+        if (own.p0 + p < P && h == 0 && query < T_len) delta[own.row_of(p, H, P, T_len) + query] = all;
+    }
+}
+
+template <int DH, int PB, int DW, bool VEC>
+__global__ __launch_bounds__(NT) void dq_kernel(const float* __restrict__ q, const float* __restrict__ k,
+                                                const float* __restrict__ v, const float* __restrict__ d_out,
+                                                const float* __restrict__ lse2, const float* __restrict__ delta,
+                                                float* __restrict__ dq, int H, int P, int T_len, int dh, float scale,
+                                                int causal, int tiles) {
+    constexpr int ROWS = NWAVE / DW * TILE, PITCH = TileStage<DH, VEC>::PITCH, NB = DH / 32;
+    extern __shared__ __align__(16) float lds[];  // [2][K tile, V tile]
+    const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const Place at = place(tiles, causal);
+    if (at.tile < 0 || at.tile >= tiles) return;
+    const QueryShare<PB, DW> own(at, wave, H, P, T_len);
+    const int q0 = own.q0, query = q0 + m;
+    float qf[1][DH / 2], gf[PB][DH / 2], dl[PB];
+    load_half_row<DH, VEC>(qf[0], q + own.kv * dh, query, h, T_len, dh);
+#pragma unroll
+    for (int p = 0; p < PB; ++p) {
+        const size_t row = own.row_of(p, H, P, T_len);
+        load_half_row<DH, VEC>(gf[p], d_out + row * dh, query, h, T_len, dh, own.p0 + p < P);
+        dl[p] = delta[row + min(query, T_len - 1)];
+    }
+    const float my_lse = query < T_len ? lse2[own.kv + query] : INFINITY;  // P = 0 past the end
     f32x16 acc[PB][NB];
 #pragma unroll
     for (int p = 0; p < PB; ++p)
@@ -328,43 +389,23 @@ __global__ __launch_bounds__(NT) void dq_kernel(const float* __restrict__ q, con
         for (int n = 0; n < NB; ++n) acc[p][n] = zero16();
     const float sc2 = scale * LOG2E;
     const int end = causal ? min(T_len, (at.tile + 1) * ROWS) : T_len;
-    const int steps = (end + TILE - 1) / TILE;
-    Stage ks, vs;
-    ks.fetch(k + kv_base, 0, T_len, dh, tid);
-    vs.fetch(v + kv_base, 0, T_len, dh, tid);
-    ks.commit(lds, 0, T_len, dh, tid);
-    vs.commit(lds + TILE * PITCH, 0, T_len, dh, tid);
-    __syncthreads();
-    auto begin = [&](int it) {  // the next tile sets out
-        if (it + 1 < steps) {
-            ks.fetch(k + kv_base, (it + 1) * TILE, T_len, dh, tid);
-            vs.fetch(v + kv_base, (it + 1) * TILE, T_len, dh, tid);
-        }
-    };
-    auto finish = [&](int it) {
-        if (it + 1 < steps) {
-            float* next = lds + ((it + 1) & 1) * BUF;
-            ks.commit(next, (it + 1) * TILE, T_len, dh, tid);
-            vs.commit(next + TILE * PITCH, (it + 1) * TILE, T_len, dh, tid);
-        }
-        __syncthreads();
-    };
+    TileStream<DH, VEC, 2> keys{{k + own.kv * dh, v + own.kv * dh}, lds, T_len, dh, tid, (end + TILE - 1) / TILE};
+    keys.start();
     // this wave's own tiles first, then the rest of the workgroup's (no branch around the products: the accumulators
     // would be copied at its join on every step)
-    const int mine = q0 >= T_len ? 0 : causal ? min(steps, q0 / TILE + 1) : steps;
+    const int mine = q0 >= T_len ? 0 : causal ? min(keys.steps, q0 / TILE + 1) : keys.steps;
     for (int it = 0; it < mine; ++it) {
         const int j0 = it * TILE;
-        begin(it);
-        const float* kt = lds + (it & 1) * BUF;
-        const float* vt = kt + TILE * PITCH;
+        keys.begin(it);
+        const float* kt = keys.tile(it, 0);
         f32x16 ss[1] = {zero16()}, dp[PB];
 #pragma unroll
         for (int p = 0; p < PB; ++p) dp[p] = zero16();
         dot_form<DH, 1>(ss, kt + m * PITCH + h * (DH / 2), qf, nothing);
         const bool masked = (causal && j0 + TILE - 1 > q0) || j0 + TILE > T_len;  // the same in all lanes
         f32x16& prob = ss[0];
-        dot_form<DH, PB>(dp, vt + m * PITCH + h * (DH / 2), gf, [&](int i) __attribute__((always_inline)) {
-            prob[i] = exp2f(prob[i] * sc2 - my_lse);
+        dot_form<DH, PB>(dp, keys.tile(it, 1) + m * PITCH + h * (DH / 2), gf, [&](int i) __attribute__((always_inline)) {
+            prob[i] = prob_of(prob[i], sc2, my_lse);
         });
         if (masked) {
 #pragma unroll
@@ -373,20 +414,20 @@ __global__ __launch_bounds__(NT) void dq_kernel(const float* __restrict__ q, con
                 if (key >= T_len || (causal && key > query)) prob[i] = 0.0f;
             }
         }
-        chain_form<NB, PITCH, PB, false>(acc, kt + 4 * h * PITCH + m, dp, [&](int i) __attribute__((always_inline)) {
+        chain_form<NB, PITCH, PB>(acc, kt + 4 * h * PITCH + m, dp, [&](int i) __attribute__((always_inline)) {
 #pragma unroll
             for (int p = 0; p < PB; ++p) dp[p][i] = prob[i] * (dp[p][i] - dl[p]);
         });
-        finish(it);
+        keys.finish(it);
     }
-    for (int it = mine; it < steps; ++it) {
-        begin(it);
-        finish(it);
+    for (int it = mine; it < keys.steps; ++it) {
+        keys.begin(it);
+        keys.finish(it);
     }
 #pragma unroll
     for (int p = 0; p < PB; ++p) {
-        if (p0 + p >= P) break;
-        float* out = dq + (((size_t)b * P + p0 + p) * H + head) * rows * dh;
+        if (own.p0 + p >= P) break;
+        float* out = dq + own.row_of(p, H, P, T_len) * dh;
 #pragma unroll
         for (int n = 0; n < NB; ++n)
 #pragma unroll
@@ -487,7 +528,7 @@ __global__ __launch_bounds__(NT) void dkdv_kernel(const float* __restrict__ q, c
             f32x16& dp = dps[0];
             if (p == 0)
                 dot_form<DH, 1>(dps, gt + m * PITCH + h * (DH / 2), vf, [&](int i) __attribute__((always_inline)) {
-                    s[i] = exp2f(s[i] * sc2 - lse4[i >> 2][i & 3]);
+                    s[i] = prob_of(s[i], sc2, lse4[i >> 2][i & 3]);
                     if (masked && key > i0 + acc_row(i, h)) s[i] = 0.0f;
                 });
             else
@@ -496,10 +537,10 @@ __global__ __launch_bounds__(NT) void dkdv_kernel(const float* __restrict__ q, c
 #pragma unroll
             for (int g = 0; g < 4; ++g)
                 d4[g] = *reinterpret_cast<const f32x4*>(stat + (1 + d0 + p) * TILE + 8 * g + 4 * h);
-            chain_form<NB, PITCH, 1, false>(acc_v[p], gt + 4 * h * PITCH + m, ss, [&](int i) __attribute__((always_inline)) {
+            chain_form<NB, PITCH, 1>(acc_v[p], gt + 4 * h * PITCH + m, ss, [&](int i) __attribute__((always_inline)) {
                 dp[i] = s[i] * (dp[i] - d4[i >> 2][i & 3]);
             });
-            chain_form<NB, PITCH, 1, false>(acc_k[p], qt + 4 * h * PITCH + m, dps, nothing);
+            chain_form<NB, PITCH, 1>(acc_k[p], qt + 4 * h * PITCH + m, dps, nothing);
         }
         if (it + 1 < steps) commit(it + 1);
         __syncthreads();
@@ -532,21 +573,23 @@ struct Args {
 template <int DH, int PB, int DW, bool VEC>
 int launch_with(const Args& a) {
     constexpr int PITCH = TileStage<DH, VEC>::PITCH, ROWS = NWAVE / DW * TILE, ND = DW * PB;
-    constexpr size_t kv_bytes = (size_t)4 * TILE * PITCH * sizeof(float);
+    constexpr size_t k_bytes = TileStream<DH, VEC, 1>::LDS_BYTES, kv_bytes = TileStream<DH, VEC, 2>::LDS_BYTES;
     constexpr size_t qg_bytes = (size_t)2 * ((1 + ND) * TILE * PITCH + 2 * NT) * sizeof(float);
     static_assert(qg_bytes <= 160 * 1024 && (1 + ND) * TILE <= 2 * NT, "LDS budget");
     const int heads = a.B * a.H, groups = heads * ((a.P + ND - 1) / ND);
     const int tiles = (a.T_len + ROWS - 1) / ROWS, stat_tiles = (a.T_len + NWAVE * TILE - 1) / (NWAVE * TILE);
     if ((long long)groups * NT >= 1LL << 32)  // before the first launch: a refused call writes nothing
         return fail(LBI_ERR_UNSUPPORTED, "lbi_attn_pullback: too many (batch, head, direction) groups for one launch");
-    if (int rc = ensure_dynamic_lds<&stats_kernel<DH, VEC>>(kv_bytes)) return rc;
+    if (int rc = ensure_dynamic_lds<&stats_kernel<DH, VEC>>(k_bytes)) return rc;
+    if (int rc = ensure_dynamic_lds<&delta_kernel<DH, PB, DW, VEC>>(kv_bytes)) return rc;
     if (int rc = ensure_dynamic_lds<&dq_kernel<DH, PB, DW, VEC>>(kv_bytes)) return rc;
     if (int rc = ensure_dynamic_lds<&dkdv_kernel<DH, PB, DW, VEC>>(qg_bytes)) return rc;
-    hipLaunchKernelGGL((stats_kernel<DH, VEC>), grid_of(stat_tiles, heads), dim3(NT), kv_bytes, a.stream,
-                       a.q, a.k, a.v, a.dk, a.lse2, a.H, a.P, a.T_len, a.dh, a.scale, a.causal, stat_tiles);
-    hipLaunchKernelGGL((dq_kernel<DH, PB, DW, VEC>), grid_of(tiles, groups), dim3(NT), kv_bytes, a.stream,
-                       a.q, a.k, a.v, a.d_out, a.dk, a.lse2, a.delta, a.dq, a.H, a.P, a.T_len, a.dh, a.scale, a.causal,
-                       tiles);
+    hipLaunchKernelGGL((stats_kernel<DH, VEC>), grid_of(stat_tiles, heads), dim3(NT), k_bytes, a.stream, a.q, a.k,
+                       a.lse2, a.T_len, a.dh, a.scale, a.causal, stat_tiles);
+    hipLaunchKernelGGL((delta_kernel<DH, PB, DW, VEC>), grid_of(tiles, groups), dim3(NT), kv_bytes, a.stream, a.q, a.k, a.v,
+                       a.d_out, a.lse2, a.delta, a.H, a.P, a.T_len, a.dh, a.scale, a.causal, tiles);
+    hipLaunchKernelGGL((dq_kernel<DH, PB, DW, VEC>), grid_of(tiles, groups), dim3(NT), kv_bytes, a.stream, a.q, a.k, a.v,
+                       a.d_out, a.lse2, a.delta, a.dq, a.H, a.P, a.T_len, a.dh, a.scale, a.causal, tiles);
     hipLaunchKernelGGL((dkdv_kernel<DH, PB, DW, VEC>), grid_of(tiles, groups), dim3(NT), qg_bytes, a.stream,
                        a.q, a.k, a.v, a.d_out, a.lse2, a.delta, a.dk, a.dv, a.H, a.P, a.T_len, a.dh, a.scale, a.causal,
                        tiles);
@@ -576,7 +619,7 @@ int launch(const void* q, const void* k, const void* v, const void* d_out, void*
                  static_cast<float*>(dv), workspace, workspace + (size_t)B * H * T_len, B, H, T_len, dh, P, causal,
                  scale, stream};
     uintptr_t bits = 0;
-    for (const void* p : {q, k, v, d_out, (const void*)dk}) bits |= reinterpret_cast<uintptr_t>(p);
+    for (const void* p : {q, k, v, d_out}) bits |= reinterpret_cast<uintptr_t>(p);
     if (dh % 4 != 0 || bits % 16 != 0) {
         if (dh <= 32) return launch_with<32, 1, 1, false>(a);
         if (dh <= 64) return launch_with<64, 1, 1, false>(a);

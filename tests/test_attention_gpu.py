@@ -93,6 +93,24 @@ def test_fp32_tile_edges_against_fp64(shape, basis, causal, device):
         assert err <= bound, (name, err, bound)
 
 
+@pytest.mark.parametrize("shape,basis", [((1, 2, 1, 64), 1), ((1, 2, 70, 64), 3), ((2, 1, 33, 33), 2), ((1, 1, 130, 128), 2),
+                                         ((1, 2, 40, 16), 9)])
+def test_fp32_rounding_of_delta_cancels(shape, basis, device):
+    """delta is summed from the same P and dP that it is subtracted from.  With one visible key dS is exactly zero; so it is
+    with zero keys and one value row repeated over a power of two of positions, where P dP sums without rounding."""
+    q, k, v, g = oattn.make_attention_inputs(*shape, basis, dtype=torch.float32, seed=shape[2])
+    dq, dk, _ = _run(q, k, v + 10.0, g, device, scale=0.3, causal=True)
+    assert torch.equal(dq[:, :, :, 0], torch.zeros_like(dq[:, :, :, 0]))
+    if shape[2] == 1:
+        assert torch.equal(dk, torch.zeros_like(dk))
+    rows = 64
+    q, g = (torch.randn(*lead, shape[1], rows, shape[3], generator=torch.Generator().manual_seed(rows))
+            for lead in ((shape[0],), (shape[0], basis)))
+    v = v[:, :, :1].expand(-1, -1, rows, -1).contiguous()
+    _, dk, _ = _run(q, torch.zeros_like(q), v, g, device, scale=0.3, causal=False)
+    assert torch.equal(dk, torch.zeros_like(dk))
+
+
 # 16-bit storage: the MFMA kernels (T % 64 == 0, Dh in {64, 128}; one fused launch for Dh = 64, T <= 128) and the
 # generic ones otherwise.
 # (121, (1, 2, 16, 64), P) are the reference's fp16 cases (tests/test_cuda_attention_pullback.py:178-243);
