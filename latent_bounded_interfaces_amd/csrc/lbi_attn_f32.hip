@@ -24,12 +24,13 @@
 // rows as far as there are any: under the causal mask neighbouring row tiles end at different steps and the waves of the
 // shorter ones wait (B=4 H=8 T=512 Dh=64 P=8: dq 145 -> 125 us, dkdv 189 -> 175 us against four row tiles).  Two
 // directions per wave share one S tile, at one wave per SIMD; one direction at two waves per SIMD took 176 / 201 us.
-// Whole call there: 5.41 ms on the scalar kernels (lbi_attn_generic.h), 0.388 ms here (46 TFLOP/s algorithmic), with the
+// Whole call there: 5.41 ms on the scalar kernels (lbi_attn_generic.h), 0.393 ms here (45 TFLOP/s algorithmic), with the
 // error of the scalar kernels: relative 2-norm against 64 bits 3.9e-7 / 6.0e-7 / 5.9e-7 in dQ / dK / dV, and 0.98 to 1.02
 // times theirs over T = 24 ... 3000, head dims 16 ... 128, V with and without an offset.
 #include "lbi_attn_f32.h"
 
 #include <initializer_list>
+#include <type_traits>
 
 namespace lbi {
 namespace attn_f32 {
@@ -116,6 +117,46 @@ __device__ __forceinline__ void chain_form(f32x16 (&acc)[N][NB], const float* la
 }
 constexpr auto nothing = [](int) __attribute__((always_inline)) {};
 
+// The tile on the diagonal: rows that an output row may not see have x = 0, but zero times a value that is not finite is
+// NaN.  If that has happened (acc, zero before the tile, holds something that is not finite), the products are repeated one
+// tile row at a time and taken over only where `sees(output row, tile row)`.  `lane_tile` points at row 0, column m.
+template <int NB, int PITCH, int N, typename Sees>
+__device__ __forceinline__ void mend_diagonal(f32x16 (&acc)[N][NB], const float* lane_tile, const f32x16 (&x)[N], int h,
+                                              Sees sees) {
+    float probe = 0.0f;
+#pragma unroll
+    for (int p = 0; p < N; ++p)
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) probe = fmaf(acc[p][n][r], 0.0f, probe);
+    if (!__any(probe != 0.0f)) return;
+#pragma unroll
+    for (int p = 0; p < N; ++p)
+#pragma unroll
+        for (int n = 0; n < NB; ++n) acc[p][n] = zero16();
+#pragma unroll 1
+    for (int row = 0; row < TILE; ++row) {
+        const int i = 4 * (row >> 3) + (row & 3);  // register and lane half that hold x of this row
+        const bool mine = h == ((row >> 2) & 1);
+        float b[NB];
+#pragma unroll
+        for (int n = 0; n < NB; ++n) b[n] = mine ? lane_tile[row * PITCH + 32 * n] : 0.0f;
+#pragma unroll
+        for (int p = 0; p < N; ++p) {
+            float a = 0.0f;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) a = mine && e == i ? x[p][e] : a;
+#pragma unroll
+            for (int n = 0; n < NB; ++n) {
+                const f32x16 sum = mma(a, b[n], acc[p][n]);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[p][n][r] = sees(acc_row(r, h), row) ? sum[r] : acc[p][n][r];
+            }
+        }
+    }
+}
+
 // Four consecutive elements of a row-major [T, dh] matrix from (row, c), zero outside it.  The load itself is never
 // predicated: it reads a clamped address and `keep` says whether the value counts, so that nothing waits for a load
 // before its value is needed (a load under a branch is waited for at the join).  VEC: dh is a multiple of four and the
@@ -188,9 +229,9 @@ inline dim3 grid_of(int tiles, int groups) {
     return dim3((unsigned)groups, (unsigned)rows, (unsigned)((tiles + rows - 1) / rows));
 }
 
-// N matrices streamed through LDS in tiles of 32 rows: two buffers of N tiles, the next tile in registers during the
-// products of the current one, one barrier per tile.
-template <int DH, bool VEC, int N>
+// N matrices streamed through LDS in tiles of 32 rows, STEP +1 from the first to the last, -1 backwards: two buffers of N
+// tiles, the next tile in registers during the products of the current one, one barrier per tile.
+template <int DH, bool VEC, int N, int STEP = 1>
 struct TileStream {
     using Stage = TileStage<DH, VEC>;
     static constexpr int MAT = TILE * Stage::PITCH, BUF = N * MAT;
@@ -208,15 +249,17 @@ struct TileStream {
         for (int n = 0; n < N; ++n) stage[n].commit(lds + (it & 1) * BUF + n * MAT, it * TILE, T_len, dh, tid);
     }
     __device__ __forceinline__ void start() {
-        fetch(0);
-        commit(0);
+        const int it = STEP > 0 ? 0 : steps - 1;
+        fetch(it);
+        commit(it);
         __syncthreads();
     }
+    __device__ __forceinline__ bool more(int it) const { return STEP > 0 ? it + 1 < steps : it > 0; }
     __device__ __forceinline__ void begin(int it) {  // the next tile sets out
-        if (it + 1 < steps) fetch(it + 1);
+        if (more(it)) fetch(it + STEP);
     }
     __device__ __forceinline__ void finish(int it) {
-        if (it + 1 < steps) commit(it + 1);
+        if (more(it)) commit(it + STEP);
         __syncthreads();
     }
     __device__ __forceinline__ const float* tile(int it, int n) const { return lds + (it & 1) * BUF + n * MAT; }
@@ -264,12 +307,12 @@ __global__ __launch_bounds__(NT) void stats_kernel(const float* __restrict__ q, 
             top = fmaxf(top, s[i]);
         }
         top = fmaxf(top, __shfl_xor(top, 32, 64));
-        // key 0 is visible to every query, so the maximum is finite from the first tile on
-        const float alpha = exp2f(m_run - top);
+        const float base2 = top == -INFINITY ? 0.0f : top;  // scores of -inf only so far: their terms are 0
+        const float alpha = exp2f(m_run - base2);
         m_run = top;
         // the terms of a tile in a tree of their own: the running sum rounds once per tile
 #pragma unroll
-        for (int i = 0; i < 16; ++i) s[i] = exp2f(s[i] - top);
+        for (int i = 0; i < 16; ++i) s[i] = exp2f(s[i] - base2);
         l_run = l_run * alpha + sum16(s);
         keys.finish(it);
     }
@@ -389,40 +432,44 @@ __global__ __launch_bounds__(NT) void dq_kernel(const float* __restrict__ q, con
         for (int n = 0; n < NB; ++n) acc[p][n] = zero16();
     const float sc2 = scale * LOG2E;
     const int end = causal ? min(T_len, (at.tile + 1) * ROWS) : T_len;
-    TileStream<DH, VEC, 2> keys{{k + own.kv * dh, v + own.kv * dh}, lds, T_len, dh, tid, (end + TILE - 1) / TILE};
+    // from the diagonal backwards: the one tile with keys that some query may not see comes first, on empty sums
+    TileStream<DH, VEC, 2, -1> keys{{k + own.kv * dh, v + own.kv * dh}, lds, T_len, dh, tid, (end + TILE - 1) / TILE};
     keys.start();
-    // this wave's own tiles first, then the rest of the workgroup's (no branch around the products: the accumulators
-    // would be copied at its join on every step)
-    const int mine = q0 >= T_len ? 0 : causal ? min(keys.steps, q0 / TILE + 1) : keys.steps;
-    for (int it = 0; it < mine; ++it) {
-        const int j0 = it * TILE;
+    auto step = [&](int it, auto first) __attribute__((always_inline)) {
         keys.begin(it);
         const float* kt = keys.tile(it, 0);
         f32x16 ss[1] = {zero16()}, dp[PB];
 #pragma unroll
         for (int p = 0; p < PB; ++p) dp[p] = zero16();
         dot_form<DH, 1>(ss, kt + m * PITCH + h * (DH / 2), qf, nothing);
-        const bool masked = (causal && j0 + TILE - 1 > q0) || j0 + TILE > T_len;  // the same in all lanes
         f32x16& prob = ss[0];
         dot_form<DH, PB>(dp, keys.tile(it, 1) + m * PITCH + h * (DH / 2), gf, [&](int i) __attribute__((always_inline)) {
             prob[i] = prob_of(prob[i], sc2, my_lse);
         });
-        if (masked) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const int key = j0 + acc_row(i, h);
-                if (key >= T_len || (causal && key > query)) prob[i] = 0.0f;
-            }
-        }
+        const int last_key = (causal ? min(query, T_len - 1) : T_len - 1) - it * TILE;
         chain_form<NB, PITCH, PB>(acc, kt + 4 * h * PITCH + m, dp, [&](int i) __attribute__((always_inline)) {
 #pragma unroll
-            for (int p = 0; p < PB; ++p) dp[p][i] = prob[i] * (dp[p][i] - dl[p]);
+            for (int p = 0; p < PB; ++p) {
+                dp[p][i] = prob[i] * (dp[p][i] - dl[p]);
+                if (first.value && acc_row(i, h) > last_key) dp[p][i] = 0.0f;
+            }
         });
+        if (first.value && causal)
+            mend_diagonal<NB, PITCH, PB>(acc, kt + m, dp, h, [&](int r, int row) __attribute__((always_inline)) {
+                return q0 + r >= it * TILE + row;
+            });
         keys.finish(it);
-    }
-    for (int it = mine; it < keys.steps; ++it) {
+    };
+    // the steps of the workgroup's later queries first, then this wave's own (no branch around the products: the
+    // accumulators would be copied at its join on every step)
+    const int top = q0 >= T_len ? -1 : causal ? q0 / TILE : keys.steps - 1;
+    for (int it = keys.steps - 1; it > top; --it) {
         keys.begin(it);
         keys.finish(it);
+    }
+    if (top >= 0) {
+        step(top, std::true_type{});
+        for (int it = top - 1; it >= 0; --it) step(it, std::false_type{});
     }
 #pragma unroll
     for (int p = 0; p < PB; ++p) {
@@ -493,10 +540,9 @@ __global__ __launch_bounds__(NT) void dkdv_kernel(const float* __restrict__ q, c
 #pragma unroll
         for (int p = 0; p < ND; ++p)
             gs[p].commit(dst + (1 + p) * TILE * PITCH, i0, dir0 + p < P ? T_len : 0, dh, tid);
-        // rows past the end: lse = +inf makes their P zero
 #pragma unroll
         for (int u = 0; u < 2; ++u)
-            dst[MATS + tid + NT * u] = i0 + tid % TILE < T_len ? row_value[u] : tid + NT * u < TILE ? INFINITY : 0.0f;
+            dst[MATS + tid + NT * u] = i0 + tid % TILE < T_len ? row_value[u] : 0.0f;
     };
     fetch(first);
     commit(first);
@@ -509,7 +555,7 @@ __global__ __launch_bounds__(NT) void dkdv_kernel(const float* __restrict__ q, c
         if (it + 1 < steps) commit(it + 1);
         __syncthreads();
     }
-    for (int it = own; it < steps; ++it) {
+    auto step = [&](int it, auto diagonal) __attribute__((always_inline)) {
         const int i0 = it * TILE;
         if (it + 1 < steps) fetch(it + 1);
         const float* qt = lds + (it & 1) * BUF;
@@ -517,33 +563,46 @@ __global__ __launch_bounds__(NT) void dkdv_kernel(const float* __restrict__ q, c
         f32x16 ss[1] = {zero16()};
         f32x16& s = ss[0];
         dot_form<DH, 1>(ss, qt + m * PITCH + h * (DH / 2), kf, nothing);
-        const bool masked = causal && i0 < k0 + TILE - 1;  // the same in all lanes
+        // queries of the tile that see the lane's key and exist
+        const int from = causal ? key - i0 : 0, to = T_len - i0;
+        auto sees = [&](int r) __attribute__((always_inline)) { return r < to && (!diagonal.value || r >= from); };
         f32x4 lse4[4];
 #pragma unroll
         for (int g = 0; g < 4; ++g) lse4[g] = *reinterpret_cast<const f32x4*>(stat + 8 * g + 4 * h);
+        f32x16 dps[PB][1];
+        auto mend = [&](int p) __attribute__((always_inline)) {
+            auto seen = [&](int r, int row) __attribute__((always_inline)) { return i0 + row >= k0 + r; };
+            mend_diagonal<NB, PITCH, 1>(acc_v[p], qt + (1 + d0 + p) * TILE * PITCH + m, ss, h, seen);
+            mend_diagonal<NB, PITCH, 1>(acc_k[p], qt + m, dps[p], h, seen);
+        };
 #pragma unroll
         for (int p = 0; p < PB; ++p) {
             const float* gt = qt + (1 + d0 + p) * TILE * PITCH;
-            f32x16 dps[1] = {zero16()};
-            f32x16& dp = dps[0];
+            f32x16& dp = dps[p][0];
+            dp = zero16();
             if (p == 0)
-                dot_form<DH, 1>(dps, gt + m * PITCH + h * (DH / 2), vf, [&](int i) __attribute__((always_inline)) {
-                    s[i] = prob_of(s[i], sc2, lse4[i >> 2][i & 3]);
-                    if (masked && key > i0 + acc_row(i, h)) s[i] = 0.0f;
+                dot_form<DH, 1>(dps[p], gt + m * PITCH + h * (DH / 2), vf, [&](int i) __attribute__((always_inline)) {
+                    s[i] = sees(acc_row(i, h)) ? prob_of(s[i], sc2, lse4[i >> 2][i & 3]) : 0.0f;
                 });
             else
-                dot_form<DH, 1>(dps, gt + m * PITCH + h * (DH / 2), vf, nothing);
+                dot_form<DH, 1>(dps[p], gt + m * PITCH + h * (DH / 2), vf, nothing);
             f32x4 d4[4];
 #pragma unroll
             for (int g = 0; g < 4; ++g)
                 d4[g] = *reinterpret_cast<const f32x4*>(stat + (1 + d0 + p) * TILE + 8 * g + 4 * h);
             chain_form<NB, PITCH, 1>(acc_v[p], gt + 4 * h * PITCH + m, ss, [&](int i) __attribute__((always_inline)) {
-                dp[i] = s[i] * (dp[i] - d4[i >> 2][i & 3]);
+                dp[i] = sees(acc_row(i, h)) ? s[i] * (dp[i] - d4[i >> 2][i & 3]) : 0.0f;
             });
-            chain_form<NB, PITCH, 1>(acc_k[p], qt + 4 * h * PITCH + m, dps, nothing);
+            chain_form<NB, PITCH, 1>(acc_k[p], qt + 4 * h * PITCH + m, dps[p], nothing);
+            if (diagonal.value && causal && p + 1 < PB) mend(p);
         }
         if (it + 1 < steps) commit(it + 1);
+        if (diagonal.value && causal) mend(PB - 1);  // the registers of the next tile are free again
         __syncthreads();
+    };
+    if (own < steps) {
+        step(own, std::true_type{});
+        for (int it = own + 1; it < steps; ++it) step(it, std::false_type{});
     }
 #pragma unroll
     for (int p = 0; p < PB; ++p) {

@@ -111,6 +111,35 @@ def test_fp32_rounding_of_delta_cancels(shape, basis, device):
     assert torch.equal(dk, torch.zeros_like(dk))
 
 
+@pytest.mark.parametrize("where", ["q", "k", "v", "d_out"])
+@pytest.mark.parametrize("value", [float("inf"), -float("inf")])
+@pytest.mark.parametrize("shape,basis,row", [((1, 2, 70, 64), 3, 37), ((1, 1, 129, 33), 1, 128), ((1, 1, 40, 128), 2, 5),
+                                             ((1, 1, 200, 96), 5, 95), ((2, 1, 64, 16), 8, 0)])
+def test_fp32_values_out_of_sight_stay_there(shape, basis, row, value, where, device):
+    """Under the causal mask a value that is not finite reaches only what may see its row: dQ of the rows behind it,
+    dK and dV of the rows before it (and its own); the rest is as with finite values, to rounding."""
+    tensors = dict(zip(("q", "k", "v", "d_out"), oattn.make_attention_inputs(*shape, basis, dtype=torch.float32, seed=row)))
+    clean = _run(*tensors.values(), device, scale=0.2, causal=True)
+    tensors[where][..., row, shape[3] // 2] = value
+    got = _run(*tensors.values(), device, scale=0.2, causal=True)
+    unseen = {"dq": slice(0, row), "dk": slice(row + 1, None), "dv": slice(row + 1, None)}
+    if where in ("k", "v"):   # row `row` spoils every later query, and through them every key up to the last
+        unseen["dk"] = unseen["dv"] = slice(0, 0)
+    for name, a, b in zip(("dq", "dk", "dv"), got, clean):
+        a, b = a[..., unseen[name], :], b[..., unseen[name], :]
+        assert torch.allclose(a, b, atol=2e-5, rtol=2e-5), name
+
+
+def test_fp32_scores_of_minus_infinity(device):
+    """Keys whose scores are -inf have P = 0 and get zero gradients, past whole tiles of them and beside rows that only
+    fill the last tile."""
+    q, k, v, g = (t.abs() for t in oattn.make_attention_inputs(1, 2, 71, 64, 2, dtype=torch.float32, seed=4))
+    k[:, :, :40] = float("-inf")
+    _, dk, dv = _run(q, k, v, g, device, scale=0.2, causal=False)
+    assert torch.isfinite(dk).all() and torch.isfinite(dv).all()
+    assert not dk[:, :, :, :40].any() and not dv[:, :, :, :40].any()
+
+
 # 16-bit storage: the MFMA kernels (T % 64 == 0, Dh in {64, 128}; one fused launch for Dh = 64, T <= 128) and the
 # generic ones otherwise.
 # (121, (1, 2, 16, 64), P) are the reference's fp16 cases (tests/test_cuda_attention_pullback.py:178-243);
