@@ -158,8 +158,9 @@ int lbi_attn_pullback(const void* q, const void* k, const void* v, const void* d
                       float softmax_scale, int causal, int dtype, void* stream);
 
 /*
- * lbi_attn_pullback for sequences and head dims that end inside a tile, on the matrix-core kernels: any T, Dh a
- * multiple of 8 up to 128, 16-bit storage, causal (short sequences, which need no workspace: causal or not).
+ * lbi_attn_pullback for sequences and head dims that end inside a tile, on the matrix-core kernels: T (rounded up to 64)
+ * times Dh below 2^30, Dh a multiple of 8 up to 128, 16-bit storage, causal (short sequences, which need no workspace:
+ * causal or not).
  * The results are those of lbi_attn_pullback on copies padded with zeros to T = 64 n and Dh = 64 or 128, without the
  * copies.  (lbi_attn_pullback itself runs such sizes on kernels that keep the probabilities in fp32, at a small
  * fraction of the speed.)  All seven tensors 16-byte aligned; other calls return LBI_ERR_UNSUPPORTED.

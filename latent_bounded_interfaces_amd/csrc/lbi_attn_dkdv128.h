@@ -45,6 +45,20 @@ __device__ __forceinline__ void dma16_at(const void* lane_ptr, unsigned lds_base
                  : "memory");
 }
 
+// One chunk per lane of a tile of a matrix of `bytes` bytes, from byte `off` (EDGE: zero from `bytes` on, see Extent).
+template <bool EDGE>
+__device__ __forceinline__ void dma_tile(const void* base, unsigned off, unsigned bytes, unsigned lds_base) {
+    if constexpr (EDGE) {
+        const u32x4 words = Extent<64, true>::descriptor(base, bytes);
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+                     :
+                     : "s"(__builtin_amdgcn_readfirstlane(lds_base)), "v"(off), "s"(words)
+                     : "memory");
+    } else {
+        dma16(base, off, lds_base);
+    }
+}
+
 template <typename T, int DH, bool CAUSAL, bool EDGE>
 __global__ __launch_bounds__(256) void dkdv_ring_kernel(const T* __restrict__ q, const T* __restrict__ k,
                                                       const T* __restrict__ v, const T* __restrict__ d_out,
@@ -103,12 +117,13 @@ __global__ __launch_bounds__(256) void dkdv_ring_kernel(const T* __restrict__ q,
     // share an allocation, so each lane carries its own 64-bit address
     const float* stat_ptr = (lane < 8 ? lse_bh : delta_p) + 4 * (lane & 7);
     const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char*)smem;
+    const unsigned bytes = ext.row_off(ext.t_rows);
     auto issue_tile = [&](int i_row, unsigned stage_base) __attribute__((always_inline)) {
 #pragma unroll
         for (int x = 0; x < NX; ++x) {
-            const unsigned off = ext.source_off(dma_off[x], (64 * (NX * wave + x) + lane) / CPR, i_row);
-            dma16(q_bh, off, lds0 + stage_base + 1024 * (NX * wave + x));
-            dma16(g_p, off, lds0 + stage_base + TILE + 1024 * (NX * wave + x));
+            const unsigned off = ext.row_off(i_row) + dma_off[x];
+            dma_tile<EDGE>(q_bh, off, bytes, lds0 + stage_base + 1024 * (NX * wave + x));
+            dma_tile<EDGE>(g_p, off, bytes, lds0 + stage_base + TILE + 1024 * (NX * wave + x));
         }
         // Every wave keeps its own copy of the 64 row statistics: no cross-wave dependency.
         if (lane < 16) dma16_at(stat_ptr + i_row, lds0 + stage_base + 2 * TILE + 256 * wave);
@@ -122,14 +137,14 @@ __global__ __launch_bounds__(256) void dkdv_ring_kernel(const T* __restrict__ q,
     for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
-            kf[t][ks] = ext.resident(k + base, j0w + 32 * t + m, 16 * ks + 8 * h);
+            kf[t][ks] = ext.load(k + base, j0w + 32 * t + m, 16 * ks + 8 * h);
     {
         char* vt_w = smem + R * STAGE + wave * 2 * TILE;
 #pragma unroll
         for (int u = 0; u < CPR; ++u) {
             const int slot = 64 * u + lane;  // 16-byte slot of the wave's 64-row block
             const int r = slot / CPR, c = slot % CPR;
-            const u32x4 val = ext.resident(v + base, j0w + r, 8 * c);
+            const u32x4 val = ext.load(v + base, j0w + r, 8 * c);
             *reinterpret_cast<u32x4*>(vt_w + (r >> 5) * TILE + tile_off<DH>(r & 31, c)) = val;
         }
     }

@@ -80,7 +80,6 @@ __global__ __launch_bounds__(256) void dkdv_pair_kernel(const T* __restrict__ q,
     const int j0s = min(j0 + 32 * wave, T_len - 32); // this wave's S tile (equals j0w + 32 d inside the sequence)
     const Extent<DH, EDGE> ext(T_len, t_rows, dh);
     const size_t base = (size_t)bh * ext.t_rows * ext.dh;
-    const T* q_bh = q + base;
     const float* lse_bh = lse2 + (size_t)bh * T_len;
     size_t prow[2 * DW];
 #pragma unroll
@@ -113,19 +112,18 @@ __global__ __launch_bounds__(256) void dkdv_pair_kernel(const T* __restrict__ q,
         const int r = sigma / CPR;
         dma_off[x] = ext.chunk_off(r, (sigma % CPR) ^ swz<DH>(r));
         dma_dst[x] = tile * TILE + 1024 * u;
-        dma_src[x] = tile == 0 ? q_bh : d_out + prow[tile - 1] * ext.dh;
+        dma_src[x] = tile == 0 ? q + base : d_out + prow[tile - 1] * ext.dh;
     }
     // lanes 0-7: lse2, 8-15: -delta of statistics slot 1, 16-23: of slot 2 (float4 each)
     const int slot_dir = DW == 1 ? (lane < 16 ? 0 : 1) : d + (lane < 16 ? 0 : 2);
     const size_t stat_row = (((size_t)b * P + min(p_first + slot_dir, P - 1)) * H + hh) * T_len;
     const float* stat_ptr = (lane < 8 ? lse_bh : delta + stat_row) + 4 * (lane & 7);
+    const unsigned bytes = ext.row_off(ext.t_rows);
     const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char*)smem;
     auto issue_tile = [&](int i_row, unsigned stage_base) __attribute__((always_inline)) {
 #pragma unroll
-        for (int x = 0; x < NXW; ++x) {
-            const int r = (64 * ((wave + 4 * x) % CPT) + lane) / CPR;
-            dma16(dma_src[x], ext.source_off(dma_off[x], r, i_row), lds0 + stage_base + dma_dst[x]);
-        }
+        for (int x = 0; x < NXW; ++x)
+            dma_tile<EDGE>(dma_src[x], ext.row_off(i_row) + dma_off[x], bytes, lds0 + stage_base + dma_dst[x]);
         if (lane < 24) dma16_at(stat_ptr + i_row, lds0 + stage_base + NTILE * TILE + 512 * wave);
     };
 
@@ -151,14 +149,14 @@ __global__ __launch_bounds__(256) void dkdv_pair_kernel(const T* __restrict__ q,
     for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks)
-            vf[t][ks] = ext.resident(v + base, j0w + 32 * t + m, 16 * ks + 8 * h);
+            vf[t][ks] = ext.load(v + base, j0w + 32 * t + m, 16 * ks + 8 * h);
     {
         char* kt_w = smem + KT0 + wave * TILE;       // wave w writes the tile it will read
 #pragma unroll
         for (int u = 0; u < CPR / 2; ++u) {
             const int slot = 64 * u + lane;
             const int r = slot / CPR, c = slot % CPR;
-            const u32x4 val = ext.resident(k + base, j0s + r, 8 * c);
+            const u32x4 val = ext.load(k + base, j0s + r, 8 * c);
             *reinterpret_cast<u32x4*>(kt_w + tile_off<DH>(r, c)) = val;
         }
     }

@@ -68,12 +68,13 @@ __global__ __launch_bounds__(256) void dq_ring_kernel(const T* __restrict__ q, c
         dma_off[x] = ext.chunk_off(r, (sigma % CPR) ^ swz<DH>(r));
     }
     const unsigned lds0 = (unsigned)(size_t)(__attribute__((address_space(3))) char*)smem;
+    const unsigned bytes = ext.row_off(ext.t_rows);
     auto issue_tile = [&](int j_row, unsigned stage_base) __attribute__((always_inline)) {
 #pragma unroll
         for (int x = 0; x < NX; ++x) {
-            const unsigned off = ext.source_off(dma_off[x], (64 * (NX * wave + x) + lane) / CPR, j_row);
-            dma16(k_bh, off, lds0 + stage_base + 1024 * (NX * wave + x));
-            dma16(v_bh, off, lds0 + stage_base + TILE + 1024 * (NX * wave + x));
+            const unsigned off = ext.row_off(j_row) + dma_off[x];
+            dma_tile<EDGE>(k_bh, off, bytes, lds0 + stage_base + 1024 * (NX * wave + x));
+            dma_tile<EDGE>(v_bh, off, bytes, lds0 + stage_base + TILE + 1024 * (NX * wave + x));
         }
     };
 
@@ -83,7 +84,7 @@ __global__ __launch_bounds__(256) void dq_ring_kernel(const T* __restrict__ q, c
     // (negated) for the dK/dV kernel: every (direction, query) has exactly one owner wave.
     u32x4 qf[KS];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[ks] = ext.resident(q + base, i0w + m, 16 * ks + 8 * h);
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = ext.load(q + base, i0w + m, 16 * ks + 8 * h);
     const float my_lse = lse2[(size_t)bh * T_len + i0w + m];
     float my_delta[PB];
     char* gf_w = smem + GF0 + wave * PB * TILE;
@@ -95,7 +96,7 @@ __global__ __launch_bounds__(256) void dq_ring_kernel(const T* __restrict__ q, c
         for (int u = 0; u < CPR / 2; ++u) {
             const int slot = 64 * u + lane;
             const int r = slot / CPR, c = slot % CPR;
-            const u32x4 val = ext.resident(g_p, i0w + r, 8 * c);
+            const u32x4 val = ext.load(g_p, i0w + r, 8 * c);
             *reinterpret_cast<u32x4*>(gf_w + pp * TILE + tile_off<DH>(r, c)) = val;
         }
         my_delta[pp] = 0.0f;

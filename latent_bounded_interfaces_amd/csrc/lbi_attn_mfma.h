@@ -128,35 +128,37 @@ template <int DH> __device__ __forceinline__ int tile_off(int r, int chunk) {
 // tile's DH.  The tile loops run over T_len, the length rounded up to 64, and the workspace has T_len rows and DH
 // columns; the caller's tensors have t_rows rows of dh elements.  Copies padded to the tile cost one extra pass over
 // every tensor and one over every result (bf16 B=8 H=12 T=1000 Dh=64 P=16: 1.19 -> 0.98 ms without them), so
-// the tiles are padded on chip instead, and the results are those of the padded call:
-//  * a row past the end is read from the last row.  As a key it lies above the diagonal of every real query; as a
-//    query its lse2 is +infinity, so its P and dS are 0 and it adds 0 to dK and dV (a value that is not finite in the
-//    last row reaches the same sums through the row itself);
-//  * the resident operands (K and V of the dK/dV kernels, Q and d_out of the dQ kernel, Q of the statistics) are
-//    zero in the columns past dh, so what a streamed tile holds there (the row's last 16 bytes again) is multiplied
-//    by zero;
-//  * neither rows nor columns past the end are stored.
+// the tiles are padded on chip instead: whatever a tile holds past the end of a tensor is zero, as in the padded copy,
+// and neither rows nor columns past the end are stored.  The results are those of the padded call, bit for bit, also for
+// values that are not finite.
+// All loads go through a raw buffer descriptor over the rows of one (b, h) or (b, p, h) (stride 0: offsets are in bytes, and
+// what lies at or past the end reads as zero); columns past dh get an offset past it.  (Clamped addresses and zeros by
+// selection cost up to 20 % of a call: the select waits for the load, and the descriptor saves the address arithmetic.)
 template <int DH, bool EDGE> struct Extent {
+    static constexpr unsigned PAST_END = 1u << 31;  // offsets inside a tensor stay below it (supports_edge)
     int t_rows, dh;
     __device__ __forceinline__ Extent(int T_len, int t_rows_, int dh_)
         : t_rows(EDGE ? t_rows_ : T_len), dh(EDGE ? dh_ : DH) {}
-    __device__ __forceinline__ int row(int r) const { return EDGE ? min(r, t_rows - 1) : r; }
-    // eight elements at column c of row r of a resident operand
-    __device__ __forceinline__ u32x4 resident(const void* base, int r, int c) const {
-        const int col = EDGE ? min(c, dh - 8) : c;
-        u32x4 v = *reinterpret_cast<const u32x4*>(static_cast<const char*>(base) + ((size_t)row(r) * dh + col) * 2);
-        if (EDGE && c >= dh) v = u32x4{0u, 0u, 0u, 0u};
-        return v;
+    // words of the descriptor of a matrix (word 3 holds only the data format, 32 bits, which must not be 0)
+    static __device__ __forceinline__ u32x4 descriptor(const void* base, unsigned bytes) {
+        return u32x4{(unsigned)(size_t)base, (unsigned)((size_t)base >> 32) & 0xffffu, bytes, 4u << 15};
+    }
+    // eight elements at column c of row r
+    __device__ __forceinline__ u32x4 load(const void* base, int r, int c) const {
+        if constexpr (EDGE) {
+            const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, row_off(t_rows), 4 << 15);
+            const unsigned off = c < dh ? (unsigned)((r * dh + c) * 2) : PAST_END;
+            return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0));
+        } else {
+            return *reinterpret_cast<const u32x4*>(static_cast<const char*>(base) + ((size_t)r * DH + c) * 2);
+        }
     }
     // byte offset of 16-byte chunk `chunk` of tile row r in the source tile (row 0 of the tile at offset 0)
     __device__ __forceinline__ unsigned chunk_off(int r, int chunk) const {
-        return (unsigned)(r * dh * 2 + ((EDGE ? min(chunk, dh / 8 - 1) : chunk) << 4));
+        return EDGE && chunk * 8 >= dh ? PAST_END : (unsigned)(r * dh * 2 + (chunk << 4));
     }
-    // the same, plus where the tile starts: row i_row, or less for a row that would lie past the end
-    __device__ __forceinline__ unsigned source_off(unsigned off, int r, int i_row) const {
-        if (!EDGE) return (unsigned)i_row * (DH * 2) + off;
-        return __umul24((unsigned)(min(i_row + r, t_rows - 1)), (unsigned)(dh * 2)) + off - (unsigned)(r * dh * 2);
-    }
+    // byte offset of row i_row
+    __device__ __forceinline__ unsigned row_off(int i_row) const { return (unsigned)i_row * (unsigned)(dh * 2); }
     __device__ __forceinline__ bool stored(int r, int c) const { return !EDGE || (r < t_rows && c < dh); }
 };
 
@@ -169,10 +171,7 @@ template <int DH> struct TileLoader {
 #pragma unroll
         for (int u = 0; u < N; ++u) {
             const int id = tid + 256 * u;
-            const int r = id / CHUNKS_PER_ROW, c = id % CHUNKS_PER_ROW;
-            const int col = EDGE ? min(c * 8, ext.dh - 8) : c * 8;
-            regs[u] = *reinterpret_cast<const u32x4*>(static_cast<const char*>(base) +
-                                                      ((size_t)ext.row(row0 + r) * ext.dh + col) * 2);
+            regs[u] = ext.load(base, row0 + id / CHUNKS_PER_ROW, id % CHUNKS_PER_ROW * 8);
         }
     }
     __device__ __forceinline__ void commit(char* tile, int tid) const {
@@ -272,7 +271,7 @@ __global__ __launch_bounds__(256) void stats_kernel(const T* __restrict__ q, con
 
     u32x4 qf[KS];
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) qf[ks] = ext.resident(q + base, i0w + m, 16 * ks + 8 * h);
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = ext.load(q + base, i0w + m, 16 * ks + 8 * h);
     f32x16 o_t[ND];
 #pragma unroll
     for (int nd = 0; nd < ND; ++nd) o_t[nd] = zero16();
@@ -353,8 +352,7 @@ __global__ __launch_bounds__(256) void stats_kernel(const T* __restrict__ q, con
     }
     if (active) {
         const float inv = 1.0f / l_run;
-        if (h == 0)
-            lse2[(size_t)bh * T_len + i0w + m] = EDGE && i0w + m >= ext.t_rows ? INFINITY : m_run + log2f(l_run);
+        if (h == 0) lse2[(size_t)bh * T_len + i0w + m] = m_run + log2f(l_run);
         float* o_row = o32 + ((size_t)bh * T_len + i0w + m) * DH;
 #pragma unroll
         for (int nd = 0; nd < ND; ++nd)
@@ -442,7 +440,8 @@ int launch(const void* q, const void* k, const void* v, const void* g, void* dq,
 // What the EDGE forms take: lengths and head dims of causal 16-bit calls that the plain forms leave out.
 inline int edge_len(int T_len) { return (T_len + 63) / 64 * 64; }
 inline bool supports_edge(int T_len, int dh, int dtype) {
-    return (dtype == LBI_F16 || dtype == LBI_BF16) && dh >= 8 && dh <= 128 && dh % 8 == 0 && T_len >= 1;
+    return (dtype == LBI_F16 || dtype == LBI_BF16) && dh >= 8 && dh <= 128 && dh % 8 == 0 && T_len >= 1 &&
+           (int64_t)edge_len(T_len) * dh * 2 < (int64_t)1 << 31;  // Extent::PAST_END
 }
 
 template <typename T>

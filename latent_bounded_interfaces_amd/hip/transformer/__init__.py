@@ -127,8 +127,10 @@ def attention_input_pullback_basis(
         long_seq = seqlen + (multiple - seqlen % multiple) if (ragged and causal) else seqlen
         if (wide_dim != head_dim or long_seq != seqlen) and long_seq % multiple == 0 \
                 and wide_dim in _MFMA_HEAD_DIMS:
-            # head dims of whole 16-byte pieces on aligned tensors: the kernels pad their tiles on chip
-            if (causal or single_launch) and head_dim % 8 == 0 and all(t.data_ptr() % 16 == 0 for t in (q, k, v, d_out)):
+            # head dims of whole 16-byte pieces on aligned tensors: the kernels pad their tiles on chip (2 GiB at most
+            # per (b, p, h): what their descriptors span)
+            if (causal or single_launch) and head_dim % 8 == 0 and long_seq * head_dim < 1 << 30 \
+                    and all(t.data_ptr() % 16 == 0 for t in (q, k, v, d_out)):
                 return _launch(q, k, v, d_out, softmax_scale, causal, dtype, True)
             pads = (0, wide_dim - head_dim, 0, long_seq - seqlen)
             padded = [torch.nn.functional.pad(t, pads) for t in (q, k, v, d_out)]

@@ -301,6 +301,32 @@ def test_tiles_padded_on_chip_equal_padded_copies(shape, basis, dtype, device):
             assert a.shape == g.shape and torch.equal(a, b[..., :seqlen, :dim]), (name, causal)
 
 
+@pytest.mark.parametrize("where", ["q", "k", "v", "d_out"])
+@pytest.mark.parametrize("value", [float("inf"), -float("inf"), float("nan")])
+@pytest.mark.parametrize("shape,basis,row", [((1, 2, 321, 64), 1, -1), ((1, 2, 1000, 64), 5, -1), ((1, 1, 300, 80), 2, -1),
+                                             ((1, 1, 333, 40), 9, 100), ((1, 2, 161, 96), 1, 0), ((1, 1, 130, 128), 3, 129)])
+def test_padding_on_chip_is_zero_beside_infinities(shape, basis, row, value, where, device):
+    """What a tile holds past the end is zero, not a copy of the last row or of its last columns: a value there that is
+    not finite gives what it gives in copies padded by hand, infinities and NaN included."""
+    from latent_bounded_interfaces_amd.hip.transformer import attention_input_pullback_basis
+
+    gen = torch.Generator().manual_seed(77)
+    bsz, heads, seqlen, dim = shape
+    t = {n: torch.randn(*shape, generator=gen).bfloat16() for n in ("q", "k", "v")}
+    t["d_out"] = torch.randn(bsz, basis, *shape[1:], generator=gen).bfloat16()
+    if where in ("q", "k"):   # one sign, so that an infinite factor gives scores of +inf or -inf and not NaN throughout
+        t = {n: x.abs() for n, x in t.items()}
+    t[where][..., row, dim - 1] = value
+    t = {n: x.to(device) for n, x in t.items()}
+    pads = (0, (64 if dim <= 64 else 128) - dim, 0, -seqlen % 64)
+    got = attention_input_pullback_basis(*t.values(), softmax_scale=0.2, causal=True, kernel_mode="hip")
+    want = attention_input_pullback_basis(*(torch.nn.functional.pad(x, pads) for x in t.values()), softmax_scale=0.2,
+                                          causal=True, kernel_mode="hip")
+    for name, a, b in zip(("dq", "dk", "dv"), got, want):
+        b = b[..., :seqlen, :dim]
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(), b.nan_to_num()), name
+
+
 def test_long_context_properties(device):
     """bf16, T=4096, Dh=128, P=16 on two (b, h) slices: size-independent checks."""
     from latent_bounded_interfaces_amd.hip.transformer import attention_input_pullback_basis
