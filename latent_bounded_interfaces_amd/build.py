@@ -25,6 +25,8 @@ HIPCC_FLAGS = [
     # Keep the compiler from forming packed-fp32 VALU instructions.
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
+    # A loop that is not unrolled as asked keeps its register arrays in scratch memory.
+    "-Werror=pass-failed",
 ]
 
 

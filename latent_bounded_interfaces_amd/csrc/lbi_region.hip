@@ -441,14 +441,18 @@ __global__ __launch_bounds__(256) void qkv_pullback_kernel(const T* __restrict__
 // projection (see the transposed convolution below), without storing the intermediate: one thread forms the
 // projection cotangent of its 2 VEC channels at RUN + KMAX - 1 consecutive positions and accumulates RUN outputs.
 //
-// Bound: memory.  The rows of a run form a serial chain only through registers, so their loads are all independent:
-// they are issued AHEAD rows before their use, from clamped addresses and under no branch (a load under a branch is
+// Bound: memory.  The rows of a run form a serial chain only through registers, so their loads are all independent.
+// RING: they are issued AHEAD rows before their use, from clamped addresses and under no branch (a load under a branch is
 // waited for at the join, which made every row cost a full memory latency).  REP is the number of query heads of a
 // key/value group, 0 for "any": then the heads are added up in a loop inside the row.  Heads of q have one source; the
 // other REP - 1 loads repeat its address and count as zero.  Consecutive workgroups share the halo rows of their runs,
 // so a contiguous eighth of them is dealt to each XCD.  bf16, H = 12, Dh = 64, T = 1024, B P = 512: 1.34 -> 1.05 ms
 // (4.6 TB/s); H = 4, Hkv = 2, T = 128, B P = 16, in runs of 4 instead of 16: 28.5 -> 7.7 us.
-template <typename T, int VEC, int KMAX, int RUN, bool INTERLEAVED, bool EXACT, int REP>
+// Without RING (long runs of any number of heads) a row is loaded when its turn comes: the loop over the heads keeps the
+// compiler from unrolling a long run around the ring, whose registers then live in scratch memory (bf16 H = 8, Hkv = 2,
+// T = 512, B P = 256: 207 us here, 1027 us so); four waves per SIMD hide the latency instead.
+// All forms round alike: a direction's result does not depend on the number of directions of the call.
+template <typename T, int VEC, int KMAX, int RUN, bool INTERLEAVED, bool EXACT, int REP, bool RING>
 __global__ __launch_bounds__(256) void qkv_conv_pullback_kernel(const T* __restrict__ dq, const T* __restrict__ dk,
                                                                 const T* __restrict__ dv,
                                                                 const float* __restrict__ cos_t,
@@ -458,7 +462,8 @@ __global__ __launch_bounds__(256) void qkv_conv_pullback_kernel(const T* __restr
                                                                 int ksize) {
     constexpr int ROWS = RUN + KMAX - 1, AHEAD = sizeof(T) == 4 ? 4 : 6;
     const unsigned per_xcd = gridDim.x / 8;
-    const unsigned block = blockIdx.x < 8 * per_xcd ? blockIdx.x % 8 * per_xcd + blockIdx.x / 8 : blockIdx.x;
+    const unsigned block =
+        RING && blockIdx.x < 8 * per_xcd ? blockIdx.x % 8 * per_xcd + blockIdx.x / 8 : blockIdx.x;
     const long long unit = (long long)block * 256 + threadIdx.x;
     if (unit >= n_units) return;
     const int half = Dh / 2;
@@ -529,45 +534,61 @@ __global__ __launch_bounds__(256) void qkv_conv_pullback_kernel(const T* __restr
         cs[slot].load(cos_t + (long long)t * half + j);
         sn[slot].load(sin_t + (long long)t * half + j);
     };
+    if constexpr (RING)
 #pragma unroll
-    for (int jj = 0; jj < AHEAD; ++jj) request(jj);
+        for (int jj = 0; jj < AHEAD; ++jj) request(jj);
 #pragma unroll
     for (int jj = 0; jj < ROWS; ++jj) {
-        const int slot = jj % AHEAD;
         const bool live = s0 + jj < T_len && jj < RUN + ksize - 1;
-        float a0[VEC], a1[VEC], c[VEC], s[VEC], g0[VEC], g1[VEC];
+        float g0[VEC], g1[VEC];
+        if constexpr (RING) {
+            const int slot = jj % AHEAD;
+            float a0[VEC], a1[VEC], c[VEC], s[VEC];
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) {
-            a0[e] = a1[e] = 0.0f;
+            for (int e = 0; e < VEC; ++e) {
+                a0[e] = a1[e] = 0.0f;
 #pragma unroll
-            for (int g = 0; g < HEADS; ++g) {
-                a0[e] += g < count ? x0[slot][g].at(e) : 0.0f;
-                a1[e] += g < count ? x1[slot][g].at(e) : 0.0f;
+                for (int g = 0; g < HEADS; ++g) {
+                    const float v0 = x0[slot][g].at(e), v1 = x1[slot][g].at(e);  // outside the selects: no branch
+                    a0[e] += g < count ? v0 : 0.0f;
+                    a1[e] += g < count ? v1 : 0.0f;
+                }
+                c[e] = cs[slot].at(e);
+                s[e] = sn[slot].at(e);
             }
-            c[e] = cs[slot].at(e);
-            s[e] = sn[slot].at(e);
-        }
-        if (REP == 0) {
-            const T* p = src + (long long)min(s0 + jj, T_len - 1) * Dh;
-            for (int g = 1; g < count; ++g) {
-                Raw<T, VEC> m0, m1;
-                m0.load(p + g * head_stride + off0);
-                m1.load(p + g * head_stride + off1);
+            if constexpr (REP == 0) {
+                const T* p = src + (long long)min(s0 + jj, T_len - 1) * Dh;
+                for (int g = 1; g < count; ++g) {
+                    Raw<T, VEC> m0, m1;
+                    m0.load(p + g * head_stride + off0);
+                    m1.load(p + g * head_stride + off1);
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) {
-                    a0[e] += m0.at(e);
-                    a1[e] += m1.at(e);
+                    for (int e = 0; e < VEC; ++e) {
+                        a0[e] += m0.at(e);
+                        a1[e] += m1.at(e);
+                    }
                 }
             }
-        }
-        qkv_unrotate<VEC, INTERLEAVED>(a0, a1, c, s, g0, g1);
+            qkv_unrotate<VEC, INTERLEAVED>(a0, a1, c, s, g0, g1);
 #pragma unroll
-        for (int e = 0; e < VEC; ++e) {  // the stored intermediate of the two-kernel form is rounded to T
-            g0[e] = live ? round_via<T>(rotary ? g0[e] : a0[e]) : 0.0f;
-            g1[e] = live ? round_via<T>(rotary ? g1[e] : a1[e]) : 0.0f;
+            for (int e = 0; e < VEC; ++e) {  // the stored intermediate of the two-kernel form is rounded to T
+                const float v0 = round_via<T>(rotary ? g0[e] : a0[e]), v1 = round_via<T>(rotary ? g1[e] : a1[e]);
+                g0[e] = live ? v0 : 0.0f;
+                g1[e] = live ? v1 : 0.0f;
+            }
+            if (jj + AHEAD < ROWS) request(jj + AHEAD);
+            __builtin_amdgcn_sched_barrier(0);
+        } else if (live) {
+            qkv_unit_values<T, VEC, INTERLEAVED>(dq, dk, dv, cos_t, sin_t, n, s0 + jj, T_len, H, Hkv, Dh, head, j, g0, g1);
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) {
+                g0[e] = round_via<T>(g0[e]);
+                g1[e] = round_via<T>(g1[e]);
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) g0[e] = g1[e] = 0.0f;
         }
-        if (jj + AHEAD < ROWS) request(jj + AHEAD);
-        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int r = 0; r < RUN; ++r) {
             const int i = jj - r;
@@ -769,13 +790,13 @@ int launch_qkv(const void* dq, const void* dk, const void* dv, const float* cos_
     return LBI_OK;
 }
 
-template <typename T, int VEC, int KMAX, int RUN, bool INTERLEAVED, bool EXACT, int REP>
+template <typename T, int VEC, int KMAX, int RUN, bool INTERLEAVED, bool EXACT, int REP, bool RING>
 int launch_qkv_conv_as(const void* dq, const void* dk, const void* dv, const float* cos_t, const float* sin_t,
                        const void* weight, void* out, long long n_seq, int T_len, int H, int Hkv, int Dh, int ksize,
                        hipStream_t stream) {
     const long long units = n_seq * ((T_len + RUN - 1) / RUN) * (long long)(H + 2 * Hkv) * (Dh / 2 / VEC);
     if (!fits_grid(units, 256)) return fail(LBI_ERR_UNSUPPORTED, "lbi_attn_qkv_conv_pullback: too many elements");
-    hipLaunchKernelGGL((qkv_conv_pullback_kernel<T, VEC, KMAX, RUN, INTERLEAVED, EXACT, REP>), dim3(blocks_for(units, 256)),
+    hipLaunchKernelGGL((qkv_conv_pullback_kernel<T, VEC, KMAX, RUN, INTERLEAVED, EXACT, REP, RING>), dim3(blocks_for(units, 256)),
                        dim3(256), 0, stream, (const T*)dq, (const T*)dk, (const T*)dv, cos_t, sin_t, (const T*)weight,
                        (T*)out, units, T_len, H, Hkv, Dh, ksize);
     LBI_HIP_CHECK(hipGetLastError());
@@ -789,28 +810,30 @@ int launch_qkv_conv_il(const void* dq, const void* dk, const void* dv, const flo
     const bool vec = (Dh / 2) % 4 == 0;
     // the 4 x 4 weights of a channel group are contiguous; 4-element loads of them need 4-element alignment
     const bool exact = vec && ksize == 4 && reinterpret_cast<uintptr_t>(weight) % (4 * sizeof(T)) == 0;
-    if (exact) {
-        // A run of RUN outputs reads RUN + 3 rows, so long runs read least; short ones where long ones would leave
-        // compute units without a workgroup.
-        const long long long_units = n_seq * ((T_len + 15) / 16) * (long long)(H + 2 * Hkv) * (Dh / 8);
-        const bool short_runs = long_units < 4LL * 256 * device_compute_units();
-        const int rep = H / Hkv;
-        if (short_runs) {
-            if (rep == 1) return launch_qkv_conv_as<T, 4, 4, 4, INTERLEAVED, true, 1>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
-            if (rep == 2) return launch_qkv_conv_as<T, 4, 4, 4, INTERLEAVED, true, 2>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
-            return launch_qkv_conv_as<T, 4, 4, 4, INTERLEAVED, true, 0>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
-        }
-        if (rep == 1) return launch_qkv_conv_as<T, 4, 4, 16, INTERLEAVED, true, 1>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
-        if (rep == 2) return launch_qkv_conv_as<T, 4, 4, 16, INTERLEAVED, true, 2>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
-        return launch_qkv_conv_as<T, 4, 4, 16, INTERLEAVED, true, 0>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
-    }
-    if (vec && ksize <= 4)
-        return launch_qkv_conv_as<T, 4, 4, 16, INTERLEAVED, false, 0>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
-    if (vec)
-        return launch_qkv_conv_as<T, 4, 8, 8, INTERLEAVED, false, 0>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);  // longer runs spill
-    if (ksize <= 4)
-        return launch_qkv_conv_as<T, 1, 4, 16, INTERLEAVED, false, 0>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
-    return launch_qkv_conv_as<T, 1, 8, 8, INTERLEAVED, false, 0>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq, T_len, H, Hkv, Dh, ksize, stream);
+    // A run of RUN outputs reads RUN + KMAX - 1 rows, so long runs read least; short ones where long ones would leave
+    // compute units without a workgroup (B P = 16, T = 128: 17-48 us in long runs loaded row by row, 9-17 us here).
+    // Long runs of three or more heads per group: see the kernel.
+    const long long long_units = n_seq * ((T_len + 15) / 16) * (long long)(H + 2 * Hkv) * (Dh / (vec ? 8 : 2));
+    const bool short_runs = long_units < 4LL * 256 * device_compute_units();
+    const int rep = H / Hkv;
+#define LBI_CONV(VEC, KMAX, RUN, EXACT, REP, RING)                                                                      \
+    launch_qkv_conv_as<T, VEC, KMAX, RUN, INTERLEAVED, EXACT, REP, RING>(dq, dk, dv, cos_t, sin_t, weight, out, n_seq,  \
+                                                                         T_len, H, Hkv, Dh, ksize, stream)
+#define LBI_CONV_RUNS(VEC, EXACT, REP)                                                                                  \
+    (short_runs ? LBI_CONV(VEC, 4, 4, EXACT, REP, true) : LBI_CONV(VEC, 4, 16, EXACT, REP, ((REP) > 0)))
+#define LBI_CONV_REPS(VEC, EXACT)                                                                                       \
+    (rep == 1 ? LBI_CONV_RUNS(VEC, EXACT, 1) : rep == 2 ? LBI_CONV_RUNS(VEC, EXACT, 2) : LBI_CONV_RUNS(VEC, EXACT, 0))
+#define LBI_CONV_LONG(VEC) /* longer runs spill */                                                                      \
+    (rep == 1 ? LBI_CONV(VEC, 8, 8, false, 1, true)                                                                     \
+              : short_runs ? LBI_CONV(VEC, 8, 8, false, 0, true) : LBI_CONV(VEC, 8, 8, false, 0, false))
+    if (ksize > 4) return vec ? LBI_CONV_LONG(4) : LBI_CONV_LONG(1);
+    if (exact) return LBI_CONV_REPS(4, true);
+    if (vec) return LBI_CONV_REPS(4, false);
+    return LBI_CONV_REPS(1, false);
+#undef LBI_CONV_LONG
+#undef LBI_CONV_REPS
+#undef LBI_CONV_RUNS
+#undef LBI_CONV
 }
 
 template <typename T>
