@@ -597,19 +597,19 @@ __global__ __launch_bounds__(256) void cotangent_staged_kernel(const Tin* __rest
 }
 
 // ---------------------------------------------------------------------------------------
-// Cotangent chain for widths up to 256 that neither fit the staged kernel (fp32 above d = 180) nor have rows of whole
-// 16-byte pieces.  One row at a time per wave, as the any-width kernel goes, a step is a serial chain of 13-32 memory
-// latencies.  The matrices do not depend on the chain, so a wave of the sixteen keeps its rows (4 NJ at most, NJ
-// elements per lane, each load 64 neighbouring elements) of the next matrix in flight in registers and refills each
-// as soon as it has been used, as cotangent256_kernel does; the sums of a lane are folded by a halving butterfly.
-// What is left is one CU's streaming rate, a batch element being one workgroup.
-// fp32 B=12 K=6 d=198: 173 -> 56 us.
-// ---------------------------------------------------------------------------------------
+// Cotangent chain for widths up to 256 that the staged kernel does not take (fp32 above d = 180, rows of no whole 16-byte
+// pieces).  One row at a time per wave, as the any-width kernel goes, a step is a serial chain of 13-32 memory
+// latencies.  The matrices do not depend on the chain, so a wave of the sixteen keeps its rows (up to 4 NJ, NJ elements per
+// lane, each load 64 neighbouring elements) of the next matrix in flight in registers and refills each as soon as it has
+// been used, as cotangent256_kernel does.  The sums of a lane are folded by a halving butterfly, four or eight rows at a
+// time: the sums of sixteen beside 64 elements in flight would not fit the 128 registers of a wave, and reloading what
+// spilled waits for every load in flight.
+// What is left is one CU's streaming rate, a batch element being one workgroup.  fp32, one row at a time -> here: B=12 K=6
+// d=198 94 -> 18 us, B=64 K=48 d=255 2.89 -> 0.28 ms.
 template <typename Tin, int NJ>
 __global__ __launch_bounds__(1024) void cotangent_rows_kernel(const Tin* __restrict__ mats, const float* __restrict__ g,
                                                               float* __restrict__ out, int K, int d) {
-    constexpr int NW = 16, R = NJ >= 3 ? 16 : 4 * NJ;  // rows of a wave
-    constexpr int SHIFT = R == 16 ? 2 : (R == 8 ? 3 : 4);  // 6 - log2 R
+    constexpr int NW = 16, R = 4 * NJ;  // rows of a wave
     __shared__ float vbuf[2][64 * NJ];
     const int b = blockIdx.x;
     const int tid = threadIdx.x, lane = tid & 63;
@@ -640,37 +640,51 @@ __global__ __launch_bounds__(1024) void cotangent_rows_kernel(const Tin* __restr
     int cur = 0;
     for (int r = K - 1; r >= 0; --r) {
         const int r_next = r > 0 ? r - 1 : 0;  // a harmless re-read at the end
-        float vv[NJ], vals[R];
+        float vv[NJ];
 #pragma unroll
         for (int j = 0; j < NJ; ++j) vv[j] = vbuf[cur][64 * j + lane];
+        // rows [first, first + n) of the wave, n = 4 or 8
+        auto fold = [&](auto first_tag, auto n_tag) __attribute__((always_inline)) {
+            constexpr int FIRST = first_tag.value, N = n_tag.value, SHIFT = N == 8 ? 3 : 4;  // 6 - log2 N
+            float vals[N];
 #pragma unroll
-        for (int i = 0; i < R; ++i) {
-            float acc = 0.0f;
+            for (int i = 0; i < N; ++i) {
+                float acc = 0.0f;
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) {
-                const float a = to_f32(buf[i][j]);
-                acc = fmaf(j < NJ - 1 || 64 * j + lane < d ? a : 0.0f, vv[j], acc);
+                for (int j = 0; j < NJ; ++j) {
+                    const float a = to_f32(buf[FIRST + i][j]);
+                    acc = fmaf(j < NJ - 1 || 64 * j + lane < d ? a : 0.0f, vv[j], acc);
+                }
+                vals[i] = acc;
+                load_row(r_next, FIRST + i);
             }
-            vals[i] = acc;
-            load_row(r_next, i);
-        }
-        // halving butterfly: lane bit `off` keeps the upper or lower half of the rows it holds
+            // halving butterfly: lane bit `off` keeps the upper or lower half of the rows it holds
 #pragma unroll
-        for (int n = R / 2, off = 32; n >= 1; n >>= 1, off >>= 1) {
-            const bool up = (lane & off) != 0;
+            for (int n = N / 2, off = 32; n >= 1; n >>= 1, off >>= 1) {
+                const bool up = (lane & off) != 0;
 #pragma unroll
-            for (int i = 0; i < n; ++i) {
-                const float send = up ? vals[i] : vals[i + n], keep = up ? vals[i + n] : vals[i];
-                vals[i] = keep + __shfl_xor(send, off, 64);
+                for (int i = 0; i < n; ++i) {
+                    const float low = vals[i], high = vals[i + n];  // ahead of the selects: no run-time index
+                    const float send = up ? low : high, keep = up ? high : low;
+                    vals[i] = keep + __shfl_xor(send, off, 64);
+                }
             }
-        }
-        float sum = vals[0];
+            float sum = vals[0];
 #pragma unroll
-        for (int off = 32 / R; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, 64);
-        const int row = wave + NW * (lane >> SHIFT);
-        if ((lane & ((1 << SHIFT) - 1)) == 0 && row < d) {
-            vbuf[cur ^ 1][row] = sum;
-            out_b[(size_t)r * d + row] = sum;
+            for (int off = 32 / N; off >= 1; off >>= 1) sum += __shfl_xor(sum, off, 64);
+            const int row = wave + NW * (FIRST + (lane >> SHIFT));
+            if ((lane & ((1 << SHIFT) - 1)) == 0 && row < d) {
+                vbuf[cur ^ 1][row] = sum;
+                out_b[(size_t)r * d + row] = sum;
+            }
+        };
+        using std::integral_constant;
+        if constexpr (NJ == 1) {
+            fold(integral_constant<int, 0>{}, integral_constant<int, 4>{});
+        } else {
+            fold(integral_constant<int, 0>{}, integral_constant<int, 8>{});
+            if constexpr (NJ == 3) fold(integral_constant<int, 8>{}, integral_constant<int, 4>{});
+            if constexpr (NJ == 4) fold(integral_constant<int, 8>{}, integral_constant<int, 8>{});
         }
         lds_barrier();
         cur ^= 1;
@@ -1383,7 +1397,11 @@ int launch_cotangent(const void* mats, const void* g, void* out, int B, int K, i
         LBI_HIP_CHECK(hipGetLastError());
         return LBI_OK;
     }
-    if (d <= 256 && d > 16) {
+    // Rows of whole 4-element pieces past 128 columns are as fast on the kernel below once every CU has several chains: four
+    // per CU (B = 1024, K = 6): bf16 d = 132 70 us there, 81 here; fp32 d = 252 274 and 292.  At two per CU this one is
+    // ahead (fp32 d = 220, B = 512, K = 8: 170 and 146).
+    const bool many_chains = d % 4 == 0 && d > 128 && B >= 4 * device_compute_units();
+    if (d <= 256 && d > 16 && !many_chains) {
         auto run = [&](auto kern) {
             hipLaunchKernelGGL(kern, dim3(B), dim3(1024), 0, stream, static_cast<const Tin*>(mats),
                                static_cast<const float*>(g), static_cast<float*>(out), K, d);

@@ -174,6 +174,24 @@ def test_cotangent_chain_rows_in_registers(rank, bsz, count, dtype, device):
     assert float(((out.double() - truth).abs() / scale)[finite].max()) <= 1e-5
 
 
+@pytest.mark.parametrize("dtype,rank", [(torch.float32, 184), (torch.float32, 252), (torch.bfloat16, 132), (torch.float16, 204)])
+@pytest.mark.parametrize("bsz", [3, 1023, 1024])
+def test_cotangent_chain_rows_of_many_chains(bsz, dtype, rank, device):
+    """Rows of whole 4-element pieces: in registers for few chains, one at a time from four chains per CU on (256 CUs)."""
+    from latent_bounded_interfaces_amd.hip.interface import suffix_scan_cotangents
+
+    gen = torch.Generator(device=device).manual_seed(rank)
+    mats = (torch.randn(bsz, 3, rank, rank, generator=gen, device=device) * rank ** -0.5).to(dtype)
+    g = torch.randn(bsz, rank, generator=gen, device=device)
+    out = suffix_scan_cotangents(mats, g)
+    assert torch.equal(out[:, 3], g)
+    want = g.double()
+    for r in (2, 1, 0):
+        want = torch.bmm(mats[:, r].double(), want.unsqueeze(-1)).squeeze(-1)
+        err = (out[:, r].double() - want).abs().amax() / want.abs().amax()
+        assert float(err) <= 1e-5
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("bsz,count", [(1, 2), (3, 5), (13, 128), (64, 128), (64, 9), (65, 11)])
 def test_cotangent_chain_on_four_workgroups_per_element(bsz, count, dtype, device):
