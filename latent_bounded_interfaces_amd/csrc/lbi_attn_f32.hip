@@ -657,15 +657,25 @@ int launch_with(const Args& a) {
 }
 
 // How many waves of a workgroup take different directions: as many as there are direction groups (MAX at most: what the
-// d_out tiles leave of the LDS), fewer where that leaves fewer waves without a direction.
-template <int DH, int PB, int MAX>
+// d_out tiles leave of the LDS), fewer where that leaves fewer waves without a direction.  One where few workgroups of one
+// or two row tiles leave half of the CUs idle anyway: a tile of one direction is loaded sooner (B=4 H=8 T=32 Dh=33 P=4:
+// 39 -> 33 us; with a workgroup for every CU or more it takes up to twice as long).
+template <int DH, int PB, int MAX, bool VEC>
 int launch_directions(const Args& a) {
     const int pgroups = (a.P + PB - 1) / PB;
     auto padded = [&](int dw) { return (pgroups + dw - 1) / dw * dw; };
+    if (a.T_len <= 2 * TILE && (long long)a.B * a.H * pgroups <= device_compute_units() / 2) return launch_with<DH, PB, 1, VEC>(a);
     if constexpr (MAX >= 4)
-        if (padded(4) == padded(2) && pgroups > 2) return launch_with<DH, PB, 4, true>(a);
-    if (padded(2) == pgroups || pgroups > 2) return launch_with<DH, PB, 2, true>(a);
-    return launch_with<DH, PB, 1, true>(a);
+        if (padded(4) == padded(2) && pgroups > 2) return launch_with<DH, PB, 4, VEC>(a);
+    if (padded(2) == pgroups || pgroups > 2) return launch_with<DH, PB, 2, VEC>(a);
+    return launch_with<DH, PB, 1, VEC>(a);
+}
+
+// Two directions per wave where that still gives every SIMD a wave: below, a call is as long as its longest wave.
+// B=1 H=2 T=1000 Dh=64 P=8: 637 us with two, 430 with one; B=4 H=8 T=512 Dh=64 P=2: 329 and 226.
+bool two_directions(const Args& a) {
+    const long long waves = (long long)a.B * a.H * ((a.P + 1) / 2) * ((a.T_len + TILE - 1) / TILE);
+    return a.P >= 2 && waves >= 4LL * device_compute_units();
 }
 
 }  // namespace
@@ -680,14 +690,14 @@ int launch(const void* q, const void* k, const void* v, const void* d_out, void*
     uintptr_t bits = 0;
     for (const void* p : {q, k, v, d_out}) bits |= reinterpret_cast<uintptr_t>(p);
     if (dh % 4 != 0 || bits % 16 != 0) {
-        if (dh <= 32) return launch_with<32, 1, 1, false>(a);
-        if (dh <= 64) return launch_with<64, 1, 1, false>(a);
-        return dh <= 96 ? launch_with<96, 1, 1, false>(a) : launch_with<128, 1, 1, false>(a);
+        if (dh <= 32) return launch_directions<32, 1, 4, false>(a);
+        if (dh <= 64) return launch_directions<64, 1, 4, false>(a);
+        return dh <= 96 ? launch_directions<96, 1, 4, false>(a) : launch_directions<128, 1, 2, false>(a);
     }
-    if (dh <= 32) return P >= 2 ? launch_directions<32, 2, 4>(a) : launch_with<32, 1, 1, true>(a);
-    if (dh <= 64) return P >= 2 ? launch_directions<64, 2, 4>(a) : launch_with<64, 1, 1, true>(a);
-    if (dh <= 96) return launch_directions<96, 1, 4>(a);
-    return launch_directions<128, 1, 2>(a);
+    if (dh <= 32) return two_directions(a) ? launch_directions<32, 2, 4, true>(a) : launch_directions<32, 1, 4, true>(a);
+    if (dh <= 64) return two_directions(a) ? launch_directions<64, 2, 4, true>(a) : launch_directions<64, 1, 4, true>(a);
+    if (dh <= 96) return launch_directions<96, 1, 4, true>(a);
+    return launch_directions<128, 1, 2, true>(a);
 }
 
 }  // namespace attn_f32

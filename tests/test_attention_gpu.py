@@ -68,6 +68,26 @@ def test_fp32_matches_oracle(seed, shape, basis, causal, device):
         assert torch.allclose(a.double(), c, atol=2e-5, rtol=2e-5)
 
 
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("shape,basis", [((4, 8, 16, 64), 1), ((4, 8, 17, 64), 1), ((16, 8, 16, 64), 8), ((16, 8, 16, 64), 7),
+                                         ((16, 8, 16, 96), 8), ((16, 8, 16, 100), 8), ((16, 32, 16, 32), 1),
+                                         ((15, 32, 16, 32), 1), ((1, 2, 48, 33), 2), ((1, 2, 49, 33), 2), ((2, 4, 48, 16), 31),
+                                         ((2, 4, 48, 16), 32), ((1, 2, 32, 8), 2), ((16, 16, 40, 33), 5), ((1, 2, 1030, 16), 2),
+                                         ((4, 8, 260, 32), 8), ((4, 8, 250, 32), 8)])
+def test_fp32_either_side_of_the_scalar_kernels(shape, basis, causal, device):
+    """Both sides of the lines between the scalar and the matrix-core kernels and between one and two directions per wave;
+    the bound of the test below."""
+    q, k, v, g = oattn.make_attention_inputs(*shape, basis, dtype=torch.float32, seed=shape[2])
+    scale = 1.0 / math.sqrt(shape[-1])
+    got = _run(q, k, v, g, device, scale=scale, causal=causal)
+    bound = (shape[2] + 2 * shape[3]) * 2.0 ** -24
+    for p in range(basis):   # one direction at a time: the dense formula holds T x T per direction
+        truth = oattn.attention_pullback_dense(q, k, v, g[:, p:p + 1], softmax_scale=scale, causal=causal, dtype=torch.float64)
+        for name, a, c in zip(("dq", "dk", "dv"), got, truth):
+            err = float((a[:, p:p + 1].double() - c).abs().max()) / max(float(c.abs().max()), float(g.abs().max()))
+            assert err <= bound, (name, p, err, bound)
+
+
 # fp32 matrix-core kernels: lengths around the 32-row tiles and the 128-row workgroups, head dims at and between the
 # compiled widths (33 and 130: scalar loads / the scalar kernels), direction counts that fill one, two or four waves of a
 # workgroup with directions and leave the last group a remainder
@@ -93,8 +113,8 @@ def test_fp32_tile_edges_against_fp64(shape, basis, causal, device):
         assert err <= bound, (name, err, bound)
 
 
-@pytest.mark.parametrize("shape,basis", [((1, 2, 1, 64), 1), ((1, 2, 70, 64), 3), ((2, 1, 33, 33), 2), ((1, 1, 130, 128), 2),
-                                         ((1, 2, 40, 16), 9)])
+@pytest.mark.parametrize("shape,basis", [((1, 2, 1, 32), 1), ((1, 2, 70, 64), 3), ((2, 1, 65, 33), 2), ((1, 1, 130, 128), 2),
+                                         ((1, 2, 30, 16), 9)])
 def test_fp32_rounding_of_delta_cancels(shape, basis, device):
     """delta is summed from the same P and dP that it is subtracted from.  With one visible key dS is exactly zero; so it is
     with zero keys and one value row repeated over a power of two of positions, where P dP sums without rounding."""
