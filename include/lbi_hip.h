@@ -163,7 +163,8 @@ int lbi_attn_pullback(const void* q, const void* k, const void* v, const void* d
  * causal or not).
  * The results are those of lbi_attn_pullback on copies padded with zeros to T = 64 n and Dh = 64 or 128, without the
  * copies.  (lbi_attn_pullback itself runs such sizes on kernels that keep the probabilities in fp32, at a small
- * fraction of the speed.)  All seven tensors 16-byte aligned; other calls return LBI_ERR_UNSUPPORTED.
+ * fraction of the speed.)  All seven tensors 16-byte aligned (LBI_ERR_INVALID otherwise, as above); other
+ * sizes, types and long non-causal calls return LBI_ERR_UNSUPPORTED, and lbi_attn_pullback takes them.
  */
 size_t lbi_attn_pullback_edge_workspace_bytes(int64_t B, int64_t H, int64_t T, int64_t Dh,
                                               int64_t P, int dtype);

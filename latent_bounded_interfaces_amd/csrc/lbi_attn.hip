@@ -153,7 +153,7 @@ extern "C" int lbi_attn_pullback_edge(const void* q, const void* k, const void* 
                        (use_small_path(t, wide, dtype) || (!causal && attn_small::supports(t, wide, dtype)));
     if (!attn_mfma::supports_edge(t, dh, dtype) || !(small || causal))
         return fail(LBI_ERR_UNSUPPORTED, "lbi_attn_pullback_edge: needs half or bfloat16, Dh a multiple of 8 up to 128, "
-                                         "and a causal call or a short sequence");
+                                         "T * Dh below 2^30, and a causal call or a short sequence");
     for (const void* ptr : {q, k, v, d_out, (const void*)dq, (const void*)dk, (const void*)dv})
         if (reinterpret_cast<uintptr_t>(ptr) % 16)
             return fail(LBI_ERR_INVALID, "lbi_attn_pullback_edge: tensors must be 16-byte aligned");

@@ -1330,8 +1330,13 @@ int launch_scan(const void* mats, void* out, const void* g, void* cot, int B, in
         // Widths between the powers of two: on matrices padded to the next one they cost three copies and
         // (128/96)^3 = 2.4, (256/160)^3 = 4.1 or (256/192)^3 = 2.4 times the products.
         // Matrices and cotangents, whole calls, padded -> here: fp32 B=16 K=50 d=96: 0.135 -> 0.068 ms; B=64 K=128,
-        // d=96 / 160 / 192: 0.78 -> 0.36, 3.1 -> 1.4, 3.4 -> 1.6 ms.  16-bit storage gains the same at 96; bf16 at 160
-        // and 192, whose padded form runs on the 16-bit matrix cores, from 1.56 to 1.50 and 1.80 to 1.70 ms.
+        // d=96 / 160 / 192: 0.78 -> 0.36, 3.1 -> 1.4, 3.4 -> 1.6 ms.  16-bit storage gains the same at 96.  bf16 is padded to
+        // 256 onto the 16-bit matrix cores with the suffix in two planes, so it gains less: at 160 and 192 0.3-0.96 times
+        // the time (1.1-1.3 for B <= 4 and K = 11), at widths padded to them 0.4-1.0 where the chain is cut into chunks and
+        // 0.8-1.6 elsewhere (B=64 K=64 d=161: 0.77 -> 1.19 ms).  It stays here for the products in fp32: error against
+        // fp64 1e-6, where two planes leave 2e-5.
+        // No wide blocks for many batch elements, as at 64 and 128: B=512 K=8 and B=1200 K=6 take 0.25-0.6 times the time
+        // of the padded form with narrow ones.
         case 96: return launch_mfma<Tin, 96, 32, 32>(mats, out, g, cot, B, K, stream);
         case 160: return launch_mfma<Tin, 160, 32, 32>(mats, out, g, cot, B, K, stream);
         case 192: return launch_mfma<Tin, 192, 32, 32>(mats, out, g, cot, B, K, stream);

@@ -124,6 +124,39 @@ def test_region_and_norm_entry_points_validate_on_the_host():
     assert f"#define LBI_ATTN_STATIC_SCRATCH_BYTES ({_lib.ATTN_STATIC_SCRATCH_BYTES >> 20}u << 20)" in header
 
 
+def test_attention_edge_entry_validates_on_the_host():
+    """What lbi_attn_pullback_edge refuses, and with which status, before any launch; a caller falls back on
+    lbi_attn_pullback for LBI_ERR_UNSUPPORTED."""
+    lib = _lib.load()
+    f16, bf16, f32 = _lib.LBI_F16, _lib.LBI_BF16, _lib.LBI_F32
+    one, odd = ctypes.c_void_p(256), ctypes.c_void_p(264)  # never dereferenced
+
+    def call(b, h, t, dh, p, *, causal=1, dtype=bf16, tensors=(one,) * 7, workspace=one, size=1 << 40):
+        return lib.lbi_attn_pullback_edge(*tensors, workspace, size, b, h, t, dh, p, 0.1, causal, dtype, None)
+
+    need = lib.lbi_attn_pullback_edge_workspace_bytes(2, 3, 1000, 40, 5, bf16)
+    assert need == 4 * (6 * 1024 + 30 * 1024 + 6 * 1024 * 64)
+    assert lib.lbi_attn_pullback_edge_workspace_bytes(2, 3, 1000, 80, 5, f16) == 4 * (6 * 1024 + 30 * 1024 + 6 * 1024 * 128)
+    for shape, dtype in (((2, 3, 200, 40, 5), bf16), ((2, 3, 128, 80, 5), f16),      # single launch: no workspace
+                         ((2, 3, 1000, 44, 5), bf16), ((2, 3, 1000, 136, 5), f16),   # not taken
+                         ((2, 3, 1000, 40, 5), f32), ((1, 1, 1 << 24, 64, 1), bf16), ((0, 3, 1000, 40, 5), bf16)):
+        assert lib.lbi_attn_pullback_edge_workspace_bytes(*shape, dtype) == 0, (shape, dtype)
+    assert call(2, 3, 1000, 44, 5) == -2 and call(2, 3, 1000, 136, 5) == -2 and call(2, 3, 1000, 40, 5, dtype=f32) == -2
+    assert call(1, 1, 1 << 24, 64, 1) == -2          # a (b, p, h) slice past 2 GiB
+    assert call(2, 3, 1000, 40, 5, causal=0) == -2   # long and non-causal
+    assert b"causal" in lib.lbi_last_error()
+    for i in range(7):
+        assert call(2, 3, 1000, 40, 5, tensors=tuple(odd if j == i else one for j in range(7))) == -1
+        assert b"aligned" in lib.lbi_last_error()
+        assert call(2, 3, 1000, 40, 5, tensors=tuple(None if j == i else one for j in range(7))) == -1
+    assert call(2, 3, 1000, 40, 5, size=need - 1) == -4 and call(2, 3, 1000, 40, 5, workspace=None) == -4
+    assert call(2, 3, 1000, 40, 5, workspace=odd) == -4
+    assert call(2, 3, -1, 40, 5) == -1 and call(2, 3, 1000, 40, 5, dtype=7) == -1
+    assert call(2, 3, 1000, 40, 0, tensors=(None,) * 7) == 0
+    header = re.sub(r"\s*\n \* ", " ", HEADER.read_text())
+    assert "All seven tensors 16-byte aligned (LBI_ERR_INVALID otherwise" in header
+
+
 def test_fp32_attention_refuses_what_no_grid_holds():
     """More groups than a grid may have threads for: refused on the host, before a kernel has written anything."""
     lib = _lib.load()
