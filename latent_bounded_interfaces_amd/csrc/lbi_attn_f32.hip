@@ -348,6 +348,8 @@ template <int PB, int DW> struct QueryShare {
 // rounding cancels as far as it can (one visible key: dS is exactly zero).  Taken as d_out . O, with O from the statistics
 // kernel, it saves these products (the whole call above 0.330 ms), but the error of dQ is 1.04 to 1.14 times as large, and
 // with an offset in V up to 1.9 times.
+// Two directions per wave at two waves per SIMD, as many as in dq: four at one wave per SIMD share S but hide less, 0.403
+// against 0.391 ms for the whole causal call (0.616 and 0.631 without the mask).
 template <int DH, int PB, int DW, bool VEC>
 __global__ __launch_bounds__(NT) void delta_kernel(const float* __restrict__ q, const float* __restrict__ k,
                                                    const float* __restrict__ v, const float* __restrict__ d_out,
