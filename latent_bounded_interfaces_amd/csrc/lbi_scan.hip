@@ -17,13 +17,14 @@
 #include <type_traits>
 
 #include "lbi_scan_colsplit.h"
+#include "lbi_scan_planes.h"
 #include "lbi_scan_split.h"
 
 namespace lbi {
 namespace {
 
 // ---------------------------------------------------------------------------------------
-// MFMA path: d in {32, 64, 128, 256}.
+// fp32 matrix cores: widths 32, 64, 96, 128 and 512.
 //
 // One wave computes an RT x CB tile of the new suffix block with
 // v_mfma_f32_32x32x2_f32.  Operand layout of that instruction (lane = 32*h + m):
@@ -47,32 +48,6 @@ namespace {
 // fragments of mats[r] that feed the MFMAs are already in registers, so a step costs
 // D/2 extra FMAs per lane (and nothing from HBM); every column block computes the chain,
 // block 0 writes it.
-// Which part of the chain a workgroup runs.  `phase` 0 is the whole chain of a batch element (K - 1 dependent
-// steps).  Phases 1-3 are the K-parallel form for batches too small to fill the chip with one chain per column
-// block: the chain is cut into C chunks; chunk c >= 1 starts at matrix b_c = cL - s and has L matrices (the last
-// one what is left), chunk 0 has the first L - s (s = 1: every chunk then has L - 1 steps in phase 3, where chunk 0,
-// which has no boundary product of its own to skip, would otherwise run one step longer than the rest), and
-//   phase 1  every chunk c >= 1 multiplies its own matrices (L - 1 steps, all chunks side by side): the last chunk's
-//            products are final results and are stored as in phase 0; a middle chunk keeps only its total
-//            T_c = mats[b_c] ... mats[b_c + L - 1], parked in out[b_c + 1], a slot phase 3 rewrites;
-//   phase 2  one chain over the totals (C - 2 steps): out[b_c] = T_c @ out[b_c + L] for c = C-2 ... 1, which are the
-//            final suffix products at the chunk boundaries (the kernel runs it with mats = the parked totals);
-//   phase 3  every chunk c <= C-2 restarts the chain from out[b_{c+1}] through its own matrices (L - 1 steps, all
-//            chunks side by side), storing each product.
-// The cotangents, if asked for, are then the finished products applied to g (suffix_apply_kernel).
-// About twice the products, a dependent depth of 2L + C - 4 instead of K - 1, no scratch memory, no atomics; the
-// summation order is fixed by (K, L), so reruns are bit-identical.
-struct ScanPlan {
-    int phase;  // 0: whole chain; 1, 2, 3: see above
-    int L;      // matrices per chunk (>= 2)
-    int C;      // chunks (>= 3)
-    // One level of the log-depth form of phase 2 (MODE 3): element c = 1 .. C-2 lives in slot out[b_c + rd], the
-    // last element is out[b_{C-1}]; the level writes elem[c] @ elem[c + off] (or elem[c] itself where c + off is
-    // past the last element) to out[b_c + wr].
-    int off, rd, wr;
-    int s;      // chunk boundaries b_c = cL - s (0 or 1)
-};
-
 // MODE 0: phase 0 only; every switch below is a compile-time constant, which keeps the whole-chain kernel at its
 // register count.  MODE 1: phases 1 and 3 (switches at run time, unit strides).  MODE 2: phase 2 (strided).
 // MODE 3: one level of phase 2 in log-depth form (one product per workgroup, all chunks side by side).
@@ -1119,7 +1094,7 @@ int launch_suffix_apply(const void* suffix, const void* g, void* cot, int64_t B,
 
 template <typename Tin, int D, int RT, int CB, bool COT, int MODE = 0>
 int launch_mfma_cot(const void* mats, void* out, const void* g, void* cot, int B, int K, hipStream_t stream,
-                    ScanPlan plan = ScanPlan{0, 0, 0, 0, 0, 0}) {
+                    ScanPlan plan = ScanPlan{0, 0, 0, 0, 0, 0, 0}) {
     constexpr int NW = D / RT;
     constexpr int NB = D / CB;
     constexpr size_t lds_bytes = ((size_t)2 * CB * (D + 4) + (COT ? 2 * D : 0)) * sizeof(float);
@@ -1156,12 +1131,12 @@ inline bool totals_in_log_depth(int L, int C) {
 // Chunking of the K-parallel scan: C chunks of L matrices.  The chunked form does twice the products, which is
 // free only while the plain form (B * nb workgroups) leaves at least half of the CUs idle (256 on a whole MI355X;
 // the count is asked of the runtime).  The dependent depth is 2L - 2 steps of the chunks plus the products of the
-// totals: C - 2 steps as a chain, or ceil(log2(C - 1)) launches of one step, each costing about 1.4 steps (12-13 us
-// against 9 us at d = 256).  L is the length with the least such depth among those whose chunks still fit two
-// workgroups per CU; where they need more than one per CU a step takes 1.7x as long.  Measured at K = 128, d = 256
-// (plain -> chunked, ms per call): B = 1: 2.36 -> 0.17 (L = 4; 0.21 at L = 8), 2: 2.36 -> 0.23, 4: 2.37 -> 0.35,
-// 8: 2.04 -> 0.59, 16: 2.05 -> 1.14, 32: 2.07 -> 2.3 (not taken); d = 128: B = 1: 0.070 at L = 4 (0.081 at L = 8),
-// 16: 0.35 -> 0.19, 48: 0.43 -> 0.57 (not taken).
+// totals: C - 2 steps as a chain, or ceil(log2(C - 1)) launches of one step, each costing about 1.4 steps.
+// L is the length with the least such depth among those whose chunks still fit two
+// workgroups per CU; where they need more than one per CU a step takes 1.7x as long.  K = 128, matrices only, us per call
+// (plain -> chunked, and the best of all lengths from 2 to 43): d = 256: B = 1: 1950 -> 126 (126), 4: 253 (253), 8: 449 (449),
+// 16: 993 -> 879 (879); d = 192: B = 1: 88 (87), 4: 152 (152); d = 160: B = 1: 79 (76), 8: 213 (196); d = 128: B = 1: 60,
+// 16: 350 -> 156, 48: 430 -> 570 (not taken).
 // Returns false when the plain chain is at least as good.  LBI_SCAN_CHUNK=0 forces the plain chain, n >= 2 chunks of n.
 inline bool plan_chunks(int B, int K, int nb, ScanPlan* plan) {
     static const int forced = std::getenv("LBI_SCAN_CHUNK") ? std::atoi(std::getenv("LBI_SCAN_CHUNK")) : -1;
@@ -1173,8 +1148,11 @@ inline bool plan_chunks(int B, int K, int nb, ScanPlan* plan) {
         const int cus = device_compute_units();
         const int groups = B * nb;  // workgroups per chunk
         if (groups > cus / 2) return false;
-        const int c_one = cus / groups + 1;      // C - 1 chunks side by side at one workgroup per CU
-        const int c_two = 2 * cus / groups + 1;  // at two
+        // C - 1 chunks side by side at one workgroup per CU, and at two.  The column blocks of a chain go to one of the eight
+        // XCDs, so what counts is how many chains the CUs of one hold: at 192 columns (6 blocks, 5 chains) 42 chunks would
+        // leave some CUs two workgroups and others none (B=1 K=128: 116 us with 43 chunks, 87 us with 33).
+        const int c_one = (cus >= 64 ? 8 * (cus / 8 / nb) : cus / nb) / B + 1;
+        const int c_two = (cus >= 64 ? 8 * (cus / 4 / nb) : 2 * cus / nb) / B + 1;
         float best = 0.0f;
         for (int cand = 2; (K + cand) / cand >= 4; ++cand) {
             const int C = (K + cand) / cand;  // ceil((K + 1) / cand): boundaries at cL - 1
@@ -1199,9 +1177,17 @@ inline bool plan_chunks(int B, int K, int nb, ScanPlan* plan) {
 
 // The three phases of ScanPlan, one launch each on `stream` (they depend on each other in that order), then the
 // cotangents from the finished products.
-template <typename Tin, int D, int RT, int CB>
-int launch_chunked(const void* mats, void* out, const void* g, void* cot, int B, int K, ScanPlan plan,
+template <typename Tin, int D>
+int launch_chunked(const void* mats, void* out, const void* g, void* cot, int B, int K, int d, ScanPlan plan,
                    hipStream_t stream) {
+    // one launch of the chunk phases on the kernel of this width
+    auto phase_launch = [&](auto in, auto mode, const void* left) {
+        using In = decltype(in);
+        constexpr int MODE = decltype(mode)::value;
+        if constexpr (D > 128) return scan_planes::launch_mode<In, D, 32, false, MODE>(left, out, nullptr, nullptr, B, K, d, stream, plan);
+        else return launch_mfma_cot<In, D, 32, 32, false, MODE>(left, out, nullptr, nullptr, B, K, stream, plan);
+    };
+    using std::integral_constant;
     // Phase 2 in log depth (totals_in_log_depth): the levels alternate between the two slots of a chunk that phase 3
     // rewrites anyway (out[cL + 1], where phase 1 parked the total, and out[cL + 2]: L >= 3) and the last one writes
     // out[cL]; no slot is read and written in the same launch.
@@ -1211,21 +1197,21 @@ int launch_chunked(const void* mats, void* out, const void* g, void* cot, int B,
         plan.phase = phase;
         int rc = LBI_OK;
         if (phase != 2) {
-            rc = launch_mfma_cot<Tin, D, RT, CB, false, 1>(mats, out, nullptr, nullptr, B, K, stream, plan);
+            rc = phase_launch(Tin{}, integral_constant<int, 1>{}, mats);
         } else if (!log_depth) {  // operands and results are fp32 products inside `out`
-            rc = launch_mfma_cot<float, D, RT, CB, false, 2>(out, out, nullptr, nullptr, B, K, stream, plan);
+            rc = phase_launch(float{}, integral_constant<int, 2>{}, out);
         } else {
             plan.rd = 1;
             for (int l = 0; l < levels && !rc; ++l) {
                 plan.off = 1 << l;
                 plan.wr = l == levels - 1 ? 0 : 3 - plan.rd;
-                rc = launch_mfma_cot<float, D, RT, CB, false, 3>(out, out, nullptr, nullptr, B, K, stream, plan);
+                rc = phase_launch(float{}, integral_constant<int, 3>{}, out);
                 plan.rd = plan.wr;
             }
         }
         if (rc) return rc;
     }
-    if (cot) return launch_suffix_apply(out, g, cot, B, K + 1, D, stream);
+    if (cot) return launch_suffix_apply(out, g, cot, B, K + 1, d, stream);
     return LBI_OK;
 }
 
@@ -1235,40 +1221,14 @@ int launch_cotangent(const void* mats, const void* g, void* out, int B, int K, i
 // batch size from which one workgroup per batch element already fills the chip (two per CU: 512 on a whole MI355X)
 inline int wide_block_batch() { return 2 * device_compute_units(); }
 
-// g / cot may be null (matrices only).  With them, the MFMA widths run the fused kernel;
+// g / cot may be null (matrices only).  With them, the matrix-core widths run the fused kernel;
 // other widths run the generic scan followed by the cotangent chain kernel.
 template <typename Tin>
 int launch_scan(const void* mats, void* out, const void* g, void* cot, int B, int K, int d, int flags,
                 hipStream_t stream) {
-    // Few batch elements: one chain per column block leaves most of the chip idle for K - 1 dependent steps, so
-    // the chain is cut into chunks that run side by side (ScanPlan), on narrow column blocks (short steps).
-    ScanPlan plan{0, 0, 0, 0, 0, 0};
-    switch (d) {
-        case 256:
-            if (plan_chunks(B, K, 8, &plan)) return launch_chunked<Tin, 256, 32, 32>(mats, out, g, cot, B, K, plan, stream);
-            break;
-        case 128:
-            if (plan_chunks(B, K, 4, &plan)) return launch_chunked<Tin, 128, 32, 32>(mats, out, g, cot, B, K, plan, stream);
-            break;
-        case 192:
-            if (plan_chunks(B, K, 6, &plan)) return launch_chunked<Tin, 192, 32, 32>(mats, out, g, cot, B, K, plan, stream);
-            break;
-        case 160:
-            if (plan_chunks(B, K, 5, &plan)) return launch_chunked<Tin, 160, 32, 32>(mats, out, g, cot, B, K, plan, stream);
-            break;
-        case 96:
-            if (plan_chunks(B, K, 3, &plan)) return launch_chunked<Tin, 96, 32, 32>(mats, out, g, cot, B, K, plan, stream);
-            break;
-        case 64:
-            if (plan_chunks(B, K, 2, &plan)) return launch_chunked<Tin, 64, 32, 32>(mats, out, g, cot, B, K, plan, stream);
-            break;
-        case 32:
-            if (plan_chunks(B, K, 1, &plan)) return launch_chunked<Tin, 32, 32, 32>(mats, out, g, cot, B, K, plan, stream);
-            break;
-        default: break;
-    }
-    switch (d) {
-        case 256: {
+    ScanPlan plan{0, 0, 0, 0, 0, 0, 0};
+    if constexpr (std::is_same<Tin, bf16_raw>::value) {
+        if (d == 256 && !plan_chunks(B, K, 8, &plan)) {
             // bf16 storage runs on the 16-bit matrix pipes: the running suffix enters each product as bf16
             // planes, the bf16 matrix as it is, accumulation in fp32.  Two planes (hi + mid, the default) round
             // that operand to 16 significand bits, 256 times finer than the bf16 rounding of the inputs
@@ -1278,38 +1238,46 @@ int launch_scan(const void* mats, void* out, const void* g, void* cot, int B, in
             // Matrices only: the column-owner kernel (a wave keeps its 16 columns of the suffix in registers, no
             // barrier between steps), with chain waves for the cotangents (below).  LBI_SCAN_ROW_OWNER=1 forces
             // the row-owner kernel, whose row dot products carry the chain.
-            // fp32 storage would need 3 x 3 planes: measured 4 % faster than the fp32-MFMA kernel and slightly
-            // less accurate (the part clocks down under dense bf16 MFMA load), so it is opt-in:
-            // LBI_SCAN_SPLIT_FP32=1.
-            if constexpr (std::is_same<Tin, bf16_raw>::value) {
-                static const bool row_owner = std::getenv("LBI_SCAN_ROW_OWNER") && std::atoi(std::getenv("LBI_SCAN_ROW_OWNER"));
-                const int planes = (flags & LBI_SCAN_EXACT_SUFFIX) ? 3 : 2;
-                if (!cot && !row_owner && K >= 1) return scan_col::launch(mats, out, B, K, planes, stream);
-                // With the chain, while all 4 B workgroups are resident at once: the same column-owner kernel with
-                // four more waves per workgroup that carry the chain (the four workgroups of a batch element
-                // exchange its vector through `cot`, which is filled with the marker word first).  Larger batches
-                // take the row-owner kernel, whose chain needs no exchange.
-                if (cot && !row_owner && K >= 1 && 4 * B <= device_compute_units()) {
-                    const size_t words = (size_t)B * (K + 1) * 256;
-                    hipLaunchKernelGGL(fill_words_kernel, dim3((unsigned)((words + 1023) / 1024)), dim3(256), 0, stream,
-                                       static_cast<unsigned*>(cot), words, kChainMarker);
-                    return scan_col::launch_with_chain(mats, out, g, cot, B, K, planes, chain_spin_limit(), stream);
-                }
-                return scan_split::launch<Tin>(mats, out, g, cot, B, K, planes, stream);
+            static const bool row_owner = std::getenv("LBI_SCAN_ROW_OWNER") && std::atoi(std::getenv("LBI_SCAN_ROW_OWNER"));
+            const int planes = (flags & LBI_SCAN_EXACT_SUFFIX) ? 3 : 2;
+            if (!cot && !row_owner && K >= 1) return scan_col::launch(mats, out, B, K, planes, stream);
+            // With the chain, while all 4 B workgroups are resident at once: the same column-owner kernel with
+            // four more waves per workgroup that carry the chain (the four workgroups of a batch element
+            // exchange its vector through `cot`, which is filled with the marker word first).  Larger batches
+            // take the row-owner kernel, whose chain needs no exchange.
+            if (cot && !row_owner && K >= 1 && 4 * B <= device_compute_units()) {
+                const size_t words = (size_t)B * (K + 1) * 256;
+                hipLaunchKernelGGL(fill_words_kernel, dim3((unsigned)((words + 1023) / 1024)), dim3(256), 0, stream,
+                                   static_cast<unsigned*>(cot), words, kChainMarker);
+                return scan_col::launch_with_chain(mats, out, g, cot, B, K, planes, chain_spin_limit(), stream);
             }
-            if constexpr (std::is_same<Tin, float>::value) {
-                static const bool split_fp32 =
-                    std::getenv("LBI_SCAN_SPLIT_FP32") && std::atoi(std::getenv("LBI_SCAN_SPLIT_FP32"));
-                if (split_fp32) return scan_split::launch<Tin>(mats, out, g, cot, B, K, 3, stream);
-            }
-            {
-                // Up to 32 batch elements the 64-wide blocks leave half the CUs or more without a workgroup: blocks
-                // of 32 columns (twice the workgroups, half the step time).
-                static const int narrow = std::getenv("LBI_SCAN_NARROW") ? std::atoi(std::getenv("LBI_SCAN_NARROW")) : -1;
-                if (narrow < 0 ? B <= device_compute_units() / 8 : narrow != 0) return launch_mfma<Tin, 256, 32, 32>(mats, out, g, cot, B, K, stream);
-            }
-            return launch_mfma<Tin, 256, 32, 64>(mats, out, g, cot, B, K, stream);
+            return scan_split::launch(mats, out, g, cot, B, K, planes, stream);
         }
+    }
+    // Few batch elements: one chain per column block leaves most of the chip idle for K - 1 dependent steps, so
+    // the chain is cut into chunks that run side by side (ScanPlan), on narrow column blocks (short steps).
+    // Widths above 128 run on the kernel of the next width it is built for, rows and columns past d empty.  (16-bit rows
+    // are brought in whole 4-byte words.)
+    if (d > 128 && d <= 256 && (sizeof(Tin) == 4 || (d % 2 == 0 && reinterpret_cast<uintptr_t>(mats) % 4 == 0))) {
+        auto run = [&](auto width) {
+            constexpr int D = decltype(width)::value;
+            if (plan_chunks(B, K, (d + 31) / 32, &plan)) return launch_chunked<Tin, D>(mats, out, g, cot, B, K, d, plan, stream);
+            // A block of 64 columns takes less than twice the time of one of 32 (about 1.4 times where those share CUs), so it is
+            // taken where it saves that in rounds over the chip.  fp32, matrices, 32 -> 64 columns, us: d = 256 B = 40 K = 60: 938
+            // -> 624; d = 192 B = 64 K = 60: 736 -> 510 (B = 100 K = 24: 445 -> 406); d = 160 B = 64 K = 60 (on the kernel of
+            // width 192): 602 -> 465, but B = 100 K = 24: 324 -> 366.  LBI_SCAN_NARROW forces one or the other.
+            static const int narrow = std::getenv("LBI_SCAN_NARROW") ? std::atoi(std::getenv("LBI_SCAN_NARROW")) : -1;
+            const int cus = device_compute_units();
+            const auto rounds = [&](int width) { return ((int64_t)B * ((d + width - 1) / width) + cus - 1) / cus; };
+            if (narrow < 0 ? 14 * rounds(64) < 10 * rounds(32) : narrow == 0)
+                return scan_planes::launch<Tin, D == 256 ? 256 : 192, 64>(mats, out, g, cot, B, K, d, stream);
+            return scan_planes::launch<Tin, D, 32>(mats, out, g, cot, B, K, d, stream);
+        };
+        if (d <= 160) return run(std::integral_constant<int, 160>{});
+        if (d <= 192) return run(std::integral_constant<int, 192>{});
+        return run(std::integral_constant<int, 256>{});
+    }
+    switch (d) {
         // Column blocks of one batch element read the same matrices.  With few batch elements, narrow blocks give
         // the chip enough workgroups, and the blocks of an element run side by side and share the matrices in L2.
         // With many, they drift apart and fetch them again (measured 1.7x / 2.4x the input bytes at d = 64 / 128),
@@ -1321,25 +1289,23 @@ int launch_scan(const void* mats, void* out, const void* g, void* cot, int B, in
             return cot ? launch_cotangent<Tin>(mats, g, cot, B, K, d, stream) : LBI_OK;
         }
         case 128:
+            if (plan_chunks(B, K, 4, &plan)) return launch_chunked<Tin, 128>(mats, out, g, cot, B, K, d, plan, stream);
             if (B >= wide_block_batch()) return launch_mfma<Tin, 128, 32, 128>(mats, out, g, cot, B, K, stream);
             return launch_mfma<Tin, 128, 32, 32>(mats, out, g, cot, B, K, stream);
         case 64:
+            if (plan_chunks(B, K, 2, &plan)) return launch_chunked<Tin, 64>(mats, out, g, cot, B, K, d, plan, stream);
             if (B >= wide_block_batch()) return launch_mfma<Tin, 64, 32, 64>(mats, out, g, cot, B, K, stream);
             return launch_mfma<Tin, 64, 32, 32>(mats, out, g, cot, B, K, stream);
-        case 32: return launch_mfma<Tin, 32, 32, 32>(mats, out, g, cot, B, K, stream);
-        // Widths between the powers of two: on matrices padded to the next one they cost three copies and
-        // (128/96)^3 = 2.4, (256/160)^3 = 4.1 or (256/192)^3 = 2.4 times the products.
-        // Matrices and cotangents, whole calls, padded -> here: fp32 B=16 K=50 d=96: 0.135 -> 0.068 ms; B=64 K=128,
-        // d=96 / 160 / 192: 0.78 -> 0.36, 3.1 -> 1.4, 3.4 -> 1.6 ms.  16-bit storage gains the same at 96.  bf16 is padded to
-        // 256 onto the 16-bit matrix cores with the suffix in two planes, so it gains less: at 160 and 192 0.3-0.96 times
-        // the time (1.1-1.3 for B <= 4 and K = 11), at widths padded to them 0.4-1.0 where the chain is cut into chunks and
-        // 0.8-1.6 elsewhere (B=64 K=64 d=161: 0.77 -> 1.19 ms).  It stays here for the products in fp32: error against
-        // fp64 1e-6, where two planes leave 2e-5.
-        // No wide blocks for many batch elements, as at 64 and 128: B=512 K=8 and B=1200 K=6 take 0.25-0.6 times the time
-        // of the padded form with narrow ones.
-        case 96: return launch_mfma<Tin, 96, 32, 32>(mats, out, g, cot, B, K, stream);
-        case 160: return launch_mfma<Tin, 160, 32, 32>(mats, out, g, cot, B, K, stream);
-        case 192: return launch_mfma<Tin, 192, 32, 32>(mats, out, g, cot, B, K, stream);
+        case 32:
+            if (plan_chunks(B, K, 1, &plan)) return launch_chunked<Tin, 32>(mats, out, g, cot, B, K, d, plan, stream);
+            return launch_mfma<Tin, 32, 32, 32>(mats, out, g, cot, B, K, stream);
+        // A width between the powers of two: matrices padded to 128 cost three copies and (128/96)^3 = 2.4 times the
+        // products.  fp32, matrices and cotangents, whole calls, padded -> here: B=16 K=50: 0.135 -> 0.068 ms; B=64 K=128:
+        // 0.78 -> 0.36 ms; 16-bit storage gains the same.  No wide blocks for many batch elements, as at 64 and 128: B=512
+        // K=8 and B=1200 K=6 take 0.25-0.6 times the time of the padded form with narrow ones.
+        case 96:
+            if (plan_chunks(B, K, 3, &plan)) return launch_chunked<Tin, 96>(mats, out, g, cot, B, K, d, plan, stream);
+            return launch_mfma<Tin, 96, 32, 32>(mats, out, g, cot, B, K, stream);
         default: break;
     }
     if (cot) {

@@ -1,15 +1,13 @@
-// Suffix scan for d = 256 on the 16-bit matrix pipes, with fp32-exact products.
+// Suffix scan for d = 256 with bf16 storage on the 16-bit matrix pipes: row-owner form with the cotangent chain.
 //
 // The fp32 MFMA rate of gfx950 is 1/16 of its bf16 rate, so the scan of d = 256 matrices
-// is bound by the matrix pipes when its products run as fp32 MFMAs.  Here every fp32
-// number x is split exactly into three bf16 numbers, x = hi + mid + lo (8 + 8 + 8
+// is bound by the matrix pipes when its products run as fp32 MFMAs.  Here every element x of the running
+// suffix is split exactly into three bf16 numbers, x = hi + mid + lo (8 + 8 + 8
 // significand bits, round-to-nearest residuals), so
-//     a * s = sum over the planes of (a_i * s_j),   each a_i * s_j exact in fp32,
-// and the products are v_mfma_f32_32x32x16_bf16 accumulated in fp32.  Nothing is dropped:
-// bf16 storage (NA = 1, the matrix is one plane) costs 3 bf16 products per fp32 product,
-// fp32 storage (NA = 3) costs 9, against 16 for one fp32 MFMA product.  The results differ
-// from the fp32-MFMA kernel only in summation order; partial products are summed in two
-// accumulators (hi*hi | everything smaller), small terms first.
+//     a * s = sum over the planes of (a * s_j),   each a * s_j exact in fp32,
+// and the products are v_mfma_f32_32x32x16_bf16 accumulated in fp32: three of them per fp32 product, against the 16 that
+// one fp32 MFMA product takes.  Partial products are summed in two
+// accumulators (hi | everything smaller), small terms first.
 //
 // Layout is that of scan_mfma_kernel: a workgroup owns 64 columns of one batch element's
 // running suffix S, streams mats[b, K-1 .. 0] once, one wave owns 32 rows.  S lives in LDS
@@ -20,12 +18,6 @@
 #pragma once
 
 #include "lbi_common.h"
-
-// Plane pairs (a_i, s_j) with i + j above this are skipped.  4 keeps all nine products of two
-// fp32 numbers (exact); 2 would drop terms of relative size 2^-24 and below.
-#ifndef LBI_SPLIT_MAX_ORDER
-#define LBI_SPLIT_MAX_ORDER 4
-#endif
 
 namespace lbi {
 namespace scan_split {
@@ -60,27 +52,17 @@ __device__ __forceinline__ f32x16 mma(u32x4 a, u32x4 b, f32x16 c) {
                                                    0);
 }
 
-// Raw chunk of a lane: 64 bytes of its row.
-//   bf16 storage: 32 consecutive k  (chunk = 64 k: the h = 0 / 1 lanes take k 0-31 / 32-63), 4 products
-//   fp32 storage: 16 consecutive k  (chunk = 32 k),                                         2 products
-template <typename Tin> struct Chunk;
-template <> struct Chunk<bf16_raw> {
-    static constexpr int K_PER_CHUNK = 64, K_PER_LANE = 32, T_STEPS = 4, NA = 1;
-};
-template <> struct Chunk<float> {
-    static constexpr int K_PER_CHUNK = 32, K_PER_LANE = 16, T_STEPS = 2, NA = 3;
-};
+// Raw chunk of a lane: 64 bytes of its row, 32 consecutive k (chunk = 64 k: the h = 0 / 1 lanes take k 0-31 / 32-63), 4 products.
+constexpr int K_PER_CHUNK = 64, K_PER_LANE = 32, T_STEPS = 4;
 
-// NP = planes of the running suffix that enter the products: 3 is exact; 2 (bf16 storage only) rounds that operand
+// NP = planes of the running suffix that enter the products: 3 is exact; 2 rounds that operand
 // to 16 significand bits (hi + mid), accumulation and stored results stay fp32.
-template <typename Tin, bool COT, int NP>
-__global__ __launch_bounds__(NT) void scan_split_kernel(const Tin* __restrict__ mats, float* __restrict__ out,
+template <bool COT, int NP>
+__global__ __launch_bounds__(NT) void scan_split_kernel(const bf16_raw* __restrict__ mats, float* __restrict__ out,
                                                         const float* __restrict__ g, float* __restrict__ cot, int B,
                                                         int K) {
-    using C = Chunk<Tin>;
-    constexpr int NCH = D / C::K_PER_CHUNK;  // chunks per step: 4 (bf16) or 8 (fp32)
+    constexpr int NCH = D / K_PER_CHUNK;  // chunks per step
     constexpr int RING = 4, AHEAD = RING - 1;
-    constexpr int NA = C::NA;
     static_assert(NCH % RING == 0, "ring slots must be compile-time constants");
 
     extern __shared__ __align__(16) char smem[];
@@ -95,13 +77,13 @@ __global__ __launch_bounds__(NT) void scan_split_kernel(const Tin* __restrict__ 
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, h = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int row0 = wave * RT;
-    const Tin* mats_b = mats + (size_t)b * K * D * D;
+    const bf16_raw* mats_b = mats + (size_t)b * K * D * D;
     float* out_b = out + (size_t)b * (K + 1) * D * D;
     auto lds_barrier = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 
     // Identity tail, first suffix (= mats[K-1]) and its planes.
     {
-        const Tin* a_last = mats_b + (size_t)(K - 1) * D * D;
+        const bf16_raw* a_last = mats_b + (size_t)(K - 1) * D * D;
         float* o_last = out_b + (size_t)(K - 1) * D * D;
         float* o_eye = out_b + (size_t)K * D * D;
         for (int idx = tid; idx < D * CB; idx += NT) {
@@ -133,17 +115,17 @@ __global__ __launch_bounds__(NT) void scan_split_kernel(const Tin* __restrict__ 
     if (K < 2) return;
 
     // lane's 64 bytes of chunk kc of mats[r]: row row0 + m, elements kc*K_PER_CHUNK + h*K_PER_LANE + [0, K_PER_LANE)
-    auto load_raw = [&](u32x4 (&dst)[4], const Tin* base) {
+    auto load_raw = [&](u32x4 (&dst)[4], const bf16_raw* base) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) dst[q] = *reinterpret_cast<const u32x4*>(reinterpret_cast<const char*>(base) + 16 * q);
     };
-    const Tin* a_lane = mats_b + (size_t)(row0 + m) * D + h * C::K_PER_LANE;  // + r*D*D + kc*K_PER_CHUNK
+    const bf16_raw* a_lane = mats_b + (size_t)(row0 + m) * D + h * K_PER_LANE;  // + r*D*D + kc*K_PER_CHUNK
     u32x4 ring[RING][4];
 #pragma unroll
-    for (int c = 0; c < AHEAD; ++c) load_raw(ring[c], a_lane + (size_t)(K - 2) * D * D + c * C::K_PER_CHUNK);
+    for (int c = 0; c < AHEAD; ++c) load_raw(ring[c], a_lane + (size_t)(K - 2) * D * D + c * K_PER_CHUNK);
 
     // byte offset of this lane's B fragments inside a plane: column m (+32 j), k = h*K_PER_LANE (+ chunk, + 8 t)
-    const unsigned b_lane = (unsigned)(m * PITCH + h * C::K_PER_LANE) * 2;
+    const unsigned b_lane = (unsigned)(m * PITCH + h * K_PER_LANE) * 2;
     int cur = 0;  // vbuf parity
     for (int r = K - 2; r >= 0; --r) {
         f32x16 acc[2][2];  // [0]: hi*hi products, [1]: all smaller ones
@@ -164,76 +146,47 @@ __global__ __launch_bounds__(NT) void scan_split_kernel(const Tin* __restrict__ 
             }
         };
         load_b(bfr[0], 0);
-        const Tin* a_r = a_lane + (size_t)r * D * D;
-        const Tin* a_wrap = a_lane + (size_t)(r > 0 ? r - 1 : 0) * D * D;
-        const float* v_old = vbuf + cur * D + h * C::K_PER_LANE;
+        const bf16_raw* a_r = a_lane + (size_t)r * D * D;
+        const bf16_raw* a_wrap = a_lane + (size_t)(r > 0 ? r - 1 : 0) * D * D;
+        const float* v_old = vbuf + cur * D + h * K_PER_LANE;
 #pragma unroll
         for (int kc = 0; kc < NCH; ++kc) {
             const int slot = kc % RING;
             const int ahead = kc + AHEAD;
             load_raw(ring[(slot + AHEAD) % RING],
-                     ahead < NCH ? a_r + ahead * C::K_PER_CHUNK : a_wrap + (ahead - NCH) * C::K_PER_CHUNK);
-            // A fragments of this chunk, one per plane and product step
-            u32x4 afr[NA][C::T_STEPS];
-            if (NA == 1) {
-#pragma unroll
-                for (int t = 0; t < C::T_STEPS; ++t) afr[0][t] = ring[slot][t];
-            } else {
-#pragma unroll
-                for (int t = 0; t < C::T_STEPS; ++t)
-#pragma unroll
-                    for (int w = 0; w < 4; ++w) {
-                        const u32x4 raw = ring[slot][2 * t + (w >> 1)];
-                        const float x0 = __uint_as_float(raw[2 * (w & 1)]), x1 = __uint_as_float(raw[2 * (w & 1) + 1]);
-                        unsigned hi, mid, lo;
-                        split2(x0, x1, hi, mid, lo);
-                        afr[0][t][w] = hi;
-                        afr[NA > 1 ? 1 : 0][t][w] = mid;
-                        afr[NA > 2 ? 2 : 0][t][w] = lo;
-                    }
-            }
+                     ahead < NCH ? a_r + ahead * K_PER_CHUNK : a_wrap + (ahead - NCH) * K_PER_CHUNK);
             if (COT) {
-                const float* vk = v_old + kc * C::K_PER_CHUNK;
+                const float* vk = v_old + kc * K_PER_CHUNK;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    if (NA == 1) {  // 8 bf16 per 16 bytes
-                        const f32x4 va = *reinterpret_cast<const f32x4*>(vk + 8 * q);
-                        const f32x4 vb = *reinterpret_cast<const f32x4*>(vk + 8 * q + 4);
-                        const u32x4 raw = ring[slot][q];
-                        vdot = fmaf(bf16_lo(raw[0]), va[0], vdot);
-                        vdot = fmaf(bf16_hi(raw[0]), va[1], vdot);
-                        vdot = fmaf(bf16_lo(raw[1]), va[2], vdot);
-                        vdot = fmaf(bf16_hi(raw[1]), va[3], vdot);
-                        vdot = fmaf(bf16_lo(raw[2]), vb[0], vdot);
-                        vdot = fmaf(bf16_hi(raw[2]), vb[1], vdot);
-                        vdot = fmaf(bf16_lo(raw[3]), vb[2], vdot);
-                        vdot = fmaf(bf16_hi(raw[3]), vb[3], vdot);
-                    } else {  // 4 floats per 16 bytes
-                        const f32x4 va = *reinterpret_cast<const f32x4*>(vk + 4 * q);
-                        const u32x4 raw = ring[slot][q];
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) vdot = fmaf(__uint_as_float(raw[e]), va[e], vdot);
-                    }
+                    const f32x4 va = *reinterpret_cast<const f32x4*>(vk + 8 * q);
+                    const f32x4 vb = *reinterpret_cast<const f32x4*>(vk + 8 * q + 4);
+                    const u32x4 raw = ring[slot][q];
+                    vdot = fmaf(bf16_lo(raw[0]), va[0], vdot);
+                    vdot = fmaf(bf16_hi(raw[0]), va[1], vdot);
+                    vdot = fmaf(bf16_lo(raw[1]), va[2], vdot);
+                    vdot = fmaf(bf16_hi(raw[1]), va[3], vdot);
+                    vdot = fmaf(bf16_lo(raw[2]), vb[0], vdot);
+                    vdot = fmaf(bf16_hi(raw[2]), vb[1], vdot);
+                    vdot = fmaf(bf16_lo(raw[3]), vb[2], vdot);
+                    vdot = fmaf(bf16_hi(raw[3]), vb[3], vdot);
                 }
             }
             // B fragments (3 planes x 2 column tiles) are read one product step ahead of use.
 #pragma unroll
-            for (int t = 0; t < C::T_STEPS; ++t) {
-                const int u = kc * C::T_STEPS + t;           // product step within the suffix step
+            for (int t = 0; t < T_STEPS; ++t) {
+                const int u = kc * T_STEPS + t;           // product step within the suffix step
                 const int slot_b = u & 1;
-                if (u + 1 < NCH * C::T_STEPS) {
-                    const int kc_n = (u + 1) / C::T_STEPS, t_n = (u + 1) % C::T_STEPS;
-                    load_b(bfr[slot_b ^ 1], kc_n * C::K_PER_CHUNK + 8 * t_n);
+                if (u + 1 < NCH * T_STEPS) {
+                    const int kc_n = (u + 1) / T_STEPS, t_n = (u + 1) % T_STEPS;
+                    load_b(bfr[slot_b ^ 1], kc_n * K_PER_CHUNK + 8 * t_n);
                 }
 #pragma unroll
-                for (int sp = NP - 1; sp >= 0; --sp)  // small planes first
-#pragma unroll
-                    for (int ap = NA - 1; ap >= 0; --ap) {
-                        if (ap + sp > LBI_SPLIT_MAX_ORDER) continue;
-                        const int o = ap + sp == 0 ? 0 : 1;
-                        acc[o][0] = mma(afr[ap][t], bfr[slot_b][sp][0], acc[o][0]);
-                        acc[o][1] = mma(afr[ap][t], bfr[slot_b][sp][1], acc[o][1]);
-                    }
+                for (int sp = NP - 1; sp >= 0; --sp) {  // small planes first
+                    const int o = sp == 0 ? 0 : 1;
+                    acc[o][0] = mma(ring[slot][t], bfr[slot_b][sp][0], acc[o][0]);
+                    acc[o][1] = mma(ring[slot][t], bfr[slot_b][sp][1], acc[o][1]);
+                }
             }
             __builtin_amdgcn_sched_barrier(0);
         }
@@ -273,31 +226,28 @@ __global__ __launch_bounds__(NT) void scan_split_kernel(const Tin* __restrict__ 
     }
 }
 
-template <typename Tin, int NP>
+template <int NP>
 int launch_planes(const void* mats, void* out, const void* g, void* cot, int B, int K, hipStream_t stream) {
     const size_t lds_bytes = (size_t)NP * PLANE * 2 + (cot ? 2 * D * sizeof(float) : 0);
     const dim3 grid(((B + 7) / 8) * 8 * NB);
-    if (cot) {
-        auto kern = scan_split_kernel<Tin, true, NP>;
-        if (int rc = ensure_dynamic_lds<&scan_split_kernel<Tin, true, NP>>(lds_bytes)) return rc;
-        hipLaunchKernelGGL(kern, grid, dim3(NT), lds_bytes, stream, static_cast<const Tin*>(mats),
+    auto run = [&](auto kern) {
+        hipLaunchKernelGGL(kern, grid, dim3(NT), lds_bytes, stream, static_cast<const bf16_raw*>(mats),
                            static_cast<float*>(out), static_cast<const float*>(g), static_cast<float*>(cot), B, K);
+    };
+    if (cot) {
+        if (int rc = ensure_dynamic_lds<&scan_split_kernel<true, NP>>(lds_bytes)) return rc;
+        run(scan_split_kernel<true, NP>);
     } else {
-        auto kern = scan_split_kernel<Tin, false, NP>;
-        if (int rc = ensure_dynamic_lds<&scan_split_kernel<Tin, false, NP>>(lds_bytes)) return rc;
-        hipLaunchKernelGGL(kern, grid, dim3(NT), lds_bytes, stream, static_cast<const Tin*>(mats),
-                           static_cast<float*>(out), static_cast<const float*>(nullptr), static_cast<float*>(nullptr),
-                           B, K);
+        if (int rc = ensure_dynamic_lds<&scan_split_kernel<false, NP>>(lds_bytes)) return rc;
+        run(scan_split_kernel<false, NP>);
     }
     LBI_HIP_CHECK(hipGetLastError());
     return LBI_OK;
 }
 
-// planes: 3 = exact; 2 = 16-bit suffix operand, bf16 storage only (fp32 storage always runs exact).
-template <typename Tin>
-int launch(const void* mats, void* out, const void* g, void* cot, int B, int K, int planes, hipStream_t stream) {
-    if (planes < 3 && Chunk<Tin>::NA == 1) return launch_planes<Tin, 2>(mats, out, g, cot, B, K, stream);
-    return launch_planes<Tin, 3>(mats, out, g, cot, B, K, stream);
+// planes: 3 = exact; 2 = 16-bit suffix operand.
+inline int launch(const void* mats, void* out, const void* g, void* cot, int B, int K, int planes, hipStream_t stream) {
+    return planes < 3 ? launch_planes<2>(mats, out, g, cot, B, K, stream) : launch_planes<3>(mats, out, g, cot, B, K, stream);
 }
 
 }  // namespace scan_split

@@ -29,21 +29,30 @@ def _validate(mats: torch.Tensor) -> tuple[int, int, int]:
     return bsz, count, rank
 
 
-#: interface widths the matrix-core scan kernels are built for
-_MFMA_WIDTHS = (32, 64, 96, 128, 160, 192, 256, 512)
+#: widths up to 128 and above 256 the matrix-core scan kernels are built for
+_MFMA_WIDTHS = (32, 64, 96, 128, 512)
 
 
-def _padded_width(rank: int) -> int:
-    """The matrix-core width a scan of ``rank x rank`` matrices is padded to, or ``rank`` itself when it is one
-    already, too small to matter (<= 16) or beyond the largest."""
+def _padded_width(mats: torch.Tensor) -> int:
+    """The width a scan is padded to by copies: a width of the list above, or the width itself where the kernels take it as
+    it is (129 ... 256), where it is too small to matter (<= 16) or beyond the largest.  Odd widths of 16-bit storage are
+    brought to an even one: rows are read in whole 4-byte words.  (Of bf16 those above 192 go to 256, whose own kernel is
+    up to 1.3 times faster when the batch fills the chip.)"""
+    rank = int(mats.shape[-1])
+    if 128 < rank <= 256:
+        if mats.element_size() == 4 or rank % 2 == 0:
+            return rank
+        return 256 if mats.dtype == torch.bfloat16 and rank > 192 else rank + 1
     if rank <= 16 or rank in _MFMA_WIDTHS:
         return rank
     return next((w for w in _MFMA_WIDTHS if w > rank), rank)
 
 
 def _aligned(t: torch.Tensor, rank: int) -> torch.Tensor:
-    """Widths whose calls on a tensor off the 16-byte grid used to run on its padded copy: on a plain copy now."""
-    return t.clone() if rank in (96, 160, 192) and t.data_ptr() % 16 else t
+    """Tensors whose calls off the 16-byte grid used to run on padded copies: on plain copies now."""
+    if rank != 96 and not 128 < rank < 256:
+        return t
+    return t.clone() if t.data_ptr() % (16 if rank % 4 == 0 else 4) else t
 
 
 def suffix_scan_pullbacks(mats: torch.Tensor, *, exact_suffix: bool = False) -> torch.Tensor:
@@ -54,7 +63,7 @@ def suffix_scan_pullbacks(mats: torch.Tensor, *, exact_suffix: bool = False) -> 
     error <= 2e-4 where 16-bit storage is asked 2e-2), with ``exact_suffix=True`` three (its exact fp32 value: only
     the rounding of fp32 accumulation is left, ~1e-5 at K = 128; half again as many products)."""
     bsz, count, rank = _validate(mats)
-    width = _padded_width(rank)
+    width = _padded_width(mats)
     if width != rank and mats.numel():
         # Products of zero-padded matrices are the zero-padded products, and the identity tail cuts to the
         # identity: run the matrix-core kernel of the next width instead of the scalar kernel (several times
@@ -108,7 +117,7 @@ def suffix_scan_pullbacks_and_cotangents(mats: torch.Tensor, g: torch.Tensor, *,
     bsz, count, rank = _validate(mats)
     if g.dim() != 2 or g.shape[0] != bsz or g.shape[1] != rank:
         raise ValueError("g must have shape [B, R]")
-    width = _padded_width(rank)
+    width = _padded_width(mats)
     if width != rank and mats.numel():
         pad = width - rank  # see suffix_scan_pullbacks; a zero-padded g leaves the first `rank` cotangents unchanged
         wide, wide_cot = suffix_scan_pullbacks_and_cotangents(torch.nn.functional.pad(mats, (0, pad, 0, pad)),

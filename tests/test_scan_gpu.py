@@ -156,6 +156,47 @@ def test_widths_between_powers_of_two(rank, bsz, count, dtype, device):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rank", [130, 192, 256])
+@pytest.mark.parametrize("bsz,count", [(1, 40), (2, 5), (40, 4)])
+@pytest.mark.parametrize("kind", ["inf", "nan", "huge", "tiny", "zero_rows"])
+def test_values_outside_the_range_of_the_planes(kind, rank, bsz, count, dtype, device):
+    """Above 128 columns an fp32 number is the sum of three bf16 ones; what they cannot hold (infinities, values next to
+    the largest, products far below 1) comes out as fp32 arithmetic gives it, and stays where it belongs."""
+    from latent_bounded_interfaces_amd.hip.interface import suffix_scan_pullbacks, suffix_scan_pullbacks_and_cotangents
+
+    if dtype == torch.bfloat16 and rank == 256 and (bsz, count) != (1, 40):
+        pytest.skip("two planes without a check: the width-256 bf16 kernels")
+    if kind in ("inf", "nan") and bsz == 1:
+        pytest.skip("chunks side by side: infinities cancel in another order than along one chain")
+    mats, g = oscan.make_scan_inputs(bsz, count, rank, kind="randn", seed=rank + count)
+    at = (bsz - 1, count // 2)
+    if kind == "inf":
+        mats[at][3, rank - 2] = float("inf")
+    elif kind == "nan":
+        mats[at][rank - 1, 0] = float("nan")
+    elif kind == "huge":   # the largest finite value, which rounds to infinity in bf16, through identities
+        mats[:] = torch.eye(rank)
+        mats[at][5, rank - 1] = torch.finfo(dtype).max
+        g *= 0.1 / g.abs().max()
+    elif kind == "tiny":   # down to 2^-120 over the chain, and one block of rows only
+        mats[at[0]] *= 2.0 ** (-120.0 / count)
+        mats[0, count - 1, 32:64] *= 2.0 ** -12
+    else:
+        mats[at][40:80] = 0.0
+    mats = mats.to(dtype)
+    truth = oscan.suffix_scan_sequential(mats.float(), dtype=torch.float64)
+    want = oscan.suffix_cotangents_sequential(mats.double(), g.double())
+    out, cot = suffix_scan_pullbacks_and_cotangents(mats.to(device), g.to(device))
+    assert torch.equal(torch.nan_to_num(out), torch.nan_to_num(suffix_scan_pullbacks(mats.to(device)))) or bsz == 40
+    for got, ref in ((out.cpu().double(), truth), (cot.cpu().double()[:, :, None], want[:, :, None])):
+        assert torch.equal(got.isnan(), ref.isnan())
+        ok = ref.isfinite()
+        assert torch.equal(got[~ok & ~ref.isnan()], ref[~ok & ~ref.isnan()])
+        scale = torch.where(ok, ref.abs(), 0.0).amax(-1, keepdim=True).clamp_min(1e-37)   # of every row
+        assert float((torch.where(ok, (got - ref).abs(), 0.0) / scale).max()) <= 5e-5     # 40 roundings a row, ~1e-5 seen
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rank", [17, 63, 65, 127, 129, 191, 193, 198, 254, 255])
 @pytest.mark.parametrize("bsz,count", [(1, 1), (3, 9)])
 def test_cotangent_chain_rows_in_registers(rank, bsz, count, dtype, device):
