@@ -51,10 +51,15 @@ namespace {
 // MODE 0: phase 0 only; every switch below is a compile-time constant, which keeps the whole-chain kernel at its
 // register count.  MODE 1: phases 1 and 3 (switches at run time, unit strides).  MODE 2: phase 2 (strided).
 // MODE 3: one level of phase 2 in log-depth form (one product per workgroup, all chunks side by side).
-template <typename Tin, int D, int RT, int CB, bool COT, int MODE>
+//
+// RAGGED: the matrices have d < D rows and columns, which are read and written where they lie.  Rows past the last one
+// are zero on chip, and so is what a row's last chunk holds past its end (of the next row or matrix: the last matrix
+// is no left operand); stores past the end go to a descriptor's outside.  Whole calls, matrices and cotangents, fp32, copies padded to
+// the next width -> here: see launch_scan.
+template <typename Tin, int D, int RT, int CB, bool COT, int MODE, bool RAGGED>
 __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
     const Tin* __restrict__ mats, float* __restrict__ out, const float* __restrict__ g,
-    float* __restrict__ cot, int B, int K, ScanPlan plan) {
+    float* __restrict__ cot, int B, int K, int d_rt, ScanPlan plan) {
     constexpr int NW = D / RT;          // waves per workgroup
     constexpr int NT = 64 * NW;         // threads
     constexpr int RTILES = RT / 32;
@@ -62,7 +67,8 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
     constexpr int NB = D / CB;          // column blocks per batch element
     constexpr int PITCH = D + 4;
     constexpr int NCH = D / 32;         // k chunks per step
-    constexpr size_t DD = (size_t)D * D;
+    const int d = RAGGED ? d_rt : D;    // rows and columns of a matrix
+    const size_t DD = (size_t)d * d;
 
     extern __shared__ __align__(16) float lds[];  // [2][CB][PITCH], then (COT) [2][D]
     float* vbuf = lds + 2 * CB * PITCH;
@@ -82,7 +88,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
         e = id / NB;
         c0 = (id % NB) * CB;
     }
-    if (e >= E) return;
+    if (e >= E || (RAGGED && c0 >= d)) return;
     const int b = e / nseg;
     const int seg = e - b * nseg;
 
@@ -134,6 +140,13 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
         const int partner = c + plan.off;
         if (partner > plan.C - 1) {
             // nothing to the right at this distance: the element is complete, it moves to the level's output slot
+            if constexpr (RAGGED) {
+                for (int idx = threadIdx.x; idx < d * CB; idx += NT) {
+                    const int row = idx / CB, col = c0 + idx % CB;
+                    if (col < d) dst[(size_t)row * d + col] = left[(size_t)row * d + col];
+                }
+                return;
+            }
             for (int idx = threadIdx.x; idx < D * CB / 4; idx += NT) {
                 const int row = idx / (CB / 4), q = idx % (CB / 4);
                 *reinterpret_cast<f32x4*>(dst + (size_t)row * D + c0 + 4 * q) =
@@ -163,7 +176,34 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
     {
         float* o_last = out_b + (size_t)(K - 1) * DD;
         float* o_eye = out_b + (size_t)K * DD;
-        if (MODE != 0) {
+        if (RAGGED) {
+            static_assert((D * CB) % NT == 0, "start-state fill");
+            constexpr int N = D * CB / NT;
+            float val[N];
+            const int col = tid % CB, first = tid / CB;
+            static_assert(NT % CB == 0, "a thread keeps its column");
+#pragma unroll
+            for (int u = 0; u < N; ++u) {
+                const int row = first + u * (NT / CB);
+                const size_t off = row < d && c0 + col < d ? (size_t)row * d + c0 + col : 0;
+                val[u] = from_a ? to_f32(init_a[off]) : init_s[off];
+            }
+#pragma unroll
+            for (int u = 0; u < N; ++u) {
+                const int row = first + u * (NT / CB);
+                if (!(row < d && c0 + col < d)) val[u] = 0.0f;
+                lds[col * PITCH + row] = val[u];
+            }
+            if (write_tail && c0 + col < d) {
+                for (int u = 0; u < N; ++u) {
+                    const int row = first + u * (NT / CB);
+                    if (row < d) {
+                        o_last[(size_t)row * d + c0 + col] = val[u];
+                        o_eye[(size_t)row * d + c0 + col] = row == c0 + col ? 1.0f : 0.0f;
+                    }
+                }
+            }
+        } else if (MODE != 0) {
             // the chunk phases are short chains: four elements per load, all loads of a thread in flight
             constexpr int Q = CB / 4;
             static_assert((D * Q) % NT == 0, "start-state fill");
@@ -197,11 +237,14 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
         }
         if (COT) {
             // first vector of the chain: (start state) @ g, one row per thread, once per kernel
-            const float* g_b = g + (size_t)b * D;
-            float* cot_b = cot + (size_t)b * (K + 1) * D;
+            const float* g_b = g + (size_t)b * d;
+            float* cot_b = cot + (size_t)b * (K + 1) * d;
             for (int row = tid; row < D; row += NT) {
                 float acc = 0.0f;
-                for (int k4 = 0; k4 < D; k4 += 4) {
+                if (RAGGED) {
+                    if (row < d)
+                        for (int k = 0; k < d; ++k) acc = fmaf(to_f32(init_a[(size_t)row * d + k]), g_b[k], acc);
+                } else for (int k4 = 0; k4 < D; k4 += 4) {
                     const f32x4 a4 = from_a ? load4(init_a + row * D + k4) : load4(init_s + row * D + k4);
                     acc = fmaf(a4[0], g_b[k4], acc);
                     acc = fmaf(a4[1], g_b[k4 + 1], acc);
@@ -209,9 +252,9 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
                     acc = fmaf(a4[3], g_b[k4 + 3], acc);
                 }
                 vbuf[row] = acc;
-                if (c0 == 0) {
-                    cot_b[(size_t)K * D + row] = g_b[row];
-                    cot_b[(size_t)(K - 1) * D + row] = acc;
+                if (c0 == 0 && row < d) {
+                    cot_b[(size_t)K * d + row] = g_b[row];
+                    cot_b[(size_t)(K - 1) * d + row] = acc;
                 }
             }
         }
@@ -220,13 +263,23 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
     if (r_top < r_lo) return;
 
     // Lane's slice of mats[r]: rows row0 + 32*i + m, k = 32*kc + 16*h + [0, 16).
+    static_assert(!RAGGED || RTILES == 1, "rows of one tile");
     auto load_a = [&](f32x4 (&dst)[RTILES][4], const Tin* base) {
 #pragma unroll
         for (int i = 0; i < RTILES; ++i)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) dst[i][q] = load4(base + (size_t)i * 32 * D + q * 4);
+            for (int q = 0; q < 4; ++q) {
+                if constexpr (RAGGED) dst[i][q] = scan_planes::load4_at(base + q * 4);
+                else dst[i][q] = load4(base + (size_t)i * 32 * D + q * 4);
+            }
     };
-    const Tin* a_lane = a_base + (size_t)(row0 + m) * D + h * 16;  // + r*a_stride + kc*32
+    const Tin* a_lane = a_base + (size_t)(!RAGGED || row0 + m < d ? row0 + m : 0) * d + h * 16;  // + r*a_stride + kc*32
+    unsigned lane_at[CTILES];   // RAGGED: byte offset of this lane's first row in a column of a result
+#pragma unroll
+    for (int j = 0; j < CTILES; ++j) {
+        const int c = c0 + 32 * j + m;
+        lane_at[j] = c < d ? (unsigned)((row0 + 4 * h) * d + c) * 4 : 0x80000000u;
+    }
 
     // mats chunks are prefetched RING-1 chunks ahead into a register ring; the ring
     // index of a chunk is kc % RING, the same in every step because RING divides NCH.
@@ -271,6 +324,13 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
             const int slot = (NCH == 1 ? sub : kc) % RING;
             const int ahead = kc + AHEAD;
             load_a(a_ring[(slot + AHEAD) % RING], ahead < NCH ? a_r + ahead * 32 : a_wrap + (ahead - NCH) * 32);
+            if (RAGGED && kc == NCH - 1) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+                        if (kc * 32 + h * 16 + q * 4 + t >= d) a_ring[slot][0][q][t] = 0.0f;
+            }
             f32x4 bfrag[CTILES][4];
 #pragma unroll
             for (int j = 0; j < CTILES; ++j)
@@ -320,6 +380,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
         const bool store = store_all || rs == r_lo;
         float* o_r = o_base + (size_t)(store_all ? rs : rs + 1) * o_stride;
         float* st_new = lds + (cur ^ 1) * (CB * PITCH);
+        const __amdgpu_buffer_rsrc_t o_rows = scan_planes::rows(o_r, store ? (unsigned)DD * 4 : 0);
 #pragma unroll
         for (int i = 0; i < RTILES; ++i)
 #pragma unroll
@@ -330,21 +391,36 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
                     const int col = j * 32 + m;
                     f32x4 v4 = {acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2],
                                 acc[i][j][4 * g + 3]};
+                    if (RAGGED) {
+#pragma unroll
+                        for (int t = 0; t < 4; ++t) {
+                            v4[t] = row + t < d ? v4[t] : 0.0f;
+                            acc[i][j][4 * g + t] = v4[t];
+                        }
+                    }
                     *reinterpret_cast<f32x4*>(st_new + col * PITCH + row) = v4;
-                    if (store) {
+                    if (!RAGGED && store) {
 #pragma unroll
                         for (int t = 0; t < 4; ++t) o_r[(size_t)(row + t) * D + c0 + col] = v4[t];
                     }
                 }
+        if (RAGGED) {   // behind the block that the next step waits for
+#pragma unroll
+            for (int j = 0; j < CTILES; ++j)
+#pragma unroll
+                for (int x = 0; x < 16; ++x)
+                    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(acc[0][j][x]), o_rows, lane_at[j] + (unsigned)((8 * (x / 4) + x % 4) * d) * 4, 0, 0);
+        }
         if (COT) {
             float* v_new = vbuf + (cur ^ 1) * D;
-            float* cot_r = cot + ((size_t)b * (K + 1) + rs) * D;
+            float* cot_r = cot + ((size_t)b * (K + 1) + rs) * d;
 #pragma unroll
             for (int i = 0; i < RTILES; ++i) {
-                const float total = vdot[i] + __shfl_xor(vdot[i], 32, 64);  // the two k halves of a row
+                float total = vdot[i] + __shfl_xor(vdot[i], 32, 64);  // the two k halves of a row
+                if (RAGGED && row0 + m >= d) total = 0.0f;
                 if (h == 0) {
                     v_new[row0 + i * 32 + m] = total;
-                    if (c0 == 0) cot_r[row0 + i * 32 + m] = total;
+                    if (c0 == 0 && (!RAGGED || row0 + m < d)) cot_r[row0 + i * 32 + m] = total;
                 }
             }
         }
@@ -1092,27 +1168,27 @@ int launch_suffix_apply(const void* suffix, const void* g, void* cot, int64_t B,
     return LBI_OK;
 }
 
-template <typename Tin, int D, int RT, int CB, bool COT, int MODE = 0>
-int launch_mfma_cot(const void* mats, void* out, const void* g, void* cot, int B, int K, hipStream_t stream,
+template <typename Tin, int D, int RT, int CB, bool COT, int MODE, bool RAGGED>
+int launch_mfma_cot(const void* mats, void* out, const void* g, void* cot, int B, int K, int d, hipStream_t stream,
                     ScanPlan plan = ScanPlan{0, 0, 0, 0, 0, 0, 0}) {
     constexpr int NW = D / RT;
     constexpr int NB = D / CB;
     constexpr size_t lds_bytes = ((size_t)2 * CB * (D + 4) + (COT ? 2 * D : 0)) * sizeof(float);
-    auto kern = scan_mfma_kernel<Tin, D, RT, CB, COT, MODE>;
-    if (int rc = ensure_dynamic_lds<&scan_mfma_kernel<Tin, D, RT, CB, COT, MODE>>(lds_bytes)) return rc;
+    auto kern = scan_mfma_kernel<Tin, D, RT, CB, COT, MODE, RAGGED>;
+    if (int rc = ensure_dynamic_lds<&scan_mfma_kernel<Tin, D, RT, CB, COT, MODE, RAGGED>>(lds_bytes)) return rc;
     // chains in this launch (the kernel derives the same number from the plan)
     const int chains = B * (MODE == 1 ? plan.C - 1 : MODE == 3 ? plan.C - 2 : 1);
     const dim3 grid(chains >= 8 ? ((chains + 7) / 8) * 8 * NB : chains * NB);
     hipLaunchKernelGGL(kern, grid, dim3(64 * NW), lds_bytes, stream, static_cast<const Tin*>(mats),
-                       static_cast<float*>(out), static_cast<const float*>(g), static_cast<float*>(cot), B, K, plan);
+                       static_cast<float*>(out), static_cast<const float*>(g), static_cast<float*>(cot), B, K, d, plan);
     LBI_HIP_CHECK(hipGetLastError());
     return LBI_OK;
 }
 
-template <typename Tin, int D, int RT, int CB>
-int launch_mfma(const void* mats, void* out, const void* g, void* cot, int B, int K, hipStream_t stream) {
-    return cot ? launch_mfma_cot<Tin, D, RT, CB, true>(mats, out, g, cot, B, K, stream)
-               : launch_mfma_cot<Tin, D, RT, CB, false>(mats, out, nullptr, nullptr, B, K, stream);
+template <typename Tin, int D, int RT, int CB, bool RAGGED = false>
+int launch_mfma(const void* mats, void* out, const void* g, void* cot, int B, int K, int d, hipStream_t stream) {
+    return cot ? launch_mfma_cot<Tin, D, RT, CB, true, 0, RAGGED>(mats, out, g, cot, B, K, d, stream)
+               : launch_mfma_cot<Tin, D, RT, CB, false, 0, RAGGED>(mats, out, nullptr, nullptr, B, K, d, stream);
 }
 
 // Whether the products of the chunk totals (phase 2) run in log depth: level l multiplies every element by the one
@@ -1185,7 +1261,8 @@ int launch_chunked(const void* mats, void* out, const void* g, void* cot, int B,
         using In = decltype(in);
         constexpr int MODE = decltype(mode)::value;
         if constexpr (D > 128) return scan_planes::launch_mode<In, D, 32, false, MODE>(left, out, nullptr, nullptr, B, K, d, stream, plan);
-        else return launch_mfma_cot<In, D, 32, 32, false, MODE>(left, out, nullptr, nullptr, B, K, stream, plan);
+        else if (d != D) return launch_mfma_cot<In, D, 32, 32, false, MODE, true>(left, out, nullptr, nullptr, B, K, d, stream, plan);
+        else return launch_mfma_cot<In, D, 32, 32, false, MODE, false>(left, out, nullptr, nullptr, B, K, d, stream, plan);
     };
     using std::integral_constant;
     // Phase 2 in log depth (totals_in_log_depth): the levels alternate between the two slots of a chunk that phase 3
@@ -1277,36 +1354,35 @@ int launch_scan(const void* mats, void* out, const void* g, void* cot, int B, in
         if (d <= 192) return run(std::integral_constant<int, 192>{});
         return run(std::integral_constant<int, 256>{});
     }
-    switch (d) {
-        // Column blocks of one batch element read the same matrices.  With few batch elements, narrow blocks give
-        // the chip enough workgroups, and the blocks of an element run side by side and share the matrices in L2.
-        // With many, they drift apart and fetch them again (measured 1.7x / 2.4x the input bytes at d = 64 / 128),
-        // so one workgroup then takes all columns.
-        case 512: {
-            // 16 column blocks of 32 per batch element, 8 waves of 64 rows.  The fused form would spill, so the
-            // cotangent chain, if asked for, runs as its own kernel behind the matrices.
-            if (int rc = launch_mfma<Tin, 512, 64, 32>(mats, out, nullptr, nullptr, B, K, stream)) return rc;
-            return cot ? launch_cotangent<Tin>(mats, g, cot, B, K, d, stream) : LBI_OK;
-        }
-        case 128:
-            if (plan_chunks(B, K, 4, &plan)) return launch_chunked<Tin, 128>(mats, out, g, cot, B, K, d, plan, stream);
-            if (B >= wide_block_batch()) return launch_mfma<Tin, 128, 32, 128>(mats, out, g, cot, B, K, stream);
-            return launch_mfma<Tin, 128, 32, 32>(mats, out, g, cot, B, K, stream);
-        case 64:
-            if (plan_chunks(B, K, 2, &plan)) return launch_chunked<Tin, 64>(mats, out, g, cot, B, K, d, plan, stream);
-            if (B >= wide_block_batch()) return launch_mfma<Tin, 64, 32, 64>(mats, out, g, cot, B, K, stream);
-            return launch_mfma<Tin, 64, 32, 32>(mats, out, g, cot, B, K, stream);
-        case 32:
-            if (plan_chunks(B, K, 1, &plan)) return launch_chunked<Tin, 32>(mats, out, g, cot, B, K, d, plan, stream);
-            return launch_mfma<Tin, 32, 32, 32>(mats, out, g, cot, B, K, stream);
-        // A width between the powers of two: matrices padded to 128 cost three copies and (128/96)^3 = 2.4 times the
-        // products.  fp32, matrices and cotangents, whole calls, padded -> here: B=16 K=50: 0.135 -> 0.068 ms; B=64 K=128:
-        // 0.78 -> 0.36 ms; 16-bit storage gains the same.  No wide blocks for many batch elements, as at 64 and 128: B=512
-        // K=8 and B=1200 K=6 take 0.25-0.6 times the time of the padded form with narrow ones.
-        case 96:
-            if (plan_chunks(B, K, 3, &plan)) return launch_chunked<Tin, 96>(mats, out, g, cot, B, K, d, plan, stream);
-            return launch_mfma<Tin, 96, 32, 32>(mats, out, g, cot, B, K, stream);
-        default: break;
+    // Widths up to 128: fp32 matrix cores (a step is a chain of dependent instructions here, which the splitting of the planes only
+    // lengthens: B=64 K=128 d=32 / 64 / 96 / 128 take 1.5 / 1.3 / 1.15 / 1.05 times as long on planes).
+    if (d > 16 && d <= 128) {
+        auto run = [&](auto width, auto wide) {
+            constexpr int D = decltype(width)::value, WIDE = decltype(wide)::value;
+            if (plan_chunks(B, K, (d + 31) / 32, &plan)) return launch_chunked<Tin, D>(mats, out, g, cot, B, K, d, plan, stream);
+            // Column blocks of one batch element read the same matrices.  With few batch elements, narrow blocks give
+            // the chip enough workgroups, and the blocks of an element run side by side and share the matrices in L2.
+            // With many, they drift apart and fetch them again (measured 1.7x / 2.4x the input bytes at d = 64 / 128),
+            // so one workgroup then takes all columns.  (At 96 narrow blocks stay ahead.)
+            const bool whole = WIDE > 32 && B >= wide_block_batch();
+            if (d != D) {
+                if (whole) return launch_mfma<Tin, D, 32, WIDE, true>(mats, out, g, cot, B, K, d, stream);
+                return launch_mfma<Tin, D, 32, 32, true>(mats, out, g, cot, B, K, d, stream);
+            }
+            if (whole) return launch_mfma<Tin, D, 32, WIDE>(mats, out, g, cot, B, K, d, stream);
+            return launch_mfma<Tin, D, 32, 32>(mats, out, g, cot, B, K, d, stream);
+        };
+        using std::integral_constant;
+        if (d <= 32) return run(integral_constant<int, 32>{}, integral_constant<int, 32>{});
+        if (d <= 64) return run(integral_constant<int, 64>{}, integral_constant<int, 64>{});
+        if (d <= 96) return run(integral_constant<int, 96>{}, integral_constant<int, 32>{});
+        return run(integral_constant<int, 128>{}, integral_constant<int, 128>{});
+    }
+    if (d == 512) {
+        // 16 column blocks of 32 per batch element, 8 waves of 64 rows.  The fused form would spill, so the
+        // cotangent chain, if asked for, runs as its own kernel behind the matrices.
+        if (int rc = launch_mfma_cot<Tin, 512, 64, 32, false, 0, false>(mats, out, nullptr, nullptr, B, K, d, stream)) return rc;
+        return cot ? launch_cotangent<Tin>(mats, g, cot, B, K, d, stream) : LBI_OK;
     }
     if (cot) {
         if (int rc = launch_cotangent<Tin>(mats, g, cot, B, K, d, stream)) return rc;

@@ -275,12 +275,12 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
     const size_t o_stride = a_stride;
 
     const Splitter splitter;
-    auto lds_barrier = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    auto lds_barrier = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 
     // This wave's RT x CB tile: the newest finished product, and of the next one the sum of the hi x hi products and that
     // of all others (the diagonal's apart).
     f32x16 tot[RTILES][CTILES], top[RTILES][CTILES], fine[RTILES][CTILES];
-    auto row_of = [&](int i, int e) { return row0 + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3); };
+    auto row_of = [&](int i, int e) __attribute__((always_inline)) { return row0 + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3); };
 
     // Results and start states by element: a descriptor over the matrix, past whose end nothing is read or written, an offset
     // per lane and column tile (past everything where the column is not there) and one per row.  (Both in the lane's offset:
@@ -293,10 +293,10 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
         lane_col[j] = c < d ? (unsigned)(4 * h * d + c) * 4 : kNowhere;
     }
     int row_elements = d;
-    auto row_bytes = [&](int i, int q, int e) { return (unsigned)((row0 + 32 * i + 8 * q + e) * row_elements) * 4; };
+    auto row_bytes = [&](int i, int q, int e) __attribute__((always_inline)) { return (unsigned)((row0 + 32 * i + 8 * q + e) * row_elements) * 4; };
     const unsigned matrix_bytes = (unsigned)dd * 4;
     // element n of the tile, n = 0 ... 16 RTILES CTILES - 1, of the finished product
-    auto store_element = [&](__amdgpu_buffer_rsrc_t o_r, int n) {
+    auto store_element = [&](__amdgpu_buffer_rsrc_t o_r, int n) __attribute__((always_inline)) {
         const int i = n / (16 * CTILES), j = n / 16 % CTILES, q = n % 16 / 4, e = n % 4;
         __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(tot[i][j][4 * q + e]), o_r, lane_col[j] + row_bytes(i, q, e), 0, 0);
     };
@@ -306,7 +306,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
     // The planes keep the 16 k of a product step in the order of the lane halves that bring them: rows 4 h + [0, 4) and
     // 8 + 4 h + [0, 4), which is how the accumulators hold a column, so that a lane writes and reads 16 bytes at a time.
     auto place = [](int k) { return (k & ~15) | ((k >> 2) & 1) << 3 | ((k >> 3) & 1) << 2 | (k & 3); };
-    auto wide_tile = [&](const Tin* a_r, bool from_planes, bool chain, float (&vdot)[RTILES], const float* v_old) {
+    auto wide_tile = [&](const Tin* a_r, bool from_planes, bool chain, float (&vdot)[RTILES], const float* v_old) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < RTILES; ++i)
 #pragma unroll
@@ -315,7 +315,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
                 for (int x = 0; x < 16; ++x) tot[i][j][x] = 0.0f;
         // lane half h brings k = 8 k8 + 4 h + [0, 4) of its row to four products (what lies behind a row's end is of the next row
         // or matrix: the last matrix is no left operand)
-#pragma unroll 4
+#pragma unroll 1
         for (int k8 = 0; k8 < D / 8; ++k8) {
             const int k = 8 * k8 + 4 * h;
             f32x4 a[RTILES];
@@ -351,7 +351,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
         }
     };
     // Whether the tile leaves the range in which three planes hold a number exactly.
-    auto out_of_range = [&]() {
+    auto out_of_range = [&]() __attribute__((always_inline)) {
         float high = 0.0f;
 #pragma unroll
         for (int i = 0; i < RTILES; ++i)
@@ -367,7 +367,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
 
     int parity = 0;
     unsigned words[RTILES][CTILES][4][NP][2];   // the finished tile as planes
-    auto split_tile = [&](int i, int j, int q) {
+    auto split_tile = [&](int i, int j, int q) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             unsigned w[NP];
@@ -377,7 +377,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
         }
     };
     // Hands the tile to the next step, once nobody reads the block before any more.
-    auto publish = [&](bool bad) {
+    auto publish = [&](bool bad) __attribute__((always_inline)) {
         parity ^= 1;
         if (bad && lane == 0) flags[parity] = 1;
         lds_barrier();
@@ -394,8 +394,8 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
                             u32x4{words[i][j][2 * x][p][0], words[i][j][2 * x][p][1], words[i][j][2 * x + 1][p][0], words[i][j][2 * x + 1][p][1]};
     };
     // Whether the block must be taken in fp32 (valid behind a barrier that follows publish).
-    auto asked_wide = [&]() { return flags[parity]; };
-    auto write_wide = [&]() {
+    auto asked_wide = [&]() __attribute__((always_inline)) { return flags[parity]; };
+    auto write_wide = [&]() __attribute__((always_inline)) {
         lds_barrier();
 #pragma unroll
         for (int i = 0; i < RTILES; ++i)
@@ -407,7 +407,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
                         f32x4{tot[i][j][4 * q], tot[i][j][4 * q + 1], tot[i][j][4 * q + 2], tot[i][j][4 * q + 3]};
         lds_barrier();
     };
-    auto split_all = [&]() {
+    auto split_all = [&]() __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < RTILES; ++i)
 #pragma unroll
@@ -419,7 +419,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
     // Rows of mats[r] come through LDS: a wave's ring of slots (32 rows x 64 bytes per row tile; 16-byte piece p of row i at
     // p ^ (i / 4) % 4, so that the 16 lanes of a read meet all banks).  Product step s of the wave's order takes k =
     // first_k(s) + 4 h + {0 ... 3, 8 ... 11}; the order begins with the k of its own rows.
-    auto first_k = [&](int s) {
+    auto first_k = [&](int s) __attribute__((always_inline)) {
         const int k = 32 * wave * RTILES + 16 * s;
         return k < D ? k : k - D;
     };
@@ -437,7 +437,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
 #pragma unroll
     for (int x = 0; x < kSlots; ++x) slot_at[x] = ring0 + x * RTILES * kSlotBytes;
     // requests the slot of product steps s ... s + HPS - 1 (past the end: of the steps that follow)
-    auto request = [&](unsigned slot, int r, int s) {
+    auto request = [&](unsigned slot, int r, int s) __attribute__((always_inline)) {
         const int rr = r - s / HALVES;
         // (reads up to 15 elements past a row, never past the tensor: the last matrix is no left operand)
         const __amdgpu_buffer_rsrc_t src = rows(a_base + (size_t)(rr > r_lo ? rr : r_lo) * a_stride,
@@ -520,7 +520,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
     float vdot[RTILES];
     f32x4 vvec[2];                          // the 8 entries of the vector that raw meets
     const unsigned piece0 = (unsigned)(m * 64), piece_swz = (unsigned)((m >> 2) & 3);
-    auto read_raw = [&](unsigned slot, int t) {
+    auto read_raw = [&](unsigned slot, int t) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < RTILES; ++i)
 #pragma unroll
@@ -534,7 +534,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
                 }
             }
     };
-    auto element_pair = [&](int i, int w, float& x0, float& x1) {
+    auto element_pair = [&](int i, int w, float& x0, float& x1) __attribute__((always_inline)) {
         if constexpr (WORDS == 2) {
             x0 = __uint_as_float(raw[i][w >> 1][2 * (w & 1)]);
             x1 = __uint_as_float(raw[i][w >> 1][2 * (w & 1) + 1]);
@@ -551,7 +551,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
     };
     // The diagonal's elements leave the matrix before it is split: the row of lane m of tile i meets them in chunk i of its
     // wave's order, product step 2 i + m / 16, lane half (m / 4) % 2.
-    auto take_diagonal = [&](int s, int buffer) {
+    auto take_diagonal = [&](int s, int buffer) __attribute__((always_inline)) {
         const int i = s / 2;
         if (i >= RTILES) return;
         const bool mine = m >> 4 == s % 2 && ((m >> 2) & 1) == h;
@@ -574,7 +574,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
     // The vector work of a product step in units: unit n takes pair w of the next step's elements one plane further.
     float left0[RTILES][4], left1[RTILES][4];
     constexpr int UNITS = 4 * NA * RTILES;
-    auto unit = [&](int n, int par, bool chain) {
+    auto unit = [&](int n, int par, bool chain) __attribute__((always_inline)) {
         const int i = n / (4 * NA), p = n % (4 * NA) / 4, w = n % 4;
         if (p == 0) {
             element_pair(i, w, left0[i][w], left1[i][w]);
@@ -592,7 +592,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
         }
     };
     const char* b_lane = smem + (size_t)(m * PITCH + h * 8) * 2;
-    auto load_b = [&](int p, int s) {       // the fragments of one plane for product step s
+    auto load_b = [&](int p, int s) __attribute__((always_inline)) {       // the fragments of one plane for product step s
 #pragma unroll
         for (int j = 0; j < CTILES; ++j)
             bfr[p][j] = *reinterpret_cast<const u32x4*>(b_lane + first_k(s) * 2 + (p * PLANE + j * 32 * PITCH) * 2);
@@ -605,7 +605,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
     bool primed = false;
     bool pending = false;                   // tot is a result that is not stored yet (it goes to o_base[(r + 1) * o_stride])
     // `apart`: the diagonal's elements were taken out of the rows
-    auto chain_out = [&](bool apart) {
+    auto chain_out = [&](bool apart) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < RTILES; ++i) {
             const int row = row0 + 32 * i + m;
@@ -625,18 +625,18 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
             }
         }
     };
-    auto load_v = [&](int s) {
+    auto load_v = [&](int s) __attribute__((always_inline)) {
         const float* v = vbuf + cur * D + 4 * h + first_k(s);
         vvec[0] = *reinterpret_cast<const f32x4*>(v);
         vvec[1] = *reinterpret_cast<const f32x4*>(v + 8);
     };
-    auto store_now = [&]() {
+    auto store_now = [&]() __attribute__((always_inline)) {
         const __amdgpu_buffer_rsrc_t o_r = rows(o_base + (size_t)(store_all ? r : r + 1) * o_stride, matrix_bytes);
 #pragma unroll
         for (int n = 0; n < NEL; ++n) store_element(o_r, n);
     };
     while (true) {
-        if (wide) {
+        if (__builtin_expect(wide, 0)) {
             write_wide();
             if (pending) {
                 ++r;
@@ -663,7 +663,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
             continue;
         }
         if (!primed) {
-            if (!requested) {
+            if (__builtin_expect(!requested, 0)) {
                 wait_vm<0>();
 #pragma unroll
                 for (int x = 0; x < kSlots; ++x) request(slot_at[x], r, x * HPS);
@@ -698,13 +698,13 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
         int asked = 0;
         f32x4 dg[RTILES][4];
         // four rows of a tile: the sums come together, with the diagonal's product, and are split
-        auto finish = [&](int i, int j, int q) {
+        auto finish = [&](int i, int j, int q) __attribute__((always_inline)) {
 #pragma unroll
             for (int x = 0; x < 4; ++x)
                 tot[i][j][4 * q + x] = fmaf(dg[i][q][x], tot[i][j][4 * q + x], top[i][j][4 * q + x] + fine[i][j][4 * q + x]);
             split_tile(i, j, q);
         };
-        auto product_step = [&](const int s) __attribute__((always_inline)) {
+        auto product_step = [&](const int s) __attribute__((always_inline)) __attribute__((always_inline)) {
             const int par = s & 1;
             const bool chain_next = s + 1 < HALVES;
             // The two waves of a SIMD would take turns by age, one idle while the other ends its step: whoever is behind goes first.
@@ -736,7 +736,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
             }
             int y = 0, done = 0, finished = 0;
             // one product and the share of the vector work that goes under it
-            auto product = [&](int sp, int ap, int i, int j) {
+            auto product = [&](int sp, int ap, int i, int j) __attribute__((always_inline)) {
                 f32x16 zero;
 #pragma unroll
                 for (int x = 0; x < 16; ++x) zero[x] = 0.0f;
@@ -836,12 +836,12 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
         asked = asked_wide();
         if constexpr (HALVES > 2) product_step(1);
         wide = __builtin_amdgcn_readfirstlane(asked) != 0;
-        if (wide) continue;                 // (nothing but raw and the planes of the rows has changed: both are made again)
+        if (__builtin_expect(wide, 0)) continue;                 // (nothing but raw and the planes of the rows has changed: both are made again)
         if constexpr (HALVES == 2) product_step(1);
 #pragma unroll
         for (int s = 2; s < HALVES; ++s) product_step(s);
         const bool bad = out_of_range();
-        if (bad) {
+        if (__builtin_expect(bad, 0)) {
             float none[RTILES];
             wide_tile(a_base + (size_t)r * a_stride, true, false, none, nullptr);
         }

@@ -29,30 +29,24 @@ def _validate(mats: torch.Tensor) -> tuple[int, int, int]:
     return bsz, count, rank
 
 
-#: widths up to 128 and above 256 the matrix-core scan kernels are built for
-_MFMA_WIDTHS = (32, 64, 96, 128, 512)
-
-
-def _padded_width(mats: torch.Tensor) -> int:
-    """The width a scan is padded to by copies: a width of the list above, or the width itself where the kernels take it as
-    it is (129 ... 256), where it is too small to matter (<= 16) or beyond the largest.  Odd widths of 16-bit storage are
-    brought to an even one: rows are read in whole 4-byte words.  (Of bf16 those above 192 go to 256, whose own kernel is
-    up to 1.3 times faster when the batch fills the chip.)"""
-    rank = int(mats.shape[-1])
-    if 128 < rank <= 256:
-        if mats.element_size() == 4 or rank % 2 == 0:
-            return rank
-        return 256 if mats.dtype == torch.bfloat16 and rank > 192 else rank + 1
-    if rank <= 16 or rank in _MFMA_WIDTHS:
+def _padded_width(rank: int, mats: torch.Tensor) -> int:
+    """The width a scan is padded to by copies: the width itself up to 256, which the kernels take as it is, and beyond 512;
+    else 512.  Of the widths above 128, odd ones of 16-bit storage are brought to an even one, since rows are read in
+    whole 4-byte words there.  (Of bf16 those above 192 go to 256, whose own kernel is up to 1.3 times faster when the
+    batch fills the chip.)"""
+    if rank <= 128:
         return rank
-    return next((w for w in _MFMA_WIDTHS if w > rank), rank)
+    if rank <= 256 and rank % 2 and mats.element_size() == 2:
+        return 256 if mats.dtype == torch.bfloat16 and rank > 192 else rank + 1
+    return 512 if 256 < rank <= 512 else rank
 
 
 def _aligned(t: torch.Tensor, rank: int) -> torch.Tensor:
     """Tensors whose calls off the 16-byte grid used to run on padded copies: on plain copies now."""
-    if rank != 96 and not 128 < rank < 256:
+    if rank in (32, 64, 128) or not 16 < rank < 256:
         return t
-    return t.clone() if t.data_ptr() % (16 if rank % 4 == 0 else 4) else t
+    grid = 16 if rank % 4 == 0 else 4 if rank > 128 else 1
+    return t.clone() if t.data_ptr() % grid else t
 
 
 def suffix_scan_pullbacks(mats: torch.Tensor, *, exact_suffix: bool = False) -> torch.Tensor:
@@ -63,7 +57,7 @@ def suffix_scan_pullbacks(mats: torch.Tensor, *, exact_suffix: bool = False) -> 
     error <= 2e-4 where 16-bit storage is asked 2e-2), with ``exact_suffix=True`` three (its exact fp32 value: only
     the rounding of fp32 accumulation is left, ~1e-5 at K = 128; half again as many products)."""
     bsz, count, rank = _validate(mats)
-    width = _padded_width(mats)
+    width = _padded_width(rank, mats)
     if width != rank and mats.numel():
         # Products of zero-padded matrices are the zero-padded products, and the identity tail cuts to the
         # identity: run the matrix-core kernel of the next width instead of the scalar kernel (several times
@@ -117,7 +111,7 @@ def suffix_scan_pullbacks_and_cotangents(mats: torch.Tensor, g: torch.Tensor, *,
     bsz, count, rank = _validate(mats)
     if g.dim() != 2 or g.shape[0] != bsz or g.shape[1] != rank:
         raise ValueError("g must have shape [B, R]")
-    width = _padded_width(mats)
+    width = _padded_width(rank, mats)
     if width != rank and mats.numel():
         pad = width - rank  # see suffix_scan_pullbacks; a zero-padded g leaves the first `rank` cotangents unchanged
         wide, wide_cot = suffix_scan_pullbacks_and_cotangents(torch.nn.functional.pad(mats, (0, pad, 0, pad)),

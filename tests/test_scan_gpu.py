@@ -156,6 +156,35 @@ def test_widths_between_powers_of_two(rank, bsz, count, dtype, device):
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rank", [17, 31, 33, 63, 97, 127, 131, 254])
+@pytest.mark.parametrize("bsz,count", [(1, 1), (2, 3), (1, 40), (520, 3)])
+def test_widths_read_where_they_lie(rank, bsz, count, dtype, device):
+    """Widths between the kernels' own, on tensors that start off the grid too; an infinity that begins a row stays out of
+    the row before, whose last chunk reads past its end."""
+    from latent_bounded_interfaces_amd.hip.interface import suffix_scan_pullbacks, suffix_scan_pullbacks_and_cotangents
+
+    mats, g = oscan.make_scan_inputs(bsz, count, rank, kind="randn", seed=rank + count)
+    mats = mats.to(dtype)
+    truth = oscan.suffix_scan_sequential(mats, dtype=torch.float64)
+    want = oscan.suffix_cotangents_sequential(mats.double(), g.double())
+    dev = torch.empty(mats.numel() + 1, dtype=dtype, device=device)[1:].view(mats.shape).copy_(mats)
+    out, cot = suffix_scan_pullbacks_and_cotangents(dev, g.to(device))
+    only = suffix_scan_pullbacks(mats.to(device))
+    bar = 2e-4 if dtype == torch.bfloat16 and rank > 192 else 1e-5   # the width-256 kernel's two planes
+    for result in (out.cpu(), only.cpu()):
+        err = (result.double() - truth).abs().flatten(2).amax(2) / truth.abs().flatten(2).amax(2)
+        assert float(err.max()) <= bar
+    scale = want.abs().amax(dim=-1, keepdim=True)
+    assert float(((cot.cpu().double() - want).abs() / scale).max()) <= max(bar, 3e-5)   # products applied to g
+    if 1 < count < 12:
+        mats[-1, 0, 9, 0] = float("inf")
+        out, cot = suffix_scan_pullbacks_and_cotangents(mats.to(device), g.to(device))
+        for result in (out[-1, 0], cot[-1, 0]):
+            bad = ~result.isfinite()
+            assert bool(bad[9].all()) and int(bad.sum()) == bad[9].numel()
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rank", [130, 192, 256])
 @pytest.mark.parametrize("bsz,count", [(1, 40), (2, 5), (40, 4)])
 @pytest.mark.parametrize("kind", ["inf", "nan", "huge", "tiny", "zero_rows"])
