@@ -264,13 +264,23 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
 
     // Lane's slice of mats[r]: rows row0 + 32*i + m, k = 32*kc + 16*h + [0, 16).
     static_assert(!RAGGED || RTILES == 1, "rows of one tile");
-    auto load_a = [&](f32x4 (&dst)[RTILES][4], const Tin* base) {
+    // fp16 elements of the whole chain without cotangents stay as they are stored until their chunk begins: the compiler widens
+    // them at the load otherwise, and waits for it (B=64 K=128: 452 -> 296 us at d = 96, 573 -> 400 at 128; the other forms,
+    // which do not wait, lose up to 10 % by widening late, narrow ones 3 %).
+    constexpr bool LATE = std::is_same<Tin, _Float16>::value && D >= 96 && !COT && MODE == 0;
+    using Stored = typename std::conditional<LATE, f16x4, f32x4>::type;
+    auto load_a = [&](Stored (&dst)[RTILES][4], const Tin* base) {
 #pragma unroll
         for (int i = 0; i < RTILES; ++i)
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                if constexpr (RAGGED) dst[i][q] = scan_planes::load4_at(base + q * 4);
-                else dst[i][q] = load4(base + (size_t)i * 32 * D + q * 4);
+                const Tin* p = base + (size_t)i * 32 * D + q * 4;
+                if constexpr (LATE) {
+                    typedef _Float16 f16x4_at __attribute__((ext_vector_type(4), aligned(2)));
+                    if constexpr (RAGGED) dst[i][q] = *reinterpret_cast<const f16x4_at*>(p);
+                    else dst[i][q] = *reinterpret_cast<const f16x4*>(p);
+                } else if constexpr (RAGGED) dst[i][q] = scan_planes::load4_at(p);
+                else dst[i][q] = load4(p);
             }
     };
     const Tin* a_lane = a_base + (size_t)(!RAGGED || row0 + m < d ? row0 + m : 0) * d + h * 16;  // + r*a_stride + kc*32
@@ -286,7 +296,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
     constexpr int RING = NCH == 1 ? 2 : NCH % 4 == 0 ? 4 : NCH % 3 == 0 ? 3 : NCH % 2 == 0 ? 2 : NCH;
     static_assert(NCH == 1 || NCH % RING == 0, "a chunk keeps its slot from step to step");
     constexpr int AHEAD = RING - 1;
-    f32x4 a_ring[RING][RTILES][4];
+    Stored a_ring[RING][RTILES][4];
     // Chunk number c (0 <= c < AHEAD) counted from the start of step r_top; when NCH == 1
     // chunk 1 is already in the next step.
 #pragma unroll
@@ -324,12 +334,22 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
             const int slot = (NCH == 1 ? sub : kc) % RING;
             const int ahead = kc + AHEAD;
             load_a(a_ring[(slot + AHEAD) % RING], ahead < NCH ? a_r + ahead * 32 : a_wrap + (ahead - NCH) * 32);
+            f32x4 a[RTILES][4];
+#pragma unroll
+            for (int i = 0; i < RTILES; ++i)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if constexpr (LATE) {
+                        asm volatile("" : "+v"(a_ring[slot][i][q]));   // not before here
+                        a[i][q] = __builtin_convertvector(a_ring[slot][i][q], f32x4);
+                    } else a[i][q] = a_ring[slot][i][q];
+                }
             if (RAGGED && kc == NCH - 1) {
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
 #pragma unroll
                     for (int t = 0; t < 4; ++t)
-                        if (kc * 32 + h * 16 + q * 4 + t >= d) a_ring[slot][0][q][t] = 0.0f;
+                        if (kc * 32 + h * 16 + q * 4 + t >= d) a[0][q][t] = 0.0f;
             }
             f32x4 bfrag[CTILES][4];
 #pragma unroll
@@ -354,7 +374,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
                                 for (int e = 0; e < 16; ++e) part[i][j][e] = 0.0f;
                             }
                             part[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-                                a_ring[slot][i][q][t], bfrag[j][q][t], part[i][j], 0, 0, 0);
+                                a[i][q][t], bfrag[j][q][t], part[i][j], 0, 0, 0);
                         }
 #pragma unroll
             for (int i = 0; i < RTILES; ++i)
@@ -369,7 +389,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
 #pragma unroll
                     for (int i = 0; i < RTILES; ++i)
 #pragma unroll
-                        for (int t = 0; t < 4; ++t) vdot[i] = fmaf(a_ring[slot][i][q][t], v4[t], vdot[i]);
+                        for (int t = 0; t < 4; ++t) vdot[i] = fmaf(a[i][q][t], v4[t], vdot[i]);
                 }
             }
             // Keep chunks from being interleaved: it only lengthens register live ranges.

@@ -704,7 +704,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
                 tot[i][j][4 * q + x] = fmaf(dg[i][q][x], tot[i][j][4 * q + x], top[i][j][4 * q + x] + fine[i][j][4 * q + x]);
             split_tile(i, j, q);
         };
-        auto product_step = [&](const int s) __attribute__((always_inline)) __attribute__((always_inline)) {
+        auto product_step = [&](const int s) __attribute__((always_inline)) {
             const int par = s & 1;
             const bool chain_next = s + 1 < HALVES;
             // The two waves of a SIMD would take turns by age, one idle while the other ends its step: whoever is behind goes first.
