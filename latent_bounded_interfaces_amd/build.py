@@ -14,7 +14,8 @@ from pathlib import Path
 PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "liblbi_hip.so"
-SOURCES = ("lbi_common.hip", "lbi_scan.hip", "lbi_attn.hip", "lbi_attn_f32.hip", "lbi_region.hip", "lbi_norms.hip", "lbi_param_grads.hip")
+SOURCES = ("lbi_common.hip", "lbi_scan.hip", "lbi_attn.hip", "lbi_attn_f32.hip", "lbi_attn_f32_f16.hip",
+           "lbi_attn_f32_bf16.hip", "lbi_region.hip", "lbi_norms.hip", "lbi_param_grads.hip")
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",
@@ -29,8 +30,8 @@ HIPCC_FLAGS = [
 
 # Flags of single sources.  Kernels that keep rows in registers index them by unrolled loops: one that the compiler does not
 # unroll puts them into scratch memory.
-SOURCE_FLAGS = {"lbi_region.hip": ["-Werror=pass-failed"], "lbi_attn_f32.hip": ["-Werror=pass-failed"],
-                "lbi_scan.hip": ["-Werror=pass-failed"]}
+SOURCE_FLAGS = {src: ["-Werror=pass-failed"] for src in ("lbi_region.hip", "lbi_attn_f32.hip", "lbi_attn_f32_f16.hip",
+                                                          "lbi_attn_f32_bf16.hip", "lbi_scan.hip")}
 
 
 def _hipcc() -> str:

@@ -114,10 +114,9 @@ extern "C" int lbi_attn_pullback(const void* q, const void* k, const void* v, co
                    ? attn_mfma::launch<_Float16>(q, k, v, d_out, dq, dk, dv, ws, b, h, t, dh, p, softmax_scale, causal, stream)
                    : attn_mfma::launch<bf16_raw>(q, k, v, d_out, dq, dk, dv, ws, b, h, t, dh, p, softmax_scale, causal, stream);
     }
-    const bool aligned = Dh % 4 == 0 && (reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
-                                         reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(d_out)) % 16 == 0;
-    if (attn_f32::supports(dh, dtype) && !attn_f32::scalar_is_faster(B, H, T, Dh, P, aligned))
-        return attn_f32::launch(q, k, v, d_out, dq, dk, dv, ws, b, h, t, dh, p, softmax_scale, causal, stream);
+    const bool aligned = attn_f32::aligned(Dh, dtype_size(dtype), {q, k, v, d_out});
+    if (attn_f32::supports(dh, dtype, B * H * P) && !attn_f32::scalar_is_faster(B, H, T, Dh, P, aligned))
+        return attn_f32::launch(q, k, v, d_out, dq, dk, dv, ws, b, h, t, dh, p, softmax_scale, causal, dtype, stream);
     switch (dtype) {
         case LBI_F32: return attn_generic::launch<float>(q, k, v, d_out, dq, dk, dv, ws, b, h, t, dh, p, softmax_scale, causal, stream);
         case LBI_F16: return attn_generic::launch<_Float16>(q, k, v, d_out, dq, dk, dv, ws, b, h, t, dh, p, softmax_scale, causal, stream);

@@ -1,5 +1,7 @@
-// Attention input-pullback for fp32 storage on the fp32 matrix cores (lbi_attn_f32.hip).
+// Attention input-pullback in fp32 on the fp32 matrix cores (lbi_attn_f32_kernels.h).
 #pragma once
+
+#include <initializer_list>
 
 #include "lbi_common.h"
 
@@ -8,7 +10,17 @@ namespace attn_f32 {
 
 constexpr int MAX_DH = 128;
 
-inline bool supports(int dh, int dtype) { return dtype == LBI_F32 && dh >= 1 && dh <= MAX_DH; }
+// 16-bit calls of more than 65535 (batch, head, direction) triples stay refused by the scalar kernels.
+inline bool supports(int dh, int dtype, int64_t groups) {
+    return dh >= 1 && dh <= MAX_DH && (dtype == LBI_F32 || groups <= 65535);
+}
+
+// Loads of four elements at a time.
+inline bool aligned(int64_t dh, size_t element_bytes, std::initializer_list<const void*> tensors) {
+    uintptr_t bits = 0;
+    for (const void* p : tensors) bits |= reinterpret_cast<uintptr_t>(p);
+    return dh % 4 == 0 && bits % (4 * element_bytes) == 0;
+}
 
 // Where the scalar kernels (lbi_attn_generic.h), whose tiles are 16 rows, are as fast or faster; both sides measured:
 //  * up to 16 positions half of a 32-row tile is empty, and with few directions waves of a workgroup have no work (B=64
@@ -17,6 +29,8 @@ inline bool supports(int dh, int dtype) { return dtype == LBI_F32 && dh >= 1 && 
 //  * a call of few workgroups is as long as one of them, and a 32-row tile of very narrow heads, or one that is loaded
 //    element by element, takes longer than two of 16 rows (B=4 H=8 T=48 Dh=8 P=2: 23 and 29 us; B=1 H=4 T=48 Dh=33 P=2: 43
 //    and 51).
+// The lines hold for 16-bit storage too (scalar kernels, here: B=16 H=8 T=16 Dh=80 P=8 63 and 40 us, B=64 H=16 T=12 Dh=96 P=4 221
+// and 126, B=2 H=8 T=32 Dh=24 P=4 30 and 19, B=1 H=2 T=20 Dh=16 P=1 22 and 18).
 inline bool scalar_is_faster(int64_t B, int64_t H, int64_t T, int64_t dh, int64_t P, bool aligned) {
     const int64_t groups = B * H * P;
     if (groups > 65535) return false;  // more than they take
@@ -28,9 +42,15 @@ inline bool scalar_is_faster(int64_t B, int64_t H, int64_t T, int64_t dh, int64_
     return T <= 48 && groups < 256 && (aligned ? dh <= 16 && T > 32 : dh > 32);
 }
 
+// One storage type each, in a source of its own.
+typedef int Launch(const void* q, const void* k, const void* v, const void* d_out, void* dq, void* dk, void* dv,
+                   float* workspace, int B, int H, int T_len, int dh, int P, float scale, int causal, hipStream_t stream);
+Launch launch_float, launch_half, launch_bf16;
+
 // Workspace: lse2[B*H*T], delta[B*P*H*T], as for the scalar kernels.
 int launch(const void* q, const void* k, const void* v, const void* d_out, void* dq, void* dk, void* dv,
-           float* workspace, int B, int H, int T_len, int dh, int P, float scale, int causal, hipStream_t stream);
+           float* workspace, int B, int H, int T_len, int dh, int P, float scale, int causal, int dtype,
+           hipStream_t stream);
 
 }  // namespace attn_f32
 }  // namespace lbi

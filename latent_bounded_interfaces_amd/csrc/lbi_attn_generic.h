@@ -1,7 +1,7 @@
 // Attention input-pullback, generic path: any T, any head dim <= 256, any storage
 // type, causal or not.  Scalar fp32 arithmetic on 16 x 16 tiles staged in LDS.
-// This is the path for shapes the matrix-core kernels do not take (fp32 head dims past 128, 16-bit shapes that cannot
-// be padded) or are slower at (short fp32 sequences, lbi_attn_f32.h); it is not tuned.
+// This is the path for shapes the matrix-core kernels do not take (head dims past 128) or are slower at (short sequences,
+// lbi_attn_f32.h); it is not tuned.
 //
 // Workspace layout (floats): lse2[B*H*T] (log2-domain logsumexp), delta[B*P*H*T].
 #pragma once

@@ -29,7 +29,7 @@ _MODE_BASIS_LIMIT = {
 }
 
 
-# what the matrix-core kernels take (the generic kernels take any length and head dim up to 256)
+# what the 16-bit matrix-core kernels take (the fp32 ones take any length and head dims up to 128, scalar kernels up to 256)
 _MFMA_SEQ_MULTIPLE = 64
 _MFMA_HEAD_DIMS = (64, 128)
 # longest sequence the single-launch kernel takes, by head dim (any length up to it)
@@ -116,7 +116,7 @@ def attention_input_pullback_basis(
     single_launch = seqlen <= _SINGLE_LAUNCH_MAX_SEQ.get(wide_dim, 0)
     if q.dtype in (torch.float16, torch.bfloat16) and d_out.numel() and (single_launch or seqlen > _MFMA_SEQ_MULTIPLE // 2):
         # The matrix-core kernels work on tiles of head dim 64 or 128 and 64 positions (short sequences, which run as
-        # a single launch, any length); what does not fill them is padded, since the generic kernels run at a small
+        # a single launch, any length); what does not fill them is padded, since the fp32 kernels run at a small
         # fraction of their speed.  Two paddings are exact:
         # * zero columns appended to the head dim add nothing to any dot product (the scale is passed explicitly)
         #   and receive zero cotangents;

@@ -113,6 +113,33 @@ def test_fp32_tile_edges_against_fp64(shape, basis, causal, device):
         assert err <= bound, (name, err, bound)
 
 
+@pytest.mark.parametrize("offset", [0, 1, 4])   # elements in front of each tensor: whole pieces, single ones, 8-byte pieces
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("shape,basis", [((1, 2, 31, 32), 1), ((1, 2, 33, 60), 3), ((1, 1, 129, 33), 5), ((1, 1, 161, 96), 3),
+                                         ((1, 2, 258, 64), 9), ((2, 1, 95, 100), 2), ((1, 1, 225, 128), 4), ((2, 2, 1, 24), 3),
+                                         ((1, 20, 321, 64), 9), ((16, 8, 16, 80), 8)])
+def test_half_storage_with_fp32_probabilities(shape, basis, causal, dtype, offset, device):
+    """16-bit tensors on the fp32 matrix cores: the bound of the test above and one rounding of the result."""
+    from latent_bounded_interfaces_amd.hip.transformer import attention_input_pullback_basis_static
+
+    inputs = oattn.make_attention_inputs(*shape, basis, dtype=dtype, seed=shape[2] * 131 + basis)
+    scale = 1.0 / math.sqrt(shape[-1])
+
+    def placed(t):
+        return torch.cat((t.new_zeros(offset), t.reshape(-1))).to(device)[offset:].view(t.shape)
+
+    got = tuple(placed(torch.full_like(inputs[3], float("nan"))) for _ in range(3))
+    attention_input_pullback_basis_static(*map(placed, inputs), got, softmax_scale=scale, causal=causal)
+    truth = oattn.attention_pullback_dense(*inputs, softmax_scale=scale, causal=causal, dtype=torch.float64)
+    eps = (shape[2] + 2 * shape[3]) * 2.0 ** -24
+    half_ulp, smallest = (2.0 ** -11, 2.0 ** -25) if dtype == torch.float16 else (2.0 ** -8, 0.0)
+    for name, a, c in zip(("dq", "dk", "dv"), got, truth):
+        fp32_error = eps * max(float(c.abs().max()), float(inputs[3].double().abs().max()))
+        excess = (a.cpu().double() - c).abs() - half_ulp * c.abs()
+        assert float(excess.max()) <= fp32_error * (1 + half_ulp) + smallest, (name, float(excess.max()), fp32_error)
+
+
 @pytest.mark.parametrize("shape,basis", [((1, 2, 1, 32), 1), ((1, 2, 70, 64), 3), ((2, 1, 65, 33), 2), ((1, 1, 130, 128), 2),
                                          ((1, 2, 30, 16), 9)])
 def test_fp32_rounding_of_delta_cancels(shape, basis, device):
