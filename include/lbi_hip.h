@@ -246,6 +246,17 @@ int lbi_gated_mlp_pullback(const void* g_down_input, const void* fc1_output, voi
                            int g_broadcast_t, int dtype, void* stream);
 
 /*
+ * Product of few rows with a weight as it lies (the pullback of y = x W^T): out = a w, sums in fp32, one rounding.
+ *
+ *   a [M,K], w [K,N]  ->  out [M/T, N/Dh, T, Dh]   (T = 1, Dh = N: [M,N])
+ *
+ * 16-bit types; N and K multiples of 8, Dh a multiple of 4, 16-byte aligned tensors, operands below 2 GiB.  For products
+ * of a few microseconds: a library product is faster on many rows.
+ */
+int lbi_rows_product(const void* a, const void* w, void* out, int64_t M, int64_t N, int64_t K, int64_t T, int64_t Dh,
+                     int dtype, void* stream);
+
+/*
  * Head split of the out_proj-input cotangent: [B,P,T,H*Dh] -> [B,P,H,T,Dh], the layout
  * lbi_attn_pullback takes as d_out (transpose of reference backends/transformer.py:152-153).
  */

@@ -10,7 +10,7 @@ backends/transformer_cuda.py:45-64) for the block the reference's backend execut
     region_output = m + res2 of the last layer
 
 The cotangent basis [B, P, T, D] is pulled back through the layers in reverse.  Matrix
-products are library GEMMs on the [B*P*T, *] cotangent rows; everything between them runs in
+products are library GEMMs on the [B*P*T, *] cotangent rows (small ones ``lbi_rows_product``); everything between them runs in
 the kernels of liblbi_hip.so (RMSNorm, gated MLP, head split, rotary embedding + KV-group
 sum, causal convolution, and the attention pullback itself).  The residual-stream cotangent
 is kept in fp32, branch cotangents in the dtype of the weights.  Inputs are read from the
@@ -256,17 +256,62 @@ def causal_conv1d_weight_grad(g_out: torch.Tensor, x: torch.Tensor, ksize: int) 
 #: rows below which the transposed copy of the weight costs more than the faster product form gains
 _TRANSPOSED_COPY_MIN_ROWS = 65536
 
+#: Multiply-adds and results up to which a product runs on the package's own kernel.  A call of the library takes 18 us of
+#: host time, one of this kernel 7; on the GPU (bf16, M x K x N, this kernel and the library): 512 x 256 x 1024 3.8 and 5.2 us,
+#: 2048 x 2048 x 256 9.0 and 11.8, 1000 x 1536 x 768 9.7 and 10.8, 3001 x 1000 x 520 14.8 and 15.5, 4096 x 256 x 1024 9.2 and 8.4;
+#: past the lines 8192 x 256 x 1024 15.4 and 11.7, 4096 x 512 x 2048 21.5 and 15.5.
+_SMALL_PRODUCT = 3 << 29
+_SMALL_PRODUCT_RESULTS = 1 << 22
+
+
+def _is_small_product(g: torch.Tensor, weight: torch.Tensor) -> bool:
+    inner, width = weight.shape
+    return (g.dtype in (torch.float16, torch.bfloat16) and g.numel() * width <= _SMALL_PRODUCT
+            and inner == g.shape[-1] and inner % 8 == 0 and width % 8 == 0 and g.dim() == 4
+            and g.numel() > 0 and g.numel() // inner * width <= _SMALL_PRODUCT_RESULTS and weight.numel() > 0 and weight.device == g.device
+            and g.is_contiguous() and weight.is_contiguous()
+            and g.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+
+
+def rows_product(g: torch.Tensor, weight: torch.Tensor, head_dim: int | None = None) -> torch.Tensor:
+    """``g [B,P,T,K] @ weight [K,N]`` for few rows of a 16-bit type; with ``head_dim`` as ``[B,P,N/head_dim,T,head_dim]``."""
+    _require_cuda(g, weight)
+    bsz, basis, seqlen, inner = g.shape
+    width = int(weight.shape[1])
+    if head_dim is None:
+        shape, seqlen, head_dim = (bsz, basis, seqlen, width), 1, width
+    else:
+        shape = (bsz, basis, width // head_dim, seqlen, head_dim)
+    out = torch.empty(shape, device=g.device, dtype=g.dtype)
+    with _lib.device_guard(g.device):
+        status = _lib.load().lbi_rows_product(g.data_ptr(), weight.data_ptr(), out.data_ptr(), g.numel() // inner, width,
+                                              inner, seqlen, head_dim, _lib.dtype_code(g.dtype), _stream(g))
+    _lib.check(status, "lbi_rows_product")
+    return out
+
 
 def _apply_transposed(g: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """``g @ weight`` for ``weight [out, in]``: the pullback of ``y = x weight^T``.  For tall ``g`` it is issued as
     the library's ``A B^T`` form on a transposed copy of the (small) weight, which is its faster path for these
-    products; for few rows (the single direction of a parameter VJP) the copy is not worth it."""
+    products; for fewer rows (the single direction of a parameter VJP) the copy is not worth it, and for few ones the
+    library's call is what takes longest."""
     if weight.dtype != g.dtype:
         # a forward run under autocast multiplied by the weight cast to the compute dtype; so does its pullback
         weight = weight.to(g.dtype)
+    if _is_small_product(g, weight):
+        return rows_product(g, weight)
     if g.numel() // g.shape[-1] < _TRANSPOSED_COPY_MIN_ROWS:
         return torch.matmul(g, weight)
     return torch.nn.functional.linear(g, weight.t().contiguous())
+
+
+def _apply_transposed_to_heads(g: torch.Tensor, weight: torch.Tensor, n_heads: int, head_dim: int) -> torch.Tensor:
+    """``g @ weight`` as ``[B,P,H,T,Dh]``."""
+    if weight.dtype != g.dtype:
+        weight = weight.to(g.dtype)
+    if head_dim % 4 == 0 and weight.shape[1] == n_heads * head_dim and _is_small_product(g, weight):
+        return rows_product(g, weight, head_dim)
+    return attn_heads_split(_apply_transposed(g, weight), n_heads, head_dim)
 
 
 def _rows(t: torch.Tensor) -> torch.Tensor:
@@ -365,10 +410,8 @@ def _layer_input_pullback(block: Any, layer_cache: Any, g_hidden: torch.Tensor |
     # attention: res2 = out_proj(heads) + res1
     if param_grads is not None:
         _linear_grads(param_grads, attn.out_proj, g_attn_out, a_cache.out_proj_input)
-    g_merged = _apply_transposed(g_attn_out, attn.out_proj.weight)
+    g_heads = _apply_transposed_to_heads(g_attn_out, attn.out_proj.weight, attn.n_heads, attn.head_dim)
     del g_attn_out
-    g_heads = attn_heads_split(g_merged, attn.n_heads, attn.head_dim)
-    del g_merged
     scale = attn.softmax_scale if attn.softmax_scale is not None else 1.0 / math.sqrt(attn.head_dim)
     dq, dk, dv = attention_input_pullback_basis(a_cache.q_rope, a_cache.k_expanded, a_cache.v_expanded, g_heads,
                                                 softmax_scale=float(scale), causal=True, kernel_mode=kernel_mode)

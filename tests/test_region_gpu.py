@@ -552,3 +552,32 @@ def test_region_pullback_at_the_end_to_end_layer_shape_matches_oracle(device):
     assert set(got_p) == set(want_p)
     for name, w in want_p.items():
         assert _max_rel(got_p[name].cpu(), w) <= 3e-2, (name, _max_rel(got_p[name].cpu(), w))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("lead,inner,width,head_dim", [
+    ((1, 1, 1), 8, 8, 4), ((1, 2, 17), 72, 104, 52), ((2, 3, 11), 256, 64, 32), ((1, 1, 129), 64, 1024, 64),
+    ((2, 1, 333), 320, 136, 8), ((1, 5, 64), 448, 256, 128), ((1, 16, 128), 2048, 256, 64), ((1, 1, 3001), 200, 520, 40),
+    ((3, 1, 1), 136, 72, 72), ((2, 4, 250), 392, 1032, 24),
+])
+def test_rows_product(lead, inner, width, head_dim, dtype, device):
+    """Rows, columns and chunks of the reduction that end inside a tile, both tile heights, one chunk to more than a turn of the
+    ring; infinities stay in their row and column."""
+    from latent_bounded_interfaces_amd.hip.transformer.region import rows_product
+
+    gen = torch.Generator().manual_seed(inner + width)
+    g = torch.randn(*lead, inner, generator=gen).to(dtype)
+    weight = torch.randn(inner, width, generator=gen).to(dtype)
+    truth = g.double() @ weight.double()
+    # a rounding per term of the sum, then one of the result
+    sums = g.double().abs() @ weight.double().abs()
+    half_ulp = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    bound = (inner + 1) * 2.0 ** -24 * sums * (1 + half_ulp) + half_ulp * truth.abs() + 2.0 ** -25
+    got = rows_product(g.to(device), weight.to(device)).cpu()
+    assert got.shape == truth.shape and got.dtype == dtype
+    assert bool(((got.double() - truth).abs() <= bound).all())
+    heads = rows_product(g.to(device), weight.to(device), head_dim).cpu()
+    assert torch.equal(heads, got.unflatten(-1, (-1, head_dim)).transpose(2, 3))
+    g[0, 0, 0, inner - 1], weight[inner - 1, width - 1] = float("inf"), float("inf")
+    got = rows_product(g.to(device), weight.to(device)).cpu().reshape(-1, width)
+    assert bool(got[1:, :-1].isfinite().all()) and not bool(got[0].isfinite().any()) and not bool(got[:, -1].isfinite().any())
