@@ -246,15 +246,21 @@ int lbi_gated_mlp_pullback(const void* g_down_input, const void* fc1_output, voi
                            int g_broadcast_t, int dtype, void* stream);
 
 /*
- * Product of few rows with a weight as it lies (the pullback of y = x W^T): out = a w, sums in fp32, one rounding.
+ * Small products of a linear layer y = x weight^T: sums in fp32, one rounding.
  *
- *   a [M,K], w [K,N]  ->  out [M/T, N/Dh, T, Dh]   (T = 1, Dh = N: [M,N])
+ *   LBI_PRODUCT_ROWS_BY_WEIGHT  out = a w    a [M,K], w [K,N]
+ *   LBI_PRODUCT_GRADIENT        out = a^T w  a [K,M], w [K,N]
+ *   LBI_PRODUCT_FORWARD         out = a w^T  a [M,K], w [N,K]
+ *   out [M/T, N/Dh, T, Dh]   (T = 1, Dh = N: [M,N])
  *
- * 16-bit types; N and K multiples of 8, Dh a multiple of 4, 16-byte aligned tensors, operands below 2 GiB.  For products
- * of a few microseconds: a library product is faster on many rows.
+ * 16-bit types; rows of a, w and out of whole 16-byte pieces, Dh a multiple of 4, 16-byte aligned tensors, operands below
+ * 2 GiB.  For products of a few microseconds: a library product is faster on large ones.
  */
-int lbi_rows_product(const void* a, const void* w, void* out, int64_t M, int64_t N, int64_t K, int64_t T, int64_t Dh,
-                     int dtype, void* stream);
+#define LBI_PRODUCT_ROWS_BY_WEIGHT 0
+#define LBI_PRODUCT_GRADIENT 1
+#define LBI_PRODUCT_FORWARD 2
+int lbi_small_product(const void* a, const void* w, void* out, int64_t M, int64_t N, int64_t K, int form, int64_t T,
+                      int64_t Dh, int dtype, void* stream);
 
 /*
  * Head split of the out_proj-input cotangent: [B,P,T,H*Dh] -> [B,P,H,T,Dh], the layout

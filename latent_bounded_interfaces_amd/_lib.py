@@ -75,7 +75,7 @@ SYMBOLS = {
         [_c.c_void_p] * 6 + [_c.c_int64] * 4 + [_c.c_float, _c.c_int, _c.c_int, _c.c_int, _c.c_void_p],
     ),
     "lbi_gated_mlp_pullback": (_c.c_int, [_c.c_void_p] * 3 + [_c.c_int64] * 4 + [_c.c_int, _c.c_int, _c.c_void_p]),
-    "lbi_rows_product": (_c.c_int, [_c.c_void_p] * 3 + [_c.c_int64] * 5 + [_c.c_int, _c.c_void_p]),
+    "lbi_small_product": (_c.c_int, [_c.c_void_p] * 3 + [_c.c_int64] * 3 + [_c.c_int] + [_c.c_int64] * 2 + [_c.c_int, _c.c_void_p]),
     "lbi_attn_heads_split": (_c.c_int, [_c.c_void_p] * 2 + [_c.c_int64] * 5 + [_c.c_int, _c.c_void_p]),
     "lbi_attn_qkv_pullback": (
         _c.c_int,

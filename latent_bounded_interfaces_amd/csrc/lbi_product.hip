@@ -1,5 +1,8 @@
-// C = A W for few rows: A [M, K] cotangent rows, W [K, N] a weight as it lies (out x in), both of one 16-bit type, sums in
-// fp32, C rounded once and written as [M, N] or, heads split, as [M / T, N / Dh, T, Dh].
+// The small products of a linear layer, y = x weight^T, in one 16-bit type, sums in fp32, C rounded once:
+//   ROWS_BY_WEIGHT  C = A W    the pullback: A [M, K] cotangent rows, W [K, N] the weight as it lies; C as [M, N] or, heads
+//                              split, as [M / T, N / Dh, T, Dh]
+//   GRADIENT        C = A^T W  the weight's gradient: A [K, M] cotangent rows, W [K, N] the layer's input
+//   FORWARD         C = A W^T  the layer itself: A [M, K], W [N, K]
 //
 // A call of this size is a few microseconds of products on the part; what it costs is the call.  (A library product takes 18 us of
 // host time, one here 7, and the layout that the next kernel wants takes no launch of its own.)
@@ -8,8 +11,8 @@
 // of a tile, and their sums are added in wave order.  Operands pass through LDS in chunks of 64 k, two buffers, the
 // next AHEAD chunks in registers: bound by the latency of those loads where K is long (0.2 us a chunk; 0.37 while the compiler
 // waited for all of them at every chunk: 512 x 6144 x 768 35.7 -> 20.5 us, 2048 x 2048 x 256 13.9 -> 9.0).  The product is formed as C^T
-// (lanes are rows of C), so that W, whose reduction index is its row, comes through transposing LDS reads, A through plain
-// ones, and a lane ends up with four consecutive columns: 8-byte stores.
+// (lanes are rows of C), so that a lane ends up with four consecutive columns: 8-byte stores.  An operand whose reduction
+// index is its row comes through transposing LDS reads, another through plain ones.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -64,8 +67,9 @@ template <int ROWS> struct Stage {
     }
 };
 
-// WN = 2: the tile of W is 64 columns wide.
-template <typename T, int WM>
+// The tile of W is 64 columns wide.  FORM: how the operands lie.
+constexpr int ROWS_BY_WEIGHT = LBI_PRODUCT_ROWS_BY_WEIGHT, GRADIENT = LBI_PRODUCT_GRADIENT, FORWARD = LBI_PRODUCT_FORWARD;
+template <typename T, int WM, int FORM>
 __global__ __launch_bounds__(256) void product_kernel(const T* __restrict__ a, const T* __restrict__ w, T* __restrict__ out,
                                                       int M, int N, int K, int T_len, int Dh, int n_tiles) {
     constexpr int KS = 2 / WM, STEPS = CHUNK / 16 / KS, ROWS = 32 * WM;
@@ -78,14 +82,17 @@ __global__ __launch_bounds__(256) void product_kernel(const T* __restrict__ a, c
     const auto a_src = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(a), 0, (unsigned)M * K * 2, 4 << 15);
     const auto w_src = __builtin_amdgcn_make_buffer_rsrc(const_cast<T*>(w), 0, (unsigned)K * N * 2, 4 << 15);
     const int steps = (K + CHUNK - 1) / CHUNK;
+    static_assert(FORM != GRADIENT || WM == 2, "a transposed tile of A has 64 columns");
     Stage<ROWS> as[AHEAD];
     Stage<CHUNK> ws[AHEAD];
     f32x16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
     auto fetch = [&](int slot, int it) __attribute__((always_inline)) {  // chunks past the last are all zero
-        as[slot].fetch(a_src, row0, it * CHUNK, K, tid);
-        ws[slot].fetch(w_src, it * CHUNK, col0, N, tid);
+        if constexpr (FORM == GRADIENT) as[slot].fetch(a_src, it * CHUNK, row0, M, tid);
+        else as[slot].fetch(a_src, row0, it * CHUNK, K, tid);
+        if constexpr (FORM == FORWARD) ws[slot].fetch(w_src, col0, it * CHUNK, K, tid);
+        else ws[slot].fetch(w_src, it * CHUNK, col0, N, tid);
     };
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u) fetch(u, u);
@@ -101,8 +108,12 @@ __global__ __launch_bounds__(256) void product_kernel(const T* __restrict__ a, c
 #pragma unroll
         for (int ks = 0; ks < STEPS; ++ks) {
             const int k = kz * STEPS + ks;
-            const u32x4 af = *reinterpret_cast<const u32x4*>(buf + tile_off<64>(32 * wm + m, 2 * k + h));
-            acc = Mma<T>::mma(frag_columns(buf + A_BYTES, lane, 16 * k, 32 * wn), af, acc);
+            u32x4 af, wf;
+            if constexpr (FORM == GRADIENT) af = frag_columns(buf, lane, 16 * k, 32 * wm);
+            else af = *reinterpret_cast<const u32x4*>(buf + tile_off<64>(32 * wm + m, 2 * k + h));
+            if constexpr (FORM == FORWARD) wf = *reinterpret_cast<const u32x4*>(buf + A_BYTES + tile_off<64>(32 * wn + m, 2 * k + h));
+            else wf = frag_columns(buf + A_BYTES, lane, 16 * k, 32 * wn);
+            acc = Mma<T>::mma(wf, af, acc);
         }
     };
     // Whole turns of the ring, then what is left, nested: a step that is left out in the middle would make the compiler wait for
@@ -149,16 +160,16 @@ __global__ __launch_bounds__(256) void product_kernel(const T* __restrict__ a, c
 }
 
 template <typename T>
-int launch(const void* a, const void* w, void* out, int M, int N, int K, int T_len, int Dh, hipStream_t stream) {
+int launch(const void* a, const void* w, void* out, int M, int N, int K, int form, int T_len, int Dh, hipStream_t stream) {
     const int n_tiles = (N + 63) / 64;
     // 64 rows of a workgroup where that gives every CU one, 32 otherwise
-    const bool tall = (long long)((M + 63) / 64) * n_tiles >= device_compute_units();
+    const bool tall = form == GRADIENT || (long long)((M + 63) / 64) * n_tiles >= device_compute_units();
     const int m_tiles = tall ? (M + 63) / 64 : (M + 31) / 32;
-    const dim3 grid((unsigned)(m_tiles * n_tiles));
-    const T *ap = static_cast<const T*>(a), *wp = static_cast<const T*>(w);
-    T* op = static_cast<T*>(out);
-    if (tall) hipLaunchKernelGGL((product_kernel<T, 2>), grid, dim3(256), 0, stream, ap, wp, op, M, N, K, T_len, Dh, n_tiles);
-    else hipLaunchKernelGGL((product_kernel<T, 1>), grid, dim3(256), 0, stream, ap, wp, op, M, N, K, T_len, Dh, n_tiles);
+    const auto kernel = form == GRADIENT ? product_kernel<T, 2, GRADIENT>
+                        : form == FORWARD ? (tall ? product_kernel<T, 2, FORWARD> : product_kernel<T, 1, FORWARD>)
+                                          : (tall ? product_kernel<T, 2, ROWS_BY_WEIGHT> : product_kernel<T, 1, ROWS_BY_WEIGHT>);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(m_tiles * n_tiles)), dim3(256), 0, stream, static_cast<const T*>(a),
+                       static_cast<const T*>(w), static_cast<T*>(out), M, N, K, T_len, Dh, n_tiles);
     LBI_HIP_CHECK(hipGetLastError());
     return LBI_OK;
 }
@@ -167,25 +178,29 @@ int launch(const void* a, const void* w, void* out, int M, int N, int K, int T_l
 }  // namespace product
 }  // namespace lbi
 
-extern "C" int lbi_rows_product(const void* a, const void* w, void* out, int64_t M, int64_t N, int64_t K, int64_t T, int64_t Dh,
-                                int dtype, void* stream) {
+extern "C" int lbi_small_product(const void* a, const void* w, void* out, int64_t M, int64_t N, int64_t K, int form, int64_t T,
+                                 int64_t Dh, int dtype, void* stream) {
     using namespace lbi;
     clear_error();
     if (M < 0 || N < 0 || K < 0 || T < 1 || Dh < 0)
-        return fail(LBI_ERR_INVALID, "lbi_rows_product: bad size (M=%lld N=%lld K=%lld T=%lld Dh=%lld)", (long long)M, (long long)N,
+        return fail(LBI_ERR_INVALID, "lbi_small_product: bad size (M=%lld N=%lld K=%lld T=%lld Dh=%lld)", (long long)M, (long long)N,
                     (long long)K, (long long)T, (long long)Dh);
     if (M == 0 || N == 0) return LBI_OK;
-    if (!a || !w || !out) return fail(LBI_ERR_INVALID, "lbi_rows_product: null pointer");
+    if (!a || !w || !out) return fail(LBI_ERR_INVALID, "lbi_small_product: null pointer");
+    if (form != LBI_PRODUCT_ROWS_BY_WEIGHT && form != LBI_PRODUCT_GRADIENT && form != LBI_PRODUCT_FORWARD)
+        return fail(LBI_ERR_INVALID, "lbi_small_product: bad form %d", form);
     constexpr int64_t kMost = 1 << 30;  // elements of a matrix: offsets are 32 bits of bytes, and one bit says "past the end"
-    if ((dtype != LBI_F16 && dtype != LBI_BF16) || K < 1 || N % 8 != 0 || K % 8 != 0 || M >= kMost || N >= kMost || K >= kMost ||
-        T >= kMost || M * K > kMost - 64 * K - 4096 || (K + 256) * N > kMost - 4096 ||
-        (M / 32 + 1) * (N / 64 + 1) >= 1 << 24)
-        return fail(LBI_ERR_UNSUPPORTED, "lbi_rows_product: needs half or bfloat16, N and K multiples of 8, operands below 2 GiB, "
-                                         "fewer than 2^24 tiles");
+    const bool by_pieces = N % 8 == 0 && (form == LBI_PRODUCT_GRADIENT ? M : K) % 8 == 0;
+    // what the tiles of the kernel span, the chunks that are asked for ahead included
+    const bool fits = M < kMost && N < kMost && K < kMost && (M + 64) * (K + 256) < kMost && (K + 256) * (N + 64) < kMost &&
+                      (M / 32 + 1) * (N / 64 + 1) < 1 << 24;
+    if ((dtype != LBI_F16 && dtype != LBI_BF16) || K < 1 || !by_pieces || !fits)
+        return fail(LBI_ERR_UNSUPPORTED, "lbi_small_product: needs half or bfloat16, rows of whole 16-byte pieces, operands below "
+                                         "2 GiB, fewer than 2^24 tiles");
     if (Dh < 1 || Dh % 4 != 0 || N % Dh != 0 || M % T != 0)
-        return fail(LBI_ERR_INVALID, "lbi_rows_product: N must be heads of Dh (a multiple of 4), M sequences of T rows");
+        return fail(LBI_ERR_INVALID, "lbi_small_product: N must be heads of Dh (a multiple of 4), M sequences of T rows");
     for (const void* ptr : {a, w, (const void*)out})
-        if (reinterpret_cast<uintptr_t>(ptr) % 16) return fail(LBI_ERR_INVALID, "lbi_rows_product: tensors must be 16-byte aligned");
+        if (reinterpret_cast<uintptr_t>(ptr) % 16) return fail(LBI_ERR_INVALID, "lbi_small_product: tensors must be 16-byte aligned");
     const auto typed = dtype == LBI_F16 ? product::launch<_Float16> : product::launch<bf16_raw>;
-    return typed(a, w, out, (int)M, (int)N, (int)K, (int)T, (int)Dh, static_cast<hipStream_t>(stream));
+    return typed(a, w, out, (int)M, (int)N, (int)K, form, (int)T, (int)Dh, static_cast<hipStream_t>(stream));
 }

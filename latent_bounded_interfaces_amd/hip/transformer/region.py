@@ -10,7 +10,7 @@ backends/transformer_cuda.py:45-64) for the block the reference's backend execut
     region_output = m + res2 of the last layer
 
 The cotangent basis [B, P, T, D] is pulled back through the layers in reverse.  Matrix
-products are library GEMMs on the [B*P*T, *] cotangent rows (small ones ``lbi_rows_product``); everything between them runs in
+products are library GEMMs on the [B*P*T, *] cotangent rows (small ones ``lbi_small_product``); everything between them runs in
 the kernels of liblbi_hip.so (RMSNorm, gated MLP, head split, rotary embedding + KV-group
 sum, causal convolution, and the attention pullback itself).  The residual-stream cotangent
 is kept in fp32, branch cotangents in the dtype of the weights.  Inputs are read from the
@@ -259,35 +259,47 @@ _TRANSPOSED_COPY_MIN_ROWS = 65536
 #: Multiply-adds and results up to which a product runs on the package's own kernel.  A call of the library takes 18 us of
 #: host time, one of this kernel 7; on the GPU (bf16, M x K x N, this kernel and the library): 512 x 256 x 1024 3.8 and 5.2 us,
 #: 2048 x 2048 x 256 9.0 and 11.8, 1000 x 1536 x 768 9.7 and 10.8, 3001 x 1000 x 520 14.8 and 15.5, 4096 x 256 x 1024 9.2 and 8.4;
-#: past the lines 8192 x 256 x 1024 15.4 and 11.7, 4096 x 512 x 2048 21.5 and 15.5.
+#: past the lines 8192 x 256 x 1024 15.4 and 11.7, 4096 x 512 x 2048 21.5 and 15.5.  Weight gradients: 256 x 1000 x 256 7.1 and 34.8,
+#: 4096 x 600 x 512 12.0 and 13.3, 6144 x 300 x 768 15.3 and 14.3, 256 x 8192 x 256 34.6 and 46.7; forward products: 500 x 768 x 2304
+#: 8.7 and 8.2, 2000 x 512 x 1024 7.4 and 7.9.
 _SMALL_PRODUCT = 3 << 29
 _SMALL_PRODUCT_RESULTS = 1 << 22
 
 
-def _is_small_product(g: torch.Tensor, weight: torch.Tensor) -> bool:
-    inner, width = weight.shape
-    return (g.dtype in (torch.float16, torch.bfloat16) and g.numel() * width <= _SMALL_PRODUCT
-            and inner == g.shape[-1] and inner % 8 == 0 and width % 8 == 0 and g.dim() == 4
-            and g.numel() > 0 and g.numel() // inner * width <= _SMALL_PRODUCT_RESULTS and weight.numel() > 0 and weight.device == g.device
-            and g.is_contiguous() and weight.is_contiguous()
-            and g.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0)
+#: how the operands of ``lbi_small_product`` lie
+_ROWS_BY_WEIGHT, _GRADIENT, _FORWARD = 0, 1, 2
 
 
-def rows_product(g: torch.Tensor, weight: torch.Tensor, head_dim: int | None = None) -> torch.Tensor:
-    """``g [B,P,T,K] @ weight [K,N]`` for few rows of a 16-bit type; with ``head_dim`` as ``[B,P,N/head_dim,T,head_dim]``."""
-    _require_cuda(g, weight)
-    bsz, basis, seqlen, inner = g.shape
-    width = int(weight.shape[1])
-    if head_dim is None:
-        shape, seqlen, head_dim = (bsz, basis, seqlen, width), 1, width
-    else:
-        shape = (bsz, basis, width // head_dim, seqlen, head_dim)
-    out = torch.empty(shape, device=g.device, dtype=g.dtype)
-    with _lib.device_guard(g.device):
-        status = _lib.load().lbi_rows_product(g.data_ptr(), weight.data_ptr(), out.data_ptr(), g.numel() // inner, width,
-                                              inner, seqlen, head_dim, _lib.dtype_code(g.dtype), _stream(g))
-    _lib.check(status, "lbi_rows_product")
+def _is_small_product(a: torch.Tensor, w: torch.Tensor, height: int, width: int, inner: int, form: int) -> bool:
+    return (a.dtype in (torch.float16, torch.bfloat16) and w.dtype == a.dtype and w.device == a.device
+            and 0 < height * width * inner <= _SMALL_PRODUCT and height * width <= _SMALL_PRODUCT_RESULTS
+            and width % 8 == 0 and (height if form == _GRADIENT else inner) % 8 == 0
+            and a.is_contiguous() and w.is_contiguous() and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+
+
+def small_product(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, height: int, width: int, inner: int, form: int,
+                  seqlen: int = 1, head_dim: int | None = None) -> torch.Tensor:
+    """``out`` filled with ``a w``, ``a^T w`` or ``a w^T`` (``form``), ``[height, width]`` with ``inner`` terms a sum; with
+    ``head_dim`` as ``[height / seqlen, width / head_dim, seqlen, head_dim]``."""
+    _require_cuda(a, w, out)
+    with _lib.device_guard(a.device):
+        status = _lib.load().lbi_small_product(a.data_ptr(), w.data_ptr(), out.data_ptr(), height, width, inner, form, seqlen,
+                                               head_dim or width, _lib.dtype_code(a.dtype), _stream(a))
+    _lib.check(status, "lbi_small_product")
     return out
+
+
+def _rows_product(g: torch.Tensor, weight: torch.Tensor, head_dim: int | None = None) -> torch.Tensor | None:
+    """``g [B,P,T,K] @ weight [K,N]``, with ``head_dim`` as ``[B,P,N/head_dim,T,head_dim]``; ``None`` where it is not a small
+    product."""
+    bsz, basis, seqlen, inner = g.shape
+    rows, width = bsz * basis * seqlen, int(weight.shape[1])
+    if weight.shape[0] != inner or not _is_small_product(g, weight, rows, width, inner, _ROWS_BY_WEIGHT):
+        return None
+    if head_dim is None:
+        return small_product(g, weight, g.new_empty(bsz, basis, seqlen, width), rows, width, inner, _ROWS_BY_WEIGHT)
+    out = g.new_empty(bsz, basis, width // head_dim, seqlen, head_dim)
+    return small_product(g, weight, out, rows, width, inner, _ROWS_BY_WEIGHT, seqlen, head_dim)
 
 
 def _apply_transposed(g: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
@@ -298,8 +310,9 @@ def _apply_transposed(g: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     if weight.dtype != g.dtype:
         # a forward run under autocast multiplied by the weight cast to the compute dtype; so does its pullback
         weight = weight.to(g.dtype)
-    if _is_small_product(g, weight):
-        return rows_product(g, weight)
+    small = _rows_product(g, weight)
+    if small is not None:
+        return small
     if g.numel() // g.shape[-1] < _TRANSPOSED_COPY_MIN_ROWS:
         return torch.matmul(g, weight)
     return torch.nn.functional.linear(g, weight.t().contiguous())
@@ -309,8 +322,10 @@ def _apply_transposed_to_heads(g: torch.Tensor, weight: torch.Tensor, n_heads: i
     """``g @ weight`` as ``[B,P,H,T,Dh]``."""
     if weight.dtype != g.dtype:
         weight = weight.to(g.dtype)
-    if head_dim % 4 == 0 and weight.shape[1] == n_heads * head_dim and _is_small_product(g, weight):
-        return rows_product(g, weight, head_dim)
+    if head_dim % 4 == 0 and weight.shape[1] == n_heads * head_dim:
+        small = _rows_product(g, weight, head_dim)
+        if small is not None:
+            return small
     return attn_heads_split(_apply_transposed(g, weight), n_heads, head_dim)
 
 
@@ -321,7 +336,13 @@ def _rows(t: torch.Tensor) -> torch.Tensor:
 def _linear_grads(sink: dict, linear: Any, g_out: torch.Tensor, x: torch.Tensor) -> None:
     """Weight (and bias) gradient of ``y = x W^T + b`` for the single direction in ``g_out [B,1,T,O]``."""
     g2 = _rows(g_out)
-    sink[id(linear.weight)] = torch.matmul(g2.t(), _rows(x).to(g2.dtype)).to(linear.weight.dtype)
+    x2 = _rows(x).to(g2.dtype)
+    (rows, height), width = g2.shape, int(x2.shape[1])
+    if x2.shape[0] == rows and _is_small_product(g2, x2, height, width, rows, _GRADIENT):
+        grad = small_product(g2, x2, g2.new_empty(height, width), height, width, rows, _GRADIENT)
+    else:
+        grad = torch.matmul(g2.t(), x2)
+    sink[id(linear.weight)] = grad.to(linear.weight.dtype)
     bias = getattr(linear, "bias", None)
     if bias is not None:
         sink[id(bias)] = g2.float().sum(dim=0).to(bias.dtype)
@@ -429,8 +450,13 @@ def _layer_input_pullback(block: Any, layer_cache: Any, g_hidden: torch.Tensor |
             if param_grads is not None:
                 # the cache keeps the projection after the convolution only: redo the projection
                 bias = getattr(attn.in_proj, "bias", None)
-                x_pre = torch.nn.functional.linear(a_cache.norm_output.to(wdtype), attn.in_proj.weight.to(wdtype),
-                                                   None if bias is None else bias.to(wdtype))
+                x_in, weight = a_cache.norm_output.to(wdtype), attn.in_proj.weight.to(wdtype)
+                (bsz, seqlen, inner), width = x_in.shape, int(weight.shape[0])
+                if bias is None and weight.shape[1] == inner and \
+                        _is_small_product(x_in, weight, bsz * seqlen, width, inner, _FORWARD):
+                    x_pre = small_product(x_in, weight, x_in.new_empty(bsz, seqlen, width), bsz * seqlen, width, inner, _FORWARD)
+                else:
+                    x_pre = torch.nn.functional.linear(x_in, weight, None if bias is None else bias.to(wdtype))
                 _conv_grads(param_grads, attn.conv1d, g_qkv, x_pre)
                 del x_pre
             g_qkv = causal_conv1d_pullback(g_qkv, attn.conv1d.weight)

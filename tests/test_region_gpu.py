@@ -560,24 +560,51 @@ def test_region_pullback_at_the_end_to_end_layer_shape_matches_oracle(device):
     ((2, 1, 333), 320, 136, 8), ((1, 5, 64), 448, 256, 128), ((1, 16, 128), 2048, 256, 64), ((1, 1, 3001), 200, 520, 40),
     ((3, 1, 1), 136, 72, 72), ((2, 4, 250), 392, 1032, 24),
 ])
-def test_rows_product(lead, inner, width, head_dim, dtype, device):
+def test_small_product(lead, inner, width, head_dim, dtype, device):
     """Rows, columns and chunks of the reduction that end inside a tile, both tile heights, one chunk to more than a turn of the
     ring; infinities stay in their row and column."""
-    from latent_bounded_interfaces_amd.hip.transformer.region import rows_product
+    from latent_bounded_interfaces_amd.hip.transformer import region
 
     gen = torch.Generator().manual_seed(inner + width)
     g = torch.randn(*lead, inner, generator=gen).to(dtype)
     weight = torch.randn(inner, width, generator=gen).to(dtype)
+    rows = math.prod(lead)
     truth = g.double() @ weight.double()
     # a rounding per term of the sum, then one of the result
     sums = g.double().abs() @ weight.double().abs()
     half_ulp = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
     bound = (inner + 1) * 2.0 ** -24 * sums * (1 + half_ulp) + half_ulp * truth.abs() + 2.0 ** -25
-    got = rows_product(g.to(device), weight.to(device)).cpu()
-    assert got.shape == truth.shape and got.dtype == dtype
+
+    def product(a, w, form, head_dim=None):
+        shape = (*lead, width) if head_dim is None else (*lead[:2], width // head_dim, lead[2], head_dim)
+        out = torch.full(shape, float("nan"), dtype=dtype, device=device)
+        return region.small_product(a.contiguous().to(device), w.contiguous().to(device), out, rows, width, inner, form,
+                                    1 if head_dim is None else lead[2], head_dim).cpu()
+
+    got = product(g, weight, 0)
     assert bool(((got.double() - truth).abs() <= bound).all())
-    heads = rows_product(g.to(device), weight.to(device), head_dim).cpu()
+    heads = product(g, weight, 0, head_dim)
     assert torch.equal(heads, got.unflatten(-1, (-1, head_dim)).transpose(2, 3))
+    assert bool(((product(g, weight.t(), 2).double() - truth).abs() <= bound).all())
+    if rows % 8 == 0:
+        assert bool(((product(g.reshape(rows, inner).t(), weight, 1).double() - truth).abs() <= bound).all())
     g[0, 0, 0, inner - 1], weight[inner - 1, width - 1] = float("inf"), float("inf")
-    got = rows_product(g.to(device), weight.to(device)).cpu().reshape(-1, width)
-    assert bool(got[1:, :-1].isfinite().all()) and not bool(got[0].isfinite().any()) and not bool(got[:, -1].isfinite().any())
+    for got in (product(g, weight, 0), product(g, weight.t(), 2)):
+        got = got.reshape(-1, width)
+        assert bool(got[1:, :-1].isfinite().all()) and not bool(got[0].isfinite().any()) and not bool(got[:, -1].isfinite().any())
+
+
+@pytest.mark.parametrize("height,width,rows", [(8, 8, 1), (72, 104, 17), (64, 136, 65), (256, 64, 384), (136, 72, 449), (520, 256, 1000)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_small_product_of_a_weight_gradient(height, width, rows, dtype, device):
+    """Any number of rows; the bound of the test above."""
+    from latent_bounded_interfaces_amd.hip.transformer import region
+
+    gen = torch.Generator().manual_seed(rows)
+    g, x = torch.randn(rows, height, generator=gen).to(dtype), torch.randn(rows, width, generator=gen).to(dtype)
+    got = region.small_product(g.to(device), x.to(device), torch.empty(height, width, dtype=dtype, device=device), height, width,
+                               rows, 1).cpu()
+    truth, sums = g.double().t() @ x.double(), g.double().abs().t() @ x.double().abs()
+    half_ulp = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    bound = (rows + 1) * 2.0 ** -24 * sums * (1 + half_ulp) + half_ulp * truth.abs() + 2.0 ** -25
+    assert bool(((got.double() - truth).abs() <= bound).all())
