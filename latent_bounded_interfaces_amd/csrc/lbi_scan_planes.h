@@ -611,14 +611,18 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
             const int row = row0 + 32 * i + m;
             float total = vdot[i] + __shfl_xor(vdot[i], 32, 64);   // the two k halves of a row
             if (apart) total = fmaf(diag[cur * D + row], vbuf[cur * D + row], total);
-            if (d != D && __builtin_amdgcn_ballot_w64(!(__builtin_fabsf(total) <= 0x1.fffffep127f))) {
-                // an element behind the end of a row that is not finite must not meet the zeros the vector ends in
+            if (apart && __builtin_amdgcn_ballot_w64(!(__builtin_fabsf(total) <= 0x1.fffffep127f))) {
+                // The rows are taken again as they lie: the first product step meets the vector with the sums of its elements'
+                // planes, which are not the elements where those are not finite or round to infinity; and an element behind the
+                // end of a row that is not finite must not meet the zeros the vector ends in.
                 total = 0.0f;
                 if (row < d) {
                     const Tin* a_row = a_base + (size_t)r * a_stride + (size_t)row * d;
+#pragma unroll 8
                     for (int k = 0; k < d; ++k) total = fmaf(to_f32(a_row[k]), vbuf[cur * D + k], total);
                 }
             }
+            if (row >= d) total = 0.0f;   // (zero rows times an infinite vector)
             if (h == 0) {
                 vbuf[(cur ^ 1) * D + row] = total;
                 if (c0 == 0 && row < d) cot[((size_t)b * (K + 1) + r) * d + row] = total;

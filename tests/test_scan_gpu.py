@@ -226,6 +226,31 @@ def test_values_outside_the_range_of_the_planes(kind, rank, bsz, count, dtype, d
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rank", [160, 192, 256])
+@pytest.mark.parametrize("at", [(3, 5), (37, 40), (158, 150), (3, 100)])
+@pytest.mark.parametrize("value", ["inf", "max"])
+def test_fused_chain_meets_what_planes_cannot_hold(value, at, rank, dtype, device):
+    """An infinity and the largest finite value, in the columns that a wave's first product step takes (its own rows') and in
+    another: the cotangents come out as fp32 arithmetic gives them."""
+    from latent_bounded_interfaces_amd.hip.interface import suffix_scan_pullbacks_and_cotangents
+
+    if dtype == torch.bfloat16 and rank == 256:
+        pytest.skip("two planes without a check: the width-256 bf16 kernels")
+    gen = torch.Generator().manual_seed(rank)
+    mats = torch.eye(rank, dtype=dtype).repeat(3, 9, 1, 1)
+    mats[1, 2][at] = torch.finfo(dtype).max if value == "max" else float("inf")
+    g = torch.rand(3, rank, generator=gen) * 0.1 + 0.01
+    _, cot = suffix_scan_pullbacks_and_cotangents(mats.to(device), g.to(device))
+    want = oscan.suffix_cotangents_sequential(mats.double(), g.double())
+    got = cot.cpu().double()
+    assert torch.equal(got.isnan(), want.isnan())
+    ok = want.isfinite()
+    assert torch.equal(got[~ok & ~want.isnan()], want[~ok & ~want.isnan()])
+    # a row has two terms: three roundings of 2^-24
+    assert float(((got - want).abs()[ok] / want.abs()[ok]).max()) <= 2e-7
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rank", [17, 63, 65, 127, 129, 191, 193, 198, 254, 255])
 @pytest.mark.parametrize("bsz,count", [(1, 1), (3, 9)])
 def test_cotangent_chain_rows_in_registers(rank, bsz, count, dtype, device):
