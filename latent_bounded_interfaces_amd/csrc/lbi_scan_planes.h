@@ -12,10 +12,14 @@
 // the rest; the hi x hi products and the smaller ones are summed apart.  Relative error against fp64 (2-norm over K = 128 products
 // at d = 256, B = 64; products of fp32 MFMAs with blocked sums -> here): identity plus update 9.6e-7 -> 2.3e-7, random
 // orthogonal-like 9.2e-7 -> 7.3e-7; the cotangents 1.7e-6 -> 3.9e-7 and 1.7e-6.
-// Three planes hold a number exactly between 2^-100 and 2^127.  A wave whose tile leaves that range (infinities and NaN too)
-// forms it again with fp32 products, and the block enters the next step in fp32: the workgroup goes on like that until
-// every tile is back in range, so the results are those of fp32 arithmetic everywhere.  (A chain below 2^-100 all the way takes 3.5
-// ms where fp32 MFMAs took 2.25; one that shrinks by 0.4 a step the same as there.)
+// Range.  bf16 ends where fp32 does, so the lower planes of a number near 2^-126 would fall below it.  The planes are those of the
+// number times 2^23: every bit of an fp32 number, down to the last of its subnormals, is then a normal number of bf16, and what
+// underflows in a product lies below 2^-172, out of sight of fp32 results.  (fp16 elements need no factor, bf16 ones are their
+// own plane, which the products take subnormal too.)  Products end at 2^81 instead, those of 16-bit elements at 2^104.  A wave whose tile holds such a
+// number, an infinity or NaN forms it again with fp32 products, and the block enters the next step in fp32: the workgroup
+// goes on like that until every tile is back in range.  The error of an element is that of fp32 arithmetic,
+// against the sizes of its own terms.  (B=64 K=128 d=256, a chain above 2^81 all the way 3.4 ms, fp32 MFMAs 2.3; one below 2^-100 1.8, random
+// matrices that shrink by 0.4 a step 1.8, that grow by 1.7 to 2^98 2.1, fp32 MFMAs 2.2-2.3 each.)
 //
 // A workgroup owns CB columns of one batch element and keeps that block of the running suffix S in LDS as three planes,
 // transposed; a wave owns 32 rows.  What a step costs was found by timing it without one thing after the other (d = 256, CB =
@@ -24,7 +28,8 @@
 //  * Rows come by 16-byte transfers into a ring in LDS, four lanes to 64 bytes of a row.  Loaded straight into the registers
 //    that the products want them in, each lane another row, they come at 36 GB/s per CU however many are in flight; like
 //    this at 61, contiguous at 72.
-//  * What is left of a number after a plane is one v_dot2_f32_bf16: 7 instead of 11 instructions for a pair.
+//  * What is left of a number after a plane is one v_dot2_f32_bf16: 7 instead of 11 instructions for a pair.  (The factor of
+//    2^23 is two more: B=64 K=128 d=256 1.77 -> 1.81 ms, B=1 122 -> 126 us; 16-bit elements 0-1 %.)
 //  * The vector work of a product step (the next step's split, the stores of the product before) is written between its
 //    products, one or two instructions' groups to each.
 //  * A step begins with the k of the wave's own rows, so that the barrier behind the handing on sits 12 products later, and
@@ -78,7 +83,7 @@ __device__ __forceinline__ unsigned pack_bf16(float lo, float hi) {
 __device__ __forceinline__ float bf16_lo(unsigned w) { return __uint_as_float(w << 16); }
 __device__ __forceinline__ float bf16_hi(unsigned w) { return __uint_as_float(w & 0xffff0000u); }
 
-// Splits pairs of fp32 numbers into packed bf16 planes, hi + mid + lo == x exactly for 2^-100 < |x| < 2^127.  What is left of a
+// Splits pairs of fp32 numbers into packed bf16 planes, hi + mid + lo == x exactly for multiples of 2^-126 below 2^127.  What is left of a
 // number after a plane is one v_dot2_f32_bf16 with (-1, 0) or (0, -1), which are kept in registers: as literals the
 // compiler would encode them as inline constants, whose value this instruction takes in another format.
 struct Splitter {
@@ -101,11 +106,12 @@ struct Splitter {
     }
 };
 
-// Planes of a stored element, and 16-byte words of the 8 elements a lane brings to a product step.
+// Planes of a stored element, what they are of it, and 16-byte words of the 8 elements a lane brings to a product step.
+constexpr float kScale = 0x1p23f;         // of the suffix block's planes
 template <typename Tin> struct Storage;
-template <> struct Storage<float> { static constexpr int NA = 3, WORDS = 2; };
-template <> struct Storage<_Float16> { static constexpr int NA = 2, WORDS = 1; };
-template <> struct Storage<bf16_raw> { static constexpr int NA = 1, WORDS = 1; };
+template <> struct Storage<float> { static constexpr int NA = 3, WORDS = 2; static constexpr float SCALE = kScale; };
+template <> struct Storage<_Float16> { static constexpr int NA = 2, WORDS = 1; static constexpr float SCALE = 1.0f; };
+template <> struct Storage<bf16_raw> { static constexpr int NA = 1, WORDS = 1; static constexpr float SCALE = 1.0f; };
 
 // Four consecutive elements, aligned as single ones are.
 __device__ __forceinline__ f32x4 load4_at(const float* p) {
@@ -168,6 +174,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
     float* __restrict__ cot, int B, int K, int d, ScanPlan plan) {
     constexpr int NW = D / RT, RTILES = RT / 32, CTILES = CB / 32, NB = D / CB;
     constexpr int NA = Storage<Tin>::NA, WORDS = Storage<Tin>::WORDS, NP = 3;
+    constexpr float SCALE = Storage<Tin>::SCALE, PRODUCT_SCALE = SCALE * kScale;
     constexpr int PITCH = D + 8;                    // bf16 elements of a column of a plane
     constexpr int PLANE = CB * PITCH;
     constexpr int WPITCH = D + 4;                   // floats of a column of the block kept in fp32
@@ -278,8 +285,10 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
     auto lds_barrier = [&]() __attribute__((always_inline)) { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 
     // This wave's RT x CB tile: the newest finished product, and of the next one the sum of the hi x hi products and that
-    // of all others (the diagonal's apart).
+    // of all others (the diagonal's apart).  The product is kept as it comes out, times PRODUCT_SCALE, unless it is past that
+    // range: `down` takes it to what it is.
     f32x16 tot[RTILES][CTILES], top[RTILES][CTILES], fine[RTILES][CTILES];
+    float down = 1.0f;
     auto row_of = [&](int i, int e) __attribute__((always_inline)) { return row0 + 32 * i + 8 * (e >> 2) + 4 * h + (e & 3); };
 
     // Results and start states by element: a descriptor over the matrix, past whose end nothing is read or written, an offset
@@ -298,7 +307,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
     // element n of the tile, n = 0 ... 16 RTILES CTILES - 1, of the finished product
     auto store_element = [&](__amdgpu_buffer_rsrc_t o_r, int n) __attribute__((always_inline)) {
         const int i = n / (16 * CTILES), j = n / 16 % CTILES, q = n % 16 / 4, e = n % 4;
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(tot[i][j][4 * q + e]), o_r, lane_col[j] + row_bytes(i, q, e), 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(tot[i][j][4 * q + e] * down), o_r, lane_col[j] + row_bytes(i, q, e), 0, 0);
     };
     constexpr int NEL = 16 * RTILES * CTILES;
 
@@ -307,6 +316,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
     // 8 + 4 h + [0, 4), which is how the accumulators hold a column, so that a lane writes and reads 16 bytes at a time.
     auto place = [](int k) { return (k & ~15) | ((k >> 2) & 1) << 3 | ((k >> 3) & 1) << 2 | (k & 3); };
     auto wide_tile = [&](const Tin* a_r, bool from_planes, bool chain, float (&vdot)[RTILES], const float* v_old) __attribute__((always_inline)) {
+        down = 1.0f;
 #pragma unroll
         for (int i = 0; i < RTILES; ++i)
 #pragma unroll
@@ -340,6 +350,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
                     const int at = (32 * j + m) * PITCH + place(k);
                     s = (load4(reinterpret_cast<const bf16_raw*>(planes) + at) + load4(reinterpret_cast<const bf16_raw*>(planes) + PLANE + at)) +
                         load4(reinterpret_cast<const bf16_raw*>(planes) + 2 * PLANE + at);
+                    s *= 1.0f / kScale;
                 } else {
                     s = *reinterpret_cast<const f32x4*>(wide_s + (32 * j + m) * WPITCH + k);
                 }
@@ -350,8 +361,8 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
             }
         }
     };
-    // Whether the tile leaves the range in which three planes hold a number exactly.
-    auto out_of_range = [&]() __attribute__((always_inline)) {
+    // Whether the tile, kept as it is or scaled, holds what planes and products do not.
+    auto out_of_range = [&](float limit) __attribute__((always_inline)) {
         float high = 0.0f;
 #pragma unroll
         for (int i = 0; i < RTILES; ++i)
@@ -360,9 +371,21 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
 #pragma unroll
                 for (int x = 0; x < 16; x += 2)
                     high = __builtin_elementwise_maximum(high, __builtin_elementwise_maximum(__builtin_fabsf(tot[i][j][x]), __builtin_fabsf(tot[i][j][x + 1])));
-        const bool large = __builtin_amdgcn_ballot_w64(!(high < 0x1p127f)) != 0;
-        const bool tiny = __builtin_amdgcn_ballot_w64(high >= 0x1p-100f) == 0 && __builtin_amdgcn_ballot_w64(high > 0.0f) != 0;
-        return large || tiny;
+        return __builtin_amdgcn_ballot_w64(!(high < limit)) != 0;
+    };
+    // A tile that is kept as it is goes on in scale, if it can.
+    auto scale_up = [&]() __attribute__((always_inline)) {
+        const bool bad = out_of_range(0x1p127f / PRODUCT_SCALE);
+        if (!bad) {
+#pragma unroll
+            for (int i = 0; i < RTILES; ++i)
+#pragma unroll
+                for (int j = 0; j < CTILES; ++j)
+#pragma unroll
+                    for (int x = 0; x < 16; ++x) tot[i][j][x] *= PRODUCT_SCALE;
+            down = 1.0f / PRODUCT_SCALE;
+        }
+        return bad;
     };
 
     int parity = 0;
@@ -371,7 +394,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             unsigned w[NP];
-            splitter.split<NP>(tot[i][j][4 * q + 2 * u], tot[i][j][4 * q + 2 * u + 1], w);
+            splitter.split<NP>(tot[i][j][4 * q + 2 * u] * (1.0f / SCALE), tot[i][j][4 * q + 2 * u + 1] * (1.0f / SCALE), w);
 #pragma unroll
             for (int p = 0; p < NP; ++p) words[i][j][q][p][u] = w[p];
         }
@@ -404,7 +427,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
 #pragma unroll
                 for (int q = 0; q < 4; ++q)
                     *reinterpret_cast<f32x4*>(wide_s + (32 * j + m) * WPITCH + row_of(i, 4 * q)) =
-                        f32x4{tot[i][j][4 * q], tot[i][j][4 * q + 1], tot[i][j][4 * q + 2], tot[i][j][4 * q + 3]};
+                        f32x4{tot[i][j][4 * q], tot[i][j][4 * q + 1], tot[i][j][4 * q + 2], tot[i][j][4 * q + 3]} * down;
         lds_barrier();
     };
     auto split_all = [&]() __attribute__((always_inline)) {
@@ -510,8 +533,9 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
     }
     if (r_top < r_lo) return;
     lds_barrier();   // the flags are zero
+    const bool past = scale_up();
     split_all();
-    publish(out_of_range());
+    publish(past);
     bool wide = false;
 
     u32x4 raw[RTILES][WORDS];               // this lane's elements of the product step that is split next
@@ -582,6 +606,10 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
                 vdot[i] = fmaf(left0[i][w], vvec[w >> 1][2 * (w & 1)], vdot[i]);
                 vdot[i] = fmaf(left1[i][w], vvec[w >> 1][2 * (w & 1) + 1], vdot[i]);
                 asm volatile("" : "+v"(vdot[i]));   // the sums stay here: sunk to their use they would keep the rows alive
+            }
+            if constexpr (SCALE != 1.0f) {
+                left0[i][w] *= SCALE;
+                left1[i][w] *= SCALE;
             }
         }
         if constexpr (NA == 1) {
@@ -659,8 +687,9 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
                 wait_vm<0>();   // no transfer into LDS outlives the workgroup
                 return;
             }
+            const bool past = scale_up();
             split_all();
-            publish(out_of_range());
+            publish(past);
             lds_barrier();
             wide = __builtin_amdgcn_readfirstlane(asked_wide()) != 0;
             --r;
@@ -830,8 +859,8 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
                             x0 += bf16_lo(afr[0][p][i][w]);
                             x1 += bf16_hi(afr[0][p][i][w]);
                         }
-                        vdot[i] = fmaf(x0, v[2 * w + (w >= 2 ? 4 : 0)], vdot[i]);
-                        vdot[i] = fmaf(x1, v[2 * w + (w >= 2 ? 4 : 0) + 1], vdot[i]);
+                        vdot[i] = fmaf(x0 * (1.0f / SCALE), v[2 * w + (w >= 2 ? 4 : 0)], vdot[i]);
+                        vdot[i] = fmaf(x1 * (1.0f / SCALE), v[2 * w + (w >= 2 ? 4 : 0) + 1], vdot[i]);
                     }
             }
         };
@@ -844,7 +873,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
         if constexpr (HALVES == 2) product_step(1);
 #pragma unroll
         for (int s = 2; s < HALVES; ++s) product_step(s);
-        const bool bad = out_of_range();
+        const bool bad = out_of_range(0x1p127f);
         if (__builtin_expect(bad, 0)) {
             float none[RTILES];
             wide_tile(a_base + (size_t)r * a_stride, true, false, none, nullptr);

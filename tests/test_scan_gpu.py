@@ -250,6 +250,40 @@ def test_fused_chain_meets_what_planes_cannot_hold(value, at, rank, dtype, devic
     assert float(((got - want).abs()[ok] / want.abs()[ok]).max()) <= 2e-7
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("rank", [140, 192, 256])
+@pytest.mark.parametrize("bsz,count", [(3, 5), (20, 14), (1, 40)])
+@pytest.mark.parametrize("kind", ["column", "row", "matrix", "subnormal", "large"])
+def test_tiny_numbers_keep_their_accuracy(kind, rank, bsz, count, dtype, device):
+    """Numbers whose lower planes would fall below the smallest that bf16 holds: one column of the products, one row of a
+    matrix, a whole small matrix times a large suffix; and products past the other end, back in range a step later.  The
+    error is that of the tiny numbers' own row or column."""
+    from latent_bounded_interfaces_amd.hip.interface import suffix_scan_pullbacks, suffix_scan_pullbacks_and_cotangents
+
+    if dtype == torch.bfloat16 and rank == 256 and (bsz, count) != (1, 40):
+        pytest.skip("two planes: the width-256 bf16 kernels")
+    mats, g = oscan.make_scan_inputs(bsz, count, rank, kind="randn", seed=rank + count)
+    if kind == "column":
+        mats[:, count - 1, :, 7] *= 2.0 ** -115
+    elif kind == "row":
+        mats[:, 1, 9] *= 2.0 ** -115
+    else:
+        mats[:, 1] *= {"matrix": 2.0 ** -118, "subnormal": 2.0 ** -126, "large": 2.0 ** -90}[kind]
+        mats[:, 2] *= 2.0 ** (90 if kind == "large" else 60)
+    mats = mats.to(dtype)
+    truth = oscan.suffix_scan_sequential(mats.float(), dtype=torch.float64)
+    want = oscan.suffix_cotangents_sequential(mats.double(), g.double())
+    out, cot = suffix_scan_pullbacks_and_cotangents(mats.to(device), g.to(device))
+    along = 2 if kind == "column" else 3
+    for got in (out, suffix_scan_pullbacks(mats.to(device))):
+        err = (got.cpu().double() - truth).abs().amax(along) / truth.abs().amax(along).clamp_min(1e-300)
+        assert float(err.max()) <= 1e-5
+    # entry by entry against the sizes of its terms, those of the chain or those of the finished product
+    size = torch.maximum(torch.einsum("bkij,bkj->bki", mats.double().abs(), want[:, 1:].abs()),
+                         torch.einsum("bkij,bj->bki", truth[:, :count].abs(), g.double().abs()))
+    assert float(((cot.cpu().double() - want).abs()[:, :count] / size).max()) <= 1e-5
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rank", [17, 63, 65, 127, 129, 191, 193, 198, 254, 255])
 @pytest.mark.parametrize("bsz,count", [(1, 1), (3, 9)])
