@@ -462,9 +462,10 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
     // requests the slot of product steps s ... s + HPS - 1 (past the end: of the steps that follow)
     auto request = [&](unsigned slot, int r, int s) __attribute__((always_inline)) {
         const int rr = r - s / HALVES;
-        // (reads up to 15 elements past a row, never past the tensor: the last matrix is no left operand)
+        // The last row's pieces end up to 15 elements past the matrix.  Those of mats are the next matrix there (the last one is no
+        // left operand); a parked total's are cut, element by element, at its end: the slot behind it may hold anything.
         const __amdgpu_buffer_rsrc_t src = rows(a_base + (size_t)(rr > r_lo ? rr : r_lo) * a_stride,
-                                                (unsigned)(dd * sizeof(Tin)) + 64);
+                                                (unsigned)(dd * sizeof(Tin)) + (MODE >= 2 ? 0 : 64));
         const unsigned k = (unsigned)first_k(s % HALVES) * (unsigned)sizeof(Tin);
 #pragma unroll
         for (int i = 0; i < RTILES; ++i)
