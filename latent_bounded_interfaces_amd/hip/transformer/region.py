@@ -270,11 +270,16 @@ _SMALL_PRODUCT_RESULTS = 1 << 22
 _ROWS_BY_WEIGHT, _GRADIENT, _FORWARD = 0, 1, 2
 
 
+def _small_product_size(height: int, width: int, inner: int, form: int) -> bool:
+    return (0 < height * width * inner <= _SMALL_PRODUCT and height * width <= _SMALL_PRODUCT_RESULTS
+            and width % 8 == 0 and (height if form == _GRADIENT else inner) % 8 == 0
+            # what the kernel's 32-bit offsets span, its tiles and the chunks asked for ahead included
+            and (max(height, width) + 64) * (inner + 256) < 1 << 30)
+
+
 def _is_small_product(a: torch.Tensor, w: torch.Tensor, height: int, width: int, inner: int, form: int) -> bool:
     return (a.dtype in (torch.float16, torch.bfloat16) and w.dtype == a.dtype and w.device == a.device
-            and 0 < height * width * inner <= _SMALL_PRODUCT and height * width <= _SMALL_PRODUCT_RESULTS
-            and width % 8 == 0 and (height if form == _GRADIENT else inner) % 8 == 0
-            and a.is_contiguous() and w.is_contiguous() and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+            and _small_product_size(height, width, inner, form) and a.is_contiguous() and w.is_contiguous() and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
 def small_product(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, height: int, width: int, inner: int, form: int,

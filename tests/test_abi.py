@@ -157,6 +157,26 @@ def test_attention_edge_entry_validates_on_the_host():
     assert "All seven tensors 16-byte aligned (LBI_ERR_INVALID otherwise" in header
 
 
+def test_small_products_are_those_that_the_entry_takes():
+    """The rule that sends a product to lbi_small_product names no size that the entry refuses (the library forms those)."""
+    import itertools
+
+    from latent_bounded_interfaces_amd.hip.transformer import region
+
+    lib = _lib.load()
+    odd = ctypes.c_void_p(264)  # refused after the sizes: nothing is launched
+    sizes = (1, 7, 8, 64, 72, 128, 256, 768, 2048, 4096, 6144, 6152, 16384, 16392, 65536, 1 << 19, 1 << 22, 25_000_000)
+    taken = 0
+    for form, height, width, inner in itertools.product((0, 1, 2), sizes, sizes, sizes):
+        if not region._small_product_size(height, width, inner, form):
+            continue
+        taken += 1
+        assert lib.lbi_small_product(odd, odd, odd, height, width, inner, form, 1, width, _lib.LBI_BF16, None) == -1
+        assert b"aligned" in lib.lbi_last_error(), (form, height, width, inner)
+    assert taken > 300
+    assert not region._small_product_size(8, 8, 25_000_000, 1) and not region._small_product_size(1, 1 << 22, 384, 0)
+
+
 def test_fp32_attention_refuses_what_no_grid_holds():
     """More groups than a grid may have threads for: refused on the host, before a kernel has written anything."""
     lib = _lib.load()
