@@ -265,13 +265,24 @@ _TRANSPOSED_COPY_MIN_ROWS = 65536
 _SMALL_PRODUCT = 3 << 29
 _SMALL_PRODUCT_RESULTS = 1 << 22
 
+#: Terms of a sum up to which it does: a tile of results is one workgroup's, which takes 0.2 us per 64 terms (0.25 in a gradient)
+#: however few tiles there are, while the library cuts long sums.  Whole calls, us, this kernel and the library: 256 x 4096 x 256 13.6 and
+#: 17.7, 512 x 6144 x 768 20.5 and 17.7 (among a parameter VJP's other calls, which wait for the host, still the better: d_model 768, B=1
+#: T=205 515 and 556 for all of it), 256 x 8192 x 256 24.1 and 17.7, 128 x 65536 x 128 178 and 104.  Gradients, for which the library is slower: 64 x 16384 x 64
+#: 65 and 86, 128 x 16384 x 128 66 and 120, 128 x 65536 x 128 253 and 196, 64 x 65536 x 64 253 and 170; with results narrower than a
+#: tile 8 x 4096 x 64 18.6 and 18.5, 8 x 8192 x 64 34 and 28.
+_SMALL_PRODUCT_TERMS = 6144
+_SMALL_GRADIENT_TERMS = 16384
+
 
 #: how the operands of ``lbi_small_product`` lie
 _ROWS_BY_WEIGHT, _GRADIENT, _FORWARD = 0, 1, 2
 
 
 def _small_product_size(height: int, width: int, inner: int, form: int) -> bool:
+    long_sums = form == _GRADIENT and min(height, width) >= 64
     return (0 < height * width * inner <= _SMALL_PRODUCT and height * width <= _SMALL_PRODUCT_RESULTS
+            and inner <= (_SMALL_GRADIENT_TERMS if long_sums else _SMALL_PRODUCT_TERMS)
             and width % 8 == 0 and (height if form == _GRADIENT else inner) % 8 == 0
             # what the kernel's 32-bit offsets span, its tiles and the chunks asked for ahead included
             and (max(height, width) + 64) * (inner + 256) < 1 << 30)

@@ -158,7 +158,8 @@ def test_attention_edge_entry_validates_on_the_host():
 
 
 def test_small_products_are_those_that_the_entry_takes():
-    """The rule that sends a product to lbi_small_product names no size that the entry refuses (the library forms those)."""
+    """The rule that sends a product to lbi_small_product names no size that the entry refuses (the library forms those), and no
+    sum so long that one workgroup takes longer over it than the library."""
     import itertools
 
     from latent_bounded_interfaces_amd.hip.transformer import region
@@ -173,7 +174,9 @@ def test_small_products_are_those_that_the_entry_takes():
         taken += 1
         assert lib.lbi_small_product(odd, odd, odd, height, width, inner, form, 1, width, _lib.LBI_BF16, None) == -1
         assert b"aligned" in lib.lbi_last_error(), (form, height, width, inner)
+        assert inner <= (16384 if form == 1 and min(height, width) >= 64 else 6144)
     assert taken > 300
+    assert region._small_product_size(128, 128, 16384, 1) and not region._small_product_size(128, 128, 65536, 1)
     assert not region._small_product_size(8, 8, 25_000_000, 1) and not region._small_product_size(1, 1 << 22, 384, 0)
 
 
