@@ -278,6 +278,9 @@ _SMALL_GRADIENT_TERMS = 16384
 #: how the operands of ``lbi_small_product`` lie
 _ROWS_BY_WEIGHT, _GRADIENT, _FORWARD = 0, 1, 2
 
+#: looked at before anything else: the shapes of a product cost a microsecond to take apart
+_SMALL_PRODUCT_TYPES = (torch.float16, torch.bfloat16)
+
 
 def _small_product_size(height: int, width: int, inner: int, form: int) -> bool:
     long_sums = form == _GRADIENT and min(height, width) >= 64
@@ -289,8 +292,9 @@ def _small_product_size(height: int, width: int, inner: int, form: int) -> bool:
 
 
 def _is_small_product(a: torch.Tensor, w: torch.Tensor, height: int, width: int, inner: int, form: int) -> bool:
-    return (a.dtype in (torch.float16, torch.bfloat16) and w.dtype == a.dtype and w.device == a.device
-            and _small_product_size(height, width, inner, form) and a.is_contiguous() and w.is_contiguous() and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+    return (a.dtype in _SMALL_PRODUCT_TYPES and w.dtype == a.dtype and w.device == a.device
+            and _small_product_size(height, width, inner, form)
+            and a.is_contiguous() and w.is_contiguous() and a.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
 def small_product(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, height: int, width: int, inner: int, form: int,
@@ -308,6 +312,8 @@ def small_product(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, height: i
 def _rows_product(g: torch.Tensor, weight: torch.Tensor, head_dim: int | None = None) -> torch.Tensor | None:
     """``g [B,P,T,K] @ weight [K,N]``, with ``head_dim`` as ``[B,P,N/head_dim,T,head_dim]``; ``None`` where it is not a small
     product."""
+    if g.dtype not in _SMALL_PRODUCT_TYPES:
+        return None
     bsz, basis, seqlen, inner = g.shape
     rows, width = bsz * basis * seqlen, int(weight.shape[1])
     if weight.shape[0] != inner or not _is_small_product(g, weight, rows, width, inner, _ROWS_BY_WEIGHT):
@@ -353,10 +359,12 @@ def _linear_grads(sink: dict, linear: Any, g_out: torch.Tensor, x: torch.Tensor)
     """Weight (and bias) gradient of ``y = x W^T + b`` for the single direction in ``g_out [B,1,T,O]``."""
     g2 = _rows(g_out)
     x2 = _rows(x).to(g2.dtype)
-    (rows, height), width = g2.shape, int(x2.shape[1])
-    if x2.shape[0] == rows and _is_small_product(g2, x2, height, width, rows, _GRADIENT):
-        grad = small_product(g2, x2, g2.new_empty(height, width), height, width, rows, _GRADIENT)
-    else:
+    grad = None
+    if g2.dtype in _SMALL_PRODUCT_TYPES:
+        (rows, height), width = g2.shape, int(x2.shape[1])
+        if x2.shape[0] == rows and _is_small_product(g2, x2, height, width, rows, _GRADIENT):
+            grad = small_product(g2, x2, g2.new_empty(height, width), height, width, rows, _GRADIENT)
+    if grad is None:
         grad = torch.matmul(g2.t(), x2)
     sink[id(linear.weight)] = grad.to(linear.weight.dtype)
     bias = getattr(linear, "bias", None)
