@@ -24,19 +24,21 @@ inline bool aligned(int64_t dh, size_t element_bytes, std::initializer_list<cons
 
 // Where the scalar kernels (lbi_attn_generic.h), whose tiles are 16 rows, are as fast or faster; both sides measured:
 //  * up to 16 positions half of a 32-row tile is empty, and with few directions waves of a workgroup have no work (B=64
-//    H=16 T=4 Dh=64 P=2: 58 us there, 111 here; P=8: 175 and 122); narrow heads in few workgroups gain from the shorter
-//    chain of a tile here (B=4 H=8 T=16 Dh=32 P=4: 23 and 21 us);
+//    H=16 T=4 Dh=64 P=2: 58 us there, 111 here; P=8: 175 and 122); heads of 17 ... 32 in few workgroups gain from the shorter
+//    chain of a tile here (B=4 H=8 T=16 Dh=32 P=4: 23 and 21 us), narrower ones do not (Dh=8: 17.5 and 20.5, one launch
+//    more), nor do many directions of heads wider than 96 (bf16 B=64 H=16 T=12 P=4, Dh=100: 230 and 277, Dh=96: 203 and 124);
 //  * a call of few workgroups is as long as one of them, and a 32-row tile of very narrow heads, or one that is loaded
 //    element by element, takes longer than two of 16 rows (B=4 H=8 T=48 Dh=8 P=2: 23 and 29 us; B=1 H=4 T=48 Dh=33 P=2: 43
 //    and 51).
-// The lines hold for 16-bit storage too (scalar kernels, here: B=16 H=8 T=16 Dh=80 P=8 63 and 40 us, B=64 H=16 T=12 Dh=96 P=4 221
-// and 126, B=2 H=8 T=32 Dh=24 P=4 30 and 19, B=1 H=2 T=20 Dh=16 P=1 22 and 18).
+// One set of lines for every storage type: over T = 4 ... 56, Dh = 8 ... 128, P = 1 ... 8, B*H = 2 ... 1024 the side they name is the
+// slower one by more than a tenth (and 2 us) in 69 of 1534 bf16 calls, by 1.53 at most (B=64 H=16 T=8 Dh=96 P=4: scalar 184, here
+// 120), and in 9 of fp32's, by 1.22 at most.
 inline bool scalar_is_faster(int64_t B, int64_t H, int64_t T, int64_t dh, int64_t P, bool aligned) {
     const int64_t groups = B * H * P;
     if (groups > 65535) return false;  // more than they take
     if (T <= 16) {
-        if (dh <= 32 && B * H < 512) return false;
-        const bool busy = (P >= 8 && dh <= 96) || (P >= 4 && dh >= 64 && T > 8);  // enough work for the waves
+        if (dh > 16 && dh <= 32 && B * H < 512) return false;
+        const bool busy = (P >= 8 && dh <= 96) || (P >= 4 && dh >= 64 && dh <= 96 && T > 8);  // enough work for the waves
         return !(aligned && busy && groups >= 1024);
     }
     return T <= 48 && groups < 256 && (aligned ? dh <= 16 && T > 32 : dh > 32);
