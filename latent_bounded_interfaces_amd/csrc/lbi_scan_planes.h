@@ -596,17 +596,28 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
             }
         if (mine) diag[buffer * D + row0 + 32 * i + m] = value;
     };
+    // The cotangents of 16-bit elements are summed by product steps, then over them (error against fp64 on random matrices, bf16 B=32
+    // K=20 d=240: 7.0e-7 as one running sum, 4.3e-7 in the chain waves of the kernel these widths were padded to; here 4.4e-7).
+    // fp32 ones were one running sum in the kernel before, too, and B=64 K=128 d=256 takes 1.84 ms like that, 1.87 by steps.
+    constexpr bool SUM_BY_STEPS = NA < 3;
     // The vector work of a product step in units: unit n takes pair w of the next step's elements one plane further.
-    float left0[RTILES][4], left1[RTILES][4];
+    float left0[RTILES][4], left1[RTILES][4], part[RTILES];
     constexpr int UNITS = 4 * NA * RTILES;
     auto unit = [&](int n, int par, bool chain) __attribute__((always_inline)) {
         const int i = n / (4 * NA), p = n % (4 * NA) / 4, w = n % 4;
         if (p == 0) {
             element_pair(i, w, left0[i][w], left1[i][w]);
             if (COT && chain) {
-                vdot[i] = fmaf(left0[i][w], vvec[w >> 1][2 * (w & 1)], vdot[i]);
-                vdot[i] = fmaf(left1[i][w], vvec[w >> 1][2 * (w & 1) + 1], vdot[i]);
-                asm volatile("" : "+v"(vdot[i]));   // the sums stay here: sunk to their use they would keep the rows alive
+                if constexpr (SUM_BY_STEPS) {
+                    part[i] = w == 0 ? left0[i][w] * vvec[0][0] : fmaf(left0[i][w], vvec[w >> 1][2 * (w & 1)], part[i]);
+                    part[i] = fmaf(left1[i][w], vvec[w >> 1][2 * (w & 1) + 1], part[i]);
+                    if (w == 3) vdot[i] += part[i];
+                    asm volatile("" : "+v"(part[i]), "+v"(vdot[i]));   // the sums stay here: sunk to their use they would keep the rows alive
+                } else {
+                    vdot[i] = fmaf(left0[i][w], vvec[w >> 1][2 * (w & 1)], vdot[i]);
+                    vdot[i] = fmaf(left1[i][w], vvec[w >> 1][2 * (w & 1) + 1], vdot[i]);
+                    asm volatile("" : "+v"(vdot[i]));
+                }
             }
             if constexpr (SCALE != 1.0f) {
                 left0[i][w] *= SCALE;
@@ -851,7 +862,8 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
                 // the first elements of the step were split before its vector was there: they are the sum of their planes
                 const float* v = vbuf + cur * D + 4 * h + first_k(0);
 #pragma unroll
-                for (int i = 0; i < RTILES; ++i)
+                for (int i = 0; i < RTILES; ++i) {
+                    float first = 0.0f;
 #pragma unroll
                     for (int w = 0; w < 4; ++w) {
                         float x0 = 0.0f, x1 = 0.0f;
@@ -860,9 +872,11 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_planes_kernel(
                             x0 += bf16_lo(afr[0][p][i][w]);
                             x1 += bf16_hi(afr[0][p][i][w]);
                         }
-                        vdot[i] = fmaf(x0 * (1.0f / SCALE), v[2 * w + (w >= 2 ? 4 : 0)], vdot[i]);
-                        vdot[i] = fmaf(x1 * (1.0f / SCALE), v[2 * w + (w >= 2 ? 4 : 0) + 1], vdot[i]);
+                        first = fmaf(x0 * (1.0f / SCALE), v[2 * w + (w >= 2 ? 4 : 0)], first);
+                        first = fmaf(x1 * (1.0f / SCALE), v[2 * w + (w >= 2 ? 4 : 0) + 1], first);
                     }
+                    vdot[i] += first;
+                }
             }
         };
         product_step(0);

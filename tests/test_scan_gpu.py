@@ -656,6 +656,21 @@ def test_backward_module_contract(device):
     assert {"jac_local_spec_mean", "jac_suffix_spec_max"} <= set(stats)
 
 
+@pytest.mark.parametrize("dtype,rank", [(torch.bfloat16, 160), (torch.float16, 192), (torch.bfloat16, 240), (torch.float16, 256)])
+def test_fused_cotangents_round_as_blocked_sums(dtype, rank, device):
+    """The fused cotangents of the plane kernel on random 16-bit matrices, 2-norm over the chain against fp64.  A sum of n terms of
+    random sign that is rounded n times is off by about sqrt(n / 2) e of itself, e = 2.5e-8 the mean rounding of one addition.
+    Summed by product steps (8 terms, then at most 16 sums) a step leaves sqrt(8 / 2 + 16 / 2) e = 0.9e-7, as one running sum of
+    up to 128 terms 2.0e-7; r steps leave sqrt(r) times that, over 20 steps 2.8e-7 and 6.4e-7 on average."""
+    from latent_bounded_interfaces_amd.hip.interface import suffix_scan_pullbacks_and_cotangents
+
+    mats, g = oscan.make_scan_inputs(32, 20, rank, kind="randn", seed=3)
+    mats = mats.to(dtype)
+    _, cot = suffix_scan_pullbacks_and_cotangents(mats.to(device), g.to(device))
+    want = oscan.suffix_cotangents_sequential(mats.double(), g.double())
+    assert float((cot.cpu().double() - want).norm() / want.norm()) <= 4.2e-7
+
+
 def test_split_fp32_variant_in_subprocess(device):
     """The opt-in bf16-split kernel for fp32 storage (LBI_SCAN_SPLIT_FP32=1) meets the same bar."""
     import os
