@@ -180,6 +180,36 @@ def test_small_products_are_those_that_the_entry_takes():
     assert not region._small_product_size(8, 8, 25_000_000, 1) and not region._small_product_size(1, 1 << 22, 384, 0)
 
 
+def test_small_product_statuses():
+    """What lbi_small_product refuses, each with its status and before anything is launched; empty results are fine."""
+    lib = _lib.load()
+    ok, odd = ctypes.c_void_p(256), ctypes.c_void_p(264)  # never dereferenced
+
+    def call(a=ok, w=ok, out=ok, m=64, n=64, k=64, form=0, t=1, dh=64, dtype=_lib.LBI_BF16):
+        return lib.lbi_small_product(a, w, out, m, n, k, form, t, dh, dtype, None), lib.lbi_last_error()
+
+    for sizes in (dict(m=-1), dict(n=-8), dict(k=-8), dict(t=0), dict(dh=-4)):
+        status, text = call(**sizes)
+        assert status == -1 and b"bad size" in text, sizes
+    assert call(m=0) == (0, b"") and call(n=0) == (0, b"")
+    for name in ("a", "w", "out"):
+        status, text = call(**{name: None})
+        assert status == -1 and b"null" in text
+        status, text = call(**{name: odd})
+        assert status == -1 and b"aligned" in text
+    for form in (-1, 3):
+        status, text = call(form=form)
+        assert status == -1 and b"form" in text
+    for bad in (dict(dtype=_lib.LBI_F32), dict(dtype=7), dict(k=0), dict(n=68, dh=68), dict(k=60), dict(form=1, m=60),
+                dict(form=1, m=64, n=64, k=1 << 25), dict(m=1 << 30)):
+        status, text = call(**bad)
+        assert status == -2 and b"needs half or bfloat16" in text, bad
+    assert call(form=1, k=60, a=odd)[0] == -1   # a gradient sums over any number of rows: refused for its alignment only
+    for heads in (dict(dh=0), dict(dh=6), dict(dh=48), dict(t=3)):
+        status, text = call(**heads)
+        assert status == -1 and b"heads of Dh" in text, heads
+
+
 def test_fp32_attention_refuses_what_no_grid_holds():
     """More groups than a grid may have threads for: refused on the host, before a kernel has written anything."""
     lib = _lib.load()
