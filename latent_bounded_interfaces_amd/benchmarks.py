@@ -488,10 +488,10 @@ def main(argv=None) -> int:
                     help="bound on max|error| / max|expected| (default 2e-5 for float32, 2e-2 for 16-bit storage)")
     ap.add_argument("--pmc-traffic", nargs=2, metavar=("FETCH_DIR", "WRITE_DIR"), default=None,
                     help="write the HBM-traffic JSON of --kernel from two rocprofv3 --pmc output folders")
-    ap.add_argument("--kernel", default="scan_mfma_kernel<float, 256, 32, 64, true, 0>")
+    ap.add_argument("--kernel", default="scan_planes_kernel<float, 256, 32, 64, true, 0>")
     ap.add_argument("--copy-kernel", default="__amd_rocclr_copyBuffer")
     ap.add_argument("--copy-bytes", type=int, default=1 << 30)
-    ap.add_argument("--sources", nargs="*", default=["csrc/lbi_scan.hip", "csrc/lbi_common.h"])
+    ap.add_argument("--sources", nargs="*", default=["csrc/lbi_scan.hip", "csrc/lbi_scan_planes.h", "csrc/lbi_common.h"])
     ap.add_argument("--out", default=None, help="--pmc-traffic: where to write the JSON (default: stdout)")
     ap.add_argument("--scan", nargs="*", default=None, help="time the fused suffix scan instead: B,K,d tuples")
     ap.add_argument("--matrices-only", action="store_true", help="--scan: the suffix matrices without the cotangents")

@@ -50,7 +50,7 @@ def test_committed_traffic_record_names_the_bench_kernel():
 
     record = json.loads(Path(bench.SCAN_TRAFFIC_JSON).read_text())
     assert record["kernel"] == bench.SCAN_KERNEL
-    assert set(record["sources"]) == {"csrc/lbi_scan.hip", "csrc/lbi_common.h"}
+    assert set(record["sources"]) == {"csrc/lbi_scan.hip", "csrc/lbi_scan_planes.h", "csrc/lbi_common.h"}
     # algorithmic bytes of the workload are 4.320e9: a figure far from it would be a unit slip
     assert 4.2e9 < record["traffic_bytes"] < 4.6e9
 
