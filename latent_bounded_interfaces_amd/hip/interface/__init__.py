@@ -52,7 +52,7 @@ def _aligned(t: torch.Tensor, rank: int) -> torch.Tensor:
 def suffix_scan_pullbacks(mats: torch.Tensor, *, exact_suffix: bool = False) -> torch.Tensor:
     """``out[:, r] = mats[:, r] @ ... @ mats[:, K-1]``, ``out[:, K] = I``; fp32, input untouched.
 
-    ``exact_suffix`` matters for bf16 storage at d = 256 only, whose products run on the 16-bit matrix cores with the
+    ``exact_suffix`` matters for bf16 storage at d = 256 (and odd widths above 192, padded to it) only, whose products run on the 16-bit matrix cores with the
     running suffix as a sum of bf16 planes: by default two planes (the suffix operand rounded to 16 significand bits,
     error <= 2e-4 where 16-bit storage is asked 2e-2), with ``exact_suffix=True`` three (its exact fp32 value: only
     the rounding of fp32 accumulation is left, ~1e-5 at K = 128; half again as many products)."""
