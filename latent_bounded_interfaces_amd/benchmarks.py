@@ -461,8 +461,9 @@ def scan_section(steps: int = 10) -> dict:
         torch.cuda.empty_cache()
     for batch in (1, 8):
         row = measure_scan(batch, 128, 256, torch.float32, iters=steps)
-        row["roofline"] = {"bound": "mfma", "achieved": row["tflops"], "peak": 157.3, "unit": "TFLOP/s",
-                           "frac": row["tflops"] / 157.3}
+        peak = PEAK_MFMA_16BIT_TFLOPS / 6  # six products of bf16 planes for one of fp32
+        row["roofline"] = {"bound": "mfma", "achieved": row["tflops"], "peak": peak, "unit": "TFLOP/s",
+                           "frac": row["tflops"] / peak}
         out[f"scan_kparallel_fp32_B{batch}_K128_d256"] = row
     return out
 
