@@ -14,7 +14,8 @@ from pathlib import Path
 PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "liblbi_hip.so"
-SOURCES = ("lbi_common.hip", "lbi_scan.hip", "lbi_attn.hip", "lbi_attn_f32.hip", "lbi_attn_f32_f16.hip",
+SOURCES = ("lbi_common.hip", "lbi_scan.hip", "lbi_scan_narrow.hip", "lbi_scan_narrow_f32.hip", "lbi_scan_narrow_f16.hip",
+           "lbi_scan_narrow_bf16.hip", "lbi_attn.hip", "lbi_attn_f32.hip", "lbi_attn_f32_f16.hip",
            "lbi_attn_f32_bf16.hip", "lbi_region.hip", "lbi_product.hip", "lbi_norms.hip", "lbi_param_grads.hip")
 
 HIPCC_FLAGS = [
@@ -31,7 +32,7 @@ HIPCC_FLAGS = [
 # Flags of single sources.  Kernels that keep rows in registers index them by unrolled loops: one that the compiler does not
 # unroll puts them into scratch memory.
 SOURCE_FLAGS = {src: ["-Werror=pass-failed"] for src in ("lbi_region.hip", "lbi_product.hip", "lbi_attn_f32.hip", "lbi_attn_f32_f16.hip",
-                                                          "lbi_attn_f32_bf16.hip", "lbi_scan.hip")}
+                                                          "lbi_attn_f32_bf16.hip", "lbi_scan.hip", "lbi_scan_narrow_f32.hip", "lbi_scan_narrow_f16.hip", "lbi_scan_narrow_bf16.hip")}
 
 
 def _hipcc() -> str:

@@ -17,6 +17,7 @@
 #include <type_traits>
 
 #include "lbi_scan_colsplit.h"
+#include "lbi_scan_narrow.h"
 #include "lbi_scan_planes.h"
 #include "lbi_scan_split.h"
 
@@ -24,7 +25,8 @@ namespace lbi {
 namespace {
 
 // ---------------------------------------------------------------------------------------
-// fp32 matrix cores: widths 32, 64, 96, 128 and 512.
+// fp32 matrix cores in 32 x 32 tiles: width 512, and widths 17 ... 128 of batches that fill the chip several times over
+// (scan_narrow::takes; the others run in 16 x 16 tiles, whose steps are shorter).
 //
 // One wave computes an RT x CB tile of the new suffix block with
 // v_mfma_f32_32x32x2_f32.  Operand layout of that instruction (lane = 32*h + m):
@@ -48,18 +50,14 @@ namespace {
 // fragments of mats[r] that feed the MFMAs are already in registers, so a step costs
 // D/2 extra FMAs per lane (and nothing from HBM); every column block computes the chain,
 // block 0 writes it.
-// MODE 0: phase 0 only; every switch below is a compile-time constant, which keeps the whole-chain kernel at its
-// register count.  MODE 1: phases 1 and 3 (switches at run time, unit strides).  MODE 2: phase 2 (strided).
-// MODE 3: one level of phase 2 in log-depth form (one product per workgroup, all chunks side by side).
-//
 // RAGGED: the matrices have d < D rows and columns, which are read and written where they lie.  Rows past the last one
 // are zero on chip, and so is what a row's last chunk holds past its end (of the next row or matrix: the last matrix
 // is no left operand); stores past the end go to a descriptor's outside.  Whole calls, matrices and cotangents, fp32, copies padded to
 // the next width -> here: see launch_scan.
-template <typename Tin, int D, int RT, int CB, bool COT, int MODE, bool RAGGED>
+template <typename Tin, int D, int RT, int CB, bool COT, bool RAGGED>
 __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
     const Tin* __restrict__ mats, float* __restrict__ out, const float* __restrict__ g,
-    float* __restrict__ cot, int B, int K, int d_rt, ScanPlan plan) {
+    float* __restrict__ cot, int B, int K, int d_rt) {
     constexpr int NW = D / RT;          // waves per workgroup
     constexpr int NT = 64 * NW;         // threads
     constexpr int RTILES = RT / 32;
@@ -73,24 +71,19 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
     extern __shared__ __align__(16) float lds[];  // [2][CB][PITCH], then (COT) [2][D]
     float* vbuf = lds + 2 * CB * PITCH;
 
-    // A launch covers E = B * (segments per batch element) chains.  With at least 8 of them the workgroups are
-    // dealt round-robin to the 8 XCDs so that all column blocks of one chain get ids that are equal mod 8 and
-    // share one L2; smaller launches are sized exactly.
-    const int nseg = MODE == 1 ? plan.C - 1 : MODE == 3 ? plan.C - 2 : 1;
-    const int E = B * nseg;
+    // With at least 8 batch elements the workgroups are dealt round-robin to the 8 XCDs so that all column blocks of one
+    // element get ids that are equal mod 8 and share one L2; smaller launches are sized exactly.
     const int id = blockIdx.x;
-    int e, c0;
-    if (E >= 8) {
+    int b, c0;
+    if (B >= 8) {
         const int slot = id >> 3;
-        e = (slot / NB) * 8 + (id & 7);
+        b = (slot / NB) * 8 + (id & 7);
         c0 = (slot % NB) * CB;
     } else {
-        e = id / NB;
+        b = id / NB;
         c0 = (id % NB) * CB;
     }
-    if (e >= E || (RAGGED && c0 >= d)) return;
-    const int b = e / nseg;
-    const int seg = e - b * nseg;
+    if (b >= B || (RAGGED && c0 >= d)) return;
 
     const int tid = threadIdx.x;
     const int wave = tid >> 6;
@@ -99,80 +92,12 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
     const int h = lane >> 5;
     const int row0 = wave * RT;
 
+    // Steps r = K - 2 ... 0 multiply mats[r] onto the running suffix and store it; it starts as mats[K - 1].
     float* out_b = out + (size_t)b * (K + 1) * DD;
-    // The chain of this workgroup: steps r = r_top ... r_lo multiply a_base[r * a_stride] onto the running suffix
-    // and store it at o_base[r * o_stride]; the suffix starts as the matrix `init_a` (storage type) or `init_s`
-    // (fp32, a product computed earlier).
     const Tin* a_base = mats + (size_t)b * K * DD;
-    float* o_base = out_b;
-    const Tin* init_a = nullptr;
-    const float* init_s = nullptr;
-    int r_top, r_lo = 0;
-    bool write_tail = false;   // the start matrix and the identity behind it are results (out[K - 1], out[K])
-    bool store_all = true;     // every step's product is a result
-    // the cotangent chain rides on the whole-chain form only; the chunk phases share no chain to carry it
-    static_assert(MODE == 0 || !COT, "chunk phases carry no cotangent chain");
-    size_t stride_rt = DD;
-    if constexpr (MODE == 0) {
-        init_a = a_base + (size_t)(K - 1) * DD;
-        r_top = K - 2;
-        write_tail = true;
-    } else if constexpr (MODE == 1) {
-        if (plan.phase == 1) {
-            const int c = seg + 1;
-            const bool last = c == plan.C - 1;
-            const int end = last ? K : (c + 1) * plan.L - plan.s;
-            init_a = a_base + (size_t)(end - 1) * DD;
-            r_top = end - 2;
-            r_lo = c * plan.L - plan.s;
-            write_tail = last;
-            store_all = last;
-        } else {
-            const int c = seg;
-            init_s = out_b + (size_t)((c + 1) * plan.L - plan.s) * DD;
-            r_top = (c + 1) * plan.L - plan.s - 1;
-            r_lo = c == 0 ? 0 : c * plan.L - plan.s + 1;   // the chunk's first product is a phase 2 result already
-        }
-    } else if constexpr (MODE == 3) {
-        const int c = seg + 1;
-        const float* left = out_b + (size_t)(c * plan.L - plan.s + plan.rd) * DD;
-        float* dst = out_b + (size_t)(c * plan.L - plan.s + plan.wr) * DD;
-        const int partner = c + plan.off;
-        if (partner > plan.C - 1) {
-            // nothing to the right at this distance: the element is complete, it moves to the level's output slot
-            if constexpr (RAGGED) {
-                for (int idx = threadIdx.x; idx < d * CB; idx += NT) {
-                    const int row = idx / CB, col = c0 + idx % CB;
-                    if (col < d) dst[(size_t)row * d + col] = left[(size_t)row * d + col];
-                }
-                return;
-            }
-            for (int idx = threadIdx.x; idx < D * CB / 4; idx += NT) {
-                const int row = idx / (CB / 4), q = idx % (CB / 4);
-                *reinterpret_cast<f32x4*>(dst + (size_t)row * D + c0 + 4 * q) =
-                    *reinterpret_cast<const f32x4*>(left + (size_t)row * D + c0 + 4 * q);
-            }
-            return;
-        }
-        a_base = reinterpret_cast<const Tin*>(left);
-        o_base = dst;
-        init_s = partner == plan.C - 1 ? out_b + (size_t)((plan.C - 1) * plan.L - plan.s) * DD
-                                       : out_b + (size_t)(partner * plan.L - plan.s + plan.rd) * DD;
-        r_top = 0;
-    } else {
-        // step j multiplies the total parked one slot above the first matrix of chunk j + 1 and stores that first slot
-        a_base = reinterpret_cast<const Tin*>(out_b + (size_t)(plan.L - plan.s + 1) * DD);
-        o_base = out_b + (size_t)(plan.L - plan.s) * DD;
-        stride_rt = (size_t)plan.L * DD;
-        init_s = out_b + (size_t)((plan.C - 1) * plan.L - plan.s) * DD;
-        r_top = plan.C - 3;
-    }
-    const bool from_a = MODE == 0 || (MODE == 1 && plan.phase == 1);  // start state: init_a, else init_s
-    // distance between the matrices (and the results) of consecutive steps: a constant except in phase 2
-    const size_t a_stride = MODE == 2 ? stride_rt : DD;
-    const size_t o_stride = a_stride;
+    const Tin* init_a = a_base + (size_t)(K - 1) * DD;
 
-    // Start state into St buffer 0 (and, with write_tail, to its place in the result with the identity behind it).
+    // Start state into St buffer 0 and to its place in the result with the identity behind it.
     {
         float* o_last = out_b + (size_t)(K - 1) * DD;
         float* o_eye = out_b + (size_t)K * DD;
@@ -186,7 +111,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
             for (int u = 0; u < N; ++u) {
                 const int row = first + u * (NT / CB);
                 const size_t off = row < d && c0 + col < d ? (size_t)row * d + c0 + col : 0;
-                val[u] = from_a ? to_f32(init_a[off]) : init_s[off];
+                val[u] = to_f32(init_a[off]);
             }
 #pragma unroll
             for (int u = 0; u < N; ++u) {
@@ -194,7 +119,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
                 if (!(row < d && c0 + col < d)) val[u] = 0.0f;
                 lds[col * PITCH + row] = val[u];
             }
-            if (write_tail && c0 + col < d) {
+            if (c0 + col < d) {
                 for (int u = 0; u < N; ++u) {
                     const int row = first + u * (NT / CB);
                     if (row < d) {
@@ -203,35 +128,13 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
                     }
                 }
             }
-        } else if (MODE != 0) {
-            // the chunk phases are short chains: four elements per load, all loads of a thread in flight
-            constexpr int Q = CB / 4;
-            static_assert((D * Q) % NT == 0, "start-state fill");
-#pragma unroll
-            for (int u = 0; u < D * Q / NT; ++u) {
-                const int idx = tid + u * NT;
-                const int row = idx / Q, q = idx % Q;
-                const size_t off = (size_t)row * D + c0 + 4 * q;
-                const f32x4 v4 = from_a ? load4(init_a + off) : load4(init_s + off);
-                if (write_tail) {
-                    f32x4 eye = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                    for (int t = 0; t < 4; ++t) eye[t] = (row == c0 + 4 * q + t) ? 1.0f : 0.0f;
-                    *reinterpret_cast<f32x4*>(o_last + off) = v4;
-                    *reinterpret_cast<f32x4*>(o_eye + off) = eye;
-                }
-#pragma unroll
-                for (int t = 0; t < 4; ++t) lds[(4 * q + t) * PITCH + row] = v4[t];
-            }
         } else {
         for (int idx = tid; idx < D * CB; idx += NT) {
             const int row = idx / CB;
             const int col = idx % CB;
-            const float val = from_a ? to_f32(init_a[row * D + c0 + col]) : init_s[row * D + c0 + col];
-            if (write_tail) {
-                o_last[row * D + c0 + col] = val;
-                o_eye[row * D + c0 + col] = (row == c0 + col) ? 1.0f : 0.0f;
-            }
+            const float val = to_f32(init_a[row * D + c0 + col]);
+            o_last[row * D + c0 + col] = val;
+            o_eye[row * D + c0 + col] = (row == c0 + col) ? 1.0f : 0.0f;
             lds[col * PITCH + row] = val;
         }
         }
@@ -245,7 +148,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
                     if (row < d)
                         for (int k = 0; k < d; ++k) acc = fmaf(to_f32(init_a[(size_t)row * d + k]), g_b[k], acc);
                 } else for (int k4 = 0; k4 < D; k4 += 4) {
-                    const f32x4 a4 = from_a ? load4(init_a + row * D + k4) : load4(init_s + row * D + k4);
+                    const f32x4 a4 = load4(init_a + row * D + k4);
                     acc = fmaf(a4[0], g_b[k4], acc);
                     acc = fmaf(a4[1], g_b[k4 + 1], acc);
                     acc = fmaf(a4[2], g_b[k4 + 2], acc);
@@ -260,14 +163,14 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
         }
     }
     __syncthreads();
-    if (r_top < r_lo) return;
+    if (K < 2) return;
 
     // Lane's slice of mats[r]: rows row0 + 32*i + m, k = 32*kc + 16*h + [0, 16).
     static_assert(!RAGGED || RTILES == 1, "rows of one tile");
     // fp16 elements of the whole chain without cotangents stay as they are stored until their chunk begins: the compiler widens
     // them at the load otherwise, and waits for it (B=64 K=128: 452 -> 296 us at d = 96, 573 -> 400 at 128; the other forms,
     // which do not wait, lose up to 10 % by widening late, narrow ones 3 %).
-    constexpr bool LATE = std::is_same<Tin, _Float16>::value && D >= 96 && !COT && MODE == 0;
+    constexpr bool LATE = std::is_same<Tin, _Float16>::value && D >= 96 && !COT;
     using Stored = typename std::conditional<LATE, f16x4, f32x4>::type;
     auto load_a = [&](Stored (&dst)[RTILES][4], const Tin* base) {
 #pragma unroll
@@ -283,7 +186,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
                 else dst[i][q] = load4(p);
             }
     };
-    const Tin* a_lane = a_base + (size_t)(!RAGGED || row0 + m < d ? row0 + m : 0) * d + h * 16;  // + r*a_stride + kc*32
+    const Tin* a_lane = a_base + (size_t)(!RAGGED || row0 + m < d ? row0 + m : 0) * d + h * 16;  // + r*DD + kc*32
     unsigned lane_at[CTILES];   // RAGGED: byte offset of this lane's first row in a column of a result
 #pragma unroll
     for (int j = 0; j < CTILES; ++j) {
@@ -297,21 +200,21 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
     static_assert(NCH == 1 || NCH % RING == 0, "a chunk keeps its slot from step to step");
     constexpr int AHEAD = RING - 1;
     Stored a_ring[RING][RTILES][4];
-    // Chunk number c (0 <= c < AHEAD) counted from the start of step r_top; when NCH == 1
+    // Chunk number c (0 <= c < AHEAD) counted from the start of the first step; when NCH == 1
     // chunk 1 is already in the next step.
 #pragma unroll
     for (int c = 0; c < AHEAD; ++c) {
-        const int rr = r_top - c / NCH;
-        load_a(a_ring[c % RING], a_lane + (size_t)(rr > r_lo ? rr : r_lo) * a_stride + (c % NCH) * 32);
+        const int rr = K - 2 - c / NCH;
+        load_a(a_ring[c % RING], a_lane + (size_t)(rr > 0 ? rr : 0) * DD + (c % NCH) * 32);
     }
 
     int cur = 0;
-    for (int r = r_top; r >= r_lo; r -= (NCH == 1 ? 2 : 1)) {
+    for (int r = K - 2; r >= 0; r -= (NCH == 1 ? 2 : 1)) {
         // NCH == 1 runs two steps per trip so ring indices stay compile-time constants.
 #pragma unroll
         for (int sub = 0; sub < (NCH == 1 ? 2 : 1); ++sub) {
         const int rs = r - sub;
-        if (rs < r_lo) break;
+        if (rs < 0) break;
         f32x16 acc[RTILES][CTILES];
 #pragma unroll
         for (int i = 0; i < RTILES; ++i)
@@ -325,10 +228,10 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
         float vdot[RTILES];
 #pragma unroll
         for (int i = 0; i < RTILES; ++i) vdot[i] = 0.0f;
-        const Tin* a_r = a_lane + (size_t)rs * a_stride;
+        const Tin* a_r = a_lane + (size_t)rs * DD;
         // Chunks past the end of this step belong to the next step's matrix (a harmless re-read of
         // the last one after the very last step).
-        const Tin* a_wrap = a_lane + (size_t)(rs > r_lo ? rs - 1 : r_lo) * a_stride;
+        const Tin* a_wrap = a_lane + (size_t)(rs > 0 ? rs - 1 : 0) * DD;
 #pragma unroll
         for (int kc = 0; kc < NCH; ++kc) {
             const int slot = (NCH == 1 ? sub : kc) % RING;
@@ -396,11 +299,9 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
             __builtin_amdgcn_sched_barrier(0);
         }
 
-        // A chunk that only forms its total parks it one slot above its first matrix (phase 1).
-        const bool store = store_all || rs == r_lo;
-        float* o_r = o_base + (size_t)(store_all ? rs : rs + 1) * o_stride;
+        float* o_r = out_b + (size_t)rs * DD;
         float* st_new = lds + (cur ^ 1) * (CB * PITCH);
-        const __amdgpu_buffer_rsrc_t o_rows = scan_planes::rows(o_r, store ? (unsigned)DD * 4 : 0);
+        const __amdgpu_buffer_rsrc_t o_rows = scan_planes::rows(o_r, (unsigned)DD * 4);
 #pragma unroll
         for (int i = 0; i < RTILES; ++i)
 #pragma unroll
@@ -419,7 +320,7 @@ __global__ __launch_bounds__(64 * (D / RT)) void scan_mfma_kernel(
                         }
                     }
                     *reinterpret_cast<f32x4*>(st_new + col * PITCH + row) = v4;
-                    if (!RAGGED && store) {
+                    if (!RAGGED) {
 #pragma unroll
                         for (int t = 0; t < 4; ++t) o_r[(size_t)(row + t) * D + c0 + col] = v4[t];
                     }
@@ -1188,27 +1089,24 @@ int launch_suffix_apply(const void* suffix, const void* g, void* cot, int64_t B,
     return LBI_OK;
 }
 
-template <typename Tin, int D, int RT, int CB, bool COT, int MODE, bool RAGGED>
-int launch_mfma_cot(const void* mats, void* out, const void* g, void* cot, int B, int K, int d, hipStream_t stream,
-                    ScanPlan plan = ScanPlan{0, 0, 0, 0, 0, 0, 0}) {
+template <typename Tin, int D, int RT, int CB, bool COT, bool RAGGED>
+int launch_mfma_cot(const void* mats, void* out, const void* g, void* cot, int B, int K, int d, hipStream_t stream) {
     constexpr int NW = D / RT;
     constexpr int NB = D / CB;
     constexpr size_t lds_bytes = ((size_t)2 * CB * (D + 4) + (COT ? 2 * D : 0)) * sizeof(float);
-    auto kern = scan_mfma_kernel<Tin, D, RT, CB, COT, MODE, RAGGED>;
-    if (int rc = ensure_dynamic_lds<&scan_mfma_kernel<Tin, D, RT, CB, COT, MODE, RAGGED>>(lds_bytes)) return rc;
-    // chains in this launch (the kernel derives the same number from the plan)
-    const int chains = B * (MODE == 1 ? plan.C - 1 : MODE == 3 ? plan.C - 2 : 1);
-    const dim3 grid(chains >= 8 ? ((chains + 7) / 8) * 8 * NB : chains * NB);
+    auto kern = scan_mfma_kernel<Tin, D, RT, CB, COT, RAGGED>;
+    if (int rc = ensure_dynamic_lds<&scan_mfma_kernel<Tin, D, RT, CB, COT, RAGGED>>(lds_bytes)) return rc;
+    const dim3 grid(B >= 8 ? ((B + 7) / 8) * 8 * NB : B * NB);
     hipLaunchKernelGGL(kern, grid, dim3(64 * NW), lds_bytes, stream, static_cast<const Tin*>(mats),
-                       static_cast<float*>(out), static_cast<const float*>(g), static_cast<float*>(cot), B, K, d, plan);
+                       static_cast<float*>(out), static_cast<const float*>(g), static_cast<float*>(cot), B, K, d);
     LBI_HIP_CHECK(hipGetLastError());
     return LBI_OK;
 }
 
 template <typename Tin, int D, int RT, int CB, bool RAGGED = false>
 int launch_mfma(const void* mats, void* out, const void* g, void* cot, int B, int K, int d, hipStream_t stream) {
-    return cot ? launch_mfma_cot<Tin, D, RT, CB, true, 0, RAGGED>(mats, out, g, cot, B, K, d, stream)
-               : launch_mfma_cot<Tin, D, RT, CB, false, 0, RAGGED>(mats, out, nullptr, nullptr, B, K, d, stream);
+    return cot ? launch_mfma_cot<Tin, D, RT, CB, true, RAGGED>(mats, out, g, cot, B, K, d, stream)
+               : launch_mfma_cot<Tin, D, RT, CB, false, RAGGED>(mats, out, nullptr, nullptr, B, K, d, stream);
 }
 
 // Whether the products of the chunk totals (phase 2) run in log depth: level l multiplies every element by the one
@@ -1231,11 +1129,11 @@ inline bool totals_in_log_depth(int L, int C) {
 // L is the length with the least such depth among those whose chunks still fit two
 // workgroups per CU; where they need more than one per CU a step takes 1.7x as long.  K = 128, matrices only, us per call
 // (plain -> chunked, and the best of all lengths from 2 to 43): d = 256: B = 1: 1950 -> 126 (126), 4: 253 (253), 8: 449 (449),
-// 16: 993 -> 879 (879); d = 192: B = 1: 88 (87), 4: 152 (152); d = 160: B = 1: 79 (76), 8: 213 (196); d = 128: B = 1: 60,
-// 16: 350 -> 156, 48: 430 -> 570 (not taken).
+// 16: 993 -> 879 (879); d = 192: B = 1: 88 (87), 4: 152 (152); d = 160: B = 1: 79 (76), 8: 213 (196).  (Widths up to 128:
+// scan_narrow::chunks.)
 // Returns false when the plain chain is at least as good.  LBI_SCAN_CHUNK=0 forces the plain chain, n >= 2 chunks of n.
 inline bool plan_chunks(int B, int K, int nb, ScanPlan* plan) {
-    static const int forced = std::getenv("LBI_SCAN_CHUNK") ? std::atoi(std::getenv("LBI_SCAN_CHUNK")) : -1;
+    const int forced = scan_forced_chunk();
     if (forced == 0 || K < 12) return false;
     int L = 0;
     if (forced > 0) {
@@ -1280,9 +1178,7 @@ int launch_chunked(const void* mats, void* out, const void* g, void* cot, int B,
     auto phase_launch = [&](auto in, auto mode, const void* left) {
         using In = decltype(in);
         constexpr int MODE = decltype(mode)::value;
-        if constexpr (D > 128) return scan_planes::launch_mode<In, D, 32, false, MODE>(left, out, nullptr, nullptr, B, K, d, stream, plan);
-        else if (d != D) return launch_mfma_cot<In, D, 32, 32, false, MODE, true>(left, out, nullptr, nullptr, B, K, d, stream, plan);
-        else return launch_mfma_cot<In, D, 32, 32, false, MODE, false>(left, out, nullptr, nullptr, B, K, d, stream, plan);
+        return scan_planes::launch_mode<In, D, 32, false, MODE>(left, out, nullptr, nullptr, B, K, d, stream, plan);
     };
     using std::integral_constant;
     // Phase 2 in log depth (totals_in_log_depth): the levels alternate between the two slots of a chunk that phase 3
@@ -1375,11 +1271,12 @@ int launch_scan(const void* mats, void* out, const void* g, void* cot, int B, in
         return run(std::integral_constant<int, 256>{});
     }
     // Widths up to 128: fp32 matrix cores (a step is a chain of dependent instructions here, which the splitting of the planes only
-    // lengthens: B=64 K=128 d=32 / 64 / 96 / 128 take 1.5 / 1.3 / 1.15 / 1.05 times as long on planes).
+    // lengthens: B=64 K=128 d=32 / 64 / 96 / 128 took 1.5 / 1.3 / 1.15 / 1.05 times as long on planes as in 32 x 32 tiles).
+    constexpr int kDtype = std::is_same<Tin, float>::value ? LBI_F32 : std::is_same<Tin, _Float16>::value ? LBI_F16 : LBI_BF16;
+    if (scan_narrow::takes(B, d, kDtype)) return scan_narrow::scan(mats, kDtype, out, g, cot, B, K, d, stream);
     if (d > 16 && d <= 128) {
         auto run = [&](auto width, auto wide) {
             constexpr int D = decltype(width)::value, WIDE = decltype(wide)::value;
-            if (plan_chunks(B, K, (d + 31) / 32, &plan)) return launch_chunked<Tin, D>(mats, out, g, cot, B, K, d, plan, stream);
             // Column blocks of one batch element read the same matrices.  With few batch elements, narrow blocks give
             // the chip enough workgroups, and the blocks of an element run side by side and share the matrices in L2.
             // With many, they drift apart and fetch them again (measured 1.7x / 2.4x the input bytes at d = 64 / 128),
@@ -1401,7 +1298,7 @@ int launch_scan(const void* mats, void* out, const void* g, void* cot, int B, in
     if (d == 512) {
         // 16 column blocks of 32 per batch element, 8 waves of 64 rows.  The fused form would spill, so the
         // cotangent chain, if asked for, runs as its own kernel behind the matrices.
-        if (int rc = launch_mfma_cot<Tin, 512, 64, 32, false, 0, false>(mats, out, nullptr, nullptr, B, K, d, stream)) return rc;
+        if (int rc = launch_mfma_cot<Tin, 512, 64, 32, false, false>(mats, out, nullptr, nullptr, B, K, d, stream)) return rc;
         return cot ? launch_cotangent<Tin>(mats, g, cot, B, K, d, stream) : LBI_OK;
     }
     if (cot) {

@@ -1,0 +1,120 @@
+// Suffix scan of narrow matrices: which form a call takes, and its launches (kernel: lbi_scan_narrow_kernel.h).
+#include "lbi_scan_narrow.h"
+
+#include "lbi_scan_planes.h"
+
+namespace lbi {
+namespace scan_narrow {
+
+// One launch, a whole chain (plan.phase 0) or a phase of the plan, on blocks of 16 `tiles` columns (1 or 2); `carry`: the vector of a whole
+// chain beside the first block of 32.  An instance per storage type in a source of its own.
+template <typename Tin>
+int launch_type(const void* mats, void* out, const void* g, void* cot, int B, int K, int d, int tiles, bool carry,
+                const ScanPlan& plan, hipStream_t stream);
+extern template int launch_type<float>(const void*, void*, const void*, void*, int, int, int, int, bool, const ScanPlan&, hipStream_t);
+extern template int launch_type<_Float16>(const void*, void*, const void*, void*, int, int, int, int, bool, const ScanPlan&, hipStream_t);
+extern template int launch_type<bf16_raw>(const void*, void*, const void*, void*, int, int, int, int, bool, const ScanPlan&, hipStream_t);
+
+int launch(const void* mats, int in_dtype, void* out, const void* g, void* cot, int B, int K, int d, int tiles, bool carry,
+           const ScanPlan& plan, hipStream_t stream) {
+    switch (in_dtype) {
+        case LBI_F32: return launch_type<float>(mats, out, g, cot, B, K, d, tiles, carry, plan, stream);
+        case LBI_F16: return launch_type<_Float16>(mats, out, g, cot, B, K, d, tiles, carry, plan, stream);
+        default: return launch_type<bf16_raw>(mats, out, g, cot, B, K, d, tiles, carry, plan, stream);
+    }
+}
+
+// Compute units of the smallest partition of the part.
+constexpr int kLeastCus = 32;
+
+// us of a step on blocks of 16 `tiles` columns: of workgroups that have a CU to themselves, fp32 (K = 128, B = 1), and how much longer it takes
+// where `groups` workgroups share the chip: up to 48 columns several run on a CU side by side, at 64 two, beyond one (the rings), and what
+// they read then counts, too (d = 128 B = 16 K = 74, inputs from memory: 1.9).
+float step_us(int nt, int tiles, int64_t groups, int cus) {
+    static constexpr float alone[8] = {0.14f, 0.24f, 0.31f, 0.41f, 0.77f, 0.88f, 1.05f, 1.22f};
+    const float full = (float)groups / (float)cus, rounds = (float)((groups + cus - 1) / cus);
+    float share = 1.0f;
+    if (nt > 4) share = rounds * (1.0f + (nt > 6 ? 1.5f : 0.6f) * full / (rounds * (float)tiles));
+    else if (groups > cus) share = nt < 4 ? 1.0f + 0.5f * (full - 1.0f) : 1.8f * (float)((groups + 2 * cus - 1) / (2 * cus));
+    return alone[nt - 1] * share * (tiles == 2 ? 1.8f : 1.0f);
+}
+
+// Chains are dealt to the eight XCDs, so it is the fullest one that counts.
+int64_t dealt(int64_t chains) { return chains >= 8 ? (chains + 7) / 8 * 8 : chains; }
+
+// Chunks of L matrices (0: the plain chain), their phases 1 and 3 on blocks of 16 `tiles` columns.
+struct Chunks { int L, tiles; };
+
+// The form with the least estimated time: chunks are three launches instead of one and about twice the products, but 2 L + C - 4
+// dependent steps instead of K - 1; blocks of 32 columns, the vector beside the first, take 1.8 times as long for a step of half as
+// many workgroups.  Room is left for the vector whether it is asked for or not: the matrices are the same bits with and without.  K = 128, fp32,
+// matrices, us, plain -> chunks: d = 16 B = 1 18 -> 12; d = 32 B = 4 31 -> 17, B = 64 32 -> 32; d = 64 B = 4 52 -> 23, B = 32 54 (59 in
+// chunks, not taken); d = 128 B = 1 156 -> 49, B = 4 154 -> 61; B = 7 K = 120, inputs from memory,
+// in chunks 122 on 16 columns, 92 on 32.
+Chunks chunks(int B, int K, int nt, int cus) {
+    const int forced = scan_forced_chunk();
+    if (forced == 0 || K < 12) return {0, 1};
+    if (forced > 0) {
+        const int L = forced < 2 ? 2 : forced;
+        return {(K + L) / L >= 4 ? L : 0, 1};
+    }
+    float best = 5.0f + (float)(K - 1) * step_us(nt, 1, dealt(B) * nt, cus);
+    Chunks form{0, 1};
+    for (int L = 2; (K + L) / L >= 4; L += 1 + L / 16) {
+        const int C = (K + L) / L;
+        const int64_t chains = dealt((int64_t)B * (C - 1));
+        const float between = 12.0f + (float)(C - 2) * step_us(nt, 1, dealt(B) * nt, cus);
+        for (int tiles = 1; tiles <= (nt > 3 ? 2 : 1); ++tiles) {
+            const float step = step_us(nt, tiles, chains * (tiles == 2 ? (nt + 1) / 2 : nt + 1), cus);
+            const float cost = between + (float)(2 * L - 2) * step;
+            if (cost < best) {
+                best = cost;
+                form = {L, tiles};
+            }
+        }
+    }
+    return form;
+}
+
+bool takes(int B, int d, int in_dtype) {
+    if (d < 2 || d > 128) return false;
+    if (d <= 16 || scan_forced_chunk() > 0) return true;   // the others take whole chains of more than 16 columns
+    const int64_t blocks = (int64_t)B * ((d + 31) / 32);
+    if (2 * blocks <= kLeastCus) return true;              // on any device: small calls do without asking the runtime
+    // Where the chip has several workgroups for every CU to run one after the other, a step's length no longer counts, and 32 x 32
+    // tiles move half the operands.  fp32, matrices, us, those -> these: d = 128 B = 64 K = 128 430 -> 380, B = 128 K = 40 227 -> 238;
+    // d = 96 B = 128 K = 40 160 -> 157, B = 512 K = 20 233 -> 265; d = 64 B = 512 K = 64 349 -> 255, B = 1024 K = 32 231 -> 262; d = 32
+    // B = 1024 K = 64 126 -> 118, B = 4096 K = 32 234 -> 228 with 240 for 232 with the cotangents.
+    const int64_t cus = device_compute_units();
+    if (d > 96) return 4 * blocks <= (in_dtype != LBI_F32 && d != 128 ? 3 : 5) * cus;
+    return blocks <= (d > 64 ? 4 : d > 32 ? 6 : 12) * cus;
+}
+
+int scan(const void* mats, int in_dtype, void* out, const void* g, void* cot, int B, int K, int d, hipStream_t stream) {
+    ScanPlan plan{0, 0, 0, 0, 0, 0, 0};
+    const int nt = row_tiles(d, in_dtype);
+    if (K < 12 && dealt(B) * (nt + 1) <= kLeastCus) return launch(mats, in_dtype, out, g, cot, B, K, d, 1, false, plan, stream);
+    const int cus = device_compute_units();
+    if (const Chunks form = chunks(B, K, nt, cus); form.L) {
+        plan.L = form.L;
+        plan.C = (K + form.L) / form.L;
+        plan.s = 1;
+        for (plan.phase = 1; plan.phase <= 3; ++plan.phase) {
+            const bool totals = plan.phase == 2;   // operands and results are fp32 products inside `out`
+            if (int rc = launch(totals ? out : mats, totals ? LBI_F32 : in_dtype, out, g, totals ? nullptr : cot, B, K, d,
+                                totals ? 1 : form.tiles, form.tiles == 2 && !totals, plan, stream))
+                return rc;
+        }
+        return LBI_OK;
+    }
+    // 16 columns a workgroup while every workgroup finds room at once, 32 beyond (a step of those takes 1.5-1.9 times as long); the vector
+    // in a workgroup of its own while that does.  fp32 K = 128 with cotangents, us, 16 / 32 / 32 with the vector beside: d = 64 B = 32
+    // 54 / 90 / -, B = 64 131 / 99 / 126; d = 128 B = 32 402 / 303 / 325, B = 64 709 / 610 / 377.
+    const int64_t room = nt <= 3 ? 8 * cus / nt : cus, more = cot ? 1 : 0;
+    const int tiles = nt > 1 && dealt(B) * (nt + more) > room ? 2 : 1;
+    const bool carry = tiles == 2 && cot && dealt(B) * ((nt + 1) / 2 + 1) > room;
+    return launch(mats, in_dtype, out, g, cot, B, K, d, tiles, carry, plan, stream);
+}
+
+}  // namespace scan_narrow
+}  // namespace lbi

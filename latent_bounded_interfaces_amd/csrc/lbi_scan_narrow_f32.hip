@@ -1,0 +1,5 @@
+// Narrow scans of fp32 matrices.
+#include "lbi_scan_narrow_kernel.h"
+
+template int lbi::scan_narrow::launch_type<float>(const void*, void*, const void*, void*, int, int, int, int, bool, const ScanPlan&,
+                                               hipStream_t);

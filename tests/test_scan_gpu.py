@@ -734,3 +734,44 @@ def test_bf16_storage_at_the_benchmark_shape_in_both_precisions(kind, device):
         cscale = want.abs().amax(dim=2, keepdim=True).clamp_min(1e-300)
         assert float(((cot.double() - want).abs() / cscale).max()) <= 1e-5
         del only, fused, cot
+
+
+# Widths up to 128 in 16 x 16 tiles: each number of row tiles with its last tile full, one short and one over, and the forms a batch
+# takes: one block of 16 columns a workgroup, blocks of 32 with the vector in a workgroup of its own and beside the first block,
+# chunks on either, one matrix.  Each product sums d terms in blocks of 32 (K of them one after the other): K (d / 32 + 32) roundings
+# of 2^-24 against the sizes of a near-identity chain bound the error; 1e-5 is less for every case here.
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rank", [2, 15, 17, 31, 48, 49, 63, 64, 66, 80, 81, 96, 111, 112, 113, 128])
+@pytest.mark.parametrize("bsz,count", [(1, 1), (3, 9), (2, 40), (13, 60), (44, 5), (70, 4)])
+def test_narrow_scan_forms(rank, bsz, count, dtype, device):
+    from latent_bounded_interfaces_amd.hip.interface import suffix_scan_pullbacks, suffix_scan_pullbacks_and_cotangents
+
+    mats, g = oscan.make_scan_inputs(bsz, count, rank, kind="near_identity", seed=rank + count)
+    mats = mats.to(dtype).to(device)
+    g = g.to(device)
+    out, cot = suffix_scan_pullbacks_and_cotangents(mats, g)
+    assert torch.equal(out, suffix_scan_pullbacks(mats))
+    truth, want = torch.eye(rank, device=device, dtype=torch.float64).expand(bsz, rank, rank), g.double()
+    assert torch.equal(out[:, count], torch.eye(rank, device=device).expand(bsz, rank, rank)) and torch.equal(cot[:, count], g)
+    for r in range(count - 1, -1, -1):
+        left = mats[:, r].double()
+        truth, want = left @ truth, (left @ want.unsqueeze(-1)).squeeze(-1)
+        assert float((out[:, r].double() - truth).abs().max() / truth.abs().max()) <= 1e-5
+        assert float((cot[:, r].double() - want).abs().max() / want.abs().max()) <= 1e-5
+
+
+@pytest.mark.parametrize("rank", [16, 30, 64, 77, 128])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_narrow_scan_keeps_other_rows_and_elements_apart(rank, value, device):
+    """What is not finite stays where plain products put it: nothing leaks through the padding of a row's last tile."""
+    from latent_bounded_interfaces_amd.hip.interface import suffix_scan_pullbacks_and_cotangents
+
+    for bsz in (2, 70):
+        mats, g = oscan.make_scan_inputs(bsz, 3, rank, kind="randn", seed=3)
+        mats[0, 1, 0, rank - 1] = value
+        out, cot = suffix_scan_pullbacks_and_cotangents(mats.to(device), g.to(device))
+        truth = oscan.suffix_scan_sequential(mats, dtype=torch.float64)
+        want = oscan.suffix_cotangents_sequential(mats.double(), g.double())
+        assert torch.equal(torch.isfinite(out.cpu()), torch.isfinite(truth))
+        assert torch.equal(torch.isfinite(cot.cpu()), torch.isfinite(want))
+        assert torch.isfinite(out[1:]).all() and torch.isfinite(cot[1:]).all()
