@@ -4,7 +4,7 @@
 //
 // Three kernels per call, all atomic-free (every output tile has one owner, sums run
 // in a fixed order, so reruns are bit-identical):
-//   stats_kernel  flash-style forward: lse2[b,h,i] (log2 domain) and O = softmax(..) V (fp32)
+//   stats_kernel, stats_split_kernel  flash-style forward: lse2[b,h,i] (log2 domain) and O = softmax(..) V (fp32)
 //   dq_ring_kernel    owner = 32 queries per wave, PB directions at once; streams K/V tiles
 //                     (lbi_attn_dq128.h); it also forms -delta[b,p,h,i] = -sum_d d_out[b,p,h,i,d] * O[b,h,i,d]
 //                     from the d_out tiles it holds anyway and leaves it in the workspace
@@ -25,6 +25,8 @@
 // 16kk + {4h..4h+3, 8+4h..8+4h+3}; the tr fragment of the other operand is read with the
 // same row assignment, so no data passes through LDS between the two products.
 #pragma once
+
+#include <type_traits>
 
 #include "lbi_common.h"
 
@@ -365,6 +367,147 @@ __global__ __launch_bounds__(256) void stats_kernel(const T* __restrict__ q, con
     }
 }
 
+// ---------------------------------------------------------------------------------------
+// stats_split_kernel: the same with an eighth of the dependent steps.  A chain of key tiles is bound by the latency of a step (loads,
+// softmax, barrier), so a workgroup has 32 queries and its four waves take every fourth key tile each, on tiles of their
+// own in LDS (no barrier between tiles); their maxima, sums and outputs are brought together at the end, in the order of the
+// waves.  K and V are read four times as often as by workgroups of 128 queries: head dim 128 comes here while those leave
+// CUs without work, head dim 64 always.  (The choice depends on B, H, T and Dh, not on the directions: their results don't depend on
+// how they are grouped.)  bf16 causal, whole calls of one direction, us, 128 queries -> 32: Dh=64 T=1024 B H=16 / 64 / 96 88 -> 69, 108 ->
+// 97, 163 -> 152; T=4096 B H=64 913 -> 896; Dh=128 T=1024 B H=16 / 24 / 64 120 -> 102, 123 -> 116, 156 -> 171.
+// ---------------------------------------------------------------------------------------
+template <typename T, int DH, bool CAUSAL, bool EDGE>
+__global__ __launch_bounds__(256) void stats_split_kernel(const T* __restrict__ q, const T* __restrict__ k,
+                                                          const T* __restrict__ v, float* __restrict__ lse2,
+                                                          float* __restrict__ o32, int n_bh, int T_len, float scale,
+                                                          int t_rows, int dh) {
+    constexpr int KS = DH / 16, ND = DH / 32, TILE_BYTES = 32 * DH * 2, CPR = DH / 8, N = 32 * CPR / 64;
+    extern __shared__ __align__(16) char smem[];  // [4 waves][K tile, V tile]; at the end [4][32][DH] floats; then [2][4][32]
+    int bh, qt;
+    const int n_qt = T_len / 32;
+    if (!map_block(n_qt, n_bh, bh, qt)) return;
+    qt = n_qt - 1 - qt;  // longest rows first
+    const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, h = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int i0 = qt * 32;
+    const Extent<DH, EDGE> ext(T_len, t_rows, dh);
+    const size_t base = (size_t)bh * ext.t_rows * ext.dh;
+    const T* k_bh = k + base;
+    const T* v_bh = v + base;
+    char* kt = smem + wave * 2 * TILE_BYTES;
+    char* vt = kt + TILE_BYTES;
+    float* row_max = reinterpret_cast<float*>(smem + 8 * TILE_BYTES);
+    float* row_sum = row_max + 4 * 32;
+
+    const int n_it = CAUSAL ? qt + 1 : T_len / 32;
+    u32x4 kr[N], vr[N];
+    auto fetch = [&](int it) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            const int id = lane + 64 * u, r = 32 * it + id / CPR, c = id % CPR * 8;
+            kr[u] = ext.load(k_bh, r, c);
+            vr[u] = ext.load(v_bh, r, c);
+        }
+    };
+    if (wave < n_it) fetch(wave);
+    u32x4 qf[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) qf[ks] = ext.load(q + base, i0 + m, 16 * ks + 8 * h);
+    f32x16 o_t[ND];
+#pragma unroll
+    for (int nd = 0; nd < ND; ++nd) o_t[nd] = zero16();
+    float m_run = -INFINITY, l_run = 0.0f;
+    const float sc2 = scale * LOG2E;
+    for (int it = wave; it < n_it; it += 4) {
+        const int j0 = it * 32;
+#pragma unroll
+        for (int u = 0; u < N; ++u) {
+            const int id = lane + 64 * u, r = id / CPR, c = id % CPR;
+            *reinterpret_cast<u32x4*>(kt + tile_off<DH>(r, c)) = kr[u];
+            *reinterpret_cast<u32x4*>(vt + tile_off<DH>(r, c)) = vr[u];
+        }
+        fetch(it + 4 < n_it ? it + 4 : it);  // the last trip re-reads its tile
+        f32x16 s = zero16();
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) s = Mma<T>::mma(frag_nat<DH>(kt, m, h, ks), qf[ks], s);
+        const bool diag = CAUSAL && it == qt;
+        float tmax = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            float x = s[r] * sc2;
+            if (diag && c_row(r, h) > m) x = -INFINITY;
+            s[r] = x;
+            tmax = fmaxf(tmax, x);
+        }
+        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+        // (the reference point of the exponentials as in stats_kernel)
+        const float m_new = fmaxf(m_run, tmax);
+        const bool grow = (m_run == -INFINITY) ? (m_new != -INFINITY) : (m_new - m_run > 8.0f);
+        const float m_use = grow ? m_new : m_run;
+        float lsum = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float pr = (m_use == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(s[r] - m_use);
+            s[r] = pr;
+            lsum += pr;
+        }
+        lsum += __shfl_xor(lsum, 32, 64);
+        if (__builtin_amdgcn_ballot_w64(grow) != 0) {  // wave-uniform
+            const float alpha = (m_run == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_use);
+            l_run *= alpha;
+#pragma unroll
+            for (int nd = 0; nd < ND; ++nd)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o_t[nd][r] *= alpha;
+        }
+        l_run += lsum;
+        m_run = m_use;
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            const u32x4 pb = pack_frag<T>(s, kk);
+#pragma unroll
+            for (int nd = 0; nd < ND; ++nd)
+                o_t[nd] = Mma<T>::mma(frag_tr<DH>(vt, lane, 16 * kk, 32 * nd), pb, o_t[nd]);
+        }
+    }
+    if (h == 0) {
+        row_max[wave * 32 + m] = m_run;
+        row_sum[wave * 32 + m] = l_run;
+    }
+    __syncthreads();  // and nobody reads a tile any more
+    float top = -INFINITY, total = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 4; ++w) top = fmaxf(top, row_max[w * 32 + m]);
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+        const float mw = row_max[w * 32 + m];
+        total += mw == -INFINITY ? 0.0f * row_sum[w * 32 + m] : row_sum[w * 32 + m] * __builtin_amdgcn_exp2f(mw - top);
+    }
+    const float part = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - top);
+    const float inv = part / total;
+    if (wave == 0 && h == 0) lse2[(size_t)bh * T_len + i0 + m] = top + log2f(total);
+    // [wave][32][DH] floats, 16-byte pieces XOR-swizzled by the row (writes: 32 rows of a piece column)
+    float* mine = reinterpret_cast<float*>(smem) + wave * 32 * DH;
+#pragma unroll
+    for (int nd = 0; nd < ND; ++nd)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const int piece = (32 * nd + 8 * g + 4 * h) / 4;
+            *reinterpret_cast<f32x4*>(mine + m * DH + 4 * (piece ^ (m & 15))) =
+                f32x4{o_t[nd][4 * g] * inv, o_t[nd][4 * g + 1] * inv, o_t[nd][4 * g + 2] * inv, o_t[nd][4 * g + 3] * inv};
+        }
+    __syncthreads();
+    float* o_rows = o32 + ((size_t)bh * T_len + i0) * DH;
+    for (int id = tid; id < 32 * DH / 4; id += 256) {
+        const int r = id / (DH / 4), piece = id % (DH / 4);
+        const float* at = reinterpret_cast<const float*>(smem) + r * DH + 4 * (piece ^ (r & 15));
+        f32x4 sum = *reinterpret_cast<const f32x4*>(at);
+#pragma unroll
+        for (int w = 1; w < 4; ++w) sum += *reinterpret_cast<const f32x4*>(at + w * 32 * DH);
+        *reinterpret_cast<f32x4*>(o_rows + (size_t)r * DH + 4 * piece) = sum;
+    }
+}
+
 inline bool supports(int T_len, int dh, int dtype) {
     return (dtype == LBI_F16 || dtype == LBI_BF16) && (dh == 64 || dh == 128) && T_len >= 64 && T_len % 64 == 0;
 }
@@ -392,25 +535,58 @@ int launch_dq(const T* q, const T* k, const T* v, const T* g, const float* lse2,
                int n_bh, int H, int P, int T_len, float scale, int t_rows, int dh,
                 hipStream_t stream);
 
+// Directions per wave of the dQ kernel, `blocks` 128-query blocks for each.  More of them share an S tile, fewer are shorter steps for
+// more workgroups: one direction while that leaves CUs free, two until the largest number fills the chip several times over without
+// idle slots.  The results are the same bits.  bf16 causal calls, us, 1 / 2 / 4 / 8 directions: Dh=64 T=1024, B H = 6, P = 6 104 / 109 /
+// 121 / 148; 24, 9 196 / 189 / 208 / 226; 64, 16 641 / 580 / 591 / 585; T=2048, 64, 16 2048 / 1839 / 1859 / 1793; Dh=128 T=1024, 6, 4
+// 117 / 125 / 147; 24, 6 221 / 219 / 232; 64, 16 1229 / 1172 / 1088.
+inline int dq_directions(int dh, int64_t blocks, int P, int64_t cus) {
+    if (P == 1) return 1;
+    if (dh == 64) {
+        if (5 * blocks * P <= 6 * cus) return 1;
+        return P % 8 == 0 || P % 8 == 7 ? (blocks * ((P + 7) / 8) > 6 * cus ? 8 : 2) : 2;
+    }
+    if (4 * blocks * P <= 3 * cus) return 1;
+    return P % 4 == 0 || P % 4 == 3 ? (4 * blocks * ((P + 3) / 4) >= 3 * cus ? 4 : 2) : 2;
+}
+
 // T_len: the length in tiles (a multiple of 64); t_rows, dh: rows and head dim of the tensors (EDGE).
 template <typename T, int DH, bool CAUSAL, bool EDGE = false>
 int launch_typed(const T* q, const T* k, const T* v, const T* g, T* dq, T* dk, T* dv, float* workspace, int B,
                  int H, int T_len, int P, float scale, int t_rows, int dh, hipStream_t stream) {
-    constexpr size_t lds_bytes = 4 * 32 * DH * 2;
+    [[maybe_unused]] constexpr size_t lds_bytes = 4 * 32 * DH * 2;
     const int n_bh = B * H;
     float* lse2 = workspace;
     float* delta = lse2 + (size_t)n_bh * T_len;
     float* o32 = delta + (size_t)n_bh * P * T_len;
     const int n_qb = (T_len + 127) / 128;
-    hipLaunchKernelGGL((stats_kernel<T, DH, CAUSAL, EDGE>), dim3(grid_size(n_qb, n_bh)), dim3(256), lds_bytes, stream, q, k,
-                       v, lse2, o32, n_bh, T_len, scale, t_rows, dh);
+    const int64_t cus = device_compute_units(), blocks = (int64_t)n_qb * n_bh;
+    auto split_stats = [&]() -> int {
+        constexpr size_t bytes = 8 * 32 * DH * 2 + 2 * 4 * 32 * 4;
+        if (int rc = ensure_dynamic_lds<&stats_split_kernel<T, DH, CAUSAL, EDGE>>(bytes)) return rc;
+        hipLaunchKernelGGL((stats_split_kernel<T, DH, CAUSAL, EDGE>), dim3(grid_size(T_len / 32, n_bh)), dim3(256), bytes, stream, q, k,
+                           v, lse2, o32, n_bh, T_len, scale, t_rows, dh);
+        return LBI_OK;
+    };
+    if constexpr (DH == 64) {
+        if (int rc = split_stats()) return rc;
+    } else if (4 * blocks <= 3 * cus) {
+        if (int rc = split_stats()) return rc;
+    } else {
+        hipLaunchKernelGGL((stats_kernel<T, DH, CAUSAL, EDGE>), dim3(grid_size(n_qb, n_bh)), dim3(256), lds_bytes, stream, q, k,
+                           v, lse2, o32, n_bh, T_len, scale, t_rows, dh);
+    }
     // the dQ kernel runs first: it writes -delta, which the dK/dV kernel reads
-    // directions per wave of the dQ kernel: as many as share one S tile, without idle slots for one or two directions
     int rc;
-    if (P == 1) rc = launch_dq<T, DH, 1, CAUSAL, EDGE>(q, k, v, g, lse2, o32, delta, dq, n_bh, H, P, T_len, scale, t_rows, dh, stream);
-    else if (P == 2) rc = launch_dq<T, DH, 2, CAUSAL, EDGE>(q, k, v, g, lse2, o32, delta, dq, n_bh, H, P, T_len, scale, t_rows, dh, stream);
-    else if (DH == 64 && P > 4) rc = launch_dq<T, DH, 8, CAUSAL, EDGE>(q, k, v, g, lse2, o32, delta, dq, n_bh, H, P, T_len, scale, t_rows, dh, stream);
-    else rc = launch_dq<T, DH, 4, CAUSAL, EDGE>(q, k, v, g, lse2, o32, delta, dq, n_bh, H, P, T_len, scale, t_rows, dh, stream);
+    auto dq_as = [&](auto pb) {
+        return launch_dq<T, DH, decltype(pb)::value, CAUSAL, EDGE>(q, k, v, g, lse2, o32, delta, dq, n_bh, H, P, T_len, scale, t_rows,
+                                                                   dh, stream);
+    };
+    switch (dq_directions(DH, blocks, P, cus)) {
+        case 1: rc = dq_as(std::integral_constant<int, 1>{}); break;
+        case 2: rc = dq_as(std::integral_constant<int, 2>{}); break;
+        default: rc = dq_as(std::integral_constant<int, DH == 64 ? 8 : 4>{}); break;
+    }
     if (rc) return rc;
     if (P >= 2) rc = launch_dkdv_pair<T, DH, CAUSAL, EDGE>(q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, t_rows, dh, stream);
     else rc = launch_dkdv<T, DH, CAUSAL, EDGE>(q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, t_rows, dh, stream);

@@ -416,3 +416,27 @@ def test_long_context_full_size_slices_match_oracle(device):
         for name, a, c in zip(("dq", "dk", "dv"), out, want):
             got = a[b:b + 1, list(dirs), h:h + 1].float().cpu()
             assert _max_rel(got, c) <= 2e-2, (name, b, h, _max_rel(got, c))
+
+
+# Calls that leave CUs without work and calls that don't, either side of the lines between the numbers of directions per workgroup and
+# between the two statistics kernels (head dim 128: 3/4 of the CUs), chains of 1 ... 5 key tiles per wave.
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape,basis", [((1, 2, 320, 64), 3), ((1, 40, 320, 64), 5), ((2, 3, 576, 64), 7), ((1, 3, 192, 128), 2),
+                                         ((1, 1, 448, 128), 9), ((1, 70, 320, 128), 3), ((1, 64, 384, 128), 1), ((1, 65, 384, 128), 4)])
+def test_directions_and_statistics_by_size(shape, basis, dtype, causal, device):
+    from latent_bounded_interfaces_amd.hip.transformer import attention_input_pullback_basis
+
+    inputs = oattn.make_attention_inputs(*shape, basis, dtype=dtype, seed=basis)
+    q, k, v, d_out = (t.to(device) for t in inputs)
+    scale = 1.0 / math.sqrt(shape[-1])
+    got = attention_input_pullback_basis(q, k, v, d_out, softmax_scale=scale, causal=causal, kernel_mode="hip")
+    want = oattn.attention_pullback_dense(*inputs, softmax_scale=scale, causal=causal, dtype=torch.float32)
+    # operands of the second products and results are rounded to the storage type: a few of its units against the largest value
+    bar = 4e-3 if dtype == torch.float16 else 3e-2
+    for name, a, b in zip(("dq", "dk", "dv"), got, want):
+        diff = a.float().cpu() - b
+        assert float(diff.norm() / b.norm()) <= bar / 2, name
+        assert float(diff.abs().max() / b.abs().max()) <= bar, name
+    one = attention_input_pullback_basis(q, k, v, d_out[:, basis - 1:].contiguous(), softmax_scale=scale, causal=causal, kernel_mode="hip")
+    assert all(torch.equal(a[:, basis - 1:], b) for a, b in zip(got, one))
