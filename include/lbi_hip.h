@@ -343,6 +343,35 @@ int lbi_causal_conv1d_weight_grad(const void* g_out, const void* x, float* grads
                                   int64_t B, int64_t T, int64_t C, int64_t ksize, int dtype, void* stream);
 
 /*
+ * One Transformer block, backwards, whose products are all small (lbi_small_product): the entries above one after the other, with the
+ * same results, as one call.  Tensors as there, all 16-byte aligned; 16-bit storage, filters of up to 8 taps, no biases.
+ *
+ *   g_residual [B,P,T,D] fp32 (g_broadcast_t: [B,P,D], the same at every position): cotangent of the block's residual output; read only
+ *   g_hidden   the cotangent of its hidden output in `dtype`, or NULL: g_residual rounded
+ *   g_input    [B,P,T,D] fp32: cotangent of the block's input;  g_input_branch: the same in `dtype`, or NULL
+ *   attn_edge  the attention is lbi_attn_pullback_edge instead of lbi_attn_pullback (causal either way)
+ * With grad_fc2 (one dense direction, P = 1) the parameter gradients, too, all in `dtype` and shaped as the parameters, from the
+ * modules' inputs down_input [B,T,hidden], norm2_output, out_input [B,T,H*Dh] and norm1_output.
+ */
+typedef struct lbi_region_layer {
+    int64_t B, P, T, D, hidden, H, Hkv, Dh, ksize;
+    int dtype, norm1_dtype, norm2_dtype;
+    int g_broadcast_t, rope_interleaved, attn_edge;
+    float norm1_eps, norm2_eps, softmax_scale;
+    const void *g_hidden, *g_residual;
+    const void *fc2_weight, *fc1_weight, *out_weight, *in_weight, *norm2_weight, *norm1_weight, *conv_weight;
+    const void *fc1_output, *norm2_input, *norm1_input, *q, *k, *v;
+    const float *rope_cos, *rope_sin;
+    void *g_input, *g_input_branch;
+    const void *down_input, *norm2_output, *out_input, *norm1_output;
+    void *grad_fc2, *grad_fc1, *grad_out, *grad_in, *grad_norm2, *grad_norm1, *grad_conv;
+} lbi_region_layer;
+
+/* 0 for a description that lbi_region_layer_pullback refuses. */
+size_t lbi_region_layer_workspace_bytes(const lbi_region_layer* layer);
+int lbi_region_layer_pullback(const lbi_region_layer* layer, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Frobenius and spectral (largest singular value) norms of N square matrices, the per-step Jacobian
  * diagnostics of the interface scan (reference backward/suffix_scan.py:105-134, which calls
  * torch.linalg.matrix_norm with ord="fro" and ord=2, a singular value decomposition per matrix).

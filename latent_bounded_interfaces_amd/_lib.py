@@ -16,13 +16,30 @@ LIB_PATH = Path(__file__).resolve().parent / "liblbi_hip.so"
 
 LBI_F32, LBI_F16, LBI_BF16 = 0, 1, 2
 ATTN_STATIC_SCRATCH_BYTES = 32 << 20  # LBI_ATTN_STATIC_SCRATCH_BYTES of include/lbi_hip.h
-ABI_VERSION = 10
+ABI_VERSION = 11
 LBI_SCAN_EXACT_SUFFIX = 1  # lbi_scan_flags of include/lbi_hip.h
 
 _DTYPE_CODES = {torch.float32: LBI_F32, torch.float16: LBI_F16, torch.bfloat16: LBI_BF16}
 
-# name -> (restype, argtypes); must list every symbol of include/lbi_hip.h.
 _c = ctypes
+
+
+class RegionLayer(_c.Structure):
+    """``lbi_region_layer`` of include/lbi_hip.h."""
+
+    _fields_ = (
+        [(name, _c.c_int64) for name in ("B", "P", "T", "D", "hidden", "H", "Hkv", "Dh", "ksize")]
+        + [(name, _c.c_int) for name in ("dtype", "norm1_dtype", "norm2_dtype", "g_broadcast_t", "rope_interleaved", "attn_edge")]
+        + [(name, _c.c_float) for name in ("norm1_eps", "norm2_eps", "softmax_scale")]
+        + [(name, _c.c_void_p) for name in (
+            "g_hidden", "g_residual", "fc2_weight", "fc1_weight", "out_weight", "in_weight", "norm2_weight", "norm1_weight",
+            "conv_weight", "fc1_output", "norm2_input", "norm1_input", "q", "k", "v", "rope_cos", "rope_sin", "g_input",
+            "g_input_branch", "down_input", "norm2_output", "out_input", "norm1_output", "grad_fc2", "grad_fc1", "grad_out",
+            "grad_in", "grad_norm2", "grad_norm1", "grad_conv")]
+    )
+
+
+# name -> (restype, argtypes); must list every symbol of include/lbi_hip.h.
 SYMBOLS = {
     "lbi_abi_version": (_c.c_int, []),
     "lbi_last_error": (_c.c_char_p, []),
@@ -86,6 +103,8 @@ SYMBOLS = {
         _c.c_int,
         [_c.c_void_p] * 7 + [_c.c_int64] * 6 + [_c.c_int, _c.c_int64, _c.c_int, _c.c_void_p],
     ),
+    "lbi_region_layer_workspace_bytes": (_c.c_size_t, [_c.POINTER(RegionLayer)]),
+    "lbi_region_layer_pullback": (_c.c_int, [_c.POINTER(RegionLayer), _c.c_void_p, _c.c_size_t, _c.c_void_p]),
     "lbi_matrix_norms_workspace_bytes": (_c.c_size_t, [_c.c_int64, _c.c_int64]),
     "lbi_matrix_norms": (
         _c.c_int,

@@ -19,13 +19,14 @@ inside the attention kernel.  GPU only.
 """
 from __future__ import annotations
 
+import ctypes
 import math
 from typing import Any
 
 import torch
 
 from ... import _lib
-from . import attention_input_pullback_basis
+from . import _MFMA_HEAD_DIMS, _MFMA_SEQ_MULTIPLE, _SINGLE_LAUNCH_MAX_SEQ, attention_input_pullback_basis
 
 
 def _stream(t: torch.Tensor) -> int:
@@ -282,9 +283,9 @@ _ROWS_BY_WEIGHT, _GRADIENT, _FORWARD = 0, 1, 2
 _SMALL_PRODUCT_TYPES = (torch.float16, torch.bfloat16)
 
 
-def _small_product_size(height: int, width: int, inner: int, form: int) -> bool:
+def _small_product_size(height: int, width: int, inner: int, form: int, times: int = 1) -> bool:
     long_sums = form == _GRADIENT and min(height, width) >= 64
-    return (0 < height * width * inner <= _SMALL_PRODUCT and height * width <= _SMALL_PRODUCT_RESULTS
+    return (0 < height * width * inner <= times * _SMALL_PRODUCT and height * width <= times * _SMALL_PRODUCT_RESULTS
             and inner <= (_SMALL_GRADIENT_TERMS if long_sums else _SMALL_PRODUCT_TERMS)
             and width % 8 == 0 and (height if form == _GRADIENT else inner) % 8 == 0
             # what the kernel's 32-bit offsets span, its tiles and the chunks asked for ahead included
@@ -412,11 +413,110 @@ def _conv_grads(sink: dict, conv: Any, g_out: torch.Tensor, x_pre: torch.Tensor)
         sink[id(conv.bias)] = g.sum(dim=(0, 1)).to(conv.bias.dtype)
 
 
+#: How many times a small product's multiply-adds and results one of a native layer may have: the library is up to twice as fast on those
+#: last ones, and the layer still the faster for the host time that it doesn't wait for.  Whole calls, us, launch by launch / native
+#: up to 1, 2, 3, 5 times: parameter VJP d_model 768, 2 layers, B=1 T=258 577 / 619, 355, 356, 354; d_model 512, 1 layer, B=2 T=1024
+#: 321 / 325, 325, 289, 289; region pullback d_model 512, 1 layer, B=2 T=65 P=9 129 / 130, 80, 79, 79; d_model 256, 2 layers, B=5 T=128
+#: P=24 281 / 292, 292, 281, 329; d_model 256, 2 layers, B=1 T=128 P=16 185 / 115 and the same on.
+_NATIVE_TIMES = 3
+
+
+def _lie_ready(dtype: torch.dtype, device: torch.device, tensors: tuple) -> bool:
+    """Whether the native layer can take these tensors as they lie."""
+    for t in tensors:
+        if t.dtype is not dtype or t.data_ptr() & 15 or not t.is_contiguous() or t.device != device:
+            return False
+    return True
+
+
+def _native_layer(block: Any, layer_cache: Any, g_hidden: torch.Tensor | None, g_residual: torch.Tensor, want_branch: bool,
+                  param_grads: dict | None) -> tuple[torch.Tensor, torch.Tensor | None] | None:
+    """:func:`_layer_input_pullback` as one native call (``lbi_region_layer_pullback``: the same launches without the host time
+    between them), for 16-bit blocks whose products are all small ones; ``None`` for others.  Nothing is updated in place."""
+    attn, mlp = block.attn, block.mlp
+    a_cache, m_cache = layer_cache.attention, layer_cache.mlp
+    q = a_cache.q_rope
+    dtype, device = q.dtype, q.device
+    if dtype not in _SMALL_PRODUCT_TYPES or attn.d_conv <= 0 or q.dim() != 4:
+        return None
+    bsz, basis, g_len, dim = g_residual.shape
+    heads, kv_heads, head_dim = attn.n_heads, attn.n_kv_heads, attn.head_dim
+    seqlen = q.shape[2]
+    fc1_output, conv = m_cache.fc1_output, attn.conv1d.weight
+    hidden, q_width, packed = fc1_output.shape[-1] // 2, heads * head_dim, (heads + 2 * kv_heads) * head_dim
+    rows = bsz * basis * seqlen
+    # the products, and the attention that runs without copies (the rule of attention_input_pullback_basis)
+    g_rows = rows if g_len == seqlen else bsz * basis
+    if not (_small_product_size(rows, dim, 2 * hidden, _ROWS_BY_WEIGHT, _NATIVE_TIMES) and _small_product_size(g_rows, hidden, dim, _ROWS_BY_WEIGHT, _NATIVE_TIMES)
+            and _small_product_size(rows, q_width, dim, _ROWS_BY_WEIGHT, _NATIVE_TIMES) and _small_product_size(rows, dim, packed, _ROWS_BY_WEIGHT, _NATIVE_TIMES)):
+        return None
+    wide_dim = next((w for w in _MFMA_HEAD_DIMS if w >= head_dim), 0)
+    single_launch = seqlen <= _SINGLE_LAUNCH_MAX_SEQ.get(wide_dim, 0)
+    if wide_dim == 0 or head_dim % 8 or heads % kv_heads or not (single_launch or seqlen > _MFMA_SEQ_MULTIPLE // 2):
+        return None
+    attn_edge = wide_dim != head_dim or not (single_launch or seqlen % _MFMA_SEQ_MULTIPLE == 0)
+    fc1, fc2, out_proj, in_proj, norm1, norm2 = (mlp.fc1.weight, mlp.fc2.weight, attn.out_proj.weight, attn.in_proj.weight,
+                                                 block.norm.weight, block.norm2.weight)
+    x1, x2, q, k, v = (t.contiguous() for t in (a_cache.norm_input, m_cache.norm_input, q, a_cache.k_expanded, a_cache.v_expanded))
+    taps = conv.shape[-1]
+    positions, matrix = (bsz, seqlen, dim), (bsz, heads, seqlen, head_dim)
+    if not (taps <= FUSED_CONV_MAX_TAPS and conv.shape == (packed, 1, taps) and fc1_output.shape == (bsz, seqlen, 2 * hidden)
+            and q.shape == matrix and k.shape == matrix and v.shape == matrix
+            and x1.shape == positions and x2.shape == positions and norm1.shape == (dim,) and norm2.shape == (dim,)
+            and fc1.shape == (2 * hidden, dim) and fc2.shape == (dim, hidden) and out_proj.shape == (dim, q_width)
+            and in_proj.shape == (packed, dim) and (g_len == seqlen or g_len == 1)
+            and g_residual.device == device
+            and _lie_ready(dtype, device, (fc1_output, q, k, v, fc1, fc2, out_proj, in_proj, norm1,
+                                           norm2, conv))
+            and (g_hidden is None or _lie_ready(dtype, device, (g_hidden,)))
+            and x1.dtype in (dtype, torch.float32) and _lie_ready(x1.dtype, device, (x1,))
+            and x2.dtype in (dtype, torch.float32) and _lie_ready(x2.dtype, device, (x2,))
+            and g_residual.dtype is torch.float32 and g_residual.is_contiguous() and g_residual.data_ptr() & 15 == 0):
+        return None
+    inputs: tuple = ()
+    if param_grads is not None:
+        inputs = (m_cache.down_input, m_cache.norm_output, a_cache.out_proj_input, a_cache.norm_output)
+        if not (basis == 1 and g_len == seqlen and dim % 4 == 0 and dim <= NORM_GRAD_MAX_WIDTH
+                and all(getattr(linear, "bias", None) is None for linear in (mlp.fc1, mlp.fc2, attn.out_proj, attn.in_proj, attn.conv1d))
+                and inputs[0].shape == (bsz, seqlen, hidden) and inputs[1].shape == positions
+                and inputs[2].shape == (bsz, seqlen, q_width) and inputs[3].shape == positions
+                and _lie_ready(dtype, device, inputs)
+                and _small_product_size(dim, hidden, rows, _GRADIENT, _NATIVE_TIMES) and _small_product_size(2 * hidden, dim, rows, _GRADIENT, _NATIVE_TIMES)
+                and _small_product_size(dim, q_width, rows, _GRADIENT, _NATIVE_TIMES) and _small_product_size(packed, dim, rows, _GRADIENT, _NATIVE_TIMES)
+                and _small_product_size(rows, packed, dim, _FORWARD, _NATIVE_TIMES)):
+            return None
+    scale = attn.softmax_scale if attn.softmax_scale is not None else 1.0 / math.sqrt(head_dim)
+    cos, sin = rope_tables(seqlen, head_dim, attn.rope_base, device)
+    g_input = torch.empty((bsz, basis, seqlen, dim), device=device, dtype=torch.float32)
+    branch = torch.empty((bsz, basis, seqlen, dim), device=device, dtype=dtype) if want_branch else None
+    grads = [torch.empty(w.shape, device=device, dtype=dtype) for w in (fc2, fc1, out_proj, in_proj, norm2, norm1, conv)] if inputs else ()
+    lib = _lib.load()
+    layer = _lib.RegionLayer(
+        bsz, basis, seqlen, dim, hidden, heads, kv_heads, head_dim, taps,
+        _lib.dtype_code(dtype), _lib.dtype_code(x1.dtype), _lib.dtype_code(x2.dtype),
+        int(g_len != seqlen), int(bool(attn.rope_interleaved)), int(attn_edge),
+        float(block.norm.eps), float(block.norm2.eps), float(scale),
+        None if g_hidden is None else g_hidden.data_ptr(), g_residual.data_ptr(),
+        fc2.data_ptr(), fc1.data_ptr(), out_proj.data_ptr(), in_proj.data_ptr(), norm2.data_ptr(), norm1.data_ptr(), conv.data_ptr(),
+        fc1_output.data_ptr(), x2.data_ptr(), x1.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
+        cos.data_ptr(), sin.data_ptr(), g_input.data_ptr(), None if branch is None else branch.data_ptr(),
+        *(t.data_ptr() for t in inputs), *(t.data_ptr() for t in grads))
+    with _lib.device_guard(device):
+        need = int(lib.lbi_region_layer_workspace_bytes(ctypes.byref(layer)))
+        workspace = torch.empty(need, device=device, dtype=torch.uint8)
+        status = lib.lbi_region_layer_pullback(ctypes.byref(layer), workspace.data_ptr(), need, _stream(q))
+    _lib.check(status, "lbi_region_layer_pullback")
+    if param_grads is not None:
+        for param, grad in zip((fc2, fc1, out_proj, in_proj, norm2, norm1, conv), grads):
+            param_grads[id(param)] = grad
+    return g_input, branch
+
+
 def _layer_input_pullback(block: Any, layer_cache: Any, g_hidden: torch.Tensor | None, g_residual: torch.Tensor,
                           kernel_mode: str, want_branch: bool, param_grads: dict | None = None,
                           keep_residual: bool = False) -> tuple[torch.Tensor, torch.Tensor | None]:
     """One block, backwards.  ``g_residual`` (fp32, [B,P,T,D]) is the cotangent of the block's
-    residual output and is updated in place (``[B,P,1,D]``: the same at every position, read only; with
+    residual output and may be updated in place (``[B,P,1,D]``: the same at every position, read only; with
     ``keep_residual`` a full-size one is left untouched too);
     ``g_hidden`` is the cotangent of its hidden output
     in the weight dtype (``None``: equal to ``g_residual``).  Returns the cotangent of
@@ -426,6 +526,10 @@ def _layer_input_pullback(block: Any, layer_cache: Any, g_hidden: torch.Tensor |
     With ``param_grads`` (a dict filled as ``id(parameter) -> gradient``; P must be 1) the
     parameter gradients of the block are formed on the way, each from the cotangent at the
     output of its module and the cached input of that module."""
+    if kernel_mode == "hip":
+        done = _native_layer(block, layer_cache, g_hidden, g_residual, want_branch, param_grads)
+        if done is not None:
+            return done
     attn, mlp = block.attn, block.mlp
     a_cache, m_cache = layer_cache.attention, layer_cache.mlp
     # Branch cotangents live in the dtype the forward's matrix products ran in, which is what the cached

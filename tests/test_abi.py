@@ -232,3 +232,23 @@ def test_wrappers_reject_bad_input_before_touching_the_device():
         suffix_scan_pullbacks(torch.zeros(2, 3, 4, 5))
     with pytest.raises(RuntimeError, match="CUDA tensor"):
         suffix_scan_pullbacks(torch.zeros(2, 3, 4, 4))
+
+
+def test_region_layer_statuses():
+    lib = _lib.load()
+    assert lib.lbi_region_layer_workspace_bytes(None) == 0 and b"null" in lib.lbi_last_error()
+    sizes = dict(B=1, P=2, T=64, D=64, hidden=128, H=2, Hkv=1, Dh=32, ksize=4, dtype=_lib.LBI_BF16, norm1_dtype=_lib.LBI_BF16,
+                 norm2_dtype=_lib.LBI_F32)
+    pointers = {name: 256 for name, kind in _lib.RegionLayer._fields_ if kind is ctypes.c_void_p and not name.startswith("grad_")}
+
+    def status(**changes):
+        layer = _lib.RegionLayer(**{**sizes, **pointers, **changes})
+        return lib.lbi_region_layer_pullback(ctypes.byref(layer), None, 0, None), lib.lbi_region_layer_workspace_bytes(ctypes.byref(layer))
+
+    assert status()[0] == -4 and status()[1] > 0            # LBI_ERR_WORKSPACE: all is well but the workspace
+    for changes in (dict(dtype=_lib.LBI_F32), dict(B=0), dict(T=1 << 31), dict(ksize=9), dict(Hkv=3), dict(Dh=30), dict(T=1 << 28),
+                    dict(q=None), dict(g_residual=None), dict(grad_fc2=256), dict(grad_fc2=256, P=1),
+                    dict(grad_fc2=256, P=1, g_broadcast_t=1)):
+        code, need = status(**changes)
+        assert code in (-1, -2) and need == 0, changes
+

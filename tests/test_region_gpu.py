@@ -608,3 +608,79 @@ def test_small_product_of_a_weight_gradient(height, width, rows, dtype, device):
     half_ulp = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
     bound = (rows + 1) * 2.0 ** -24 * sums * (1 + half_ulp) + half_ulp * truth.abs() + 2.0 ** -25
     assert bool(((got.double() - truth).abs() <= bound).all())
+
+
+def _small_block(dtype, device, *, dim=64, heads=2, kv=1, hd=32, hidden=96, layers=2, b=2, t=40, **more):
+    backend = oreg.make_backend(dim=dim, n_heads=heads, n_kv_heads=kv, head_dim=hd, hidden=hidden, layers=layers, d_conv=4, dtype=dtype,
+                                seed=7, **more).to(device)
+    gen = torch.Generator().manual_seed(8)
+    with torch.no_grad():
+        _, cache = backend.forward_region(region_input=torch.randn(b, t, dim, generator=gen).to(dtype).to(device), region_index=0)
+    return backend, cache, gen
+
+
+def _launch_by_launch(monkeypatch, call):
+    from latent_bounded_interfaces_amd.hip.transformer import region
+
+    taken = []
+    native = region._native_layer
+    with monkeypatch.context() as patch:
+        patch.setattr(region, "_native_layer", lambda *a: taken.append(native(*a)) or taken[-1])
+        got = call()
+    with monkeypatch.context() as patch:
+        patch.setattr(region, "_native_layer", lambda *a: None)
+        return got, call(), [one is not None for one in taken]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("sizes", [dict(), dict(hd=64, t=64), dict(hd=64, heads=3, kv=3, t=300), dict(hd=128, t=130, rope_interleaved=True),
+                                   dict(hd=40, dim=80, t=129, softmax_scale=0.2, residual_in_fp32=False), dict(t=1, b=1, layers=1)])
+def test_native_layer_equals_its_launches(sizes, dtype, device, monkeypatch):
+    """One call per block, and the same launches one by one: the same bits; dense and position-constant bases, parameter gradients."""
+    from latent_bounded_interfaces_amd.backends import HipTransformerLowering
+
+    backend, cache, gen = _small_block(dtype, device, **sizes)
+    lowering = HipTransformerLowering()
+    b, t, dim = cache.region_input.shape
+    basis = torch.randn(b, 3, t, dim, generator=gen).to(device)
+    for cotangent in (basis, basis[:, :, :1].expand(b, 3, t, dim), basis.to(dtype)):
+        keep = cotangent.clone()
+        got, want, taken = _launch_by_launch(monkeypatch, lambda: lowering.input_pullback_basis(
+            backend=backend, cache=cache, output_cotangent_basis=cotangent))
+        assert all(taken) and torch.equal(got, want) and torch.equal(cotangent, keep)
+    got, want, taken = _launch_by_launch(monkeypatch, lambda: lowering.parameter_vjp_with_input_cotangent(
+        backend=backend, cache=cache, output_cotangent=basis[:, 0]))
+    assert all(taken) and torch.equal(got[1], want[1]) and got[0].keys() == want[0].keys()
+    for name, grad in want[0].items():
+        assert torch.equal(got[0][name], grad) and got[0][name].dtype == grad.dtype, name
+
+
+def test_native_layer_leaves_what_it_does_not_take(device, monkeypatch):
+    from latent_bounded_interfaces_amd.backends import HipTransformerLowering
+
+    lowering = HipTransformerLowering()
+    for dtype, sizes, expect in ((torch.float32, dict(), False), (torch.bfloat16, dict(bias=True), None), (torch.bfloat16, dict(hd=36, dim=72), False)):
+        backend, cache, gen = _small_block(dtype, device, **sizes)
+        b, t, dim = cache.region_input.shape
+        basis = torch.randn(b, 2, t, dim, generator=gen).to(device)
+        got, want, taken = _launch_by_launch(monkeypatch, lambda: lowering.input_pullback_basis(
+            backend=backend, cache=cache, output_cotangent_basis=basis))
+        assert torch.equal(got, want) and (expect is None or not any(taken))   # (biases take no part in the input pullback)
+        got, want, taken = _launch_by_launch(monkeypatch, lambda: lowering.parameter_vjp(
+            backend=backend, cache=cache, output_cotangent=basis[:, 0]))
+        assert not any(taken) and all(torch.equal(got[name], grad) for name, grad in want.items())
+    # weights off the 16-byte grid, and a cache that is not contiguous
+    backend, cache, gen = _small_block(torch.bfloat16, device)
+    block = backend.backbone.blocks[0]
+    room = torch.empty(block.mlp.fc1.weight.numel() + 1, device=device, dtype=torch.bfloat16)
+    moved = room[1:].view_as(block.mlp.fc1.weight)
+    moved.copy_(block.mlp.fc1.weight.detach())
+    block.mlp.fc1.weight.data = moved
+    cache.layer_caches[1].attention.q_rope = cache.layer_caches[1].attention.q_rope.transpose(1, 2).contiguous().transpose(1, 2)
+    b, t, dim = cache.region_input.shape
+    basis = torch.randn(b, 2, t, dim, generator=gen).to(device)
+    got, want, taken = _launch_by_launch(monkeypatch, lambda: lowering.input_pullback_basis(
+        backend=backend, cache=cache, output_cotangent_basis=basis))
+    assert taken == [True, False]
+    assert _max_rel(got.cpu(), want.cpu()) <= 2e-2
+
