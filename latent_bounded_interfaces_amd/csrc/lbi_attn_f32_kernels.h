@@ -27,7 +27,7 @@
 // rows as far as there are any: under the causal mask neighbouring row tiles end at different steps and the waves of the
 // shorter ones wait (B=4 H=8 T=512 Dh=64 P=8: dq 145 -> 125 us, dkdv 189 -> 175 us against four row tiles).  Two
 // directions per wave share one S tile, at one wave per SIMD; one direction at two waves per SIMD took 176 / 201 us.
-// Whole call there: 5.41 ms on the scalar kernels (lbi_attn_generic.h), 0.393 ms here (45 TFLOP/s algorithmic), with the
+// Whole call there: 5.41 ms on the scalar kernels (lbi_attn_generic.h), 0.355 ms here (50 TFLOP/s algorithmic), with the
 // error of the scalar kernels: relative 2-norm against 64 bits 3.9e-7 / 6.0e-7 / 5.9e-7 in dQ / dK / dV, and 0.98 to 1.02
 // times theirs over T = 24 ... 3000, head dims 16 ... 128, V with and without an offset.
 // 16-bit storage, no mask, scalar kernels -> here: bf16 B=4 H=8 T=1000 Dh=64 P=8 26.2 -> 2.36 ms, B=1 H=2 T=333 Dh=64 P=3 388 ->
@@ -36,6 +36,8 @@
 
 #include "lbi_attn_f32.h"
 
+#include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace lbi {
@@ -239,14 +241,27 @@ __device__ __forceinline__ void load_half_row(float (&dst)[DH / 2], const T* __r
 }
 
 // Workgroup -> (row tile, group).  The groups lie along x, which is dealt first, and the row tiles along y and z: all
-// groups of the longest row tile come first, so that the short tiles of a causal call fill the end of the launch.  A grid
+// groups of the longest row tile come first, so that the short tiles of a causal call fill the end of the launch.  Only the first
+// `turned` workgroups, one for every CU, come shortest first: where a CU holds two of them, the longest of the second lot joins the
+// shortest of the first (B=4 H=8 T=512 Dh=64 P=8, all four kernels: 393 us with both lots longest first, 360 so).  A grid
 // may hold fewer than 2^32 threads along x and 65535 workgroups along y and z, so neither lies along x alone.
 struct Place {
     int tile, group;
 };
-__device__ __forceinline__ Place place(int tiles, bool last_first) {
-    const int t = (int)(blockIdx.z * gridDim.y + blockIdx.y);  // past `tiles` in the last row of z: no work
-    return {last_first ? tiles - 1 - t : t, (int)blockIdx.x};
+__device__ __forceinline__ Place place(bool last_first, int tiles, int turned) {
+    int t = (int)(blockIdx.z * gridDim.y + blockIdx.y), group = (int)blockIdx.x;  // past `tiles` in the last row of z: no work
+    const long long id = (long long)t * gridDim.x + group;
+    if (id < turned) {
+        const unsigned from_end = (unsigned)turned - 1 - (unsigned)id;
+        t = (int)(from_end / gridDim.x);
+        group = (int)(from_end - (unsigned)t * gridDim.x);
+    }
+    return {last_first ? tiles - 1 - t : t, group};
+}
+// the workgroups that come shortest first
+inline int turned_of(int tiles, int groups) {
+    const long long all = (long long)tiles * groups, cus = device_compute_units();
+    return (int)(all < cus ? all : cus);
 }
 inline dim3 grid_of(int tiles, int groups) {
     const int rows = tiles < 65535 ? tiles : 65535;
@@ -296,20 +311,41 @@ __device__ __forceinline__ float sum16(const f32x16& x) {
     return (t[0] + t[1]) + (t[2] + t[3]);
 }
 
+// The largest score (log2 domain) of a query so far and the sum of 2^(score - largest); the two lanes of a query share `top`.
+struct RowSums {
+    float top = -INFINITY, sum = 0.0f;
+    __device__ __forceinline__ void add(f32x16& s, int j0, int h, int last_key, float sc2) {
+        float most = top;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            s[i] = j0 + acc_row(i, h) <= last_key ? s[i] * sc2 : -INFINITY;
+            most = fmaxf(most, s[i]);
+        }
+        most = fmaxf(most, __shfl_xor(most, 32, 64));
+        const float base = most == -INFINITY ? 0.0f : most;  // scores of -inf only so far: their terms are 0
+        const float alpha = exp2f(top - base);
+        top = most;
+        // the terms of a tile in a tree of their own: the running sum rounds once per tile
+#pragma unroll
+        for (int i = 0; i < 16; ++i) s[i] = exp2f(s[i] - base);
+        sum = sum * alpha + sum16(s);
+    }
+};
+
 template <typename T, int DH, bool VEC>
 __global__ __launch_bounds__(NT) void stats_kernel(const T* __restrict__ q, const T* __restrict__ k,
                                                    float* __restrict__ lse2, int T_len, int dh, float scale, int causal,
-                                                   int tiles) {
+                                                   int tiles, int turned) {
     constexpr int ROWS = NWAVE * TILE, PITCH = TileStage<T, DH, VEC>::PITCH;
     extern __shared__ __align__(16) float lds[];  // [2][K tile]
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, h = lane >> 5, wave = tid >> 6;
-    const Place at = place(tiles, causal);
+    const Place at = place(causal, tiles, turned);
     if (at.tile < 0 || at.tile >= tiles) return;
     const size_t base = (size_t)at.group * T_len * dh;
     const int q0 = at.tile * ROWS + wave * TILE, query = q0 + m;
     float qf[1][DH / 2];
     load_half_row<T, DH, VEC>(qf[0], q + base, query, h, T_len, dh);
-    float m_run = -INFINITY, l_run = 0.0f;
+    RowSums run;
     const float sc2 = scale * LOG2E;
     const int end = causal ? min(T_len, (at.tile + 1) * ROWS) : T_len;
     TileStream<T, DH, VEC, 1> keys{{k + base}, lds, T_len, dh, tid, (end + TILE - 1) / TILE};
@@ -323,21 +359,7 @@ __global__ __launch_bounds__(NT) void stats_kernel(const T* __restrict__ q, cons
         f32x16 ss[1] = {zero16()};
         f32x16& s = ss[0];
         dot_form<DH, 1>(ss, keys.tile(it, 0) + m * PITCH + h * (DH / 2), qf, nothing);
-        float top = m_run;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const int key = j0 + acc_row(i, h);
-            s[i] = (key < T_len && (!causal || key <= query)) ? s[i] * sc2 : -INFINITY;
-            top = fmaxf(top, s[i]);
-        }
-        top = fmaxf(top, __shfl_xor(top, 32, 64));
-        const float base2 = top == -INFINITY ? 0.0f : top;  // scores of -inf only so far: their terms are 0
-        const float alpha = exp2f(m_run - base2);
-        m_run = top;
-        // the terms of a tile in a tree of their own: the running sum rounds once per tile
-#pragma unroll
-        for (int i = 0; i < 16; ++i) s[i] = exp2f(s[i] - base2);
-        l_run = l_run * alpha + sum16(s);
+        run.add(s, j0, h, causal ? min(query, T_len - 1) : T_len - 1, sc2);
         keys.finish(it);
     }
     for (int it = mine; it < keys.steps; ++it) {
@@ -345,8 +367,62 @@ __global__ __launch_bounds__(NT) void stats_kernel(const T* __restrict__ q, cons
         keys.finish(it);
     }
     if (query >= T_len) return;
-    const float l_all = l_run + __shfl_xor(l_run, 32, 64);
-    if (h == 0) lse2[(size_t)at.group * T_len + query] = m_run + log2f(l_all);
+    const float l_all = run.sum + __shfl_xor(run.sum, 32, 64);
+    if (h == 0) lse2[(size_t)at.group * T_len + query] = run.top + log2f(l_all);
+}
+
+// The statistics of few rows: a workgroup owns 32 queries and its waves every fourth tile of their keys, each read straight into the
+// operand registers, a tile ahead; the four sums of a query meet at the end.  (The kernel above has a workgroup for every 128
+// queries, as long as the last of them: a whole call of B=4 H=8 T=512 Dh=64 P=8 370 -> 355 us, B=2 H=8 T=1000 Dh=64 P=4 448 ->
+// 415, B=2 H=4 T=512 Dh=128 P=4 387 -> 369.)
+template <typename T, int DH, bool VEC>
+__global__ __launch_bounds__(NT) void stats_split_kernel(const T* __restrict__ q, const T* __restrict__ k,
+                                                         float* __restrict__ lse2, int T_len, int dh, float scale, int causal,
+                                                         int tiles, int turned) {
+    __shared__ float part[NWAVE][2][TILE];  // largest score and sum, by wave
+    const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const Place at = place(causal, tiles, turned);
+    if (at.tile < 0 || at.tile >= tiles) return;
+    const size_t base = (size_t)at.group * T_len * dh;
+    const int query = at.tile * TILE + m;
+    float qf[1][DH / 2];
+    load_half_row<T, DH, VEC>(qf[0], q + base, query, h, T_len, dh);
+    const int last_key = causal ? min(query, T_len - 1) : T_len - 1, steps = causal ? at.tile + 1 : tiles;
+    const float sc2 = scale * LOG2E;
+    RowSums run;
+    Raw<T, VEC> next[DH / 8];
+    auto fetch = [&](int it) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < DH / 8; ++c) next[c] = load_piece<T, VEC>(k + base, it * TILE + m, h * (DH / 2) + 4 * c, T_len, dh);
+    };
+    if (wave < steps) fetch(wave);
+    for (int it = wave; it < steps; it += NWAVE) {
+        f32x4 key[DH / 8];
+#pragma unroll
+        for (int c = 0; c < DH / 8; ++c) key[c] = keep<T>(next[c], it * TILE + m < T_len, h * (DH / 2) + 4 * c, dh);
+        fetch(min(it + NWAVE, steps - 1));
+        f32x16 s = zero16();
+#pragma unroll
+        for (int c = 0; c < DH / 8; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s = mma(key[c][e], qf[0][4 * c + e], s);
+        run.add(s, it * TILE, h, last_key, sc2);
+    }
+    const float sum = run.sum + __shfl_xor(run.sum, 32, 64);
+    if (h == 0) {
+        part[wave][0][m] = run.top;
+        part[wave][1][m] = sum;
+    }
+    __syncthreads();
+    if (tid >= TILE || query >= T_len) return;
+    float top = part[0][0][m];
+#pragma unroll
+    for (int w = 1; w < NWAVE; ++w) top = fmaxf(top, part[w][0][m]);
+    const float base2 = top == -INFINITY ? 0.0f : top;
+    float terms[NWAVE];
+#pragma unroll
+    for (int w = 0; w < NWAVE; ++w) terms[w] = part[w][1][m] * exp2f(part[w][0][m] - base2);
+    lse2[(size_t)at.group * T_len + query] = top + log2f((terms[0] + terms[1]) + (terms[2] + terms[3]));
 }
 
 // The wave's share of a dq or delta launch.  DW of the four waves own different direction groups of the same rows, 4 / DW
@@ -373,16 +449,17 @@ template <int PB, int DW> struct QueryShare {
 // kernel, it saves these products (the whole call above 0.330 ms), but the error of dQ is 1.04 to 1.14 times as large, and
 // with an offset in V up to 1.9 times.
 // Two directions per wave at two waves per SIMD, as many as in dq: four at one wave per SIMD share S but hide less, 0.403
-// against 0.391 ms for the whole causal call (0.616 and 0.631 without the mask).
+// against 0.391 ms for the whole causal call (0.616 and 0.631 without the mask).  The matrix cores are at work for 47 % of its time (61
+// and 58 in dq and dkdv, one wave per SIMD).
 template <typename T, int DH, int PB, int DW, bool VEC>
 __global__ __launch_bounds__(NT) void delta_kernel(const T* __restrict__ q, const T* __restrict__ k,
                                                    const T* __restrict__ v, const T* __restrict__ d_out,
                                                    const float* __restrict__ lse2, float* __restrict__ delta, int H, int P,
-                                                   int T_len, int dh, float scale, int causal, int tiles) {
+                                                   int T_len, int dh, float scale, int causal, int tiles, int turned) {
     constexpr int ROWS = NWAVE / DW * TILE, PITCH = TileStage<T, DH, VEC>::PITCH;
     extern __shared__ __align__(16) float lds[];  // [2][K tile, V tile]
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const Place at = place(tiles, causal);
+    const Place at = place(causal, tiles, turned);
     if (at.tile < 0 || at.tile >= tiles) return;
     const QueryShare<PB, DW> own(at, wave, H, P, T_len);
     const int query = own.q0 + m;
@@ -434,11 +511,11 @@ __global__ __launch_bounds__(NT) void dq_kernel(const T* __restrict__ q, const T
                                                 const T* __restrict__ v, const T* __restrict__ d_out,
                                                 const float* __restrict__ lse2, const float* __restrict__ delta,
                                                 T* __restrict__ dq, int H, int P, int T_len, int dh, float scale,
-                                                int causal, int tiles) {
+                                                int causal, int tiles, int turned) {
     constexpr int ROWS = NWAVE / DW * TILE, PITCH = TileStage<T, DH, VEC>::PITCH, NB = DH / 32;
     extern __shared__ __align__(16) float lds[];  // [2][K tile, V tile]
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const Place at = place(tiles, causal);
+    const Place at = place(causal, tiles, turned);
     if (at.tile < 0 || at.tile >= tiles) return;
     const QueryShare<PB, DW> own(at, wave, H, P, T_len);
     const int q0 = own.q0, query = q0 + m;
@@ -516,14 +593,14 @@ __global__ __launch_bounds__(NT) void dkdv_kernel(const T* __restrict__ q, const
                                                   const T* __restrict__ v, const T* __restrict__ d_out,
                                                   const float* __restrict__ lse2, const float* __restrict__ delta,
                                                   T* __restrict__ dk, T* __restrict__ dv, int H, int P,
-                                                  int T_len, int dh, float scale, int causal, int tiles) {
+                                                  int T_len, int dh, float scale, int causal, int tiles, int turned) {
     using Stage = TileStage<T, DH, VEC>;
     constexpr int PITCH = Stage::PITCH, NB = DH / 32, ROWS = NWAVE / DW * TILE;
     constexpr int ND = DW * PB;  // directions of the workgroup
     constexpr int MATS = (1 + ND) * TILE * PITCH, BUF = MATS + 2 * NT;
     extern __shared__ __align__(16) float lds[];  // [2][Q tile, ND d_out tiles, lse of the rows, ND deltas of the rows]
     const int tid = threadIdx.x, lane = tid & 63, m = lane & 31, h = lane >> 5, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const Place at = place(tiles, false);  // the first keys see the most queries
+    const Place at = place(false, tiles, turned);  // the first keys see the most queries
     if (at.tile >= tiles) return;
     const int pgroups = (P + ND - 1) / ND;
     const int head = at.group % H, b = at.group / (H * pgroups);
@@ -670,15 +747,22 @@ int launch_with(const Args<T>& a) {
     if (int rc = ensure_dynamic_lds<&delta_kernel<T, DH, PB, DW, VEC>>(kv_bytes)) return rc;
     if (int rc = ensure_dynamic_lds<&dq_kernel<T, DH, PB, DW, VEC>>(kv_bytes)) return rc;
     if (int rc = ensure_dynamic_lds<&dkdv_kernel<T, DH, PB, DW, VEC>>(qg_bytes)) return rc;
-    hipLaunchKernelGGL((stats_kernel<T, DH, VEC>), grid_of(stat_tiles, heads), dim3(NT), k_bytes, a.stream, a.q, a.k,
-                       a.lse2, a.T_len, a.dh, a.scale, a.causal, stat_tiles);
+    const int key_tiles = (a.T_len + TILE - 1) / TILE, turned = turned_of(tiles, groups);
+    // the largest number of workgroups of the other statistics kernel at which this one was as fast or faster: B=8 H=8 T=512 P=1 224 -> 217 us
+    // with a mask (256), 223 -> 226 without; B=4 H=8 T=2048 Dh=128 (512) 1579 -> 1610 and 2841 -> 2924
+    if (4LL * stat_tiles * heads <= (a.causal ? 4LL : 3LL) * device_compute_units())
+        hipLaunchKernelGGL((stats_split_kernel<T, DH, VEC>), grid_of(key_tiles, heads), dim3(NT), 0, a.stream, a.q, a.k, a.lse2,
+                           a.T_len, a.dh, a.scale, a.causal, key_tiles, turned_of(key_tiles, heads));
+    else
+        hipLaunchKernelGGL((stats_kernel<T, DH, VEC>), grid_of(stat_tiles, heads), dim3(NT), k_bytes, a.stream, a.q, a.k,
+                           a.lse2, a.T_len, a.dh, a.scale, a.causal, stat_tiles, turned_of(stat_tiles, heads));
     hipLaunchKernelGGL((delta_kernel<T, DH, PB, DW, VEC>), grid_of(tiles, groups), dim3(NT), kv_bytes, a.stream, a.q, a.k, a.v,
-                       a.d_out, a.lse2, a.delta, a.H, a.P, a.T_len, a.dh, a.scale, a.causal, tiles);
+                       a.d_out, a.lse2, a.delta, a.H, a.P, a.T_len, a.dh, a.scale, a.causal, tiles, turned);
     hipLaunchKernelGGL((dq_kernel<T, DH, PB, DW, VEC>), grid_of(tiles, groups), dim3(NT), kv_bytes, a.stream, a.q, a.k, a.v,
-                       a.d_out, a.lse2, a.delta, a.dq, a.H, a.P, a.T_len, a.dh, a.scale, a.causal, tiles);
+                       a.d_out, a.lse2, a.delta, a.dq, a.H, a.P, a.T_len, a.dh, a.scale, a.causal, tiles, turned);
     hipLaunchKernelGGL((dkdv_kernel<T, DH, PB, DW, VEC>), grid_of(tiles, groups), dim3(NT), qg_bytes, a.stream,
                        a.q, a.k, a.v, a.d_out, a.lse2, a.delta, a.dk, a.dv, a.H, a.P, a.T_len, a.dh, a.scale, a.causal,
-                       tiles);
+                       tiles, turned);
     LBI_HIP_CHECK(hipGetLastError());
     return LBI_OK;
 }
@@ -687,22 +771,36 @@ int launch_with(const Args<T>& a) {
 // d_out tiles leave of the LDS), fewer where that leaves fewer waves without a direction.  One where few workgroups of one
 // or two row tiles leave half of the CUs idle anyway: a tile of one direction is loaded sooner (B=4 H=8 T=32 Dh=33 P=4:
 // 39 -> 33 us; with a workgroup for every CU or more it takes up to twice as long).
-template <int DH, int PB, int MAX, bool VEC, typename T>
-int launch_directions(const Args<T>& a) {
+template <int PB, int MAX, typename T> int waves_apart(const Args<T>& a) {
     const int pgroups = (a.P + PB - 1) / PB;
     auto padded = [&](int dw) { return (pgroups + dw - 1) / dw * dw; };
-    if (a.T_len <= 2 * TILE && (long long)a.B * a.H * pgroups <= device_compute_units() / 2) return launch_with<DH, PB, 1, VEC>(a);
-    if constexpr (MAX >= 4)
-        if (padded(4) == padded(2) && pgroups > 2) return launch_with<DH, PB, 4, VEC>(a);
-    if (padded(2) == pgroups || pgroups > 2) return launch_with<DH, PB, 2, VEC>(a);
-    return launch_with<DH, PB, 1, VEC>(a);
+    if (a.T_len <= 2 * TILE && (long long)a.B * a.H * pgroups <= device_compute_units() / 2) return 1;
+    if (MAX >= 4 && padded(4) == padded(2) && pgroups > 2) return 4;
+    return padded(2) == pgroups || pgroups > 2 ? 2 : 1;
 }
 
-// Two directions per wave where that still gives every SIMD a wave: below, a call is as long as its longest wave.
-// B=1 H=2 T=1000 Dh=64 P=8: 637 us with two, 430 with one; B=4 H=8 T=512 Dh=64 P=2: 329 and 226.
+template <int DH, int PB, int MAX, bool VEC, typename T> int launch_directions(const Args<T>& a) {
+    const int dw = waves_apart<PB, MAX>(a);
+    if constexpr (MAX >= 4)
+        if (dw == 4) return launch_with<DH, PB, 4, VEC>(a);
+    return dw == 2 ? launch_with<DH, PB, 2, VEC>(a) : launch_with<DH, PB, 1, VEC>(a);
+}
+
+// Tiles that a CU goes through at PB directions per wave, one workgroup after another: those of the longest one at least.
+template <int PB, typename T> double steps_of_a_cu(const Args<T>& a) {
+    const int dw = waves_apart<PB, 4>(a), rows = NWAVE / dw, nd = dw * PB;
+    const double steps = (a.T_len + TILE - 1) / TILE, tiles = (a.T_len + rows * TILE - 1) / (rows * TILE);
+    const double cus = device_compute_units(), groups = (double)a.B * a.H * ((a.P + nd - 1) / nd);
+    if (!a.causal) return steps * ceil(groups * tiles / cus);
+    return std::max(steps, groups * tiles * (steps + rows) / (2 * cus));
+}
+
+// Two directions per wave share S: 15 products for the two and not 18.  One makes for twice the workgroups, half as long: taken
+// where few long ones leave CUs idle.  The line lies at 3 / 2, below 5 / 3, since a wave does less well with one (us, with one and
+// with two): B=1 H=2 T=1000 Dh=64 P=8 430 and 637, B=4 H=8 T=512 P=2 226 and 329, B=2 H=8 T=1000 P=4 417 and 591, B=5 H=1 T=1761 Dh=32
+// P=8 430 and 589; B=4 H=8 T=512 Dh=64 P=8 427 and 354, B=8 H=5 T=320 P=8 248 and 215.
 template <typename T> bool two_directions(const Args<T>& a) {
-    const long long waves = (long long)a.B * a.H * ((a.P + 1) / 2) * ((a.T_len + TILE - 1) / TILE);
-    return a.P >= 2 && waves >= 4LL * device_compute_units();
+    return a.P >= 2 && 1.5 * steps_of_a_cu<2>(a) <= steps_of_a_cu<1>(a);
 }
 
 template <typename T>

@@ -113,6 +113,22 @@ def test_fp32_tile_edges_against_fp64(shape, basis, causal, device):
         assert err <= bound, (name, err, bound)
 
 
+# more and fewer workgroups than CUs, row tiles and groups either side of one for every CU and of two; the statistics by workgroups of
+# 128 queries and of 32
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("shape,basis", [((16, 17, 40, 32), 1), ((12, 16, 33, 64), 2), ((5, 13, 129, 64), 4), ((3, 11, 250, 64), 8),
+                                         ((2, 8, 520, 64), 4), ((1, 1, 1055, 128), 2), ((1, 43, 95, 96), 5)])
+def test_fp32_workgroups_and_cus(shape, basis, causal, device):
+    q, k, v, g = oattn.make_attention_inputs(*shape, basis, dtype=torch.float32, seed=shape[2] + basis)
+    scale = 1.0 / math.sqrt(shape[-1])
+    got = _run(q, k, v, g, device, scale=scale, causal=causal)
+    truth = oattn.attention_pullback_blocked(q, k, v, g, softmax_scale=scale, causal=causal, dtype=torch.float64)
+    bound = (shape[2] + 2 * shape[3]) * 2.0 ** -24  # as above
+    for name, a, c in zip(("dq", "dk", "dv"), got, truth):
+        err = float((a.double() - c).abs().max()) / max(float(c.abs().max()), float(g.abs().max()))
+        assert err <= bound, (name, err, bound)
+
+
 @pytest.mark.parametrize("offset", [0, 1, 4])   # elements in front of each tensor: whole pieces, single ones, 8-byte pieces
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("causal", [True, False])
