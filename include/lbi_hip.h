@@ -263,6 +263,15 @@ int lbi_small_product(const void* a, const void* w, void* out, int64_t M, int64_
                       int64_t Dh, int dtype, void* stream);
 
 /*
+ * The weight gradient of a linear layer: out = a^T w, a [K,M], w [K,N], out [M,N], sums in fp32, one rounding; the gradient form of
+ * lbi_small_product where that is the faster one, with its sizes and types.  Otherwise long sums are cut into ranges of K and added
+ * in order; workspace: lbi_weight_gradient_workspace_bytes(M,N,K) bytes, none if that is 0.
+ */
+size_t lbi_weight_gradient_workspace_bytes(int64_t M, int64_t N, int64_t K);
+int lbi_weight_gradient(const void* a, const void* w, void* out, void* workspace, size_t workspace_bytes,
+                        int64_t M, int64_t N, int64_t K, int dtype, void* stream);
+
+/*
  * Head split of the out_proj-input cotangent: [B,P,T,H*Dh] -> [B,P,H,T,Dh], the layout
  * lbi_attn_pullback takes as d_out (transpose of reference backends/transformer.py:152-153).
  */

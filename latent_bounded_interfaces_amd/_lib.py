@@ -16,7 +16,7 @@ LIB_PATH = Path(__file__).resolve().parent / "liblbi_hip.so"
 
 LBI_F32, LBI_F16, LBI_BF16 = 0, 1, 2
 ATTN_STATIC_SCRATCH_BYTES = 32 << 20  # LBI_ATTN_STATIC_SCRATCH_BYTES of include/lbi_hip.h
-ABI_VERSION = 11
+ABI_VERSION = 12
 LBI_SCAN_EXACT_SUFFIX = 1  # lbi_scan_flags of include/lbi_hip.h
 
 _DTYPE_CODES = {torch.float32: LBI_F32, torch.float16: LBI_F16, torch.bfloat16: LBI_BF16}
@@ -93,6 +93,8 @@ SYMBOLS = {
     ),
     "lbi_gated_mlp_pullback": (_c.c_int, [_c.c_void_p] * 3 + [_c.c_int64] * 4 + [_c.c_int, _c.c_int, _c.c_void_p]),
     "lbi_small_product": (_c.c_int, [_c.c_void_p] * 3 + [_c.c_int64] * 3 + [_c.c_int] + [_c.c_int64] * 2 + [_c.c_int, _c.c_void_p]),
+    "lbi_weight_gradient_workspace_bytes": (_c.c_size_t, [_c.c_int64] * 3),
+    "lbi_weight_gradient": (_c.c_int, [_c.c_void_p] * 4 + [_c.c_size_t] + [_c.c_int64] * 3 + [_c.c_int, _c.c_void_p]),
     "lbi_attn_heads_split": (_c.c_int, [_c.c_void_p] * 2 + [_c.c_int64] * 5 + [_c.c_int, _c.c_void_p]),
     "lbi_attn_qkv_pullback": (
         _c.c_int,

@@ -16,7 +16,7 @@ CSRC = PKG_DIR / "csrc"
 LIB_PATH = PKG_DIR / "liblbi_hip.so"
 SOURCES = ("lbi_common.hip", "lbi_scan.hip", "lbi_scan_narrow.hip", "lbi_scan_narrow_f32.hip", "lbi_scan_narrow_f16.hip",
            "lbi_scan_narrow_bf16.hip", "lbi_attn.hip", "lbi_attn_f32.hip", "lbi_attn_f32_f16.hip",
-           "lbi_attn_f32_bf16.hip", "lbi_region.hip", "lbi_product.hip", "lbi_region_layer.hip", "lbi_norms.hip", "lbi_param_grads.hip")
+           "lbi_attn_f32_bf16.hip", "lbi_region.hip", "lbi_product.hip", "lbi_gradient.hip", "lbi_region_layer.hip", "lbi_norms.hip", "lbi_param_grads.hip")
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950",

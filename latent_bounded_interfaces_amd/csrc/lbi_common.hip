@@ -22,6 +22,6 @@ void clear_error() { g_error[0] = '\0'; }
 
 }  // namespace lbi
 
-extern "C" int lbi_abi_version(void) { return 11; }
+extern "C" int lbi_abi_version(void) { return 12; }
 
 extern "C" const char* lbi_last_error(void) { return g_error; }

@@ -1,4 +1,4 @@
-// One Transformer block, backwards, in one call: the launches of lbi_gated_mlp_pullback, lbi_small_product, lbi_rmsnorm_pullback,
+// One Transformer block, backwards, in one call: the launches of lbi_gated_mlp_pullback, lbi_small_product, lbi_weight_gradient, lbi_rmsnorm_pullback,
 // lbi_attn_pullback, lbi_attn_qkv_conv_pullback (and of the parameter gradients) one after the other, on buffers of one workspace.
 //
 // For blocks whose products are all small ones.  A block is nine launches of a few microseconds each (nineteen with the parameter
@@ -49,9 +49,9 @@ struct Pieces {
 
 struct Buffers {
     void *g_hidden, *g_down, *g_fc1, *g_norm2, *g_res2, *g_attn_out, *g_heads, *dq, *dk, *dv, *attn, *g_qkv, *g_in_proj, *g_norm1, *x_pre,
-        *norm_ws, *conv_ws;
+        *norm_ws, *conv_ws, *sums;
     float* small_grads;   // norm2, norm, convolution
-    size_t attn_bytes, norm_bytes, conv_bytes, used;
+    size_t attn_bytes, norm_bytes, conv_bytes, sums_bytes, used;
 };
 
 Buffers lay_out(const lbi_region_layer& s, void* base) {
@@ -82,6 +82,9 @@ Buffers lay_out(const lbi_region_layer& s, void* base) {
         b.conv_bytes = lbi_causal_conv1d_weight_grad_workspace_bytes(s.B, s.T, (int64_t)packed, s.ksize);
         b.norm_ws = ws.take(b.norm_bytes);
         b.conv_ws = ws.take(b.conv_bytes);
+        for (const auto& [m, n] : {std::pair<int64_t, int64_t>{s.D, s.hidden}, {2 * s.hidden, s.D}, {s.D, (int64_t)q_width}, {(int64_t)packed, s.D}})
+            b.sums_bytes = std::max(b.sums_bytes, lbi_weight_gradient_workspace_bytes(m, n, (int64_t)rows));
+        b.sums = ws.take(b.sums_bytes);
         b.small_grads = static_cast<float*>(ws.take((2 * s.D + packed * (s.ksize + 1)) * 4));
     }
     b.used = ws.used;
@@ -128,6 +131,9 @@ int run(const lbi_region_layer& s, const Buffers& b, void* stream_v) {
     auto product = [&](const void* a, const void* w, void* out, int64_t m, int64_t n, int64_t k, int form, int64_t t, int64_t dh) {
         return lbi_small_product(a, w, out, m, n, k, form, t, dh, s.dtype, stream_v);
     };
+    auto weight_gradient = [&](const void* a, const void* w, void* out, int64_t m, int64_t n) {
+        return lbi_weight_gradient(a, w, out, b.sums_bytes ? b.sums : nullptr, b.sums_bytes, m, n, rows, s.dtype, stream_v);
+    };
     const void* g_hidden = s.g_hidden;
     if (!g_hidden) {
         const int64_t n = g_rows * s.D;
@@ -135,10 +141,10 @@ int run(const lbi_region_layer& s, const Buffers& b, void* stream_v) {
         g_hidden = b.g_hidden;
     }
     // gated MLP
-    if (grads) LBI_STEP(product(g_hidden, s.down_input, s.grad_fc2, s.D, s.hidden, rows, LBI_PRODUCT_GRADIENT, 1, s.hidden));
+    if (grads) LBI_STEP(weight_gradient(g_hidden, s.down_input, s.grad_fc2, s.D, s.hidden));
     LBI_STEP(product(g_hidden, s.fc2_weight, b.g_down, g_rows, s.hidden, s.D, LBI_PRODUCT_ROWS_BY_WEIGHT, 1, s.hidden));
     LBI_STEP(lbi_gated_mlp_pullback(b.g_down, s.fc1_output, b.g_fc1, s.B, s.P, s.T, s.hidden, s.g_broadcast_t, s.dtype, stream_v));
-    if (grads) LBI_STEP(product(b.g_fc1, s.norm2_output, s.grad_fc1, 2 * s.hidden, s.D, rows, LBI_PRODUCT_GRADIENT, 1, s.D));
+    if (grads) LBI_STEP(weight_gradient(b.g_fc1, s.norm2_output, s.grad_fc1, 2 * s.hidden, s.D));
     LBI_STEP(product(b.g_fc1, s.fc1_weight, b.g_norm2, rows, s.D, 2 * s.hidden, LBI_PRODUCT_ROWS_BY_WEIGHT, 1, s.D));
     if (grads)
         LBI_STEP(lbi_rmsnorm_weight_grad(b.g_norm2, s.norm2_input, b.small_grads, b.norm_ws, b.norm_bytes, rows, s.D, s.norm2_eps, s.dtype,
@@ -146,7 +152,7 @@ int run(const lbi_region_layer& s, const Buffers& b, void* stream_v) {
     LBI_STEP(lbi_rmsnorm_pullback(b.g_norm2, s.norm2_input, s.norm2_weight, s.g_residual, b.g_res2, b.g_attn_out, s.B, s.P, s.T, s.D,
                                   s.norm2_eps, s.g_broadcast_t, s.dtype, s.norm2_dtype, stream_v));
     // attention
-    if (grads) LBI_STEP(product(b.g_attn_out, s.out_input, s.grad_out, s.D, q_width, rows, LBI_PRODUCT_GRADIENT, 1, q_width));
+    if (grads) LBI_STEP(weight_gradient(b.g_attn_out, s.out_input, s.grad_out, s.D, q_width));
     LBI_STEP(product(b.g_attn_out, s.out_weight, b.g_heads, rows, q_width, s.D, LBI_PRODUCT_ROWS_BY_WEIGHT, s.T, s.Dh));
     LBI_STEP((s.attn_edge ? lbi_attn_pullback_edge : lbi_attn_pullback)(s.q, s.k, s.v, b.g_heads, b.dq, b.dk, b.dv, b.attn, b.attn_bytes, s.B,
                                                                         s.H, s.T, s.Dh, s.P, s.softmax_scale, 1, s.dtype, stream_v));
@@ -161,7 +167,7 @@ int run(const lbi_region_layer& s, const Buffers& b, void* stream_v) {
         LBI_STEP(lbi_causal_conv1d_weight_grad(b.g_qkv, b.x_pre, b.small_grads + 2 * s.D, b.conv_ws, b.conv_bytes, s.B, s.T, packed, s.ksize,
                                                s.dtype, stream_v));
         LBI_STEP(lbi_causal_conv1d_pullback(b.g_qkv, s.conv_weight, b.g_in_proj, s.B * s.P, s.T, packed, s.ksize, s.dtype, stream_v));
-        LBI_STEP(product(b.g_in_proj, s.norm1_output, s.grad_in, packed, s.D, rows, LBI_PRODUCT_GRADIENT, 1, s.D));
+        LBI_STEP(weight_gradient(b.g_in_proj, s.norm1_output, s.grad_in, packed, s.D));
     }
     LBI_STEP(product(b.g_in_proj, s.in_weight, b.g_norm1, rows, s.D, packed, LBI_PRODUCT_ROWS_BY_WEIGHT, 1, s.D));
     if (grads) {

@@ -10,8 +10,9 @@ backends/transformer_cuda.py:45-64) for the block the reference's backend execut
     region_output = m + res2 of the last layer
 
 The cotangent basis [B, P, T, D] is pulled back through the layers in reverse.  Matrix
-products are library GEMMs on the [B*P*T, *] cotangent rows (small ones ``lbi_small_product``); everything between them runs in
-the kernels of liblbi_hip.so (RMSNorm, gated MLP, head split, rotary embedding + KV-group
+products are library GEMMs on the [B*P*T, *] cotangent rows (small ones
+``lbi_small_product``, weight gradients ``lbi_weight_gradient``); everything between them
+runs in the kernels of liblbi_hip.so (RMSNorm, gated MLP, head split, rotary embedding + KV-group
 sum, causal convolution, and the attention pullback itself).  The residual-stream cotangent
 is kept in fp32, branch cotangents in the dtype of the weights.  Inputs are read from the
 forward cache the backend recorded; nothing is recomputed except the softmax statistics
@@ -260,8 +261,7 @@ _TRANSPOSED_COPY_MIN_ROWS = 65536
 #: Multiply-adds and results up to which a product runs on the package's own kernel.  A call of the library takes 18 us of
 #: host time, one of this kernel 7; on the GPU (bf16, M x K x N, this kernel and the library): 512 x 256 x 1024 3.8 and 5.2 us,
 #: 2048 x 2048 x 256 9.0 and 11.8, 1000 x 1536 x 768 9.7 and 10.8, 3001 x 1000 x 520 14.8 and 15.5, 4096 x 256 x 1024 9.2 and 8.4;
-#: past the lines 8192 x 256 x 1024 15.4 and 11.7, 4096 x 512 x 2048 21.5 and 15.5.  Weight gradients: 256 x 1000 x 256 7.1 and 34.8,
-#: 4096 x 600 x 512 12.0 and 13.3, 6144 x 300 x 768 15.3 and 14.3, 256 x 8192 x 256 34.6 and 46.7; forward products: 500 x 768 x 2304
+#: past the lines 8192 x 256 x 1024 15.4 and 11.7, 4096 x 512 x 2048 21.5 and 15.5; forward products: 500 x 768 x 2304
 #: 8.7 and 8.2, 2000 x 512 x 1024 7.4 and 7.9.
 _SMALL_PRODUCT = 3 << 29
 _SMALL_PRODUCT_RESULTS = 1 << 22
@@ -269,9 +269,8 @@ _SMALL_PRODUCT_RESULTS = 1 << 22
 #: Terms of a sum up to which it does: a tile of results is one workgroup's, which takes 0.2 us per 64 terms (0.25 in a gradient)
 #: however few tiles there are, while the library cuts long sums.  Whole calls, us, this kernel and the library: 256 x 4096 x 256 13.6 and
 #: 17.7, 512 x 6144 x 768 20.5 and 17.7 (among a parameter VJP's other calls, which wait for the host, still the better: d_model 768, B=1
-#: T=205 515 and 556 for all of it), 256 x 8192 x 256 24.1 and 17.7, 128 x 65536 x 128 178 and 104.  Gradients, for which the library is slower: 64 x 16384 x 64
-#: 65 and 86, 128 x 16384 x 128 66 and 120, 128 x 65536 x 128 253 and 196, 64 x 65536 x 64 253 and 170; with results narrower than a
-#: tile 8 x 4096 x 64 18.6 and 18.5, 8 x 8192 x 64 34 and 28.
+#: T=205 515 and 556 for all of it), 256 x 8192 x 256 24.1 and 17.7, 128 x 65536 x 128 178 and 104.  Gradients, in a block that is one native call, for which
+#: the library is slower still: 64 x 16384 x 64 65 and 86, 128 x 16384 x 128 66 and 120.
 _SMALL_PRODUCT_TERMS = 6144
 _SMALL_GRADIENT_TERMS = 16384
 
@@ -307,6 +306,39 @@ def small_product(a: torch.Tensor, w: torch.Tensor, out: torch.Tensor, height: i
         status = _lib.load().lbi_small_product(a.data_ptr(), w.data_ptr(), out.data_ptr(), height, width, inner, form, seqlen,
                                                head_dim or width, _lib.dtype_code(a.dtype), _stream(a))
     _lib.check(status, "lbi_small_product")
+    return out
+
+
+#: Results and multiply-adds up to which a weight gradient runs on the package's own kernels, the library's product not cutting its long
+#: sums (us, 8192 rows, own and library): 768 x 768 22 and 57, 768 x 3072 60 and 96, 6144 x 768 95 and 114; past the lines 2048 x 4096 165 and 132,
+#: 1024 x 4096 with 32768 rows 342 and 291.
+_WEIGHT_GRADIENT_RESULTS = 5 << 20
+_WEIGHT_GRADIENT = 3 << 34
+
+
+def _is_weight_gradient(g: torch.Tensor, x: torch.Tensor) -> bool:
+    """Whether ``lbi_weight_gradient`` takes ``g^T x``."""
+    if g.dtype not in _SMALL_PRODUCT_TYPES or x.dtype != g.dtype or x.device != g.device or x.shape[0] != g.shape[0]:
+        return False
+    (rows, height), width = g.shape, int(x.shape[1])
+    return (0 < height * width <= _WEIGHT_GRADIENT_RESULTS and 0 < height * width * rows <= _WEIGHT_GRADIENT and height % 8 == 0 and width % 8 == 0
+            # what the kernels' 32-bit offsets span, the steps asked for ahead included
+            and (max(height, width) + 128) * (rows + 256) < 1 << 30
+            and g.is_contiguous() and x.is_contiguous() and g.data_ptr() % 16 == 0 and x.data_ptr() % 16 == 0)
+
+
+def weight_gradient(g: torch.Tensor, x: torch.Tensor) -> torch.Tensor:
+    """``g^T x`` for ``g [rows, M]`` and ``x [rows, N]`` of one 16-bit type, sums in fp32."""
+    _require_cuda(g, x)
+    rows, height, width = int(g.shape[0]), int(g.shape[1]), int(x.shape[1])
+    out = g.new_empty(height, width)
+    lib = _lib.load()
+    with _lib.device_guard(g.device):
+        need = int(lib.lbi_weight_gradient_workspace_bytes(height, width, rows))
+        workspace = torch.empty(need, device=g.device, dtype=torch.uint8) if need else None
+        status = lib.lbi_weight_gradient(g.data_ptr(), x.data_ptr(), out.data_ptr(), None if workspace is None else workspace.data_ptr(), need,
+                                         height, width, rows, _lib.dtype_code(g.dtype), _stream(g))
+    _lib.check(status, "lbi_weight_gradient")
     return out
 
 
@@ -360,13 +392,7 @@ def _linear_grads(sink: dict, linear: Any, g_out: torch.Tensor, x: torch.Tensor)
     """Weight (and bias) gradient of ``y = x W^T + b`` for the single direction in ``g_out [B,1,T,O]``."""
     g2 = _rows(g_out)
     x2 = _rows(x).to(g2.dtype)
-    grad = None
-    if g2.dtype in _SMALL_PRODUCT_TYPES:
-        (rows, height), width = g2.shape, int(x2.shape[1])
-        if x2.shape[0] == rows and _is_small_product(g2, x2, height, width, rows, _GRADIENT):
-            grad = small_product(g2, x2, g2.new_empty(height, width), height, width, rows, _GRADIENT)
-    if grad is None:
-        grad = torch.matmul(g2.t(), x2)
+    grad = weight_gradient(g2, x2) if _is_weight_gradient(g2, x2) else torch.matmul(g2.t(), x2)
     sink[id(linear.weight)] = grad.to(linear.weight.dtype)
     bias = getattr(linear, "bias", None)
     if bias is not None:

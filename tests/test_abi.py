@@ -210,6 +210,24 @@ def test_small_product_statuses():
         assert status == -1 and b"heads of Dh" in text, heads
 
 
+def test_weight_gradient_statuses():
+    """What lbi_weight_gradient refuses before anything is launched, for sums that are cut and for those that lbi_small_product takes."""
+    lib = _lib.load()
+    ok, odd = ctypes.c_void_p(256), ctypes.c_void_p(264)  # never dereferenced
+
+    def call(a=ok, w=ok, out=ok, ws=ok, need=1 << 40, m=768, n=768, k=8192, dtype=_lib.LBI_BF16):
+        return lib.lbi_weight_gradient(a, w, out, ws, need, m, n, k, dtype, None)
+
+    need = lib.lbi_weight_gradient_workspace_bytes(768, 768, 8192)
+    assert need > 0 and need % (128 * 128 * 4 * 36) == 0 and lib.lbi_weight_gradient_workspace_bytes(64, 64, 64) == 0
+    assert call(need=need - 1) == call(ws=None) == -4 and b"workspace" in lib.lbi_last_error()
+    for k in (64, 8192):
+        assert call(m=-1, k=k) == -1 and call(m=0, k=k) == 0
+        assert all(call(**{name: bad}, k=k) == -1 for name in ("a", "w", "out") for bad in (None, odd))
+        assert all(call(**bad, k=k) == -2 for bad in (dict(m=12), dict(n=12), dict(dtype=_lib.LBI_F32)))
+    assert call(k=0) == -2 and call(k=1 << 30) == -2 and call(m=1 << 29, n=1 << 29) == -2
+
+
 def test_fp32_attention_refuses_what_no_grid_holds():
     """More groups than a grid may have threads for: refused on the host, before a kernel has written anything."""
     lib = _lib.load()

@@ -610,6 +610,32 @@ def test_small_product_of_a_weight_gradient(height, width, rows, dtype, device):
     assert bool(((got.double() - truth).abs() <= bound).all())
 
 
+# uncut with tiles that the results end in, cut into two to many ranges (the last one short, or of a single step), results narrower than a
+# tile; the first is one for the kernel above
+@pytest.mark.parametrize("height,width,rows", [(136, 72, 449), (4104, 520, 700), (768, 3080, 1801), (264, 520, 2991), (8, 8, 8200), (136, 8, 4097),
+                                               (64, 256, 20000), (1536, 520, 6000)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_weight_gradient_cut_into_ranges(height, width, rows, dtype, device):
+    """The bound of the test above; a row past the end or of the next range in a sum would show in what is exact for small whole numbers; a
+    value that is not finite stays in its row and column of the results."""
+    from latent_bounded_interfaces_amd.hip.transformer import region
+
+    gen = torch.Generator(device=device).manual_seed(rows)
+    g, x = (torch.randn(rows, n, generator=gen, device=device).to(dtype) for n in (height, width))
+    got = region.weight_gradient(g, x)
+    assert torch.equal(got, region.weight_gradient(g, x))
+    truth, sums = g.double().t().contiguous() @ x.double(), g.double().abs().t().contiguous() @ x.double().abs()
+    half_ulp = 2.0 ** -11 if dtype == torch.float16 else 2.0 ** -8
+    bound = (rows + 1) * 2.0 ** -24 * sums * (1 + half_ulp) + half_ulp * truth.abs() + 2.0 ** -25
+    assert bool(((got.double() - truth).abs() <= bound).all())
+    g, x = (torch.randint(-1, 2, (rows, n), generator=gen, device=device).to(dtype) for n in (height, width))
+    assert torch.equal(region.weight_gradient(g, x), (g.double().t().contiguous() @ x.double()).to(dtype))
+    g[rows - 1, 3], x[rows // 2, 5] = float("inf"), float("nan")
+    got = region.weight_gradient(g, x)
+    got[3], got[:, 5] = 0, 0
+    assert bool(got.isfinite().all())
+
+
 def _small_block(dtype, device, *, dim=64, heads=2, kv=1, hd=32, hidden=96, layers=2, b=2, t=40, **more):
     backend = oreg.make_backend(dim=dim, n_heads=heads, n_kv_heads=kv, head_dim=hd, hidden=hidden, layers=layers, d_conv=4, dtype=dtype,
                                 seed=7, **more).to(device)
