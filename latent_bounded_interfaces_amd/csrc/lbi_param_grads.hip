@@ -160,18 +160,21 @@ int launch_norm(const void* g_out, const void* x, float* out, float* partials, l
 // A thread owns VEC consecutive channels and walks a slab of TS positions of one batch element, keeping the
 // last k-1 inputs in registers.  Partial layout per workgroup row: [C][k] weights, then [C] bias.
 // ---------------------------------------------------------------------------------------
-constexpr int CONV_TS = 64, CONV_AHEAD = 8;
+// A slab is CONV_TS positions, half or a quarter of that where the partial rows are no more than CONV_SLABS then: every eight positions wait
+// for memory once (B=3 T=600 C=1024 15.7 -> 8.3 us, B=1 T=128 C=1536 15.8 -> 7.8, and the rows fold in the time they took; past the line
+// B=8 T=1024 C=2304 22.8 -> 24.4, bound by its partial rows).
+constexpr int CONV_TS = 64, CONV_AHEAD = 8, CONV_SLABS = 128;
 
 template <typename T, int VEC, int KMAX>
 __global__ __launch_bounds__(THREADS) void conv_weight_grad_kernel(const T* __restrict__ g_out,
                                                                    const T* __restrict__ x,
                                                                    float* __restrict__ partials, int T_len, int C,
-                                                                   int ksize, int slabs_per_seq) {
+                                                                   int ksize, int slabs_per_seq, int slab_len) {
     const int c0 = (blockIdx.x * THREADS + threadIdx.x) * VEC;
     if (c0 >= C) return;
     const int b = blockIdx.y / slabs_per_seq, slab = blockIdx.y % slabs_per_seq;
-    const int t0 = slab * CONV_TS;
-    const int t1 = t0 + CONV_TS < T_len ? t0 + CONV_TS : T_len;
+    const int t0 = slab * slab_len;
+    const int t1 = t0 + slab_len < T_len ? t0 + slab_len : T_len;
     const size_t seq = (size_t)b * T_len;
     auto load = [&](const T* base, int t, float (&dst)[VEC]) {
         const T* p = base + (seq + t) * C + c0;
@@ -240,12 +243,20 @@ __global__ __launch_bounds__(THREADS) void conv_weight_grad_kernel(const T* __re
     for (int e = 0; e < VEC; ++e) row[(size_t)C * ksize + c0 + e] = acc_bias[e];
 }
 
-inline int conv_slabs_per_seq(int T_len) { return (T_len + CONV_TS - 1) / CONV_TS; }
+inline int conv_slab_len(long long B, int T_len) {
+    int len = CONV_TS / 4;
+    while (len < CONV_TS && B * ((T_len + len - 1) / len) > CONV_SLABS) len *= 2;
+    return len;
+}
+inline int conv_slabs_per_seq(long long B, int T_len) {
+    const int len = conv_slab_len(B, T_len);
+    return (T_len + len - 1) / len;
+}
 
 template <typename T>
 int launch_conv(const void* g_out, const void* x, float* out, float* partials, int B, int T_len, int C, int ksize,
                 hipStream_t stream) {
-    const int sps = conv_slabs_per_seq(T_len);
+    const int sps = conv_slabs_per_seq(B, T_len), len = conv_slab_len(B, T_len);
     const int slabs = B * sps;
     const int width = C * ksize + C;
     const T* gp = static_cast<const T*>(g_out);
@@ -254,11 +265,11 @@ int launch_conv(const void* g_out, const void* x, float* out, float* partials, i
     const int per_block = THREADS * (vec4 ? 4 : 1);
     const dim3 grid((C + per_block - 1) / per_block, slabs);
     if (vec4 && ksize <= 4)
-        hipLaunchKernelGGL((conv_weight_grad_kernel<T, 4, 4>), grid, dim3(THREADS), 0, stream, gp, xp, partials, T_len, C, ksize, sps);
+        hipLaunchKernelGGL((conv_weight_grad_kernel<T, 4, 4>), grid, dim3(THREADS), 0, stream, gp, xp, partials, T_len, C, ksize, sps, len);
     else if (vec4)
-        hipLaunchKernelGGL((conv_weight_grad_kernel<T, 4, 8>), grid, dim3(THREADS), 0, stream, gp, xp, partials, T_len, C, ksize, sps);
+        hipLaunchKernelGGL((conv_weight_grad_kernel<T, 4, 8>), grid, dim3(THREADS), 0, stream, gp, xp, partials, T_len, C, ksize, sps, len);
     else
-        hipLaunchKernelGGL((conv_weight_grad_kernel<T, 1, 8>), grid, dim3(THREADS), 0, stream, gp, xp, partials, T_len, C, ksize, sps);
+        hipLaunchKernelGGL((conv_weight_grad_kernel<T, 1, 8>), grid, dim3(THREADS), 0, stream, gp, xp, partials, T_len, C, ksize, sps, len);
     hipLaunchKernelGGL(fold_partials_kernel, fold_grid(width), dim3(THREADS), 0, stream, partials, out, slabs, width);
     LBI_HIP_CHECK(hipGetLastError());
     return LBI_OK;
@@ -318,7 +329,7 @@ extern "C" int lbi_rmsnorm_weight_grad(const void* g_out, const void* x, float* 
 
 extern "C" size_t lbi_causal_conv1d_weight_grad_workspace_bytes(int64_t B, int64_t T, int64_t C, int64_t ksize) {
     if (B <= 0 || T <= 0 || C <= 0 || ksize <= 0) return 0;
-    return (size_t)B * (size_t)param_grads::conv_slabs_per_seq((int)T) * ((size_t)C * ksize + C) * sizeof(float);
+    return (size_t)B * (size_t)param_grads::conv_slabs_per_seq(B, (int)T) * ((size_t)C * ksize + C) * sizeof(float);
 }
 
 extern "C" int lbi_causal_conv1d_weight_grad(const void* g_out, const void* x, float* grads, void* workspace,

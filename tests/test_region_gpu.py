@@ -98,6 +98,21 @@ def test_gated_mlp_pullback(dtype, hidden, device):
     assert torch.allclose(got.double(), want, atol=_tol(dtype) * 4, rtol=_tol(dtype) * 4)
 
 
+# directions of a token in one workgroup and in several, the last with fewer; a dense and a broadcast cotangent
+@pytest.mark.parametrize("b,p,t,hidden", [(1, 4, 5, 40), (1, 5, 3, 264), (2, 13, 7, 64), (1, 40, 300, 72), (2, 3, 600, 8)])
+@pytest.mark.parametrize("broadcast", [False, True])
+def test_gated_mlp_pullback_by_direction(b, p, t, hidden, broadcast, device):
+    """A direction's result is the one it has alone, bit for bit."""
+    from latent_bounded_interfaces_amd.hip.transformer import region
+
+    gen = torch.Generator().manual_seed(p)
+    g = torch.randn(b, p, 1 if broadcast else t, hidden, generator=gen).bfloat16().to(device)
+    fc1 = torch.randn(b, t, 2 * hidden, generator=gen).bfloat16().to(device)
+    got = region.gated_mlp_pullback(g, fc1)
+    for i in range(p):
+        assert torch.equal(got[:, i:i + 1], region.gated_mlp_pullback(g[:, i:i + 1].contiguous(), fc1)), i
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("heads,head_dim", [(3, 4), (2, 64), (5, 6)])
 def test_heads_split(dtype, heads, head_dim, device):
@@ -221,6 +236,13 @@ def test_causal_conv1d_weight_grad(dtype, bsz, seqlen, channels, ksize, device):
     assert _max_rel(g_w.cpu(), want_w) <= 2e-5 and _max_rel(g_b.cpu(), want_b) <= 2e-5
     again = region.causal_conv1d_weight_grad(g.to(device), x.to(device), ksize)
     assert torch.equal(g_w, again[0]) and torch.equal(g_b, again[1])
+
+
+@pytest.mark.parametrize("bsz,seqlen,channels,ksize", [(1, 15, 8, 4), (1, 17, 8, 4), (3, 33, 12, 8), (8, 256, 8, 4), (8, 257, 5, 4), (1, 4095, 4, 3),
+                                                      (2, 2049, 4, 4)])
+def test_causal_conv1d_weight_grad_by_slab_length(bsz, seqlen, channels, ksize, device):
+    """Slabs of 16, 32 and 64 positions, whole and cut, at the lines between them."""
+    test_causal_conv1d_weight_grad(torch.float32, bsz, seqlen, channels, ksize, device)
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
