@@ -106,8 +106,8 @@ def suffix_scan_cotangents(mats: torch.Tensor, g: torch.Tensor) -> torch.Tensor:
 def suffix_scan_pullbacks_and_cotangents(mats: torch.Tensor, g: torch.Tensor, *,
                                          exact_suffix: bool = False) -> tuple[torch.Tensor, torch.Tensor]:
     """Both results of the two functions above: ``(suffix [B, K+1, d, d], cotangents [B, K+1, d])``, fp32.  One pass over
-    ``mats`` in one kernel for d = 17 ... 256; few batch elements, whose chains are cut into chunks, get the finished
-    products applied to ``g``, and other widths the matrices and the chain in a kernel each.
+    ``mats`` in one kernel for d = 2 ... 256 (three launches where few chains are cut into chunks; beyond d = 128 those get the
+    finished products applied to ``g``), and other widths the matrices and the chain in a kernel each.
     ``exact_suffix``: see :func:`suffix_scan_pullbacks`."""
     bsz, count, rank = _validate(mats)
     if g.dim() != 2 or g.shape[0] != bsz or g.shape[1] != rank:
