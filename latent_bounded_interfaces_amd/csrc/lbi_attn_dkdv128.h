@@ -64,7 +64,7 @@ __global__ __launch_bounds__(256) void dkdv_ring_kernel(const T* __restrict__ q,
                                                       const T* __restrict__ v, const T* __restrict__ d_out,
                                                       const float* __restrict__ lse2, const float* __restrict__ delta,
                                                       T* __restrict__ dk, T* __restrict__ dv, int n_bh, int H, int P,
-                                                      int T_len, float scale, int t_rows, int dh) {
+                                                      int T_len, float scale, int t_rows, int dh, int turned) {
     constexpr int KS = DH / 16, ND = DH / 32;
     constexpr int RB = DH * 2;                     // bytes per tile row
     constexpr int CPR = DH / 8;                    // 16-byte chunks per tile row
@@ -77,10 +77,15 @@ __global__ __launch_bounds__(256) void dkdv_ring_kernel(const T* __restrict__ q,
     extern __shared__ __align__(16) char smem[];   // [R][STAGE], then V
 
     const int n_kb = (T_len + 255) / 256;
-    int bh, rem;
-    if (!map_block(n_kb * P, n_bh, bh, rem)) return;
-    const int p = rem / n_kb;
-    const int kb = rem % n_kb;
+    int bh, p, kb;
+    if (turned) {
+        if (!map_long_first(n_kb, P, n_bh, turned, bh, kb, p)) return;
+    } else {
+        int rem;
+        if (!map_block(n_kb * P, n_bh, bh, rem)) return;
+        p = rem / n_kb;
+        kb = rem % n_kb;
+    }
     const int b = bh / H, hh = bh % H;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, m = lane & 31, h = lane >> 5;
     const bool active = kb * 256 + wave * 64 < T_len;
@@ -414,7 +419,7 @@ int launch_dkdv(const T* q, const T* k, const T* v, const T* g, const float* lse
     static_assert(lds_bytes <= 160 * 1024, "LDS budget");
     if (int rc = ensure_dynamic_lds<&dkdv_ring_kernel<T, DH, CAUSAL, EDGE>>(lds_bytes)) return rc;
     hipLaunchKernelGGL((dkdv_ring_kernel<T, DH, CAUSAL, EDGE>), dim3(grid_size(n_kb * P, n_bh)), dim3(256), lds_bytes, stream,
-                       q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, t_rows, dh);
+                       q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, t_rows, dh, turned_of(CAUSAL, grid_size(n_kb * P, n_bh)));
     return LBI_OK;
 }
 

@@ -37,7 +37,7 @@ __global__ __launch_bounds__(256) void dkdv_pair_kernel(const T* __restrict__ q,
                                                       const T* __restrict__ v, const T* __restrict__ d_out,
                                                       const float* __restrict__ lse2, const float* __restrict__ delta,
                                                       T* __restrict__ dk, T* __restrict__ dv, int n_bh, int H, int P,
-                                                      int T_len, float scale, int t_rows, int dh) {
+                                                      int T_len, float scale, int t_rows, int dh, int turned) {
     constexpr int KS = DH / 16, ND = DH / 32;
     constexpr int RB = DH * 2;                       // bytes per tile row
     constexpr int CPR = DH / 8;                      // 16-byte chunks per tile row
@@ -62,10 +62,15 @@ __global__ __launch_bounds__(256) void dkdv_pair_kernel(const T* __restrict__ q,
 
     const int n_kb = (T_len + 127) / 128;
     const int n_pp = (P + 2 * DW - 1) / (2 * DW);
-    int bh, rem;
-    if (!map_block(n_kb * n_pp, n_bh, bh, rem)) return;
-    const int pp = rem / n_kb;
-    const int kb = rem % n_kb;                       // ascending: longest key blocks first
+    int bh, pp, kb;                                  // ascending: longest key blocks first
+    if (turned) {
+        if (!map_long_first(n_kb, n_pp, n_bh, turned, bh, kb, pp)) return;
+    } else {
+        int rem;
+        if (!map_block(n_kb * n_pp, n_bh, bh, rem)) return;
+        pp = rem / n_kb;
+        kb = rem % n_kb;
+    }
     const int b = bh / H, hh = bh % H;
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, m = lane & 31,
               h = lane >> 5;
@@ -468,7 +473,7 @@ int launch_dkdv_pair_as(const T* q, const T* k, const T* v, const T* g, const fl
     static_assert(lds_bytes <= 160 * 1024, "LDS budget");
     if (int rc = ensure_dynamic_lds<&dkdv_pair_kernel<T, DH, CAUSAL, DW, EDGE>>(lds_bytes)) return rc;
     hipLaunchKernelGGL((dkdv_pair_kernel<T, DH, CAUSAL, DW, EDGE>), dim3(grid_size(n_kb * n_pp, n_bh)), dim3(256), lds_bytes,
-                       stream, q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, t_rows, dh);
+                       stream, q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, t_rows, dh, turned_of(CAUSAL, grid_size(n_kb * n_pp, n_bh)));
     return LBI_OK;
 }
 

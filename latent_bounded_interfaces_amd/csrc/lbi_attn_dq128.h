@@ -29,7 +29,7 @@ __global__ __launch_bounds__(256) void dq_ring_kernel(const T* __restrict__ q, c
                                                     const T* __restrict__ v, const T* __restrict__ d_out,
                                                     const float* __restrict__ lse2, const float* __restrict__ o32,
                                                     float* __restrict__ delta, T* __restrict__ dq, int n_bh, int H,
-                                                    int P, int T_len, float scale, int t_rows, int dh) {
+                                                    int P, int T_len, float scale, int t_rows, int dh, int turned) {
     constexpr int KS = DH / 16, ND = DH / 32;
     constexpr int RB = DH * 2;               // bytes per tile row
     constexpr int CPR = DH / 8;              // 16-byte chunks per tile row
@@ -42,10 +42,17 @@ __global__ __launch_bounds__(256) void dq_ring_kernel(const T* __restrict__ q, c
 
     const int n_qb = (T_len + 127) / 128;
     const int n_pb = (P + PB - 1) / PB;
-    int bh, rem;
-    if (!map_block(n_qb * n_pb, n_bh, bh, rem)) return;
-    const int qb = n_qb - 1 - rem / n_pb;  // longest rows first
-    const int p0 = (rem % n_pb) * PB;
+    int bh, qb, p0;  // longest rows first
+    if (turned) {
+        if (!map_long_first(n_qb, n_pb, n_bh, turned, bh, qb, p0)) return;
+    } else {
+        int rem;
+        if (!map_block(n_qb * n_pb, n_bh, bh, rem)) return;
+        qb = rem / n_pb;
+        p0 = rem % n_pb;
+    }
+    qb = n_qb - 1 - qb;
+    p0 *= PB;
     const int b = bh / H, hh = bh % H;
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, m = lane & 31, h = lane >> 5;
     const bool active = qb * 128 + wave * 32 < T_len;
@@ -307,7 +314,7 @@ int launch_dq(const T* q, const T* k, const T* v, const T* g, const float* lse2,
     static_assert(lds_bytes <= 160 * 1024, "LDS budget");
     if (int rc = ensure_dynamic_lds<&dq_ring_kernel<T, DH, PBK, CAUSAL, EDGE>>(lds_bytes)) return rc;
     hipLaunchKernelGGL((dq_ring_kernel<T, DH, PBK, CAUSAL, EDGE>), dim3(grid_size(n_qb * n_pb, n_bh)), dim3(256), lds_bytes,
-                       stream, q, k, v, g, lse2, o32, delta, dq, n_bh, H, P, T_len, scale, t_rows, dh);
+                       stream, q, k, v, g, lse2, o32, delta, dq, n_bh, H, P, T_len, scale, t_rows, dh, turned_of(CAUSAL, grid_size(n_qb * n_pb, n_bh)));
     return LBI_OK;
 }
 

@@ -456,3 +456,30 @@ def test_directions_and_statistics_by_size(shape, basis, dtype, causal, device):
         assert float(diff.abs().max() / b.abs().max()) <= bar, name
     one = attention_input_pullback_basis(q, k, v, d_out[:, basis - 1:].contiguous(), softmax_scale=scale, causal=causal, kernel_mode="hip")
     assert all(torch.equal(a[:, basis - 1:], b) for a, b in zip(got, one))
+
+
+# Launches of one to sixteen workgroups a CU, whose order is by length over all heads, heads that fill the eight XCDs or not
+@pytest.mark.parametrize("shape,basis", [((3, 13, 640, 64), 3), ((2, 20, 1000, 64), 1), ((4, 24, 1024, 64), 1), ((2, 7, 815, 64), 9),
+                                         ((1, 56, 700, 128), 2), ((5, 9, 1100, 96), 1)])
+def test_order_of_workgroups_changes_nothing(shape, basis, device):
+    """The heads of a call, and the same heads in calls of a few workgroups each."""
+    from latent_bounded_interfaces_amd.hip.transformer import attention_input_pullback_basis
+
+    b, h, t, dh = shape
+    gen = torch.Generator(device=device).manual_seed(t)
+    q, k, v = (torch.randn(shape, generator=gen, device=device).bfloat16() for _ in range(3))
+    d_out = torch.randn(b, basis, h, t, dh, generator=gen, device=device).bfloat16()
+
+    def run(rows, heads):
+        return attention_input_pullback_basis(*(x[rows, heads].contiguous() for x in (q, k, v)), d_out[rows, :, heads].contiguous(),
+                                              softmax_scale=dh ** -0.5, causal=True, kernel_mode="hip")
+
+    whole = run(slice(0, b), slice(0, h))
+    for row, head in ((0, 0), (b - 1, h - 1), (b // 2, h // 2), (0, h - 1)):
+        alone = run(slice(row, row + 1), slice(head, head + 1))
+        for a, c in zip(whole, alone):
+            a = a[row:row + 1, :, head:head + 1]
+            if dh == 64:
+                assert torch.equal(a, c)
+            else:  # the statistics' order of summation depends on the heads: results differ by a unit of the storage type
+                assert bool(((a.float() - c.float()).abs() <= 2.0 ** -7 * c.float().abs() + 2.0 ** -8 * float(c.float().abs().max())).all())
