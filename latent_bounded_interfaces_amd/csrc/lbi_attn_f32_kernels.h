@@ -449,8 +449,8 @@ template <int PB, int DW> struct QueryShare {
 // kernel, it saves these products (the whole call above 0.330 ms), but the error of dQ is 1.04 to 1.14 times as large, and
 // with an offset in V up to 1.9 times.
 // Two directions per wave at two waves per SIMD, as many as in dq: four at one wave per SIMD share S but hide less, 0.403
-// against 0.391 ms for the whole causal call (0.616 and 0.631 without the mask).  The matrix cores are at work for 47 % of its time (61
-// and 58 in dq and dkdv, one wave per SIMD).
+// against 0.391 ms for the whole causal call (0.616 and 0.631 without the mask).  The matrix cores are at work for 58 % of its time (47 with
+// both lots of workgroups longest first; 61 and 58 in dq and dkdv, one wave per SIMD).
 template <typename T, int DH, int PB, int DW, bool VEC>
 __global__ __launch_bounds__(NT) void delta_kernel(const T* __restrict__ q, const T* __restrict__ k,
                                                    const T* __restrict__ v, const T* __restrict__ d_out,
