@@ -90,6 +90,26 @@ bool takes(int B, int d, int in_dtype) {
     return blocks <= (d > 64 ? 4 : d > 32 ? 6 : 12) * cus;
 }
 
+// A chain of vectors is its vector's block of a scan (15 of the 16 columns are empty: a step is as long as the fp32 products of one tile
+// column). The kernels for whole 16-byte pieces of rows (fold of a staged copy) and for other rows (a row a lane group) take 0.6 to 3 us a
+// step for d = 16 ... 128; they move more a step, which counts where the chains fill the chip. us, those -> this, fp32 / bf16: B = 64 K = 128
+// d = 32 86 / 74 -> 35 / 39; d = 64 140 / 112 -> 66 / 69; d = 96 265 / 191 -> 142 / 141; d = 128 B = 40 K = 90 295 -> 168, B = 64 K = 128 232 -> 188
+// (bf16). d < 17 (scalar before unless in whole pieces): B = 64 K = 128 d = 12 fp16 550 -> 28. Past the lines: B = 512 K = 20 d = 80 bf16 32 -> 55, d =
+// 101 B = 64 K = 128 150 / 123 -> 219 / 240, d = 112 fp16 B = 16 K = 90 154 -> 156, B = 64 K = 12 d = 47
+// bf16 9.5 -> 10.3.
+bool takes_chain(int B, int K, int d, int in_dtype) {
+    if (d < 2 || d > 128) return false;
+    if (d <= 16) return true;
+    const bool pieces = d % (in_dtype == LBI_F32 ? 4 : 8) == 0;
+    if (!pieces && (d > 48 || (d > 32 && K < 20))) return false;
+    if (in_dtype != LBI_F32 && d > 96 && d != 128) return false;
+    return B <= (d <= 64 ? 4 : 1) * (int64_t)device_compute_units();
+}
+
+int chain(const void* mats, int in_dtype, const void* g, void* cot, int B, int K, int d, hipStream_t stream) {
+    return launch(mats, in_dtype, nullptr, g, cot, B, K, d, 1, false, ScanPlan{0, 0, 0, 0, 0, 0, 0}, stream);
+}
+
 int scan(const void* mats, int in_dtype, void* out, const void* g, void* cot, int B, int K, int d, hipStream_t stream) {
     ScanPlan plan{0, 0, 0, 0, 0, 0, 0};
     const int nt = row_tiles(d, in_dtype);

@@ -88,7 +88,8 @@ __global__ __launch_bounds__(64 * NT, 2) void scan_narrow_kernel(const Tin* __re
     const int phase = plan.phase;
     const int nseg = phase == 1 || phase == 3 ? plan.C - 1 : 1;
     const bool carried = CT > 1 && carry && cot;   // the first column block carries the vector, too
-    const int nbx = NB + (cot && !carried ? 1 : 0);
+    const bool alone = !out;                       // the cotangent chain without the matrices
+    const int nbx = alone ? 1 : NB + (cot && !carried ? 1 : 0);
     const int E = B * nseg;
     const int id = blockIdx.x;
     int e, block;
@@ -101,7 +102,7 @@ __global__ __launch_bounds__(64 * NT, 2) void scan_narrow_kernel(const Tin* __re
         block = id % nbx;
     }
     if (e >= E) return;
-    const bool chain = block == NB;
+    const bool chain = alone || block == NB;
     const int c0 = block * CB;
     const int b = e / nseg, seg = e - b * nseg;
 
@@ -513,7 +514,7 @@ int launch_one(const void* mats, void* out, const void* g, void* cot, int B, int
     static_assert(bytes <= 160 * 1024, "LDS budget");
     if (int rc = ensure_dynamic_lds<&scan_narrow_kernel<Tin, NT, CT, RAGGED, RING>>(bytes)) return rc;
     const int64_t chains = (int64_t)B * (plan.phase == 1 || plan.phase == 3 ? plan.C - 1 : 1);
-    const int64_t blocks = (chains >= 8 ? (chains + 7) / 8 * 8 : chains) * (NB + (cot && !(CT > 1 && carry) ? 1 : 0));
+    const int64_t blocks = (chains >= 8 ? (chains + 7) / 8 * 8 : chains) * (out ? NB + (cot && !(CT > 1 && carry) ? 1 : 0) : 1);
     hipLaunchKernelGGL((scan_narrow_kernel<Tin, NT, CT, RAGGED, RING>), dim3((unsigned)blocks), dim3(64 * NT), bytes, stream,
                        static_cast<const Tin*>(mats), static_cast<float*>(out), static_cast<const float*>(g),
                        static_cast<float*>(cot), B, K, d, (int)carry, plan);

@@ -309,6 +309,36 @@ def test_chunked_scan_takes_nothing_from_the_result_buffer(shape, dtype, device)
     assert _rel_err(results[0].cpu(), truth) <= 1e-5
 
 
+# widths of one to eight row tiles, whole and not, in whole 16-byte pieces or not, either side of the lines of the narrow chain; one matrix
+# and chains that end anywhere in a trip of the rows' ring
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rank,bsz,count", [(2, 1, 1), (7, 9, 13), (15, 3, 40), (16, 300, 2), (17, 8, 3), (33, 2, 19), (33, 2, 21), (48, 65, 6),
+                                            (56, 4, 17), (64, 5, 31), (72, 3, 9), (80, 17, 14), (96, 2, 12), (112, 3, 7), (128, 9, 23), (120, 257, 2),
+                                            (32, 1025, 3)])
+def test_narrow_cotangent_chain(rank, bsz, count, dtype, device):
+    from latent_bounded_interfaces_amd.hip.interface import suffix_scan_cotangents
+
+    gen = torch.Generator(device=device).manual_seed(rank + count)
+    mats = torch.randn(bsz, count, rank, rank, generator=gen, device=device) * (0.01 / rank) ** 0.5
+    mats.diagonal(dim1=-2, dim2=-1).add_(1.0)
+    mats, g = mats.to(dtype), torch.randn(bsz, rank, generator=gen, device=device)
+    got = suffix_scan_cotangents(mats, g)
+    v, want = g.double(), [g.double()]
+    for r in range(count - 1, -1, -1):
+        v = (mats[:, r].double() @ v.unsqueeze(-1)).squeeze(-1)
+        want.append(v)
+    want = torch.stack(want[::-1], dim=1)
+    # each step rounds each of its rank terms and sums once, of terms whose absolute values sum to at most twice the result's norm
+    bound = 2 * count * (rank + 8) * 2.0 ** -24 * float(want.norm(dim=-1).max())
+    assert got.shape == want.shape and float((got.double() - want).abs().max()) <= bound
+    at = count // 2
+    mats[bsz - 1, at, rank - 1, 0] = float("inf")
+    again = suffix_scan_cotangents(mats, g)
+    finite = again.isfinite()
+    assert bool(finite[:bsz - 1].all()) and bool(finite[bsz - 1, at + 1:].all()) and bool(finite[bsz - 1, at, :rank - 1].all())
+    assert not bool(finite[bsz - 1, at, rank - 1]) and torch.equal(again[:bsz - 1], got[:bsz - 1])
+
+
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("rank", [17, 63, 65, 127, 129, 191, 193, 198, 254, 255])
 @pytest.mark.parametrize("bsz,count", [(1, 1), (3, 9)])
