@@ -466,11 +466,13 @@ def _native_layer(block: Any, layer_cache: Any, g_hidden: torch.Tensor | None, g
     if dtype not in _SMALL_PRODUCT_TYPES or attn.d_conv <= 0 or q.dim() != 4:
         return None
     bsz, basis, g_len, dim = g_residual.shape
-    heads, kv_heads, head_dim = attn.n_heads, attn.n_kv_heads, attn.head_dim
     seqlen = q.shape[2]
-    fc1_output, conv = m_cache.fc1_output, attn.conv1d.weight
+    rows, fc1_output = bsz * basis * seqlen, m_cache.fc1_output
+    if rows * dim * fc1_output.shape[-1] > _NATIVE_TIMES * _SMALL_PRODUCT:  # most calls that are not taken leave here
+        return None
+    heads, kv_heads, head_dim = attn.n_heads, attn.n_kv_heads, attn.head_dim
+    conv = attn.conv1d.weight
     hidden, q_width, packed = fc1_output.shape[-1] // 2, heads * head_dim, (heads + 2 * kv_heads) * head_dim
-    rows = bsz * basis * seqlen
     # the products, and the attention that runs without copies (the rule of attention_input_pullback_basis)
     g_rows = rows if g_len == seqlen else bsz * basis
     if not (_small_product_size(rows, dim, 2 * hidden, _ROWS_BY_WEIGHT, _NATIVE_TIMES) and _small_product_size(g_rows, hidden, dim, _ROWS_BY_WEIGHT, _NATIVE_TIMES)
