@@ -248,7 +248,8 @@ __device__ __forceinline__ bool map_block(int per_bh, int n_bh, int& bh, int& re
 // after the other, a CU that holds two workgroups gets two long ones and the next two short ones; here the first `turned` workgroups of
 // an XCD, one for each of its CUs, come shortest first, so that the longest of the second lot joins the shortest of the first.
 // bf16 causal, whole calls, map_block -> this, us: B H=96 T=1024 Dh=64 P=1 164 -> 124, P=16 T=1000 877 -> 829; B H=14 T=815 P=9 110 -> 91; B H=20
-// T=960 P=8 139 -> 110; Dh=128 B H=56 T=2560 P=1 596 -> 525.  The results are the same bits.
+// T=960 P=8 139 -> 110; Dh=128 B H=56 T=2560 P=1 596 -> 525, and with the
+// statistics of 128 queries in this order, too, 480; Dh=96 B H=28 T=3000 P=1 those alone 408 -> 364.  The results are the same bits.
 __device__ __forceinline__ bool map_long_first(int n_tiles, int n_groups, int n_bh, int turned, int& bh, int& tile, int& group) {
     int slot = blockIdx.x >> 3;
     if (slot < turned) slot = turned - 1 - slot;
@@ -276,12 +277,12 @@ template <typename T, int DH, bool CAUSAL, bool EDGE>
 __global__ __launch_bounds__(256) void stats_kernel(const T* __restrict__ q, const T* __restrict__ k,
                                                     const T* __restrict__ v, float* __restrict__ lse2,
                                                     float* __restrict__ o32, int n_bh, int T_len, float scale,
-                                                    int t_rows, int dh) {
+                                                    int t_rows, int dh, int turned) {
     constexpr int KS = DH / 16, ND = DH / 32, TILE_BYTES = 32 * DH * 2;
     extern __shared__ __align__(16) char smem[];  // [2][K tile, V tile]
-    int bh, qb;
+    int bh, qb, group;
     const int n_qb = (T_len + 127) / 128;
-    if (!map_block(n_qb, n_bh, bh, qb)) return;
+    if (turned ? !map_long_first(n_qb, 1, n_bh, turned, bh, qb, group) : !map_block(n_qb, n_bh, bh, qb)) return;
     qb = n_qb - 1 - qb;  // longest rows first
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, m = lane & 31, h = lane >> 5;
     // Waves past the end of the sequence redo the last 32 rows and store nothing; the
@@ -597,7 +598,7 @@ int launch_typed(const T* q, const T* k, const T* v, const T* g, T* dq, T* dk, T
         if (int rc = split_stats()) return rc;
     } else {
         hipLaunchKernelGGL((stats_kernel<T, DH, CAUSAL, EDGE>), dim3(grid_size(n_qb, n_bh)), dim3(256), lds_bytes, stream, q, k,
-                           v, lse2, o32, n_bh, T_len, scale, t_rows, dh);
+                           v, lse2, o32, n_bh, T_len, scale, t_rows, dh, turned_of(CAUSAL, grid_size(n_qb, n_bh)));
     }
     // the dQ kernel runs first: it writes -delta, which the dK/dV kernel reads
     int rc;
