@@ -1319,7 +1319,7 @@ int launch_scan(const void* mats, void* out, const void* g, void* cot, int B, in
 template <typename Tin>
 int launch_cotangent(const void* mats, const void* g, void* out, int B, int K, int d, hipStream_t stream) {
     constexpr int kDtype = std::is_same<Tin, float>::value ? LBI_F32 : std::is_same<Tin, _Float16>::value ? LBI_F16 : LBI_BF16;
-    if (K >= 1 && scan_narrow::takes_chain(B, K, d, kDtype)) return scan_narrow::chain(mats, kDtype, g, out, B, K, d, stream);
+    if (K >= 1 && scan_narrow::takes_chain(mats, B, K, d, kDtype)) return scan_narrow::chain(mats, kDtype, g, out, B, K, d, stream);
     const int dpad = (d + 3) & ~3;
     const size_t lds_bytes = (size_t)2 * dpad * sizeof(float);
     if (lds_bytes > 64 * 1024) return fail(LBI_ERR_UNSUPPORTED, "suffix cotangents: d=%d is too large (max 8192)", d);

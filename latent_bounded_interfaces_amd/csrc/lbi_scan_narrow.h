@@ -24,7 +24,7 @@ bool takes(int B, int d, int in_dtype);
 // The scan of K >= 1 matrices, with the cotangents where `cot` is given.
 int scan(const void* mats, int in_dtype, void* out, const void* g, void* cot, int B, int K, int d, hipStream_t stream);
 // The cotangents alone.
-bool takes_chain(int B, int K, int d, int in_dtype);
+bool takes_chain(const void* mats, int B, int K, int d, int in_dtype);
 int chain(const void* mats, int in_dtype, const void* g, void* cot, int B, int K, int d, hipStream_t stream);
 }  // namespace scan_narrow
 }  // namespace lbi

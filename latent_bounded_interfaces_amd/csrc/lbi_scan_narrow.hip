@@ -96,11 +96,12 @@ bool takes(int B, int d, int in_dtype) {
 // d = 32 86 / 74 -> 35 / 39; d = 64 140 / 112 -> 66 / 69; d = 96 265 / 191 -> 142 / 141; d = 128 B = 40 K = 90 295 -> 168, B = 64 K = 128 232 -> 188
 // (bf16). d < 17 (scalar before unless in whole pieces): B = 64 K = 128 d = 12 fp16 550 -> 28. Past the lines: B = 512 K = 20 d = 80 bf16 32 -> 55, d =
 // 101 B = 64 K = 128 150 / 123 -> 219 / 240, d = 112 fp16 B = 16 K = 90 154 -> 156, B = 64 K = 12 d = 47
-// bf16 9.5 -> 10.3.
-bool takes_chain(int B, int K, int d, int in_dtype) {
+// bf16 9.5 -> 10.3; 16-bit matrices that start off the 4-byte grid (their rows would not come through LDS here), bf16 B = 16 K = 20, d = 64 19.8 ->
+// 25.3, d = 128 42.6 -> 82.7.
+bool takes_chain(const void* mats, int B, int K, int d, int in_dtype) {
     if (d < 2 || d > 128) return false;
     if (d <= 16) return true;
-    const bool pieces = d % (in_dtype == LBI_F32 ? 4 : 8) == 0;
+    const bool pieces = d % (in_dtype == LBI_F32 ? 4 : 8) == 0 && reinterpret_cast<uintptr_t>(mats) % 4 == 0;
     if (!pieces && (d > 48 || (d > 32 && K < 20))) return false;
     if (in_dtype != LBI_F32 && d > 96 && d != 128) return false;
     return B <= (d <= 64 ? 4 : 1) * (int64_t)device_compute_units();

@@ -528,11 +528,11 @@ int launch_width(const void* mats, void* out, const void* g, void* cot, int B, i
                  ScanPlan plan, hipStream_t stream) {
     auto run = [&](auto ct) {
         constexpr int CT = decltype(ct)::value, RING = ring_steps(NT, CT, sizeof(Tin));
+        // transfers into LDS move whole 4-byte words: 16-bit rows of an odd width or start come straight into registers
+        if (sizeof(Tin) == 2 && (d % 2 != 0 || reinterpret_cast<uintptr_t>(mats) % 4 != 0))
+            return launch_one<Tin, NT, CT, true, 0>(mats, out, g, cot, B, K, d, carry, plan, stream);
         if (d == 16 * NT) return launch_one<Tin, NT, CT, false, RING>(mats, out, g, cot, B, K, d, carry, plan, stream);
-        // transfers into LDS move whole 4-byte words
-        if (sizeof(Tin) == 4 || (d % 2 == 0 && reinterpret_cast<uintptr_t>(mats) % 4 == 0))
-            return launch_one<Tin, NT, CT, true, RING>(mats, out, g, cot, B, K, d, carry, plan, stream);
-        return launch_one<Tin, NT, CT, true, 0>(mats, out, g, cot, B, K, d, carry, plan, stream);
+        return launch_one<Tin, NT, CT, true, RING>(mats, out, g, cot, B, K, d, carry, plan, stream);
     };
     if constexpr (NT > 1)
         if (tiles == 2) return run(std::integral_constant<int, 2>{});

@@ -766,6 +766,26 @@ def test_bf16_storage_at_the_benchmark_shape_in_both_precisions(kind, device):
         del only, fused, cot
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rank", [16, 32, 48, 64, 80, 96, 128])
+@pytest.mark.parametrize("bsz,count", [(1, 2), (3, 25)])
+def test_cotangent_chain_off_the_grid(rank, bsz, count, dtype, device):
+    """Matrices that start one element behind the allocation's grid (16-bit ones off the 4-byte words that transfers into LDS move)."""
+    from latent_bounded_interfaces_amd.hip.interface import suffix_scan_cotangents
+
+    mats, g = oscan.make_scan_inputs(bsz, count, rank, kind="near_identity", seed=rank + count)
+    mats, g = mats.to(dtype).to(device), g.to(device)
+    off = torch.empty(mats.numel() + 1, dtype=dtype, device=device)[1:].view(mats.shape).copy_(mats)
+    g_off = torch.empty(g.numel() + 1, device=device)[1:].view(g.shape).copy_(g)
+    assert off.data_ptr() % 16 == mats.element_size() and off.is_contiguous()
+    got, again = suffix_scan_cotangents(off, g_off), suffix_scan_cotangents(mats, g)
+    want = oscan.suffix_cotangents_sequential(mats.cpu().double(), g.cpu().double())
+    # the bound of the test above
+    bound = 2 * count * (rank + 8) * 2.0 ** -24 * float(want.norm(dim=-1).max())
+    for one in (got, again):
+        assert float((one.cpu().double() - want).abs().max()) <= bound
+
+
 # Widths up to 128 in 16 x 16 tiles: each number of row tiles with its last tile full, one short and one over, and the forms a batch
 # takes: one block of 16 columns a workgroup, blocks of 32 with the vector in a workgroup of its own and beside the first block,
 # chunks on either, one matrix.  Each product sums d terms in blocks of 32 (K of them one after the other): K (d / 32 + 32) roundings
