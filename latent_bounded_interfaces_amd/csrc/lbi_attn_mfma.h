@@ -342,10 +342,11 @@ __global__ __launch_bounds__(256) void stats_kernel(const T* __restrict__ q, con
             const float m_new = fmaxf(m_run, tmax);
             const bool grow = (m_run == -INFINITY) ? (m_new != -INFINITY) : (m_new - m_run > 8.0f);
             const float m_use = grow ? m_new : m_run;
+            const float base = m_use == -INFINITY ? 0.0f : m_use;  // scores of -inf only so far: their terms are 0, NaN stays NaN
             float lsum = 0.0f;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const float pr = (m_use == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(s[r] - m_use);
+                const float pr = __builtin_amdgcn_exp2f(s[r] - base);
                 s[r] = pr;
                 lsum += pr;
             }
@@ -468,10 +469,11 @@ __global__ __launch_bounds__(256) void stats_split_kernel(const T* __restrict__ 
         const float m_new = fmaxf(m_run, tmax);
         const bool grow = (m_run == -INFINITY) ? (m_new != -INFINITY) : (m_new - m_run > 8.0f);
         const float m_use = grow ? m_new : m_run;
+        const float base = m_use == -INFINITY ? 0.0f : m_use;
         float lsum = 0.0f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const float pr = (m_use == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(s[r] - m_use);
+            const float pr = __builtin_amdgcn_exp2f(s[r] - base);
             s[r] = pr;
             lsum += pr;
         }
@@ -505,7 +507,7 @@ __global__ __launch_bounds__(256) void stats_split_kernel(const T* __restrict__ 
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
         const float mw = row_max[w * 32 + m];
-        total += mw == -INFINITY ? 0.0f * row_sum[w * 32 + m] : row_sum[w * 32 + m] * __builtin_amdgcn_exp2f(mw - top);
+        total += mw == -INFINITY ? row_sum[w * 32 + m] : row_sum[w * 32 + m] * __builtin_amdgcn_exp2f(mw - top);
     }
     const float part = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - top);
     const float inv = part / total;

@@ -458,6 +458,25 @@ def test_directions_and_statistics_by_size(shape, basis, dtype, causal, device):
     assert all(torch.equal(a[:, basis - 1:], b) for a, b in zip(got, one))
 
 
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("shape", [(1, 2, 320, 64), (1, 2, 384, 128), (1, 70, 320, 128)])
+@pytest.mark.parametrize("block", [0, 2, 9])
+def test_keys_that_are_nan_show(block, shape, dtype, causal, device):
+    """A whole tile of 32 keys that are NaN, wherever it lies among the tiles of a wave: every query that sees one of them has no statistics, and
+    with it neither its dQ nor a dK or dV that it takes part in is finite."""
+    from latent_bounded_interfaces_amd.hip.transformer import attention_input_pullback_basis
+
+    inputs = oattn.make_attention_inputs(*shape, 2, dtype=dtype, seed=block)
+    q, k, v, d_out = (t.to(device) for t in inputs)
+    k[:, 0, 32 * block:32 * block + 32] = float("nan")
+    dq, dk, dv = attention_input_pullback_basis(q, k, v, d_out, softmax_scale=shape[-1] ** -0.5, causal=causal, kernel_mode="hip")
+    first = 32 * block if causal else 0
+    assert bool(dq[:, :, 0, first:].isnan().all())
+    assert bool(dk[:, :, 0].isnan().all()) and bool(dv[:, :, 0].isnan().all())
+    assert all(bool(t[:, :, 1:].isfinite().all()) for t in (dq, dk, dv))
+
+
 # Launches of one to sixteen workgroups a CU, whose order is by length over all heads, heads that fill the eight XCDs or not
 @pytest.mark.parametrize("shape,basis", [((3, 13, 640, 64), 3), ((2, 20, 1000, 64), 1), ((4, 24, 1024, 64), 1), ((2, 7, 815, 64), 9),
                                          ((1, 56, 700, 128), 2), ((5, 9, 1100, 96), 1)])
