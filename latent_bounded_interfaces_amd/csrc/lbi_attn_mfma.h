@@ -451,6 +451,8 @@ __global__ __launch_bounds__(256) void stats_split_kernel(const T* __restrict__ 
             *reinterpret_cast<u32x4*>(kt + tile_off<DH>(r, c)) = kr[u];
             *reinterpret_cast<u32x4*>(vt + tile_off<DH>(r, c)) = vr[u];
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // the tiles are the wave's own: LDS runs in order
+        __builtin_amdgcn_wave_barrier();
         fetch(it + 4 < n_it ? it + 4 : it);  // the last trip re-reads its tile
         f32x16 s = zero16();
 #pragma unroll
@@ -495,6 +497,8 @@ __global__ __launch_bounds__(256) void stats_split_kernel(const T* __restrict__ 
             for (int nd = 0; nd < ND; ++nd)
                 o_t[nd] = Mma<T>::mma(frag_tr<DH>(vt, lane, 16 * kk, 32 * nd), pb, o_t[nd]);
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // read, before the next tile is written over them
+        __builtin_amdgcn_wave_barrier();
     }
     if (h == 0) {
         row_max[wave * 32 + m] = m_run;
