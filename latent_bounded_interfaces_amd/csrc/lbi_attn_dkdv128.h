@@ -419,7 +419,7 @@ int launch_dkdv(const T* q, const T* k, const T* v, const T* g, const float* lse
     static_assert(lds_bytes <= 160 * 1024, "LDS budget");
     if (int rc = ensure_dynamic_lds<&dkdv_ring_kernel<T, DH, CAUSAL, EDGE>>(lds_bytes)) return rc;
     hipLaunchKernelGGL((dkdv_ring_kernel<T, DH, CAUSAL, EDGE>), dim3(grid_size(n_kb * P, n_bh)), dim3(256), lds_bytes, stream,
-                       q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, t_rows, dh, turned_of(CAUSAL, grid_size(n_kb * P, n_bh)));
+                       q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, t_rows, dh, turned_of(CAUSAL, grid_size(n_kb * P, n_bh), most_dkdv(n_kb)));
     return LBI_OK;
 }
 

@@ -473,7 +473,7 @@ int launch_dkdv_pair_as(const T* q, const T* k, const T* v, const T* g, const fl
     static_assert(lds_bytes <= 160 * 1024, "LDS budget");
     if (int rc = ensure_dynamic_lds<&dkdv_pair_kernel<T, DH, CAUSAL, DW, EDGE>>(lds_bytes)) return rc;
     hipLaunchKernelGGL((dkdv_pair_kernel<T, DH, CAUSAL, DW, EDGE>), dim3(grid_size(n_kb * n_pp, n_bh)), dim3(256), lds_bytes,
-                       stream, q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, t_rows, dh, turned_of(CAUSAL, grid_size(n_kb * n_pp, n_bh)));
+                       stream, q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, t_rows, dh, turned_of(CAUSAL, grid_size(n_kb * n_pp, n_bh), most_dkdv(n_kb)));
     return LBI_OK;
 }
 

@@ -314,7 +314,7 @@ int launch_dq(const T* q, const T* k, const T* v, const T* g, const float* lse2,
     static_assert(lds_bytes <= 160 * 1024, "LDS budget");
     if (int rc = ensure_dynamic_lds<&dq_ring_kernel<T, DH, PBK, CAUSAL, EDGE>>(lds_bytes)) return rc;
     hipLaunchKernelGGL((dq_ring_kernel<T, DH, PBK, CAUSAL, EDGE>), dim3(grid_size(n_qb * n_pb, n_bh)), dim3(256), lds_bytes,
-                       stream, q, k, v, g, lse2, o32, delta, dq, n_bh, H, P, T_len, scale, t_rows, dh, turned_of(CAUSAL, grid_size(n_qb * n_pb, n_bh)));
+                       stream, q, k, v, g, lse2, o32, delta, dq, n_bh, H, P, T_len, scale, t_rows, dh, turned_of(CAUSAL, grid_size(n_qb * n_pb, n_bh), most_dq(DH, n_qb)));
     return LBI_OK;
 }
 

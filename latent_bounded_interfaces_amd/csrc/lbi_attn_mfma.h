@@ -260,13 +260,20 @@ __device__ __forceinline__ bool map_long_first(int n_tiles, int n_groups, int n_
     group = rest % n_groups;
     return bh < n_bh;
 }
-// `turned` of a launch of `count` workgroups; 0: map_block, where none shares a CU and where there are so many that they level out by themselves
-// and the workgroups of a head had better run together (40 random calls, geometric mean of the time against map_block with this from one to 2 / 4 /
-// 8 / 16 / any number of workgroups a CU: 0.960 / 0.937 / 0.930 / 0.927 / 0.929; B H=96 T=1000 P=16, 12 a CU in dK/dV, 829 and, all so, 852 us).
-inline int turned_of(bool causal, unsigned count) {
+// `turned` of a launch of `count` workgroups; 0: map_block, where none shares a CU and where there are more than `most` a CU, so that they level
+// out by themselves and the workgroups of a head had better run together (40 random calls, geometric mean of the time against map_block with
+// this from one to 2 / 4 / 8 / 16 / any number of workgroups a CU: 0.960 / 0.937 / 0.930 / 0.927 / 0.929).
+inline int turned_of(bool causal, unsigned count, unsigned most) {
     const unsigned cus = device_compute_units();
-    return causal && count > cus && count <= 16 * cus ? (int)(cus / 8) : 0;
+    return causal && count > cus && count <= most * cus ? (int)(cus / 8) : 0;
 }
+// `most` of the dK/dV and the dQ kernels by the tiles of a head.  map_block deals these to the CUs in turn: an even number of them brings a CU
+// the same few lengths all the time, an odd number all of them, and only the last workgroups differ.  Those kernels' part of 520
+// random calls (whole calls, geometric mean against map_block), 4 ... 6, 6 ... 8 and 8 ... 12 workgroups a CU: dK/dV head dim 64, 4 tiles 0.89
+// 0.86 0.89, 3 tiles 1.03 1.03 1.04; 128, 2 tiles 0.95 0.94 -, 3 1.00 1.03 1.04, 5 1.00 1.01 1.02, 8 0.93 0.95 0.95.  dQ, whose workgroups of
+// one tile lie together, at 128: 3 tiles 1.02 1.03 1.01, 4 0.96 - -, 5 1.00 1.01 1.02, 8 0.97 0.98 0.98; at 64 0.95 ... 1.00.
+inline unsigned most_dkdv(int n_tiles) { return n_tiles % 2 == 0 || n_tiles > 8 ? 16 : 4; }
+inline unsigned most_dq(int dh, int n_tiles) { return dh == 64 || n_tiles % 4 == 0 || n_tiles > 8 ? 16 : n_tiles < 4 ? 2 : 4; }
 inline unsigned grid_size(int per_bh, int n_bh) { return (unsigned)(((n_bh + 7) / 8) * 8 * per_bh); }
 
 // ---------------------------------------------------------------------------------------
@@ -595,7 +602,7 @@ int launch_typed(const T* q, const T* k, const T* v, const T* g, T* dq, T* dk, T
         constexpr size_t bytes = 8 * 32 * DH * 2 + 2 * 4 * 32 * 4;
         if (int rc = ensure_dynamic_lds<&stats_split_kernel<T, DH, CAUSAL, EDGE>>(bytes)) return rc;
         hipLaunchKernelGGL((stats_split_kernel<T, DH, CAUSAL, EDGE>), dim3(grid_size(T_len / 32, n_bh)), dim3(256), bytes, stream, q, k,
-                           v, lse2, o32, n_bh, T_len, scale, t_rows, dh, turned_of(CAUSAL, grid_size(T_len / 32, n_bh)));
+                           v, lse2, o32, n_bh, T_len, scale, t_rows, dh, turned_of(CAUSAL, grid_size(T_len / 32, n_bh), 16));
         return LBI_OK;
     };
     if constexpr (DH == 64) {
@@ -604,7 +611,7 @@ int launch_typed(const T* q, const T* k, const T* v, const T* g, T* dq, T* dk, T
         if (int rc = split_stats()) return rc;
     } else {
         hipLaunchKernelGGL((stats_kernel<T, DH, CAUSAL, EDGE>), dim3(grid_size(n_qb, n_bh)), dim3(256), lds_bytes, stream, q, k,
-                           v, lse2, o32, n_bh, T_len, scale, t_rows, dh, turned_of(CAUSAL, grid_size(n_qb, n_bh)));
+                           v, lse2, o32, n_bh, T_len, scale, t_rows, dh, turned_of(CAUSAL, grid_size(n_qb, n_bh), 16));
     }
     // the dQ kernel runs first: it writes -delta, which the dK/dV kernel reads
     int rc;
