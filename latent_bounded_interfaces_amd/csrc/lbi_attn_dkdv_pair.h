@@ -478,7 +478,7 @@ int launch_dkdv_pair_as(const T* q, const T* k, const T* v, const T* g, const fl
 }
 
 // Head dim 64 with three directions or more: two directions per wave (four per workgroup), unless workgroups of two still find a CU each, or
-// five or six directions would leave slots idle.  bf16 causal calls, us, one / two per wave: T=1024, B H = 12, P = 4 107 / 121; 24, 4 124 /
+// idle slots take what that gives (`fours`).  bf16 causal calls, us, one / two per wave: T=1024, B H = 12, P = 4 107 / 121; 24, 4 124 /
 // 123; 6, 6 136 / 149; 64, 6 331 / 342; 24, 9 236 / 228; 64, 16 653 / 583.
 template <typename T, int DH, bool CAUSAL, bool EDGE>
 int launch_dkdv_pair(const T* q, const T* k, const T* v, const T* g, const float* lse2, const float* delta, T* dk,
@@ -486,7 +486,7 @@ int launch_dkdv_pair(const T* q, const T* k, const T* v, const T* g, const float
                      hipStream_t stream) {
     if constexpr (DH == 64) {
         const int64_t workgroups = (int64_t)((T_len + 127) / 128) * n_bh * ((P + 1) / 2);
-        if (P >= 3 && P != 5 && P != 6 && 10 * workgroups > 9 * (int64_t)device_compute_units())
+        if (fours(P) && 10 * workgroups > 9 * (int64_t)device_compute_units())
             return launch_dkdv_pair_as<T, DH, CAUSAL, 2, EDGE>(q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, t_rows, dh, stream);
     }
     return launch_dkdv_pair_as<T, DH, CAUSAL, 1, EDGE>(q, k, v, g, lse2, delta, dk, dv, n_bh, H, P, T_len, scale, t_rows, dh, stream);

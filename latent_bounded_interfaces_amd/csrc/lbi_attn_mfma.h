@@ -572,6 +572,11 @@ int launch_dq(const T* q, const T* k, const T* v, const T* g, const float* lse2,
                int n_bh, int H, int P, int T_len, float scale, int t_rows, int dh,
                 hipStream_t stream);
 
+// Whether P directions are better off in fours than in twos: what four of them share makes one of them 5/6 as long, idle slots included.  (dQ at
+// head dim 128, whole calls, us, fours / twos: B H=64 T=369 P=21 376 / 395; 94, 588, 17 900 / 942; 45, 517, 13 350 / 363; 206, 396, 14 1220 / 1257; dK/dV at 64,
+// twos and fours per workgroup: T=1024 B H=6 P=6 149 / 136, 24, 9 228 / 236.)
+inline bool fours(int P) { return 5 * 4 * ((P + 3) / 4) <= 6 * 2 * ((P + 1) / 2); }
+
 // Directions per wave of the dQ kernel, `blocks` 128-query blocks for each.  More of them share an S tile, fewer are shorter steps for
 // more workgroups: one direction while that leaves CUs free, two until the largest number fills the chip several times over without
 // idle slots.  The results are the same bits.  bf16 causal calls, us, 1 / 2 / 4 / 8 directions: Dh=64 T=1024, B H = 6, P = 6 104 / 109 /
@@ -584,7 +589,7 @@ inline int dq_directions(int dh, int64_t blocks, int P, int64_t cus) {
         return P % 8 == 0 || P % 8 == 7 ? (blocks * ((P + 7) / 8) > 6 * cus ? 8 : 2) : 2;
     }
     if (4 * blocks * P <= 3 * cus) return 1;
-    return P % 4 == 0 || P % 4 == 3 ? (4 * blocks * ((P + 3) / 4) >= 3 * cus ? 4 : 2) : 2;
+    return fours(P) && 4 * blocks * ((P + 3) / 4) >= 3 * cus ? 4 : 2;
 }
 
 // T_len: the length in tiles (a multiple of 64); t_rows, dh: rows and head dim of the tensors (EDGE).
