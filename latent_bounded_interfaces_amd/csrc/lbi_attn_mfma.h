@@ -272,7 +272,7 @@ inline int turned_of(bool causal, unsigned count, unsigned most) {
 // random calls (whole calls, geometric mean against map_block), 4 ... 6, 6 ... 8 and 8 ... 12 workgroups a CU: dK/dV head dim 64, 4 tiles 0.89
 // 0.86 0.89, 3 tiles 1.03 1.03 1.04; 128, 2 tiles 0.95 0.94 -, 3 1.00 1.03 1.04, 5 1.00 1.01 1.02, 8 0.93 0.95 0.95.  dQ, whose workgroups of
 // one tile lie together, at 128: 3 tiles 1.02 1.03 1.01, 4 0.96 - -, 5 1.00 1.01 1.02, 8 0.97 0.98 0.98; at 64 0.95 ... 1.00.
-inline unsigned most_dkdv(int n_tiles) { return n_tiles % 2 == 0 || n_tiles > 8 ? 16 : 4; }
+inline unsigned most_dkdv(int n_tiles) { return n_tiles % 2 == 0 || n_tiles > 8 ? 16 : n_tiles < 4 ? 4 : 6; }
 inline unsigned most_dq(int dh, int n_tiles) { return dh == 64 || n_tiles % 4 == 0 || n_tiles > 8 ? 16 : n_tiles < 4 ? 2 : 4; }
 inline unsigned grid_size(int per_bh, int n_bh) { return (unsigned)(((n_bh + 7) / 8) * 8 * per_bh); }
 
