@@ -1273,7 +1273,7 @@ int launch_scan(const void* mats, void* out, const void* g, void* cot, int B, in
     // Widths up to 128: fp32 matrix cores (a step is a chain of dependent instructions here, which the splitting of the planes only
     // lengthens: B=64 K=128 d=32 / 64 / 96 / 128 took 1.5 / 1.3 / 1.15 / 1.05 times as long on planes as in 32 x 32 tiles).
     constexpr int kDtype = std::is_same<Tin, float>::value ? LBI_F32 : std::is_same<Tin, _Float16>::value ? LBI_F16 : LBI_BF16;
-    if (scan_narrow::takes(B, d, kDtype)) return scan_narrow::scan(mats, kDtype, out, g, cot, B, K, d, stream);
+    if (scan_narrow::takes(mats, B, K, d, kDtype)) return scan_narrow::scan(mats, kDtype, out, g, cot, B, K, d, stream);
     if (d > 16 && d <= 128) {
         auto run = [&](auto width, auto wide) {
             constexpr int D = decltype(width)::value, WIDE = decltype(wide)::value;

@@ -19,8 +19,8 @@ inline int row_tiles(int d, int dtype) {
     const int nt = (d + 15) / 16;
     return dtype != LBI_F32 && nt > 4 ? nt + nt % 2 : nt;
 }
-// Whether a scan of B chains of this width runs here.
-bool takes(int B, int d, int in_dtype);
+// Whether a scan of B chains of K matrices runs here.
+bool takes(const void* mats, int B, int K, int d, int in_dtype);
 // The scan of K >= 1 matrices, with the cotangents where `cot` is given.
 int scan(const void* mats, int in_dtype, void* out, const void* g, void* cot, int B, int K, int d, hipStream_t stream);
 // The cotangents alone.

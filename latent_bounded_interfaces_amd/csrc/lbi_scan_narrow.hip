@@ -58,7 +58,11 @@ Chunks chunks(int B, int K, int nt, int cus) {
         const int L = forced < 2 ? 2 : forced;
         return {(K + L) / L >= 4 ? L : 0, 1};
     }
-    float best = 5.0f + (float)(K - 1) * step_us(nt, 1, dealt(B) * nt, cus);
+    // Beyond 64 columns a plain chain whose blocks of 16 don't find a CU each runs on 32, and chunks have never been the better form then.  (13 widths,
+    // B = 8 ... 768, K = 13 ... 100: 253 calls 1.18 times as long in chunks.)  The estimate is good to a tenth: chunks are taken for less than that only
+    // where they save 8 %.
+    if (nt > 4 && dealt(B) * nt > cus) return {0, 1};
+    float best = 0.92f * (5.0f + (float)(K - 1) * step_us(nt, 1, dealt(B) * nt, cus));
     Chunks form{0, 1};
     for (int L = 2; (K + L) / L >= 4; L += 1 + L / 16) {
         const int C = (K + L) / L;
@@ -76,18 +80,33 @@ Chunks chunks(int B, int K, int nt, int cus) {
     return form;
 }
 
-bool takes(int B, int d, int in_dtype) {
+// 16-bit rows that are no whole 4-byte words come straight into registers at all widths.
+static bool in_words(const void* mats, int d, int in_dtype) {
+    return in_dtype == LBI_F32 || (d % 2 == 0 && reinterpret_cast<uintptr_t>(mats) % 4 == 0);
+}
+
+// Where the chip has several workgroups for every CU to run one after the other, a step's length no longer counts, and 32 x 32
+// tiles move half the operands.  The matrices are the same bits with the cotangents and without, so it is one rule for both, and its lines lie where
+// the two together begin to take longer here (15492 calls: 14 widths, three types, B = 8 ... 2048, K = 2 ... 100, inputs from memory
+// and from the caches).  us, 32 x 32 tiles -> here, matrices / with the cotangents:
+//  * up to 32 columns several small workgroups share a CU: fp32 d = 32 B = 1024 K = 50 150 -> 150 / 173 -> 169, B = 1536 K = 24 118 -> 145 / 133 -> 154.
+//  * 33 ... 48, and 49 ... 64 where 16-bit rows come through LDS: bf16 d = 64 B = 768 K = 24 136 -> 98 / 149 -> 120.  In registers at most one
+//    workgroup of 32 columns a CU twice over: fp32 d = 49 B = 256 K = 24 46 -> 35 / 57 -> 46, B = 288 47 -> 52 / 57 -> 66.
+//  * beyond 64 columns while a step's blocks of 32 find a CU each: fp32 d = 81 B = 80 K = 24 56 -> 57 / 70 -> 63, B = 96 58 -> 71 / 72 -> 83; d = 128 B = 64
+//    K = 100 319 -> 293 / 350 -> 315, B = 72 323 -> 353 / 352 -> 381; three quarters of them for 16-bit rows of 97 ... 127.  Odd 16-bit widths, whose
+//    rows come straight into registers, take them in chains of a dozen matrices and more: bf16 d = 65 B = 64 K = 8 20 -> 24 / 28 -> 27.
+bool takes(const void* mats, int B, int K, int d, int in_dtype) {
     if (d < 2 || d > 128) return false;
     if (d <= 16 || scan_forced_chunk() > 0) return true;   // the others take whole chains of more than 16 columns
-    const int64_t blocks = (int64_t)B * ((d + 31) / 32);
-    if (2 * blocks <= kLeastCus) return true;              // on any device: small calls do without asking the runtime
-    // Where the chip has several workgroups for every CU to run one after the other, a step's length no longer counts, and 32 x 32
-    // tiles move half the operands.  fp32, matrices, us, those -> these: d = 128 B = 64 K = 128 430 -> 380, B = 128 K = 40 227 -> 238;
-    // d = 96 B = 128 K = 40 160 -> 157, B = 512 K = 20 233 -> 265; d = 64 B = 512 K = 64 349 -> 255, B = 1024 K = 32 231 -> 262; d = 32
-    // B = 1024 K = 64 126 -> 118, B = 4096 K = 32 234 -> 228 with 240 for 232 with the cotangents.
+    const int nt = row_tiles(d, in_dtype);
+    if (dealt(B) * nt <= kLeastCus) return true;           // on any device: small calls do without asking the runtime
     const int64_t cus = device_compute_units();
-    if (d > 96) return 4 * blocks <= (in_dtype != LBI_F32 && d != 128 ? 3 : 5) * cus;
-    return blocks <= (d > 64 ? 4 : d > 32 ? 6 : 12) * cus;
+    const bool words = in_words(mats, d, in_dtype), half = in_dtype != LBI_F32, whole = d == 16 * nt;
+    if (nt <= 2) return B <= (whole || K >= 24 ? 4 : 2) * cus;
+    if (nt == 3 || (nt == 4 && half && words)) return B <= (K < (whole ? 4 : 8) ? 1 : 3) * cus;
+    if (nt == 4) return 2 * B <= (whole || K >= 8 ? 2 : 1) * cus;
+    if (!words && K < 12) return dealt(B) * nt <= cus;
+    return 4 * dealt(B) * ((nt + 1) / 2) <= (half && nt == 8 && !whole ? 3 : 4) * cus;
 }
 
 // A chain of vectors is its vector's block of a scan (15 of the 16 columns are empty: a step is as long as the fp32 products of one tile
