@@ -235,8 +235,9 @@ __global__ __launch_bounds__(64 * NT, 2) void scan_narrow_kernel(const Tin* __re
 #pragma unroll
             for (int u = 0; u < AHEAD; ++u) {
                 const int rr = r_top - u;
+                if (rr < r_lo) break;   // (rows that nothing uses: bf16 B = 32 K = 2, d = 65 9.6 -> 7.2 us without, d = 113 11.2 -> 8.2)
 #pragma unroll
-                for (int j = 0; j < NT; ++j) ring[u][j] = load_tile(a_base + (size_t)(rr > r_lo ? rr : r_lo) * stride, j);
+                for (int j = 0; j < NT; ++j) ring[u][j] = load_tile(a_base + (size_t)rr * stride, j);
                 __builtin_amdgcn_sched_barrier(0);   // in the order in which they are used
             }
         }
