@@ -1273,7 +1273,15 @@ int launch_scan(const void* mats, void* out, const void* g, void* cot, int B, in
     // Widths up to 128: fp32 matrix cores (a step is a chain of dependent instructions here, which the splitting of the planes only
     // lengthens: B=64 K=128 d=32 / 64 / 96 / 128 took 1.5 / 1.3 / 1.15 / 1.05 times as long on planes as in 32 x 32 tiles).
     constexpr int kDtype = std::is_same<Tin, float>::value ? LBI_F32 : std::is_same<Tin, _Float16>::value ? LBI_F16 : LBI_BF16;
-    if (scan_narrow::takes(mats, B, K, d, kDtype)) return scan_narrow::scan(mats, kDtype, out, g, cot, B, K, d, stream);
+    if (scan_narrow::takes(mats, B, K, d, kDtype)) {
+        // a chain that is better off on the scalar kernel is so beside the matrices, too, where it takes longer than a launch (d = 2, as part of the
+        // scan -> behind it, us: B = 1048576 K = 1 896 -> 630, B = 65536 K = 2 83 -> 59; B = 8192 K = 1 9.6 -> 11.8)
+        if (cot && d <= 16 && !scan_narrow::takes_chain(mats, B, K, d, kDtype) && B >= 64 * (int64_t)device_compute_units()) {
+            if (int rc = launch_cotangent<Tin>(mats, g, cot, B, K, d, stream)) return rc;
+            cot = nullptr;
+        }
+        return scan_narrow::scan(mats, kDtype, out, cot ? g : nullptr, cot, B, K, d, stream);
+    }
     if (d > 16 && d <= 128) {
         auto run = [&](auto width, auto wide) {
             constexpr int D = decltype(width)::value, WIDE = decltype(wide)::value;

@@ -786,6 +786,32 @@ def test_cotangent_chain_off_the_grid(rank, bsz, count, dtype, device):
         assert float((one.cpu().double() - want).abs().max()) <= bound
 
 
+# a few small matrices each, either side of the lines between the narrow scan's chain and the scalar kernel's, alone and behind the matrices
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rank,bsz,count", [(2, 4096, 2), (2, 4097, 4), (2, 4097, 5), (3, 16384, 2), (4, 16385, 1), (4, 4099, 2)])
+def test_many_chains_of_a_few_small_matrices(rank, bsz, count, dtype, device):
+    from latent_bounded_interfaces_amd.hip.interface import (suffix_scan_cotangents, suffix_scan_pullbacks,
+                                                             suffix_scan_pullbacks_and_cotangents)
+
+    gen = torch.Generator(device=device).manual_seed(bsz + count)
+    mats = (torch.randn(bsz, count, rank, rank, generator=gen, device=device) * rank ** -0.5).to(dtype)
+    g = torch.randn(bsz, rank, generator=gen, device=device)
+    out, cot = suffix_scan_pullbacks_and_cotangents(mats, g)
+    assert torch.equal(out, suffix_scan_pullbacks(mats))
+    eye = torch.eye(rank, device=device, dtype=torch.float64).expand(bsz, rank, rank)
+    truth, want, terms = eye, g.double(), g.double().abs()
+    alone = suffix_scan_cotangents(mats, g)
+    for r in range(count - 1, -1, -1):
+        left = mats[:, r].double()
+        truth, want = left @ truth, (left @ want.unsqueeze(-1)).squeeze(-1)
+        terms = (left.abs() @ terms.unsqueeze(-1)).squeeze(-1)
+        # rank products and sums a step, of terms whose absolute values sum to `terms`
+        bound = (count - r) * (rank + 1) * 2.0 ** -24 * terms
+        assert bool(((cot[:, r].double() - want).abs() <= bound).all()) and bool(((alone[:, r].double() - want).abs() <= bound).all())
+        assert float((out[:, r].double() - truth).abs().max() / truth.abs().max()) <= 1e-6
+    assert torch.equal(cot[:, count], g) and torch.equal(alone[:, count], g)
+
+
 # Widths up to 128 in 16 x 16 tiles: each number of row tiles with its last tile full, one short and one over, and the forms a batch
 # takes: one block of 16 columns a workgroup, blocks of 32 with the vector in a workgroup of its own and beside the first block,
 # chunks on either, one matrix.  Each product sums d terms in blocks of 32 (K of them one after the other): K (d / 32 + 32) roundings
