@@ -116,15 +116,20 @@ bool takes(const void* mats, int B, int K, int d, int in_dtype) {
 // (bf16).  d < 17 (scalar before unless in whole pieces): B = 64 K = 128 d = 12 fp16 550 -> 28; fp32 B = 4096 K = 64 d = 16 310 -> 64; but a chain of
 // one to four matrices of two to four columns is less than a workgroup's start here: fp32 B = 65536 d = 2 K = 1 17 -> 30, K = 4 45 -> 49, K = 6 69 -> 59; d = 3
 // K = 2 39 -> 44, K = 3 52 -> 47.  Past the other lines: B = 512 K = 20 d = 80 bf16 32 -> 55, d = 101 B = 64 K = 128 150 / 123 -> 219 / 240, d = 112
-// fp16 B = 16 K = 90 154 -> 156, B = 64 K = 12 d = 47 bf16 9.5 -> 10.3; 16-bit matrices that start off the 4-byte grid (their rows would not come
+// fp16 B = 16 K = 90 154 -> 156, B = 64 K = 12 d = 47 bf16 9.5 -> 10.3, d = 72 fp16 B = 64 K = 8 12 -> 14 (six row tiles for five), d = 56 fp32 B = 512
+// K = 4 9 -> 11, d = 128 bf16 B = 256 K = 4 11 -> 13, d = 31 B = 1024 K = 2 7 -> 10; 16-bit matrices that start off the 4-byte grid (their rows would not come
 // through LDS here), bf16 B = 16 K = 20, d = 64 19.8 -> 25.3, d = 128 42.6 -> 82.7.
 bool takes_chain(const void* mats, int B, int K, int d, int in_dtype) {
     if (d < 2 || d > 128) return false;
     const bool pieces = d % (in_dtype == LBI_F32 ? 4 : 8) == 0 && reinterpret_cast<uintptr_t>(mats) % 4 == 0;
     if (d <= 16) return pieces || (int64_t)K * d * d > 18 || B <= 16 * (int64_t)device_compute_units();
     if (!pieces && (d > 48 || (d > 32 && K < 20))) return false;
-    if (in_dtype != LBI_F32 && d > 96 && d != 128) return false;
-    return B <= (d <= 64 ? 4 : 1) * (int64_t)device_compute_units();
+    const bool half = in_dtype != LBI_F32;
+    if (half && ((d > 96 && d != 128) || (d > 64 && d <= 80 && K < 24))) return false;
+    const int64_t cus = device_compute_units();
+    if (d <= 48) return B <= (K < 4 ? 3 : 4) * cus;
+    if (d <= 64) return B <= (K >= 13 && (half || d == 64) ? 4 : 1) * cus;
+    return 4 * B <= (half && d == 128 && K < 8 ? 1 : 4) * cus;
 }
 
 int chain(const void* mats, int in_dtype, const void* g, void* cot, int B, int K, int d, hipStream_t stream) {
