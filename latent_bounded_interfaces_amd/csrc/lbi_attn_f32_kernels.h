@@ -791,14 +791,15 @@ template <int PB, typename T> double steps_of_a_cu(const Args<T>& a) {
     const int dw = waves_apart<PB, 4>(a), rows = NWAVE / dw, nd = dw * PB;
     const double steps = (a.T_len + TILE - 1) / TILE, tiles = (a.T_len + rows * TILE - 1) / (rows * TILE);
     const double cus = device_compute_units(), groups = (double)a.B * a.H * ((a.P + nd - 1) / nd);
-    if (!a.causal) return steps * ceil(groups * tiles / cus);
+    if (!a.causal || tiles == 1.0) return steps * ceil(groups * tiles / cus);
     return std::max(steps, groups * tiles * (steps + rows) / (2 * cus));
 }
 
 // Two directions per wave share S: 15 products for the two and not 18.  One makes for twice the workgroups, half as long: taken
 // where few long ones leave CUs idle.  The line lies at 3 / 2, below 5 / 3, since a wave does less well with one (us, with one and
 // with two): B=1 H=2 T=1000 Dh=64 P=8 430 and 637, B=4 H=8 T=512 P=2 226 and 329, B=2 H=8 T=1000 P=4 417 and 591, B=5 H=1 T=1761 Dh=32
-// P=8 430 and 589; B=4 H=8 T=512 Dh=64 P=8 427 and 354, B=8 H=5 T=320 P=8 248 and 215.
+// P=8 430 and 589; B=4 H=8 T=512 Dh=64 P=8 427 and 354, B=8 H=5 T=320 P=8 248 and 215.  Where a row tile is all there is, workgroups are alike, and whole
+// rounds of them count under the mask, too: B H=100 T=21 Dh=64 P=9 45 and 67, 54 T=62 P=18 79 and 118.
 template <typename T> bool two_directions(const Args<T>& a) {
     return a.P >= 2 && 1.5 * steps_of_a_cu<2>(a) <= steps_of_a_cu<1>(a);
 }
