@@ -749,8 +749,9 @@ int launch_with(const Args<T>& a) {
     if (int rc = ensure_dynamic_lds<&dkdv_kernel<T, DH, PB, DW, VEC>>(qg_bytes)) return rc;
     const int key_tiles = (a.T_len + TILE - 1) / TILE, turned = turned_of(tiles, groups);
     // the largest number of workgroups of the other statistics kernel at which this one was as fast or faster: B=8 H=8 T=512 P=1 224 -> 217 us
-    // with a mask (256), 223 -> 226 without; B=4 H=8 T=2048 Dh=128 (512) 1579 -> 1610 and 2841 -> 2924
-    if (4LL * stat_tiles * heads <= (a.causal ? 4LL : 3LL) * device_compute_units())
+    // with a mask (256), 223 -> 226 without; B=4 H=8 T=2048 Dh=128 (512) 1579 -> 1610 and 2841 -> 2924.  One tile of keys has nothing to split (B H=28 T=21
+    // Dh=128 P=15 48 -> 49)
+    if (key_tiles > 1 && 4LL * stat_tiles * heads <= (a.causal ? 4LL : 3LL) * device_compute_units())
         hipLaunchKernelGGL((stats_split_kernel<T, DH, VEC>), grid_of(key_tiles, heads), dim3(NT), 0, a.stream, a.q, a.k, a.lse2,
                            a.T_len, a.dh, a.scale, a.causal, key_tiles, turned_of(key_tiles, heads));
     else
