@@ -468,7 +468,8 @@ def _native_layer(block: Any, layer_cache: Any, g_hidden: torch.Tensor | None, g
     bsz, basis, g_len, dim = g_residual.shape
     seqlen = q.shape[2]
     rows, fc1_output = bsz * basis * seqlen, m_cache.fc1_output
-    if rows * dim * fc1_output.shape[-1] > _NATIVE_TIMES * _SMALL_PRODUCT:  # most calls that are not taken leave here
+    # most calls that are not taken leave here: the largest product is not a small one, or its sums are too long
+    if fc1_output.shape[-1] > _SMALL_PRODUCT_TERMS or rows * dim * fc1_output.shape[-1] > _NATIVE_TIMES * _SMALL_PRODUCT:
         return None
     heads, kv_heads, head_dim = attn.n_heads, attn.n_kv_heads, attn.head_dim
     conv = attn.conv1d.weight
