@@ -21,7 +21,7 @@
 // Rows come straight into registers up to 48 columns.  Beyond that each lane loading another row would be what bounds a step: sixteen
 // 64-byte pieces an instruction come at 35 GB/s per CU (d = 128 1.85 us a step, 1.06 without the loads).  They go through LDS there, by
 // 16-byte transfers into a ring of the wave's own, four lanes to 64 bytes of a row (1.23 us).
-// A step takes (fp32, B = 1, K = 128) 0.18 / 0.26 / 0.45 / 1.0 / 1.3 us at d = 16 / 32 / 64 / 96 / 128, of which 0.06 / 0.11 / 0.23 / 0.7 /
+// A step takes (fp32, B = 1, K = 256 less K = 56) 0.15 / 0.24 / 0.42 / 0.98 / 1.30 us at d = 16 / 32 / 64 / 96 / 128, of which 0.06 / 0.11 / 0.23 / 0.7 /
 // 0.9 are the fp32 products at the rate of the matrix cores.  Whole calls, old (scalar or 32 x 32 tiles) -> here, us, matrices and cotangents,
 // inputs from memory: fp32 B = 17 K = 73 d = 16 133 -> 14; B = 18 K = 101 d = 64 86 -> 47; B = 3 K = 10 d = 128 36 -> 17; B = 64 K = 45 d = 128
 // 176 -> 145.  Error against fp64 (2-norm, identity plus update), over 400 random calls: 0.54 of before (matrices), 0.68 (cotangents).
@@ -530,8 +530,9 @@ int launch_width(const void* mats, void* out, const void* g, void* cot, int B, i
     auto run = [&](auto ct) {
         constexpr int CT = decltype(ct)::value, RING = ring_steps(NT, CT, sizeof(Tin));
         // transfers into LDS move whole 4-byte words: 16-bit rows of an odd width or start come straight into registers
-        if (sizeof(Tin) == 2 && (d % 2 != 0 || reinterpret_cast<uintptr_t>(mats) % 4 != 0))
-            return launch_one<Tin, NT, CT, true, 0>(mats, out, g, cot, B, K, d, carry, plan, stream);
+        if constexpr (sizeof(Tin) == 2)
+            if (d % 2 != 0 || reinterpret_cast<uintptr_t>(mats) % 4 != 0)
+                return launch_one<Tin, NT, CT, true, 0>(mats, out, g, cot, B, K, d, carry, plan, stream);
         if (d == 16 * NT) return launch_one<Tin, NT, CT, false, RING>(mats, out, g, cot, B, K, d, carry, plan, stream);
         return launch_one<Tin, NT, CT, true, RING>(mats, out, g, cot, B, K, d, carry, plan, stream);
     };
