@@ -353,7 +353,8 @@ int lbi_causal_conv1d_weight_grad(const void* g_out, const void* x, float* grads
 
 /*
  * One Transformer block, backwards, whose products are all small (lbi_small_product): the entries above one after the other, with the
- * same results, as one call.  Tensors as there, all 16-byte aligned; 16-bit storage, filters of up to 8 taps, no biases.
+ * same results, as one call.  Tensors as there, all 16-byte aligned; 16-bit storage, the weights included (`dtype`; fp32 ones are not cast here),
+ * filters of up to 8 taps, no biases.
  *
  *   g_residual [B,P,T,D] fp32 (g_broadcast_t: [B,P,D], the same at every position): cotangent of the block's residual output; read only
  *   g_hidden   the cotangent of its hidden output in `dtype`, or NULL: g_residual rounded

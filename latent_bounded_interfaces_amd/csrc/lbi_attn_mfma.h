@@ -399,7 +399,7 @@ __global__ __launch_bounds__(256) void stats_kernel(const T* __restrict__ q, con
 }
 
 // ---------------------------------------------------------------------------------------
-// stats_split_kernel: the same with an eighth of the dependent steps.  A chain of key tiles is bound by the latency of a step (loads,
+// stats_split_kernel: the same with a quarter of the dependent steps.  A chain of key tiles is bound by the latency of a step (loads,
 // softmax, barrier), so a workgroup has 32 queries and its four waves take every fourth key tile each, on tiles of their
 // own in LDS (no barrier between tiles); their maxima, sums and outputs are brought together at the end, in the order of the
 // waves.  K and V are read four times as often as by workgroups of 128 queries: head dim 128 comes here while those leave

@@ -1285,9 +1285,9 @@ int launch_scan(const void* mats, void* out, const void* g, void* cot, int B, in
     if (d > 16 && d <= 128) {
         auto run = [&](auto width, auto wide) {
             constexpr int D = decltype(width)::value, WIDE = decltype(wide)::value;
-            // Column blocks of one batch element read the same matrices.  With few batch elements, narrow blocks give
-            // the chip enough workgroups, and the blocks of an element run side by side and share the matrices in L2.
-            // With many, they drift apart and fetch them again (measured 1.7x / 2.4x the input bytes at d = 64 / 128),
+            // Column blocks of one batch element read the same matrices.  Where whole ones would leave CUs with less than two (batches past the lines of
+            // scan_narrow::takes, below this one), blocks of 32 run side by side and share the matrices in L2.
+            // With more batch elements they drift apart and fetch them again (measured 1.7x / 2.4x the input bytes at d = 64 / 128),
             // so one workgroup then takes all columns.  (At 96 narrow blocks stay ahead.)
             const bool whole = WIDE > 32 && B >= wide_block_batch();
             if (d != D) {

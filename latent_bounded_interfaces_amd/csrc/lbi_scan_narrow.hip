@@ -27,7 +27,8 @@ int launch(const void* mats, int in_dtype, void* out, const void* g, void* cot, 
 // Compute units of the smallest partition of the part.
 constexpr int kLeastCus = 32;
 
-// us of a step on blocks of 16 `tiles` columns: of workgroups that have a CU to themselves, fp32 (K = 128, B = 1), and how much longer it takes
+// us of a step on blocks of 16 `tiles` columns: of workgroups that have a CU to themselves (fp32, fitted with the other constants, up to a tenth below
+// the 0.15 ... 1.30 that a step alone takes), and how much longer it takes
 // where `groups` workgroups share the chip: up to 48 columns several run on a CU side by side, at 64 two, beyond one (the rings), and what
 // they read then counts, too (d = 128 B = 16 K = 74, inputs from memory: 1.9).
 float step_us(int nt, int tiles, int64_t groups, int cus) {

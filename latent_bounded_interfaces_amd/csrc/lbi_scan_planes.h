@@ -56,7 +56,8 @@ namespace lbi {
 //            final suffix products at the chunk boundaries (the kernel runs it with mats = the parked totals);
 //   phase 3  every chunk c <= C-2 restarts the chain from out[b_{c+1}] through its own matrices (L - 1 steps, all
 //            chunks side by side), storing each product.
-// The cotangents, if asked for, are then the finished products applied to g (suffix_apply_kernel).
+// The cotangents, if asked for, are then the finished products applied to g (suffix_apply_kernel) above 128 columns; up to 128 the vector rides on the
+// last chunk of phase 1 and on phase 3 (scan_narrow).
 // About twice the products, a dependent depth of 2L + C - 4 instead of K - 1, no scratch memory, no atomics; the
 // summation order is fixed by (K, L), so reruns are bit-identical.
 struct ScanPlan {
