@@ -703,17 +703,62 @@ def test_native_layer_equals_its_launches(sizes, dtype, device, monkeypatch):
         assert torch.equal(got[0][name], grad) and got[0][name].dtype == grad.dtype, name
 
 
+def _widened(node):
+    """The same values in fp32, all the way down."""
+    for name, value in vars(node).items():
+        if torch.is_tensor(value) and value.is_floating_point():
+            setattr(node, name, value.float())
+        elif isinstance(value, list):
+            for one in value:
+                _widened(one)
+        elif hasattr(value, "__dict__") and not torch.is_tensor(value):
+            _widened(value)
+
+
+# products of one to three times a small product's size, which the launches one by one leave to the library
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("dim,b,t,p", [(512, 2, 65, 9), (768, 1, 258, 1), (512, 2, 512, 1)])
+def test_native_layer_of_products_past_the_small_ones(dim, b, t, p, dtype, device, monkeypatch):
+    """The two ways round differ in the order of fp32 sums: both are as far from fp32 arithmetic on the same values (a tenth of the error for
+    what rounding does by chance, a quarter in gradients of a few hundred values)."""
+    from latent_bounded_interfaces_amd.backends import HipTransformerLowering
+    from latent_bounded_interfaces_amd.hip.transformer import region
+
+    backend, cache, gen = _small_block(dtype, device, dim=dim, heads=dim // 64, kv=dim // 64, hd=64, hidden=4 * dim, layers=1, b=b, t=t)
+    work, grads = b * t * p * dim * 8 * dim / region._SMALL_PRODUCT, 8 * dim * dim / region._SMALL_PRODUCT_RESULTS  # the largest product and gradient
+    assert 1 < max(work, grads) <= region._NATIVE_TIMES
+    lowering = HipTransformerLowering()
+    basis = torch.randn(b, p, t, dim, generator=gen).to(device)
+
+    def pullback():
+        return {"input": lowering.input_pullback_basis(backend=backend, cache=cache, output_cotangent_basis=basis)}
+
+    def vjp():
+        return lowering.parameter_vjp(backend=backend, cache=cache, output_cotangent=basis[:, 0])
+
+    call = vjp if p == 1 else pullback
+    got, want, taken = _launch_by_launch(monkeypatch, call)
+    assert taken == [True] and got.keys() == want.keys()
+    backend.float()
+    _widened(cache)
+    for name, truth in call().items():
+        truth = truth.double()
+        errors = [float((one[name].double() - truth).norm() / truth.norm()) for one in (got, want)]
+        assert errors[0] <= (1.1 if truth.dim() > 1 else 1.25) * errors[1], (name, errors)
+        assert errors[0] <= (2e-3 if dtype == torch.float16 else 1.5e-2), (name, errors)
+
+
 def test_native_layer_leaves_what_it_does_not_take(device, monkeypatch):
     from latent_bounded_interfaces_amd.backends import HipTransformerLowering
 
     lowering = HipTransformerLowering()
-    for dtype, sizes, expect in ((torch.float32, dict(), False), (torch.bfloat16, dict(bias=True), None), (torch.bfloat16, dict(hd=36, dim=72), False)):
+    for dtype, sizes, expect in ((torch.float32, dict(), False), (torch.bfloat16, dict(bias=True), True), (torch.bfloat16, dict(hd=36, dim=72), False)):
         backend, cache, gen = _small_block(dtype, device, **sizes)
         b, t, dim = cache.region_input.shape
         basis = torch.randn(b, 2, t, dim, generator=gen).to(device)
         got, want, taken = _launch_by_launch(monkeypatch, lambda: lowering.input_pullback_basis(
             backend=backend, cache=cache, output_cotangent_basis=basis))
-        assert torch.equal(got, want) and (expect is None or not any(taken))   # (biases take no part in the input pullback)
+        assert torch.equal(got, want) and all(one is expect for one in taken)   # (biases take no part in the input pullback)
         got, want, taken = _launch_by_launch(monkeypatch, lambda: lowering.parameter_vjp(
             backend=backend, cache=cache, output_cotangent=basis[:, 0]))
         assert not any(taken) and all(torch.equal(got[name], grad) for name, grad in want.items())
@@ -729,6 +774,5 @@ def test_native_layer_leaves_what_it_does_not_take(device, monkeypatch):
     basis = torch.randn(b, 2, t, dim, generator=gen).to(device)
     got, want, taken = _launch_by_launch(monkeypatch, lambda: lowering.input_pullback_basis(
         backend=backend, cache=cache, output_cotangent_basis=basis))
-    assert taken == [True, False]
-    assert _max_rel(got.cpu(), want.cpu()) <= 2e-2
+    assert taken == [True, False] and torch.equal(got, want)
 

@@ -836,6 +836,14 @@ def test_narrow_scan_forms(rank, bsz, count, dtype, device):
         assert float((cot[:, r].double() - want).abs().max() / want.abs().max()) <= 1e-5
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rank,bsz", [(49, 90), (64, 90), (66, 70), (80, 70), (96, 70), (113, 60), (128, 60)])
+def test_narrow_scan_carries_the_vector_over_several_trips(rank, bsz, dtype, device):
+    """Plain chains on blocks of 32 columns with the vector beside the first block (below the twelve matrices from which on chains are cut): ten
+    steps, more than two trips through the rings.  Bounds as above."""
+    test_narrow_scan_forms(bsz, 11, rank, dtype, device)
+
+
 @pytest.mark.parametrize("rank", [16, 30, 64, 77, 128])
 @pytest.mark.parametrize("value", [float("inf"), float("nan")])
 def test_narrow_scan_keeps_other_rows_and_elements_apart(rank, value, device):
