@@ -841,7 +841,16 @@ def test_narrow_scan_forms(rank, bsz, count, dtype, device):
 def test_narrow_scan_carries_the_vector_over_several_trips(rank, bsz, dtype, device):
     """Plain chains on blocks of 32 columns with the vector beside the first block (below the twelve matrices from which on chains are cut): ten
     steps, more than two trips through the rings.  Bounds as above."""
-    test_narrow_scan_forms(bsz, 11, rank, dtype, device)
+    test_narrow_scan_forms(rank, bsz, 11, dtype, device)
+
+
+# either side of the lines between the narrow scan and the 32 x 32 tiles (256 CUs), blocks of 32 columns and whole ones there
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rank,bsz", [(24, 512), (24, 513), (41, 257), (57, 128), (57, 300), (64, 300), (64, 800), (75, 40), (75, 81), (96, 81), (105, 33), (105, 65),
+                                      (120, 40), (128, 65), (128, 513)])
+def test_batches_at_the_lines_of_the_narrow_scan(rank, bsz, dtype, device):
+    """Sums in blocks of 32 on either side: the bound above."""
+    test_narrow_scan_forms(rank, bsz, 5, dtype, device)
 
 
 @pytest.mark.parametrize("rank", [16, 30, 64, 77, 128])
