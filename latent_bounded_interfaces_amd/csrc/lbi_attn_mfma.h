@@ -518,7 +518,7 @@ __global__ __launch_bounds__(256) void stats_split_kernel(const T* __restrict__ 
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
         const float mw = row_max[w * 32 + m];
-        total += mw == -INFINITY ? row_sum[w * 32 + m] : row_sum[w * 32 + m] * __builtin_amdgcn_exp2f(mw - top);
+        total += mw == -INFINITY ? 0.0f * row_sum[w * 32 + m] : row_sum[w * 32 + m] * __builtin_amdgcn_exp2f(mw - top);
     }
     const float part = m_run == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m_run - top);
     const float inv = part / total;
