@@ -52,33 +52,40 @@ struct Chunks { int L, tiles; };
 // matrices, us, plain -> chunks: d = 16 B = 1 18 -> 12; d = 32 B = 4 31 -> 17, B = 64 32 -> 32; d = 64 B = 4 52 -> 23, B = 32 54 (59 in
 // chunks, not taken); d = 128 B = 1 156 -> 49, B = 4 154 -> 61; B = 7 K = 120, inputs from memory,
 // in chunks 122 on 16 columns, 92 on 32.
-Chunks chunks(int B, int K, int nt, int cus) {
+Chunks chunks(int B, int K, int nt, bool half, int cus) {
     const int forced = scan_forced_chunk();
     if (forced == 0 || K < 12) return {0, 1};
     if (forced > 0) {
         const int L = forced < 2 ? 2 : forced;
         return {(K + L) / L >= 4 ? L : 0, 1};
     }
-    // Beyond 64 columns a plain chain whose blocks of 16 don't find a CU each runs on 32, and chunks have never been the better form then.  (13 widths,
-    // B = 8 ... 768, K = 13 ... 100: 253 calls 1.18 times as long in chunks.)  The estimate is good to a tenth: chunks are taken for less than that only
-    // where they save 8 %.
+    // Beyond 64 columns a plain chain whose blocks of 16 don't find a CU each runs on 32, and chunks have never been the better form then (13 widths,
+    // B = 8 ... 768, K = 13 ... 100: 253 calls 1.18 times as long in chunks).
     if (nt > 4 && dealt(B) * nt > cus) return {0, 1};
-    float best = 0.92f * (5.0f + (float)(K - 1) * step_us(nt, 1, dealt(B) * nt, cus));
+    const float plain = 5.0f + (float)(K - 1) * step_us(nt, 1, dealt(B) * nt, cus);
+    float best = plain;
+    int64_t groups = 0;
     Chunks form{0, 1};
     for (int L = 2; (K + L) / L >= 4; L += 1 + L / 16) {
         const int C = (K + L) / L;
         const int64_t chains = dealt((int64_t)B * (C - 1));
         const float between = 12.0f + (float)(C - 2) * step_us(nt, 1, dealt(B) * nt, cus);
         for (int tiles = 1; tiles <= (nt > 3 ? 2 : 1); ++tiles) {
-            const float step = step_us(nt, tiles, chains * (tiles == 2 ? (nt + 1) / 2 : nt + 1), cus);
-            const float cost = between + (float)(2 * L - 2) * step;
+            const int64_t blocks = chains * (tiles == 2 ? (nt + 1) / 2 : nt + 1);
+            const float cost = between + (float)(2 * L - 2) * step_us(nt, tiles, blocks, cus);
             if (cost < best) {
                 best = cost;
+                groups = blocks;
                 form = {L, tiles};
             }
         }
     }
-    return form;
+    // The estimate is good to a tenth, and what it misses where chunks fill the CUs is the same for calls alike (measured / estimated part of the plain chain): 7 and 8
+    // row tiles 1.17 / 0.91 (bf16 d = 128 B = 16 K = 24), 0.90 / 0.90 (B = 8 K = 24); 5 and 6 1.13 / 0.99 (bf16 d = 80 B = 24 K = 50), 0.80 / 0.93 (B = 8 K =
+    // 24); fp32 at 4 1.19 / 0.97 (d = 64 B = 32 K = 100); at 3, ten workgroups a CU, 1.29 / 0.94 (d = 33 B = 40 K = 100).
+    const bool crowd = !half && nt == 3 && groups >= 8 * (int64_t)cus;
+    const float full = nt > 7 ? 0.905f : nt > 6 ? 0.93f : nt > 4 ? 0.97f : crowd ? 0.85f : nt == 4 && !half ? 0.95f : 1.0f;
+    return best < (5 * groups >= 4 * (int64_t)cus ? full : 1.0f) * plain ? form : Chunks{0, 1};
 }
 
 // 16-bit rows that are no whole 4-byte words come straight into registers at all widths.
@@ -95,7 +102,7 @@ static bool in_words(const void* mats, int d, int in_dtype) {
 //    workgroup of 32 columns a CU twice over: fp32 d = 49 B = 256 K = 24 46 -> 35 / 57 -> 46, B = 288 47 -> 52 / 57 -> 66.
 //  * beyond 64 columns while a step's blocks of 32 find a CU each: fp32 d = 81 B = 80 K = 24 56 -> 57 / 70 -> 63, B = 96 58 -> 71 / 72 -> 83; d = 128 B = 64
 //    K = 100 319 -> 293 / 350 -> 315, B = 72 323 -> 353 / 352 -> 381; three quarters of them for 16-bit rows of 97 ... 127.  Odd 16-bit widths, whose
-//    rows come straight into registers, take them in chains of a dozen matrices and more: bf16 d = 65 B = 64 K = 8 20 -> 24 / 28 -> 27.
+//    rows come straight into registers, take them in chains of eight matrices and more: bf16 d = 81 B = 64 K = 4 11 -> 15 / 19 -> 15, K = 8 20 -> 22 / 28 -> 24.
 bool takes(const void* mats, int B, int K, int d, int in_dtype) {
     if (d < 2 || d > 128) return false;
     if (d <= 16 || scan_forced_chunk() > 0) return true;   // the others take whole chains of more than 16 columns
@@ -106,7 +113,7 @@ bool takes(const void* mats, int B, int K, int d, int in_dtype) {
     if (nt <= 2) return B <= (whole || K >= 24 ? 4 : 2) * cus;
     if (nt == 3 || (nt == 4 && half && words)) return B <= (K < (whole ? 4 : 8) ? 1 : 3) * cus;
     if (nt == 4) return 2 * B <= (whole || K >= 8 ? 2 : 1) * cus;
-    if (!words && K < 12) return dealt(B) * nt <= cus;
+    if (!words && K < 8) return dealt(B) * nt <= cus;
     return 4 * dealt(B) * ((nt + 1) / 2) <= (half && nt == 8 && !whole ? 3 : 4) * cus;
 }
 
@@ -142,7 +149,7 @@ int scan(const void* mats, int in_dtype, void* out, const void* g, void* cot, in
     const int nt = row_tiles(d, in_dtype);
     if (K < 12 && dealt(B) * (nt + 1) <= kLeastCus) return launch(mats, in_dtype, out, g, cot, B, K, d, 1, false, plan, stream);
     const int cus = device_compute_units();
-    if (const Chunks form = chunks(B, K, nt, cus); form.L) {
+    if (const Chunks form = chunks(B, K, nt, in_dtype != LBI_F32, cus); form.L) {
         plan.L = form.L;
         plan.C = (K + form.L) / form.L;
         plan.s = 1;
